@@ -293,16 +293,11 @@ extern "C" int pb_coord_counts(pb_sys *s, float rmax2t, uint32_t *counts) {
   hipLaunchKernelGGL(k_coord_counts, dim3(pb_blocks(s->n, 256)), dim3(256), 0, st, s->r, s->perm,
                      s->cellid, s->cstart, s->n, ref_grid(s), c[0], c[1], c[2], rmax2t,
                      s->ref_periodic, dcnt);
-  hipError_t e = hipGetLastError();
-  std::vector<uint32_t> h(s->npad), o(s->npad);
-  if (e == hipSuccess) e = hipMemcpyAsync(h.data(), dcnt, 4 * (size_t)s->npad, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipMemcpyAsync(o.data(), s->orig, 4 * (size_t)s->npad, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
+  int e = PB_OK;
+  if (hipError_t he = hipGetLastError()) e = pb_hip_check(s->ctx, he, "pb_coord_counts");
+  if (e == PB_OK) e = pb_io_gather_u32(s, dcnt, counts);
   pb_free(dcnt);
-  if (e != hipSuccess) return pb_hip_check(s->ctx, e, "pb_coord_counts");
-  for (uint32_t k = 0; k < s->npad; ++k)
-    if (o[k] != PB_NONE) counts[o[k]] = h[k];
-  return PB_OK;
+  return e;
 }
 
 // ------------------------------------------------------------------ g(r)

@@ -1,4 +1,4 @@
-// pb_core.hip -- context, particle storage, import/export, integrators,
+// pb_core.hip -- context, particle storage, integrators,
 // boundaries and FP64 reductions of the MI355X particle engine.
 //
 // Reference counterparts: cudaFrame (cudaFrame.cu), cudaParticleBase
@@ -66,6 +66,7 @@ extern "C" int pb_ctx_destroy(pb_ctx *ctx) {
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) {
     (void)hipStreamSynchronize(ctx->stream);
+    pb_io_release(ctx);
     (void)hipStreamDestroy(ctx->stream);
   }
   delete ctx;
@@ -192,7 +193,7 @@ extern "C" void pb_sys_destroy(pb_sys *s) {
   pb_free(s->w); pb_free(s->Lm); pb_free(s->T); pb_free(s->radius);
   pb_free(s->move); pb_free(s->type); pb_free(s->orig); pb_free(s->waveRep);
   pb_free(s->d_reps); pb_free(s->partials); pb_free(s->d_counter); pb_free(s->d_out);
-  pb_free(s->d_hash); pb_free(s->lj_queue);
+  pb_free(s->d_hash); pb_free(s->lj_queue); pb_free(s->io);
   pb_free(s->gt); pb_free(s->gt_bad);
   pb_free(s->md_row); pb_free(s->md_col); pb_free(s->md_inv);
   pb_free(s->ref_table); pb_free(s->ref_bid); pb_free(s->ref_pid); pb_free(s->ref_bindex);
@@ -241,74 +242,6 @@ extern "C" int pb_sys_set_cell(pb_sys *s, const double *cells) {
   return upload_reps(s);
 }
 
-// host-side packing: original order <-> storage order
-std::vector<uint32_t> pb_download_orig(pb_sys *s, int *rc) {
-  std::vector<uint32_t> o(s->npad);
-  *rc = PB_OK;
-  if (hipMemcpyAsync(o.data(), s->orig, 4 * (size_t)s->npad, hipMemcpyDeviceToHost,
-                     s->ctx->stream) != hipSuccess ||
-      hipStreamSynchronize(s->ctx->stream) != hipSuccess)
-    *rc = pb_fail(s->ctx, PB_ERR_HIP, "download orig");
-  return o;
-}
-
-extern "C" int pb_sys_import(pb_sys *s, const double *r, const double *v, const double *a,
-                             const double *m, const uint32_t *type, const uint8_t *is_fixed) {
-  if (!s || !r || !m) return pb_fail(s ? s->ctx : nullptr, PB_ERR_ARG, "pb_sys_import: r and m required");
-  PB_HIP(s->ctx, hipSetDevice(s->ctx->device));
-  int rc = PB_OK;
-  std::vector<uint32_t> o = pb_download_orig(s, &rc);
-  if (rc) return rc;
-  const size_t np = s->npad;
-  std::vector<double4> hr(np), hv(np), ha(np);
-  std::vector<uint16_t> ht(np);
-  std::vector<uint8_t> hm(np);
-  for (size_t k = 0; k < np; ++k) {
-    const uint32_t g = o[k];
-    if (g == PB_NONE) {
-      hr[k] = make_double4(0, 0, 0, (double)PB_PAD_TYPE);
-      hv[k] = make_double4(0, 0, 0, 0);
-      ha[k] = make_double4(0, 0, 0, 0);
-      ht[k] = (uint16_t)PB_PAD_TYPE;
-      hm[k] = 0;
-      continue;
-    }
-    if (type && type[g] >= PB_MAXT) return pb_fail(s->ctx, PB_ERR_ARG, "pb_sys_import: type >= 5");
-    if (!(m[g] > 0)) return pb_fail(s->ctx, PB_ERR_ARG, "pb_sys_import: mass must be > 0");
-    const double t = type ? (double)type[g] : 0.0;
-    hr[k] = make_double4(r[3 * g], r[3 * g + 1], r[3 * g + 2], t);
-    hv[k] = v ? make_double4(v[3 * g], v[3 * g + 1], v[3 * g + 2], 1.0 / m[g])
-              : make_double4(0, 0, 0, 1.0 / m[g]);
-    ha[k] = a ? make_double4(a[3 * g], a[3 * g + 1], a[3 * g + 2], 0) : make_double4(0, 0, 0, 0);
-    ht[k] = type ? (uint16_t)type[g] : 0;
-    hm[k] = is_fixed ? (is_fixed[g] ? 0 : 1) : 1;
-  }
-  hipStream_t st = s->ctx->stream;
-  PB_HIP(s->ctx, hipMemcpyAsync(s->r, hr.data(), sizeof(double4) * np, hipMemcpyHostToDevice, st));
-  PB_HIP(s->ctx, hipMemcpyAsync(s->v, hv.data(), sizeof(double4) * np, hipMemcpyHostToDevice, st));
-  PB_HIP(s->ctx, hipMemcpyAsync(s->a, ha.data(), sizeof(double4) * np, hipMemcpyHostToDevice, st));
-  PB_HIP(s->ctx, hipMemcpyAsync(s->type, ht.data(), 2 * np, hipMemcpyHostToDevice, st));
-  PB_HIP(s->ctx, hipMemcpyAsync(s->move, hm.data(), np, hipMemcpyHostToDevice, st));
-  PB_HIP(s->ctx, hipMemsetAsync(s->F, 0, sizeof(double4) * np, st));
-  PB_HIP(s->ctx, hipStreamSynchronize(st));
-  s->ref_binned = false;
-  return PB_OK;
-}
-
-static double4 *vec_field(pb_sys *s, int field) {
-  switch (field) {
-    case PB_FIELD_R: return s->r;
-    case PB_FIELD_V: return s->v;
-    case PB_FIELD_A: return s->a;
-    case PB_FIELD_F: return s->F;
-    case PB_FIELD_W: return s->w;
-    case PB_FIELD_L: return s->Lm;
-    case PB_FIELD_T: return s->T;
-    case PB_FIELD_SPH_NUM: return s->sph_num;
-    default: return nullptr;
-  }
-}
-
 int pb_ensure_rotation(pb_sys *s) {
   if (s->w) return PB_OK;
   int rc;
@@ -327,161 +260,6 @@ int pb_ensure_radius(pb_sys *s) {
   if (rc) return rc;
   PB_HIP(s->ctx, hipMemsetAsync(s->radius, 0, sizeof(double) * s->npad, s->ctx->stream));
   return PB_OK;
-}
-
-extern "C" int pb_sys_get(pb_sys *s, int field, void *host) {
-  if (!s || !host) return PB_ERR_ARG;
-  PB_HIP(s->ctx, hipSetDevice(s->ctx->device));
-  int rc = PB_OK;
-  std::vector<uint32_t> o = pb_download_orig(s, &rc);
-  if (rc) return rc;
-  const size_t np = s->npad;
-  hipStream_t st = s->ctx->stream;
-  if (double4 *src = vec_field(s, field)) {
-    std::vector<double4> h(np);
-    PB_HIP(s->ctx, hipMemcpyAsync(h.data(), src, sizeof(double4) * np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    double *out = (double *)host;
-    for (size_t k = 0; k < np; ++k)
-      if (o[k] != PB_NONE) {
-        out[3 * (size_t)o[k]] = h[k].x;
-        out[3 * (size_t)o[k] + 1] = h[k].y;
-        out[3 * (size_t)o[k] + 2] = h[k].z;
-      }
-    return PB_OK;
-  }
-  if (field == PB_FIELD_W || field == PB_FIELD_L || field == PB_FIELD_T)
-    return pb_fail(s->ctx, PB_ERR_STATE, "pb_sys_get: rotation state not allocated");
-  if (field == PB_FIELD_SPH_NUM || field == PB_FIELD_SPH_RHOINV) {
-    if (!s->sph_num) return pb_fail(s->ctx, PB_ERR_STATE, "pb_sys_get: no SPH density yet");
-    if (field == PB_FIELD_SPH_RHOINV) {
-      std::vector<double> h(np);
-      PB_HIP(s->ctx, hipMemcpyAsync(h.data(), s->sph_rhoinv, 8 * np, hipMemcpyDeviceToHost, st));
-      PB_HIP(s->ctx, hipStreamSynchronize(st));
-      double *out = (double *)host;
-      for (size_t k = 0; k < np; ++k)
-        if (o[k] != PB_NONE) out[o[k]] = h[k];
-      return PB_OK;
-    }
-  }
-  if (field == PB_FIELD_MINV) {
-    std::vector<double4> h(np);
-    PB_HIP(s->ctx, hipMemcpyAsync(h.data(), s->v, sizeof(double4) * np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    double *out = (double *)host;
-    for (size_t k = 0; k < np; ++k)
-      if (o[k] != PB_NONE) out[o[k]] = h[k].w;
-    return PB_OK;
-  }
-  if (field == PB_FIELD_TYPE) {
-    std::vector<uint16_t> h(np);
-    PB_HIP(s->ctx, hipMemcpyAsync(h.data(), s->type, 2 * np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    uint16_t *out = (uint16_t *)host;
-    for (size_t k = 0; k < np; ++k)
-      if (o[k] != PB_NONE) out[o[k]] = h[k];
-    return PB_OK;
-  }
-  if (field == PB_FIELD_MOVE) {
-    std::vector<uint8_t> h(np);
-    PB_HIP(s->ctx, hipMemcpyAsync(h.data(), s->move, np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    uint8_t *out = (uint8_t *)host;
-    for (size_t k = 0; k < np; ++k)
-      if (o[k] != PB_NONE) out[o[k]] = h[k];
-    return PB_OK;
-  }
-  if (field == PB_FIELD_RADIUS) {
-    if (!s->radius) return pb_fail(s->ctx, PB_ERR_STATE, "pb_sys_get: radius not set");
-    std::vector<double> h(np);
-    PB_HIP(s->ctx, hipMemcpyAsync(h.data(), s->radius, 8 * np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    double *out = (double *)host;
-    for (size_t k = 0; k < np; ++k)
-      if (o[k] != PB_NONE) out[o[k]] = h[k];
-    return PB_OK;
-  }
-  return pb_fail(s->ctx, PB_ERR_ARG, "pb_sys_get: unknown field");
-}
-
-extern "C" int pb_sys_set(pb_sys *s, int field, const void *host) {
-  if (!s || !host) return PB_ERR_ARG;
-  PB_HIP(s->ctx, hipSetDevice(s->ctx->device));
-  int rc = PB_OK;
-  if ((field == PB_FIELD_W || field == PB_FIELD_L || field == PB_FIELD_T) && (rc = pb_ensure_rotation(s)))
-    return rc;
-  if (field == PB_FIELD_RADIUS && (rc = pb_ensure_radius(s))) return rc;
-  if (field == PB_FIELD_SPH_NUM && !s->sph_num)
-    return pb_fail(s->ctx, PB_ERR_STATE, "pb_sys_set: no SPH density yet");
-  std::vector<uint32_t> o = pb_download_orig(s, &rc);
-  if (rc) return rc;
-  const size_t np = s->npad;
-  hipStream_t st = s->ctx->stream;
-  if (double4 *dst = vec_field(s, field)) {
-    std::vector<double4> h(np);
-    PB_HIP(s->ctx, hipMemcpyAsync(h.data(), dst, sizeof(double4) * np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    const double *in = (const double *)host;
-    for (size_t k = 0; k < np; ++k)
-      if (o[k] != PB_NONE) {
-        h[k].x = in[3 * (size_t)o[k]];
-        h[k].y = in[3 * (size_t)o[k] + 1];
-        h[k].z = in[3 * (size_t)o[k] + 2];
-      }
-    PB_HIP(s->ctx, hipMemcpyAsync(dst, h.data(), sizeof(double4) * np, hipMemcpyHostToDevice, st));
-    if (field == PB_FIELD_SPH_NUM && s->sph_rhoinv) {
-      // 1/rho follows the imported rho (calcDensityPost's reciprocal,
-      // cudaParticleSPH_NS.cu:190-195), so an acceleration after a density
-      // import uses the imported densities throughout
-      std::vector<double> hr(np, 0.0);
-      for (size_t k = 0; k < np; ++k)
-        if (o[k] != PB_NONE) hr[k] = 1.0 / in[3 * (size_t)o[k] + 1];
-      PB_HIP(s->ctx, hipMemcpyAsync(s->sph_rhoinv, hr.data(), 8 * np, hipMemcpyHostToDevice, st));
-    }
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    return PB_OK;
-  }
-  if (field == PB_FIELD_MINV || field == PB_FIELD_TYPE) {
-    std::vector<double4> hr(np), hv(np);
-    std::vector<uint16_t> ht(np);
-    PB_HIP(s->ctx, hipMemcpyAsync(hv.data(), s->v, sizeof(double4) * np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipMemcpyAsync(hr.data(), s->r, sizeof(double4) * np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipMemcpyAsync(ht.data(), s->type, 2 * np, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    for (size_t k = 0; k < np; ++k)
-      if (o[k] != PB_NONE) {
-        if (field == PB_FIELD_MINV) {
-          hv[k].w = ((const double *)host)[o[k]];
-        } else {
-          const uint16_t t = ((const uint16_t *)host)[o[k]];
-          if (t >= PB_MAXT) return pb_fail(s->ctx, PB_ERR_ARG, "pb_sys_set: type >= 5");
-          ht[k] = t;
-          hr[k].w = (double)t;
-        }
-      }
-    PB_HIP(s->ctx, hipMemcpyAsync(s->v, hv.data(), sizeof(double4) * np, hipMemcpyHostToDevice, st));
-    PB_HIP(s->ctx, hipMemcpyAsync(s->r, hr.data(), sizeof(double4) * np, hipMemcpyHostToDevice, st));
-    PB_HIP(s->ctx, hipMemcpyAsync(s->type, ht.data(), 2 * np, hipMemcpyHostToDevice, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    return PB_OK;
-  }
-  if (field == PB_FIELD_MOVE || field == PB_FIELD_RADIUS) {
-    const bool isr = field == PB_FIELD_RADIUS;
-    std::vector<uint8_t> hm(np, 0);
-    std::vector<double> hrad(np, 0.0);
-    for (size_t k = 0; k < np; ++k)
-      if (o[k] != PB_NONE) {
-        if (isr) hrad[k] = ((const double *)host)[o[k]];
-        else hm[k] = ((const uint8_t *)host)[o[k]];
-      }
-    if (isr)
-      PB_HIP(s->ctx, hipMemcpyAsync(s->radius, hrad.data(), 8 * np, hipMemcpyHostToDevice, st));
-    else
-      PB_HIP(s->ctx, hipMemcpyAsync(s->move, hm.data(), np, hipMemcpyHostToDevice, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
-    return PB_OK;
-  }
-  return pb_fail(s->ctx, PB_ERR_ARG, "pb_sys_set: unknown field");
 }
 
 // ======================================================= element-wise kernels

@@ -357,20 +357,23 @@ __global__ void k_set_inertia(const double4 *v, const double *r0, uint32_t n, do
 }
 
 // ------------------------------------------------------------------ host
+// a radius per particle (r0, or r0_all for every one) in storage order
+static int scatter_radius(pb_sys *s, const double *r0, double r0_all, double *dst,
+                          const char *msg) {
+  std::vector<double> all;
+  if (!r0) {
+    all.assign(s->n, r0_all);
+    r0 = all.data();
+  }
+  for (size_t g = 0; g < s->n; ++g)
+    if (!(r0[g] > 0)) return pb_fail(s->ctx, PB_ERR_ARG, msg);
+  return pb_io_scatter(s, r0, dst, false);
+}
+
 static int upload_radius(pb_sys *s, const double *r0, double r0_all) {
   int rc = pb_ensure_radius(s);
   if (rc) return rc;
-  std::vector<uint32_t> o = pb_download_orig(s, &rc);
-  if (rc) return rc;
-  std::vector<double> h(s->npad, 0.0);
-  for (size_t k = 0; k < s->npad; ++k)
-    if (o[k] != PB_NONE) {
-      const double x = r0 ? r0[o[k]] : r0_all;
-      if (!(x > 0)) return pb_fail(s->ctx, PB_ERR_ARG, "DEM: radius must be > 0");
-      h[k] = x;
-    }
-  PB_HIP(s->ctx, hipMemcpyAsync(s->radius, h.data(), 8 * (size_t)s->npad, hipMemcpyHostToDevice,
-                                s->ctx->stream));
+  if ((rc = scatter_radius(s, r0, r0_all, s->radius, "DEM: radius must be > 0"))) return rc;
   PB_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
   return PB_OK;
 }
@@ -438,30 +441,21 @@ extern "C" int pb_rot_set_inertia(pb_sys *s, const double *r0, double r0_all) {
   PB_HIP(s->ctx, hipSetDevice(s->ctx->device));
   int rc = pb_ensure_rotation(s);
   if (rc) return rc;
-  // the inertia radius may differ from the contact radius: stage it in a
+  // the inertia radius may differ from the contact radius: it is staged in a
   // temporary device array in storage order
-  std::vector<uint32_t> o = pb_download_orig(s, &rc);
-  if (rc) return rc;
-  std::vector<double> h(s->npad, 0.0);
-  for (size_t k = 0; k < s->npad; ++k)
-    if (o[k] != PB_NONE) {
-      const double x = r0 ? r0[o[k]] : r0_all;
-      if (!(x > 0)) return pb_fail(s->ctx, PB_ERR_ARG, "setInertia: radius must be > 0");
-      h[k] = x;
-    }
   double *d = nullptr;
   if ((rc = pb_alloc(s->ctx, &d, s->npad))) return rc;
-  if (!s->m0inv && (rc = pb_alloc(s->ctx, &s->m0inv, s->npad))) {
+  hipStream_t st = s->ctx->stream;
+  rc = scatter_radius(s, r0, r0_all, d, "setInertia: radius must be > 0");
+  if (!rc && !s->m0inv) rc = pb_alloc(s->ctx, &s->m0inv, s->npad);
+  if (rc) {
+    (void)hipStreamSynchronize(st);
     pb_free(d);
     return rc;
   }
-  hipStream_t st = s->ctx->stream;
-  hipError_t e = hipMemcpyAsync(d, h.data(), 8 * (size_t)s->npad, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_set_inertia, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->v, d,
-                       s->npad, s->m0inv);
-    e = hipGetLastError();
-  }
+  hipLaunchKernelGGL(k_set_inertia, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->v, d,
+                     s->npad, s->m0inv);
+  hipError_t e = hipGetLastError();
   if (e == hipSuccess) e = hipMemsetAsync(s->w, 0, sizeof(double4) * s->npad, st);
   if (e == hipSuccess) e = hipMemsetAsync(s->Lm, 0, sizeof(double4) * s->npad, st);
   if (e == hipSuccess) e = hipStreamSynchronize(st);

@@ -46,6 +46,11 @@ struct LJTable {
 struct pb_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
+  // pinned staging ring of the host boundary (pb_io.hip; 2 MiB, allocated on
+  // first use, released with the context), its device address and an event
+  // per slot
+  uint8_t *io_stage = nullptr, *io_dev = nullptr;
+  hipEvent_t io_ev[2] = {};
   // device address of pb_bin.hip's static g(r) scratch array on this
   // context's device (pb_gr_hist_noalloc); set when the context is created
   void *gr_scratch = nullptr;
@@ -84,6 +89,7 @@ struct pb_sys {
   double *partials = nullptr;     // per-wave partial sums, 4 per wave
   uint32_t *d_counter = nullptr;  // last-block counters / flags (16 words)
   double *d_out = nullptr;        // small reduction outputs (16 per replica)
+  uint8_t *io = nullptr;          // a packed field in the caller's order (24 B a particle, lazy)
 
   // reference cell grid (pb_setup_cells), single replica
   bool ref_cells = false;
@@ -242,8 +248,14 @@ int pb_counting_sort(pb_sys *sys, uint32_t ncell, const uint32_t *key);
 int pb_counting_sort_counted(pb_sys *sys, uint32_t ncell, const uint32_t *key);
 // per-replica reduction of K per-wave partial components into out[rep*8+c]
 int pb_reduce_waves(pb_sys *sys, int K);
-// storage slot -> original index (PB_NONE for padding), downloaded
-std::vector<uint32_t> pb_download_orig(pb_sys *sys, int *rc);
+// host boundary (pb_io.hip): the packed-field device buffer, an upload into
+// it, a scalar per particle from the caller's order into storage order
+// (squared if asked; padding 0) and a uint32 per slot to the caller's order
+int pb_io_buffer(pb_sys *sys);
+int pb_io_upload(pb_sys *sys, const void *host, size_t bytes, size_t off);
+int pb_io_scatter(pb_sys *sys, const double *host, double *dst, bool square);
+int pb_io_gather_u32(pb_sys *sys, const uint32_t *src, uint32_t *host);
+void pb_io_release(pb_ctx *ctx);
 // rotation / radius state, allocated on first use
 int pb_ensure_rotation(pb_sys *sys);
 int pb_gr_scratch_init(pb_ctx *ctx);          // pb_bin.hip: device address of the g(r) scratch

@@ -24,7 +24,6 @@
 // pb_sph_set_wcsph, with the same gathered views, cell grid and launches.
 #include "pb_internal.h"
 #include <cmath>
-#include <vector>
 
 struct SphGrid {
   uint32_t nb[3];
@@ -471,24 +470,16 @@ extern "C" int pb_sph_set_properties(pb_sys *s, const double *mu0, const double 
   if (s->nrep != 1) return pb_fail(s->ctx, PB_ERR_ARG, "SPH: single replica only");
   PB_HIP(s->ctx, hipSetDevice(s->ctx->device));
   int rc = PB_OK;
-  std::vector<uint32_t> o = pb_download_orig(s, &rc);
-  if (rc) return rc;
   const size_t np = s->npad;
-  std::vector<double> hm(np, 0.0), hc(np, 0.0);
-  for (size_t k = 0; k < np; ++k)
-    if (o[k] != PB_NONE) {
-      hm[k] = mu0[o[k]];
-      hc[k] = c[o[k]] * c[o[k]];                    // c^2, cudaParticleSPH_NS.cu:63-64
-    }
   if (!s->sph_mu0) {
     if ((rc = pb_alloc(s->ctx, &s->sph_mu0, np)) || (rc = pb_alloc(s->ctx, &s->sph_c2, np)))
       return rc;
   }
   if ((rc = sph_alloc_views(s))) return rc;
-  hipStream_t st = s->ctx->stream;
-  PB_HIP(s->ctx, hipMemcpyAsync(s->sph_mu0, hm.data(), 8 * np, hipMemcpyHostToDevice, st));
-  PB_HIP(s->ctx, hipMemcpyAsync(s->sph_c2, hc.data(), 8 * np, hipMemcpyHostToDevice, st));
-  PB_HIP(s->ctx, hipStreamSynchronize(st));
+  if ((rc = pb_io_scatter(s, mu0, s->sph_mu0, false)) ||
+      (rc = pb_io_scatter(s, c, s->sph_c2, true)))              // c^2, cudaParticleSPH_NS.cu:63-64
+    return rc;
+  PB_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
   s->sph_h = h;
   s->sph_rho0 = 1.0;
   s->sph_kind = 0;
