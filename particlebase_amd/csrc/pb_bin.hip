@@ -6,6 +6,7 @@
 #include "pb_internal.h"
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 int pb_ensure_sort_ws(pb_sys *s, uint32_t ncell);
 int pb_counting_sort(pb_sys *s, uint32_t ncell, const uint32_t *key);
@@ -304,163 +305,213 @@ extern "C" int pb_coord_counts(pb_sys *s, float rmax2t, uint32_t *counts) {
 // All unordered pairs of every replica (the pair set of
 // calcF_IJpairWithBlock5_F4 over makePairInfo's tiles, kerneltemplate.hh:
 // 423-512, cudaCalcGR.cu:30-84), binned by calcGR_F4 (kernelinline.hh:
-// 440-448).  Work = triangular tile pairs of every replica, found by a
-// binary search over the per-replica tile-pair prefix.  Each workgroup bins
-// into an LDS histogram and flushes it with 64-bit atomics: integer sums, so
-// the result is independent of the order.  Bin 0 (the pairs the reference
-// drops: r < dr/2 and r beyond the last bin, about half of all pairs in a
-// periodic box) is counted in registers and added once per tile pair, so
-// it is not a serialising LDS atomic hot spot.
+// 440-448).  A work item is a slice (1/1 to 1/8) of the j particles of one of
+// the triangular pairs of 256-particle tiles; a workgroup takes consecutive
+// items, so it stays with a replica and flushes its LDS histogram seldom.
+// Integer sums: the result is independent of the order.
+//
+// Bound by VALU issue.  The reference's rounding (per axis
+// d2 + 4 (c - sqrt(c d2)) with correctly rounded roots, then sqrt and a
+// double-precision bin) takes 102 instructions a pair; but the bin is decided
+// by far less unless the distance lies next to a bin boundary.  So a lane
+// computes r from the folded axes min(|d|, ||d| - L|) and the hardware rsqrt
+// (26 instructions), with a bound on how far its bin coordinate t can be from
+// the reference's, and counts the pair when no boundary (an integer t) lies
+// within the bound.  The others -- about 1 % at 200 bins -- go to a queue in
+// LDS that the wavefront works off 64 at a time with the reference's exact
+// arithmetic.  The bound, with u = 2^-24 and c the squared half edges:
+//   the reference's sum is within (34 + 5) u (cx + cy + cz) of the exact fold
+//   of the same d (the root's 20 u c, c - root, d2 and sum roundings, for
+//   |d| <= 1.25 L), this one within (8 + 8 + 3) u (cx + cy + cz) (the rounding
+//   of L and |d| - L, the other side of the fold test, the sum), together
+//   below E = 64 u (cx + cy + cz) (largest difference seen in 6e7 random
+//   pairs: 0.23 E).  So t differs by at most K / (t - 0.5), K = rstepinv^2 E,
+//   plus k0 = 2^-20 (rnum + 2) for the relative errors of rsqrt and products.
+// Particles further than L / 8 outside the box (or not finite) and bins finer
+// than the bound void it: those tile pairs take the exact arithmetic.
+// 256 replicas, 7.17e9 pairs, 200 bins: 13.4 ms before, 4.1 ms now.  (The
+// fold by 32-bit box fractions, one subtraction and one conversion an axis,
+// took 5.5 ms: conversions issue slowly.  Copies of the histogram against
+// atomics on one LDS address changed nothing.)
 #define GR_T 256
+#define GR_MAX_SLICES 8u
 // A tile pair adds at most GR_T * GR_T = 2^16 pairs to one bin of the
-// workgroup's uint32 LDS histogram; flushing at least every 2^15 tile pairs
-// keeps every bin below 2^31, whatever the replica's size.
-#define GR_FLUSH_TILES 32768u
+// workgroup's uint32 LDS histogram; flushing at least every 2^14 work items
+// keeps every bin and the pair count below 2^31, whatever the replica's size.
+#define GR_FLUSH_ITEMS 16384u
 struct GrRep {
   uint32_t atom0, natoms, ntile;
   uint64_t pair0;      // first tile-pair index of this replica
   float cx, cy, cz, rstepinv;
+  float lo[3], hi[3];  // FP32 box
 };
 
+// the reference's bin of a pair (0: dropped), calcGR_F4
+__device__ __forceinline__ uint32_t gr_bin(const float4 &pi, const float4 &pj, const GrRep &R,
+                                           uint32_t rnum) {
+  const float R2 = distance2p(pi.x, pi.y, pi.z, pj.x, pj.y, pj.z, R.cx, R.cy, R.cz);
+  const float r0 = sqrtf(R2) * R.rstepinv;
+  const double tt = (double)r0 + 0.5;
+  return (tt < (double)rnum) ? (uint32_t)tt : 0u;
+}
+
+// Bin 0 (the pairs the reference drops: r < dr/2 and r beyond the last bin,
+// about half of all pairs in a periodic box) is what is left of the items'
+// pairs when a histogram is flushed.
 __global__ void __launch_bounds__(GR_T) k_gr(const double4 *r, const GrRep *reps, uint32_t nrep,
-                                             uint64_t npairs, uint32_t rnum, uint64_t *hist) {
+                                             uint64_t nitem, uint32_t slices, uint32_t rnum,
+                                             uint64_t *hist) {
   extern __shared__ uint32_t h[];
-  __shared__ float4 tj[GR_T];
-  for (uint32_t b = threadIdx.x; b < rnum; b += GR_T) h[b] = 0;
-  uint32_t since = 0;                  // tile pairs in the LDS histogram since its last flush
-  for (uint64_t p = blockIdx.x; p < npairs; p += gridDim.x) {
-    uint32_t lo = 0, hi = nrep;
-    while (hi - lo > 1) {
-      const uint32_t mid = (lo + hi) / 2;
-      if (reps[mid].pair0 <= p) lo = mid;
-      else hi = mid;
-    }
-    const GrRep R = reps[lo];
-    // triangular index -> (ti <= tj)
-    uint64_t t = p - R.pair0;
-    uint32_t ti = 0;
-    uint32_t row = R.ntile;
-    while (t >= row) {
-      t -= row;
-      ++ti;
-      --row;
-    }
-    const uint32_t tjx = ti + (uint32_t)t;
-    uint32_t zero = 0;                 // this thread's bin-0 pairs of the tile pair
-    __syncthreads();
-    const uint32_t j = tjx * GR_T + threadIdx.x;
-    if (j < R.natoms) {
-      const double4 q = r[R.atom0 + j];
-      tj[threadIdx.x] = make_float4((float)q.x, (float)q.y, (float)q.z, 0.f);
-    }
-    __syncthreads();
-    const uint32_t i = ti * GR_T + threadIdx.x;
-    if (i < R.natoms) {
-      const double4 q = r[R.atom0 + i];
-      const float xi = (float)q.x, yi = (float)q.y, zi = (float)q.z;
-      const uint32_t jn = min(GR_T, R.natoms - tjx * GR_T);
-      const uint32_t jb = (ti == tjx) ? threadIdx.x + 1 : 0;
-      for (uint32_t jj = jb; jj < jn; ++jj) {
-        const float4 pj = tj[jj];
-        const float R2 = distance2p(xi, yi, zi, pj.x, pj.y, pj.z, R.cx, R.cy, R.cz);
-        const float r0 = sqrtf(R2) * R.rstepinv;
-        const double tt = (double)r0 + 0.5;
-        const uint32_t bin = (tt < (double)rnum) ? (uint32_t)tt : 0u;
-        if (bin == 0u) ++zero;
-        else atomicAdd(&h[bin], 1u);
+  __shared__ float4 ti[GR_T], tj[GR_T + 4];   // 4: read, not used, by the last group of j
+  __shared__ uint32_t queue[GR_T / 64][5 * 64];   // fewer than 64, and a group's 4 x 64
+  __shared__ uint32_t binned;
+  const uint32_t tid = threadIdx.x, lane = pb_lane(), wave = tid / 64;
+  for (uint32_t b = tid; b < rnum; b += GR_T) h[b] = 0;
+  if (tid == 0) binned = 0;
+  const uint64_t per = (nitem + gridDim.x - 1) / gridDim.x;
+  const uint64_t w0 = (uint64_t)blockIdx.x * per, w1 = min(w0 + per, nitem);
+  uint32_t pairs = 0, since = 0;           // of the items in the LDS histogram
+  uint32_t rep = 0;
+  for (uint64_t w = w0; w < w1; ++w) {     // block-uniform
+    const uint64_t p = w / slices;
+    const uint32_t slice = (uint32_t)(w % slices);
+    if (w == w0 || (rep + 1 < nrep && p >= reps[rep + 1].pair0)) {
+      uint32_t lo = rep, hi = nrep;
+      while (hi - lo > 1) {
+        const uint32_t mid = (lo + hi) / 2;
+        if (reps[mid].pair0 <= p) lo = mid;
+        else hi = mid;
       }
+      rep = lo;
     }
-    {
-      const uint32_t wz = pb_wave_sum_u32(zero);
-      if (pb_lane() == 0 && wz) atomicAdd(&h[0], wz);
-      zero = 0;
+    const GrRep R = reps[rep];
+    // triangular index t -> (it <= jt): row it starts at it ntile - it (it - 1) / 2
+    const uint64_t t = p - R.pair0;
+    const double b2 = 2.0 * R.ntile + 1.0;
+    uint32_t it = (uint32_t)(0.5 * (b2 - sqrt(fmax(b2 * b2 - 8.0 * (double)t, 0.0))));
+    auto row0 = [&](uint32_t k) { return (uint64_t)k * R.ntile - (uint64_t)k * (k - 1) / 2; };
+    it = min(it, R.ntile - 1u);
+    while (it > 0 && row0(it) > t) --it;
+    while (it + 1 < R.ntile && row0(it + 1) <= t) ++it;
+    const uint32_t jt = it + (uint32_t)(t - row0(it));
+    const uint32_t ni = min(GR_T, R.natoms - it * GR_T), nj = min(GR_T, R.natoms - jt * GR_T);
+    const uint32_t j0 = min(nj, slice * (GR_T / slices)), j1 = min(nj, j0 + GR_T / slices);
+    const bool diag = it == jt;
+    pairs += diag ? (j1 * j1 - j1 - (j0 * j0 - j0)) / 2u : ni * (j1 - j0);
+    const float L[3] = {R.hi[0] - R.lo[0], R.hi[1] - R.lo[1], R.hi[2] - R.lo[2]};
+    __syncthreads();                       // the tiles of the item before are consumed
+    // FP32 position of a particle; whether the bound holds for it
+    auto load = [&](uint32_t k, float4 &q) {
+      const double4 x = r[R.atom0 + k];
+      q = make_float4((float)x.x, (float)x.y, (float)x.z, 0.f);
+      const float c[3] = {q.x, q.y, q.z};
+      bool in = true;
+#pragma unroll
+      for (int a = 0; a < 3; ++a) {
+        const float s = 0.125f * L[a];
+        in = in && c[a] >= R.lo[a] - s && c[a] <= R.hi[a] + s;
+      }
+      return in;
+    };
+    float4 pi = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float K = R.rstepinv * R.rstepinv * (64.0f * 5.9604645e-8f * 1.0001f) * (R.cx + R.cy + R.cz);
+    bool ok = K < 0.25f * (float)rnum;
+    if (tid < ni) {
+      ok = load(it * GR_T + tid, pi) && ok;
+      ti[tid] = pi;
+    }
+    if (tid >= j0 && tid < j1) ok = load(jt * GR_T + tid, tj[tid]) && ok;
+    if (!__syncthreads_and(ok)) {
+      if (tid < ni)
+        for (uint32_t jj = diag ? max(j0, tid + 1) : j0; jj < j1; ++jj) {
+          const uint32_t bin = gr_bin(pi, tj[jj], R, rnum);
+          if (bin) atomicAdd(&h[bin], 1u);
+        }
+    } else {
+      const float sc = R.rstepinv, ke = -K / sc;
+      const float k0 = 0.5f - 9.5367432e-7f * (float)(rnum + 2u);
+      const float tin = (float)rnum, tout = (float)(rnum + 1u);
+      const uint32_t first = tid >= ni ? GR_T : (diag ? tid + 1u : 0u);
+      uint32_t qn = 0;                     // queued pairs (wave-uniform)
+      auto work_off = [&](uint32_t n) {    // the last n <= 64 queued pairs, exactly
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (lane < n) {
+          const uint32_t e = queue[wave][qn - n + lane];
+          const uint32_t bin = gr_bin(ti[e >> 16], tj[e & 0xFFFFu], R, rnum);
+          if (bin) atomicAdd(&h[bin], 1u);
+        }
+        qn -= n;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+      };
+      // four consecutive j: their loads and arithmetic interleave, and one
+      // branch asks whether any lane has a pair for the queue
+      auto four = [&](uint32_t jj, auto masked) {
+        constexpr uint32_t U = 4;
+        bool slow[U], any = false;
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+          const float4 pj = tj[jj + u];
+          const float dx = fabsf(pi.x - pj.x), dy = fabsf(pi.y - pj.y), dz = fabsf(pi.z - pj.z);
+          const float ax = fminf(dx, fabsf(dx - L[0])), ay = fminf(dy, fabsf(dy - L[1])),
+                      az = fminf(dz, fabsf(dz - L[2]));
+          const float R2 = fmaf(az, az, fmaf(ay, ay, ax * ax));
+          const float y = __builtin_amdgcn_rsqf(R2);
+          const float tc = fmaf(R2 * sc, y, 0.5f);    // NaN at R2 = 0: exact arithmetic
+          // half a bin less the bound; beyond rnum the bound is below 1
+          const float room = fmaf(ke, y, k0);
+          const bool valid = !decltype(masked)::value || (jj + u >= first && jj + u < j1);
+          const bool safe = fabsf(__builtin_amdgcn_fractf(tc) - 0.5f) < room;
+          if (valid && safe && tc < tin) atomicAdd(&h[(uint32_t)tc], 1u);
+          slow[u] = valid && !safe && !(tc >= tout);
+          any |= slow[u];
+        }
+        if (__ballot(any) == 0ull) return;
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+          const uint64_t m = __ballot(slow[u]);
+          if (slow[u])
+            queue[wave][qn + __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32),
+                                                       __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u))] =
+                (tid << 16) + jj + u;
+          qn += (uint32_t)__popcll(m);
+        }
+        while (qn >= 64u) work_off(64u);
+      };
+      uint32_t jj = j0;
+      if (!diag && ni == GR_T)
+        for (; jj + 4 <= j1; jj += 4) four(jj, std::false_type{});
+      for (; jj < j1; jj += 4) four(jj, std::true_type{});
+      if (qn) work_off(qn);                // fewer than 64
     }
     // flush when the replica changes, at the end (histograms are per
-    // replica) and every GR_FLUSH_TILES tile pairs (no uint32 bin can wrap)
-    const uint64_t pn = p + gridDim.x;
-    bool flush = pn >= npairs || ++since >= GR_FLUSH_TILES;
-    if (!flush) {
-      flush = !(pn >= R.pair0 && (lo + 1 >= nrep || pn < reps[lo + 1].pair0));
-    }
-    __syncthreads();
+    // replica) and every GR_FLUSH_ITEMS items (no uint32 count can wrap)
+    const bool flush = w + 1 >= w1 || ++since >= GR_FLUSH_ITEMS ||
+                       (rep + 1 < nrep && (w + 1) / slices >= reps[rep + 1].pair0);
     if (flush) {
-      for (uint32_t b = threadIdx.x; b < rnum; b += GR_T) {
+      __syncthreads();
+      uint32_t mine = 0;
+      for (uint32_t b = tid; b < rnum; b += GR_T) {
         const uint32_t v = h[b];
-        if (v) atomicAdd((unsigned long long *)&hist[(uint64_t)lo * rnum + b], (unsigned long long)v);
         h[b] = 0;
+        if (b && v) {
+          mine += v;
+          atomicAdd((unsigned long long *)&hist[(uint64_t)rep * rnum + b], (unsigned long long)v);
+        }
       }
+      mine = pb_wave_sum_u32(mine);
+      if (lane == 0 && mine) atomicAdd(&binned, mine);
+      __syncthreads();
+      if (tid == 0) {
+        if (pairs != binned)
+          atomicAdd((unsigned long long *)&hist[(uint64_t)rep * rnum], (unsigned long long)(pairs - binned));
+        binned = 0;
+      }
+      pairs = 0;
       since = 0;
     }
   }
-}
-
-extern "C" int pb_gr_hist(pb_sys *s, const float *rstep, uint32_t rnum, uint64_t *hist) {
-  if (!s || !rstep || !hist || rnum == 0) return PB_ERR_ARG;
-  if (rnum > 16384) return pb_fail(s->ctx, PB_ERR_ARG, "pb_gr_hist: rnum > 16384");
-  if (!s->cell_set) return pb_fail(s->ctx, PB_ERR_STATE, "pb_gr_hist: cell not set");
-  std::vector<GrRep> hr(s->nrep);
-  uint64_t tot = 0;
-  for (uint32_t q = 0; q < s->nrep; ++q) {
-    GrRep &g = hr[q];
-    g.atom0 = s->reps[q].atom0;
-    g.natoms = s->reps[q].natoms;
-    g.ntile = (g.natoms + GR_T - 1) / GR_T;
-    g.pair0 = tot;
-    tot += (uint64_t)g.ntile * (g.ntile + 1) / 2;
-    float c[3];
-    half_cell2(s, q, c);
-    g.cx = c[0];
-    g.cy = c[1];
-    g.cz = c[2];
-    // cudaCalcGR::setup: rstepinv = 1.0 / rstep (double) stored as real
-    g.rstepinv = (float)(1.0 / (double)rstep[q]);
-  }
-  // storage order must hold each replica's real particles at [atom0, atom0+natoms):
-  // true at all times (padding sorts after real particles of its replica).
-  GrRep *dreps = nullptr;
-  const size_t hn = (size_t)s->nrep * rnum;
-  if (s->gr_cap < hn) {
-    if (int rc = pb_alloc(s->ctx, &s->gr_hist, hn)) return rc;
-    s->gr_cap = hn;
-  }
-  if (int rc = pb_alloc(s->ctx, &dreps, s->nrep)) return rc;
-  hipStream_t st = s->ctx->stream;
-  hipError_t e = hipMemcpyAsync(dreps, hr.data(), sizeof(GrRep) * s->nrep, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) e = hipMemsetAsync(s->gr_hist, 0, sizeof(uint64_t) * hn, st);
-  if (e == hipSuccess) {
-    const uint32_t grid = (uint32_t)std::min<uint64_t>(tot, 8192);
-    hipLaunchKernelGGL(k_gr, dim3(grid), dim3(GR_T), sizeof(uint32_t) * rnum, st, s->r, dreps,
-                       s->nrep, tot, rnum, s->gr_hist);
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipMemcpyAsync(hist, s->gr_hist, sizeof(uint64_t) * hn, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  pb_free(dreps);
-  if (e != hipSuccess) return pb_hip_check(s->ctx, e, "pb_gr_hist");
-  return PB_OK;
-}
-
-// ---------------------------------------- g(r) without allocations
-// pb_gr_hist_noalloc keeps its replica table and histograms in this
-// file-scope device array instead of library-allocated memory: each device
-// holds its own copy for the life of the process.  Host code never passes
-// the array's name to a kernel (on the host it is only a stand-in symbol);
-// it uses the device address that pb_gr_scratch_init stores in the context.
-#define GR_NA_MAX_REPS 4096u                          // replicas per call
-#define GR_NA_MAX_SLOTS 131072u                       // nrep * rnum histogram slots
-#define GR_NA_REP_BYTES ((size_t)GR_NA_MAX_REPS * sizeof(GrRep))
-#define GR_NA_RSTEP_BYTES ((size_t)GR_NA_MAX_REPS * sizeof(float))
-#define GR_NA_BYTES (GR_NA_REP_BYTES + GR_NA_RSTEP_BYTES + (size_t)GR_NA_MAX_SLOTS * 8)
-static __device__ __align__(256) unsigned char scratch[GR_NA_BYTES];
-
-// the device address of `scratch` on the context's (current) device
-int pb_gr_scratch_init(pb_ctx *c) {
-  void *ptr = nullptr;
-  const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
-  if (e != hipSuccess || !ptr) return pb_hip_check(c, e != hipSuccess ? e : hipErrorUnknown,
-                                                   "hipGetSymbolAddress(g(r) scratch)");
-  c->gr_scratch = ptr;
-  return PB_OK;
 }
 
 // replica table of the g(r) kernel from the device replica records: one
@@ -487,8 +538,7 @@ __global__ void __launch_bounds__(256) k_gr_prep(const RepInfo *reps, const floa
     g.ntile = (R.natoms + GR_T - 1) / GR_T;
     g.pair0 = base;
     base += (unsigned long long)g.ntile * (g.ntile + 1) / 2;
-    // cudaFrame::setCell (cudaFrame.cu:85-91) on the FP32 cell values, as
-    // the host-side table of pb_gr_hist
+    // cudaFrame::setCell (cudaFrame.cu:85-91) on the FP32 cell values
     float c[3];
     for (int a = 0; a < 3; ++a) {
       const float lo = (float)R.lo[a], hi = (float)R.hi[a];
@@ -498,14 +548,89 @@ __global__ void __launch_bounds__(256) k_gr_prep(const RepInfo *reps, const floa
     g.cx = c[0];
     g.cy = c[1];
     g.cz = c[2];
+    // cudaCalcGR::setup: rstepinv = 1.0 / rstep (double) stored as real
     g.rstepinv = (float)(1.0 / (double)rstep[q]);
+    for (int a = 0; a < 3; ++a) {
+      g.lo[a] = (float)R.lo[a];
+      g.hi[a] = (float)R.hi[a];
+    }
     out[q] = g;
   }
 }
 
-__global__ void k_zero_u64(uint64_t *x, uint32_t n) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void k_zero_u64(uint64_t *x, size_t n) {
+  const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) x[i] = 0;
+}
+
+// Table, cleared histograms, pairs and the histograms back to the host, on
+// given device memory (rstep first written by an upload).  Storage order
+// holds each replica's real particles at [atom0, atom0 + natoms) at all times
+// (padding sorts after the real particles of its replica).
+static int gr_run(pb_sys *s, const float *rstep, uint32_t rnum, uint64_t *hist, GrRep *dreps,
+                  float *drstep, uint64_t *dhist) {
+  uint64_t tot = 0;
+  for (uint32_t q = 0; q < s->nrep; ++q) {
+    const uint64_t nt = (s->reps[q].natoms + GR_T - 1) / GR_T;
+    tot += nt * (nt + 1) / 2;
+  }
+  // few tile pairs: their j particles split so that 4096 workgroups (16 a
+  // compute unit) have work
+  uint32_t slices = 1;
+  while (slices < GR_MAX_SLICES && tot * slices < 4096) slices *= 2;
+  const size_t hn = (size_t)s->nrep * rnum;
+  hipStream_t st = s->ctx->stream;
+  if (int rc = pb_io_upload(s->ctx, drstep, rstep, sizeof(float) * s->nrep)) return rc;
+  hipLaunchKernelGGL(k_gr_prep, dim3(1), dim3(256), 0, st, s->d_reps, drstep, s->nrep, dreps);
+  hipLaunchKernelGGL(k_zero_u64, dim3(pb_blocks(hn, 256)), dim3(256), 0, st, dhist, hn);
+  if (tot) {
+    // a few items a workgroup: their number varies by the diagonal and the
+    // ragged tiles (16384 workgroups at most: 6 % slower on the 256 replicas)
+    const uint32_t grid = (uint32_t)std::min<uint64_t>(tot * slices, 65536);
+    hipLaunchKernelGGL(k_gr, dim3(grid), dim3(GR_T), sizeof(uint32_t) * rnum, st,
+                       s->r, dreps, s->nrep, tot * slices, slices, rnum, dhist);
+  }
+  PB_LAUNCH_CHECK(s->ctx, "k_gr");
+  return pb_io_download(s->ctx, hist, dhist, sizeof(uint64_t) * hn);
+}
+
+extern "C" int pb_gr_hist(pb_sys *s, const float *rstep, uint32_t rnum, uint64_t *hist) {
+  if (!s || !rstep || !hist || rnum == 0) return PB_ERR_ARG;
+  if (rnum > 16384) return pb_fail(s->ctx, PB_ERR_ARG, "pb_gr_hist: rnum > 16384");
+  if (!s->cell_set) return pb_fail(s->ctx, PB_ERR_STATE, "pb_gr_hist: cell not set");
+  // one workspace, kept: histograms, replica table, steps
+  const size_t hb = sizeof(uint64_t) * (size_t)s->nrep * rnum, rb = sizeof(GrRep) * (size_t)s->nrep;
+  const size_t need = hb + rb + sizeof(float) * (size_t)s->nrep;
+  if (s->gr_cap < need) {
+    s->gr_cap = 0;
+    if (int rc = pb_alloc(s->ctx, (uint8_t **)&s->gr_hist, need)) return rc;
+    s->gr_cap = need;
+  }
+  uint8_t *base = (uint8_t *)s->gr_hist;
+  return gr_run(s, rstep, rnum, hist, (GrRep *)(base + hb), (float *)(base + hb + rb), s->gr_hist);
+}
+
+// ---------------------------------------- g(r) without allocations
+// pb_gr_hist_noalloc keeps its replica table and histograms in this
+// file-scope device array instead of library-allocated memory: each device
+// holds its own copy for the life of the process.  Host code never passes
+// the array's name to a kernel (on the host it is only a stand-in symbol);
+// it uses the device address that pb_gr_scratch_init stores in the context.
+#define GR_NA_MAX_REPS 4096u                          // replicas per call
+#define GR_NA_MAX_SLOTS 131072u                       // nrep * rnum histogram slots
+#define GR_NA_REP_BYTES ((size_t)GR_NA_MAX_REPS * sizeof(GrRep))
+#define GR_NA_RSTEP_BYTES ((size_t)GR_NA_MAX_REPS * sizeof(float))
+#define GR_NA_BYTES (GR_NA_REP_BYTES + GR_NA_RSTEP_BYTES + (size_t)GR_NA_MAX_SLOTS * 8)
+static __device__ __align__(256) unsigned char scratch[GR_NA_BYTES];
+
+// the device address of `scratch` on the context's (current) device
+int pb_gr_scratch_init(pb_ctx *c) {
+  void *ptr = nullptr;
+  const hipError_t e = hipGetSymbolAddress(&ptr, HIP_SYMBOL(scratch));
+  if (e != hipSuccess || !ptr) return pb_hip_check(c, e != hipSuccess ? e : hipErrorUnknown,
+                                                   "hipGetSymbolAddress(g(r) scratch)");
+  c->gr_scratch = ptr;
+  return PB_OK;
 }
 
 extern "C" int pb_gr_hist_noalloc(pb_sys *s, const float *rstep, uint32_t rnum, uint64_t *hist) {
@@ -521,33 +646,10 @@ extern "C" int pb_gr_hist_noalloc(pb_sys *s, const float *rstep, uint32_t rnum, 
     return pb_fail(s->ctx, PB_ERR_STATE, "pb_gr_hist_noalloc: no scratch address");
   for (uint32_t q = 0; q < s->nrep; ++q)
     if (!(rstep[q] > 0.0f)) return pb_fail(s->ctx, PB_ERR_ARG, "pb_gr_hist_noalloc: rstep <= 0");
-  // tile pairs of all replicas (host replica records, no allocation)
-  uint64_t tot = 0;
-  for (uint32_t q = 0; q < s->nrep; ++q) {
-    const uint64_t nt = (s->reps[q].natoms + GR_T - 1) / GR_T;
-    tot += nt * (nt + 1) / 2;
-  }
   unsigned char *base = static_cast<unsigned char *>(s->ctx->gr_scratch);
-  GrRep *dreps = reinterpret_cast<GrRep *>(base);
-  float *drstep = reinterpret_cast<float *>(base + GR_NA_REP_BYTES);
-  uint64_t *dhist = reinterpret_cast<uint64_t *>(base + GR_NA_REP_BYTES + GR_NA_RSTEP_BYTES);
-  const uint32_t hn = s->nrep * rnum;
-  hipStream_t st = s->ctx->stream;
-  hipError_t e = hipMemcpyAsync(drstep, rstep, sizeof(float) * s->nrep, hipMemcpyHostToDevice, st);
-  if (e == hipSuccess) {
-    hipLaunchKernelGGL(k_gr_prep, dim3(1), dim3(256), 0, st, s->d_reps, drstep, s->nrep, dreps);
-    hipLaunchKernelGGL(k_zero_u64, dim3(pb_blocks(hn, 256)), dim3(256), 0, st, dhist, hn);
-    if (tot) {
-      const uint32_t grid = (uint32_t)std::min<uint64_t>(tot, 8192);
-      hipLaunchKernelGGL(k_gr, dim3(grid), dim3(GR_T), sizeof(uint32_t) * rnum, st, s->r, dreps,
-                         s->nrep, tot, rnum, dhist);
-    }
-    e = hipGetLastError();
-  }
-  if (e == hipSuccess) e = hipMemcpyAsync(hist, dhist, sizeof(uint64_t) * hn, hipMemcpyDeviceToHost, st);
-  if (e == hipSuccess) e = hipStreamSynchronize(st);
-  if (e != hipSuccess) return pb_hip_check(s->ctx, e, "pb_gr_hist_noalloc");
-  return PB_OK;
+  return gr_run(s, rstep, rnum, hist, reinterpret_cast<GrRep *>(base),
+                reinterpret_cast<float *>(base + GR_NA_REP_BYTES),
+                reinterpret_cast<uint64_t *>(base + GR_NA_REP_BYTES + GR_NA_RSTEP_BYTES));
 }
 
 __global__ void k_clear4_bin(double4 *x, uint32_t n) {

@@ -166,8 +166,8 @@ struct pb_sys {
   bool md_valid = false;
 
   // g(r)
-  uint64_t *gr_hist = nullptr;
-  size_t gr_cap = 0;
+  uint64_t *gr_hist = nullptr;     // histograms, replica table, rstep
+  size_t gr_cap = 0;               // bytes
 
   // SPH (cudaParticleSPH_NS), storage order unless noted
   double *sph_mu0 = nullptr, *sph_c2 = nullptr, *sph_rhoinv = nullptr;
@@ -248,11 +248,13 @@ int pb_counting_sort(pb_sys *sys, uint32_t ncell, const uint32_t *key);
 int pb_counting_sort_counted(pb_sys *sys, uint32_t ncell, const uint32_t *key);
 // per-replica reduction of K per-wave partial components into out[rep*8+c]
 int pb_reduce_waves(pb_sys *sys, int K);
-// host boundary (pb_io.hip): the packed-field device buffer, an upload into
-// it, a scalar per particle from the caller's order into storage order
+// host boundary (pb_io.hip): copies through the context's pinned ring (an
+// upload is stream ordered, a download waits); the packed-field device
+// buffer; a scalar per particle from the caller's order into storage order
 // (squared if asked; padding 0) and a uint32 per slot to the caller's order
+int pb_io_upload(pb_ctx *ctx, void *dev, const void *host, size_t bytes);
+int pb_io_download(pb_ctx *ctx, void *host, const void *dev, size_t bytes);
 int pb_io_buffer(pb_sys *sys);
-int pb_io_upload(pb_sys *sys, const void *host, size_t bytes, size_t off);
 int pb_io_scatter(pb_sys *sys, const double *host, double *dst, bool square);
 int pb_io_gather_u32(pb_sys *sys, const uint32_t *src, uint32_t *host);
 void pb_io_release(pb_ctx *ctx);

@@ -48,16 +48,16 @@ void pb_io_release(pb_ctx *ctx) {
   }
 }
 
-// Both return with the ring free: every DMA that used it has completed.
-static int download(pb_ctx *ctx, void *host, const uint8_t *dev, size_t bytes) {
+// Device to host.  Every DMA that wrote the ring has completed on return.
+int pb_io_download(pb_ctx *ctx, void *host, const void *dev, size_t bytes) {
   if (int rc = ensure_stage(ctx)) return rc;
   hipStream_t st = ctx->stream;
   const size_t nchunk = (bytes + IO_CHUNK - 1) / IO_CHUNK;
   for (size_t c = 0; c <= nchunk; ++c) {
     if (c < nchunk) {
       const size_t len = std::min(IO_CHUNK, bytes - c * IO_CHUNK);
-      PB_HIP(ctx, hipMemcpyAsync(ctx->io_stage + (c & 1u) * IO_CHUNK, dev + c * IO_CHUNK, len,
-                                 hipMemcpyDeviceToHost, st));
+      PB_HIP(ctx, hipMemcpyAsync(ctx->io_stage + (c & 1u) * IO_CHUNK,
+                                 (const uint8_t *)dev + c * IO_CHUNK, len, hipMemcpyDeviceToHost, st));
       PB_HIP(ctx, hipEventRecord(ctx->io_ev[c & 1u], st));
     }
     if (c > 0) {
@@ -69,20 +69,21 @@ static int download(pb_ctx *ctx, void *host, const uint8_t *dev, size_t bytes) {
   return PB_OK;
 }
 
-int pb_io_upload(pb_sys *s, const void *host, size_t bytes, size_t off) {
-  pb_ctx *ctx = s->ctx;
+// Host to device, stream ordered; the caller's buffer is free on return.  A
+// slot's last event tells when the host may write it again (an event that was
+// never recorded, or one of a finished download, does not wait).
+int pb_io_upload(pb_ctx *ctx, void *dev, const void *host, size_t bytes) {
   if (int rc = ensure_stage(ctx)) return rc;
   hipStream_t st = ctx->stream;
   const size_t nchunk = (bytes + IO_CHUNK - 1) / IO_CHUNK;
   for (size_t c = 0; c < nchunk; ++c) {
     const size_t len = std::min(IO_CHUNK, bytes - c * IO_CHUNK);
     uint8_t *slot = ctx->io_stage + (c & 1u) * IO_CHUNK;
-    if (c >= 2) PB_HIP(ctx, hipEventSynchronize(ctx->io_ev[c & 1u]));
+    PB_HIP(ctx, hipEventSynchronize(ctx->io_ev[c & 1u]));
     std::memcpy(slot, (const uint8_t *)host + c * IO_CHUNK, len);
-    PB_HIP(ctx, hipMemcpyAsync(s->io + off + c * IO_CHUNK, slot, len, hipMemcpyHostToDevice, st));
+    PB_HIP(ctx, hipMemcpyAsync((uint8_t *)dev + c * IO_CHUNK, slot, len, hipMemcpyHostToDevice, st));
     PB_HIP(ctx, hipEventRecord(ctx->io_ev[c & 1u], st));
   }
-  if (nchunk) PB_HIP(ctx, hipEventSynchronize(ctx->io_ev[(nchunk - 1) & 1u]));
   return PB_OK;
 }
 
@@ -199,12 +200,12 @@ static int download_packed(pb_sys *s, void *host, size_t bytes, F &&pack) {
   if (int rc = pb_io_buffer(s)) return rc;
   pack((void *)s->io);
   PB_LAUNCH_CHECK(ctx, "pb_sys_get");
-  return download(ctx, host, s->io, bytes);
+  return pb_io_download(ctx, host, s->io, bytes);
 }
 
 int pb_io_scatter(pb_sys *s, const double *host, double *dst, bool square) {
   if (int rc = pb_io_buffer(s)) return rc;
-  if (int rc = pb_io_upload(s, host, 8 * (size_t)s->n, 0)) return rc;
+  if (int rc = pb_io_upload(s->ctx, s->io, host, 8 * (size_t)s->n)) return rc;
   const double *in = (const double *)s->io;
   if (square) hipLaunchKernelGGL(k_pack_square, IO_GRID(s), in, s->orig, s->npad, dst);
   else hipLaunchKernelGGL(k_pack1<double>, IO_GRID(s), in, s->orig, s->npad, dst);
@@ -238,8 +239,9 @@ extern "C" int pb_sys_import(pb_sys *s, const double *r, const double *v, const 
   A.n = s->npad;
   A.r = s->r; A.v = s->v; A.a = s->a; A.F = s->F;
   A.type = s->type; A.move = s->move;
-  if ((rc = pb_io_upload(s, m, 8 * n, 0)) || (type && (rc = pb_io_upload(s, type, 4 * n, 8 * n))) ||
-      (is_fixed && (rc = pb_io_upload(s, is_fixed, n, 12 * n))))
+  if ((rc = pb_io_upload(s->ctx, s->io, m, 8 * n)) ||
+      (type && (rc = pb_io_upload(s->ctx, s->io + 8 * n, type, 4 * n))) ||
+      (is_fixed && (rc = pb_io_upload(s->ctx, s->io + 12 * n, is_fixed, n))))
     return rc;
   hipLaunchKernelGGL(k_import_scalars, IO_GRID(s), A);
   PB_LAUNCH_CHECK(s->ctx, "k_import_scalars");
@@ -248,7 +250,7 @@ extern "C" int pb_sys_import(pb_sys *s, const double *r, const double *v, const 
   for (int k = 0; k < 3; ++k) {
     if (!src[k]) continue;
     // the stream orders the upload behind the kernels that read the buffer
-    if ((rc = pb_io_upload(s, src[k], 24 * n, 0))) return rc;
+    if ((rc = pb_io_upload(s->ctx, s->io, src[k], 24 * n))) return rc;
     hipLaunchKernelGGL(k_pack3, IO_GRID(s), (const double *)s->io, s->orig, s->npad, dst[k]);
     PB_LAUNCH_CHECK(s->ctx, "k_pack3");
   }
@@ -334,7 +336,7 @@ extern "C" int pb_sys_set(pb_sys *s, int field, const void *host) {
       default: return pb_fail(s->ctx, PB_ERR_ARG, "pb_sys_set: unknown field");
     }
   }
-  if ((rc = pb_io_buffer(s)) || (rc = pb_io_upload(s, host, bytes, 0))) return rc;
+  if ((rc = pb_io_buffer(s)) || (rc = pb_io_upload(s->ctx, s->io, host, bytes))) return rc;
   if (vec) {
     hipLaunchKernelGGL(k_pack3, IO_GRID(s), (const double *)s->io, s->orig, s->npad, vec);
     if (field == PB_FIELD_SPH_NUM && s->sph_rhoinv)
