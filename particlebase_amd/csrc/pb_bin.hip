@@ -8,9 +8,6 @@
 #include <cstring>
 #include <type_traits>
 
-int pb_ensure_sort_ws(pb_sys *s, uint32_t ncell);
-int pb_counting_sort(pb_sys *s, uint32_t ncell, const uint32_t *key);
-
 // CUDA's float->uint conversion saturates; calcBID_F4 relies on it.
 __device__ __host__ __forceinline__ uint32_t f2u_sat(float q) {
   if (!(q > 0.0f)) return 0u;
@@ -43,34 +40,27 @@ struct RefGrid {
 };
 
 // calcBID_F4, kernelfuncs.cu:807-841; padding slots go to the extra cell
-// ncell so they sort after every real particle.
+// ncell so they sort after every real particle.  The cell's particles are
+// counted in the same pass.
 __global__ void k_ref_bid(const double4 *r, const uint32_t *orig, uint32_t n, RefGrid g,
-                          uint32_t ncell, uint32_t *cellid) {
+                          uint32_t ncell, uint32_t *cellid, uint32_t *counts, uint32_t *rank) {
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n) return;
-  if (orig[s] == PB_NONE) {
-    cellid[s] = ncell;
-    return;
+  const bool valid = s < n;
+  uint32_t c = PB_NONE;
+  if (valid) {
+    c = ncell;
+    if (orig[s] != PB_NONE) {
+      const double4 p = r[s];
+      const float x = (float)p.x, y = (float)p.y, z = (float)p.z;
+      const uint32_t d0 = clamp_axis(f2u_sat((x - g.lo[0]) / g.len[0]), g.nb[0]);
+      const uint32_t d1 = clamp_axis(f2u_sat((y - g.lo[1]) / g.len[1]), g.nb[1]);
+      const uint32_t d2 = clamp_axis(f2u_sat((z - g.lo[2]) / g.len[2]), g.nb[2]);
+      c = d2 + d1 * g.nb[2] + d0 * g.nb[1] * g.nb[2];
+    }
+    cellid[s] = c;
   }
-  const double4 p = r[s];
-  const float x = (float)p.x, y = (float)p.y, z = (float)p.z;
-  const uint32_t d0 = clamp_axis(f2u_sat((x - g.lo[0]) / g.len[0]), g.nb[0]);
-  const uint32_t d1 = clamp_axis(f2u_sat((y - g.lo[1]) / g.len[1]), g.nb[1]);
-  const uint32_t d2 = clamp_axis(f2u_sat((z - g.lo[2]) / g.len[2]), g.nb[2]);
-  cellid[s] = d2 + d1 * g.nb[2] + d0 * g.nb[1] * g.nb[2];
-}
-
-__global__ void k_ref_outputs(const uint32_t *perm, const uint32_t *cellid, const uint32_t *orig,
-                              const uint32_t *count, const uint32_t *start, uint32_t nreal,
-                              uint32_t ncell, uint32_t *pid, uint32_t *bid, uint32_t *bindex) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k < nreal) {
-    const uint32_t s = perm[k];
-    pid[k] = orig[s];
-    bid[k] = cellid[s];
-  }
-  if (k < ncell) bindex[k] = count[k] ? start[k] : PB_NONE;
-  if (k == 0) bindex[ncell] = nreal;
+  const uint32_t k = pb_count_rank(c, valid, counts);
+  if (valid) rank[s] = k;
 }
 
 static void host_neighbor_table(const uint32_t bn[3], int w, int periodic, uint32_t *table) {
@@ -194,14 +184,11 @@ extern "C" int pb_bin(pb_sys *s) {
   hipStream_t st = s->ctx->stream;
   const uint32_t nc = s->ref_ncell;
   hipLaunchKernelGGL(k_ref_bid, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->r, s->orig,
-                     s->npad, ref_grid(s), nc, s->cellid);
+                     s->npad, ref_grid(s), nc, s->cellid, s->ccount, s->rank);
   PB_LAUNCH_CHECK(s->ctx, "k_ref_bid");
-  if (int rc = pb_counting_sort(s, nc + 1, s->orig)) return rc;
-  const uint32_t m = (s->n > nc + 1) ? s->n : nc + 1;
-  hipLaunchKernelGGL(k_ref_outputs, dim3(pb_blocks(m, 256)), dim3(256), 0, st, s->perm, s->cellid,
-                     s->orig, s->ccount, s->cstart, s->n, nc, s->ref_pid, s->ref_bid,
-                     s->ref_bindex);
-  PB_LAUNCH_CHECK(s->ctx, "k_ref_outputs");
+  PbCellOrder O;
+  if (int rc = pb_counting_sort(s, nc + 1, s->orig, &O)) return rc;
+  if (int rc = pb_cell_order(s, O, nc)) return rc;
   s->ref_binned = true;
   return PB_OK;
 }

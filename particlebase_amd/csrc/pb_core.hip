@@ -198,6 +198,7 @@ extern "C" void pb_sys_destroy(pb_sys *s) {
   pb_free(s->md_row); pb_free(s->md_col); pb_free(s->md_inv);
   pb_free(s->ref_table); pb_free(s->ref_bid); pb_free(s->ref_pid); pb_free(s->ref_bindex);
   pb_free(s->cellid); pb_free(s->rank); pb_free(s->perm); pb_free(s->ccount);
+  pb_free(s->skey); pb_free(s->sslot); pb_free(s->scell);
   pb_free(s->cstart); pb_free(s->scan_tmp); pb_free(s->d_lj);
   pb_free(s->nl); pb_free(s->nn); pb_free(s->rbuild); pb_free(s->r2buf); pb_free(s->v2buf);
   pb_free(s->orig2); pb_free(s->type2); pb_free(s->move2); pb_free(s->a2buf);

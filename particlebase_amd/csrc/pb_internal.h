@@ -103,6 +103,7 @@ struct pb_sys {
 
   // counting-sort workspace (shared by pb_bin and the list rebuild)
   uint32_t *cellid = nullptr, *rank = nullptr, *perm = nullptr;
+  uint32_t *skey = nullptr, *sslot = nullptr, *scell = nullptr;   // grouped by cell
   uint32_t *ccount = nullptr, *cstart = nullptr;  // ncell_cap + 1
   uint32_t ncell_cap = 0;
   uint32_t *scan_tmp = nullptr;
@@ -242,10 +243,17 @@ static inline uint32_t pb_blocks(size_t n, uint32_t bs) {
 int pb_ensure_sort_ws(pb_sys *sys, uint32_t ncell);
 // exclusive scan of in[0..n) into out[0..n], out[n] = total
 int pb_exclusive_scan(pb_sys *sys, const uint32_t *in, uint32_t *out, uint32_t n);
-// cellid[s] given (PB_NONE never); builds perm (sorted slot -> storage slot)
-// ordered by (cell, key[s]); counts/starts in sys->ccount / sys->cstart.
-int pb_counting_sort(pb_sys *sys, uint32_t ncell, const uint32_t *key);
-int pb_counting_sort_counted(pb_sys *sys, uint32_t ncell, const uint32_t *key);
+// (key, slot, cell) grouped by cell, in no particular order inside a cell
+struct PbCellOrder {
+  const uint32_t *start;       // cell -> first position (start[c + 1] ends it)
+  const uint32_t *skey, *sslot, *scell;
+};
+// cellid[s] (PB_NONE never), the counts of every cell and the rank of s among
+// them given; cells start in sys->cstart
+int pb_counting_sort(pb_sys *sys, uint32_t ncell, const uint32_t *key, PbCellOrder *O);
+// sys->perm (sorted position -> storage slot, by cell and key) and
+// calcBlockID's outputs of the reference cell grid
+int pb_cell_order(pb_sys *sys, const PbCellOrder &O, uint32_t ncell);
 // per-replica reduction of K per-wave partial components into out[rep*8+c]
 int pb_reduce_waves(pb_sys *sys, int K);
 // host boundary (pb_io.hip): copies through the context's pinned ring (an
@@ -289,6 +297,32 @@ __device__ __forceinline__ uint32_t pb_count_rank(uint32_t c, bool valid, uint32
   }
   base = __shfl(base, (int)hl, 64);
   return base + (lane - hl);
+}
+
+// Sorted position of the pair at i: its cell's start plus the number of
+// smaller keys in the cell (equal keys, which only padding has, by slot).
+// Lanes of a wavefront share cells, so the reads are mostly broadcast L1 hits;
+// eight are in flight at a time.
+__device__ __forceinline__ uint32_t pb_cell_position(const PbCellOrder &O, uint32_t i,
+                                                     uint32_t *slot, uint32_t *cell) {
+  const uint32_t s = O.sslot[i], k = O.skey[i], c = O.scell[i];
+  const uint32_t b = O.start[c], e = O.start[c + 1];
+  uint32_t rank = 0, same = 0;
+  for (uint32_t j = b; j < e; j += 8) {
+    uint32_t q[8];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) q[u] = O.skey[min(j + u, e - 1u)];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) {
+      rank += (j + u < e && q[u] < k) ? 1u : 0u;
+      same += (j + u < e && q[u] == k) ? 1u : 0u;
+    }
+  }
+  if (same > 1)
+    for (uint32_t j = b; j < e; ++j) rank += (O.skey[j] == k && O.sslot[j] < s) ? 1u : 0u;
+  *slot = s;
+  *cell = c;
+  return b + rank;
 }
 
 __device__ __forceinline__ double pb_wave_sum(double x) {

@@ -4,15 +4,19 @@
 // pre-sort, single-block odd-even sortByBID and makeBindex,
 // kernelfuncs.cu:844-932, cudaCutoffBlock.cu:241-256), whose in-cell order is
 // unstable and timing dependent.  Here:
-//   1. k_count   : wave64 atomics on per-cell counters; equal keys in
-//                  neighbouring lanes are aggregated into one atomic.
-//   2. scan      : exclusive prefix sum, LDS-tiled (block sums, then
-//                  scan-and-add with each block summing the sums before it),
-//                  any length.
-//   3. k_scatter : slot = start[cell] + rank.
-//   4. k_cell_sort: inside every cell, order by a key (the original particle
-//                  index) -- the in-cell order produced by the atomics is
+//   1. counting  : wave64 atomics on per-cell counters by the caller's cell-id
+//                  kernel (pb_count_rank); equal cells in neighbouring lanes
+//                  are aggregated into one atomic.
+//   2. scan      : exclusive prefix sum, LDS-tiled (each block adds the sums,
+//                  or the elements, before it), any length.
+//   3. k_scatter : (key, slot, cell) to start[cell] + rank; clears the counters for
+//                  the next sort.
+//   4. ordering  : inside every cell, by a key (the original particle index):
+//                  one thread an element counts the smaller keys of its cell
+//                  (pb_cell_position) -- the order produced by the atomics is
 //                  discarded, so the permutation is the canonical stable one.
+//                  Done by the kernel that uses the order (k_cell_order here,
+//                  k_reorder of the LJ path), not by a pass of its own.
 #include "pb_internal.h"
 
 #define SCAN_BS 256
@@ -93,18 +97,65 @@ __global__ void __launch_bounds__(SCAN_BS) k_scan_final(const uint32_t *in, uint
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = before + tot;
 }
 
-int pb_exclusive_scan(pb_sys *s, const uint32_t *in, uint32_t *out, uint32_t n) {
-  const uint32_t nb = (n + SCAN_CH - 1) / SCAN_CH;
-  const size_t need = (size_t)nb + 1;
-  if (s->scan_tmp_n < need) {
-    if (int rc = pb_alloc(s->ctx, &s->scan_tmp, need)) return rc;
-    s->scan_tmp_n = need;
+// Short arrays in one launch: every block sums all elements before its own
+// (at most SCAN_ONE_MAX reads a block, coalesced).  The rebuild of a small
+// system is a chain of launches of about 2 us each, so one fewer is worth
+// more than the extra reads; the line lies where they reach a launch's time.
+#define SCAN_ONE_BS 1024
+#define SCAN_ONE_CH 4096
+#define SCAN_ONE_MAX 16384u
+__global__ void __launch_bounds__(SCAN_ONE_BS) k_scan_one(const uint32_t *in, uint32_t n,
+                                                          uint32_t *out) {
+  __shared__ uint32_t wsum[SCAN_ONE_BS / 64], wpre[SCAN_ONE_BS / 64];
+  const uint32_t b0 = blockIdx.x * SCAN_ONE_CH, lane = pb_lane(), w = threadIdx.x / 64;
+  uint32_t pre = 0;
+  for (uint32_t k = threadIdx.x; k < b0; k += SCAN_ONE_BS) pre += in[k];
+  const uint32_t base = b0 + threadIdx.x * 4u;
+  uint32_t v[4], x = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k) {
+    v[k] = base + k < n ? in[base + k] : 0u;
+    x += v[k];
   }
+  const uint32_t inc = wave_incl_scan(x);
+  pre = pb_wave_sum_u32(pre);
+  if (lane == 63) wsum[w] = inc;
+  if (lane == 0) wpre[w] = pre;
+  __syncthreads();
+  uint32_t run = inc - x, before = 0, tot = 0;
+  for (uint32_t k = 0; k < SCAN_ONE_BS / 64; ++k) {
+    if (k < w) run += wsum[k];
+    tot += wsum[k];
+    before += wpre[k];
+  }
+  run += before;
+#pragma unroll
+  for (uint32_t k = 0; k < 4; ++k)
+    if (base + k < n) {
+      out[base + k] = run;
+      run += v[k];
+    }
+  if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = before + tot;
+}
+
+int pb_exclusive_scan(pb_sys *s, const uint32_t *in, uint32_t *out, uint32_t n) {
   hipStream_t st = s->ctx->stream;
   if (n == 0) {
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, out, 1u, 0u);
     PB_LAUNCH_CHECK(s->ctx, "scan(empty)");
     return PB_OK;
+  }
+  if (n <= SCAN_ONE_MAX) {
+    hipLaunchKernelGGL(k_scan_one, dim3(pb_blocks(n, SCAN_ONE_CH)), dim3(SCAN_ONE_BS), 0, st, in, n,
+                       out);
+    PB_LAUNCH_CHECK(s->ctx, "pb_exclusive_scan");
+    return PB_OK;
+  }
+  const uint32_t nb = (n + SCAN_CH - 1) / SCAN_CH;
+  const size_t need = (size_t)nb + 1;
+  if (s->scan_tmp_n < need) {
+    if (int rc = pb_alloc(s->ctx, &s->scan_tmp, need)) return rc;
+    s->scan_tmp_n = need;
   }
   hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(SCAN_BS), 0, st, in, n, s->scan_tmp);
   hipLaunchKernelGGL(k_scan_final, dim3(nb), dim3(SCAN_BS), 0, st, in, n, s->scan_tmp, out);
@@ -112,108 +163,41 @@ int pb_exclusive_scan(pb_sys *s, const uint32_t *in, uint32_t *out, uint32_t n) 
   return PB_OK;
 }
 
-// Wave-aggregated counting: lanes holding the same cell as their left
-// neighbour form a run; the run head does one atomicAdd for the whole run and
-// broadcasts the base.  Correct for any input; one atomic per run when the
-// input is already nearly cell-ordered (the steady state after a re-sort).
-__global__ void k_count(const uint32_t *cellid, uint32_t n, uint32_t *counts, uint32_t *rank) {
-  const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-  const bool valid = s < n;
-  const uint32_t c = valid ? cellid[s] : PB_NONE;
-  const uint32_t r = pb_count_rank(c, valid, counts);
-  if (valid) rank[s] = r;
-}
-
 __global__ void k_scatter(const uint32_t *cellid, const uint32_t *rank, const uint32_t *start,
-                          uint32_t n, uint32_t *perm) {
+                          const uint32_t *key, uint32_t n, uint32_t *skey, uint32_t *sslot,
+                          uint32_t *scell, uint32_t *counts, uint32_t ncell) {
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s < n) perm[start[cellid[s]] + rank[s]] = s;
+  if (s < ncell) counts[s] = 0;
+  if (s < n) {
+    const uint32_t c = cellid[s], pos = start[c] + rank[s];
+    skey[pos] = key[s];
+    sslot[pos] = s;
+    scell[pos] = c;
+  }
 }
 
-// CS_CELLS consecutive cells per workgroup own one contiguous range of perm
-// (64 cells: about 900 particles at liquid density, so a 1M-particle sort
-// is ~1200 workgroups and fills the chip).
-// The range is sorted in passes: each pass stages the longest run of the
-// remaining cells whose particles fit the LDS stage (at least one cell).
-// Every element then finds its cell and its rank in it -- the number of
-// elements of the cell with a smaller key (equal keys: smaller position) --
-// and is written to cell start + rank.  The rank loops are independent LDS
-// reads, so a crowded cell costs O(n) per element in parallel instead of a
-// serial O(n^2) insertion sort.  A single cell larger than the stage (a
-// pathological pile-up) is insertion-sorted in global memory by its thread.
-#define CS_CELLS 64
-#define CS_THREADS 256
-#define CS_CAP 3072
-__global__ void __launch_bounds__(CS_THREADS) k_cell_sort(const uint32_t *start, uint32_t ncell,
-                                                        const uint32_t *key, uint32_t *perm) {
-  __shared__ uint32_t sv[CS_CAP], sk[CS_CAP];
-  __shared__ uint32_t cst[CS_CELLS + 1];
-  __shared__ uint32_t s_next;
-  const uint32_t c0 = blockIdx.x * CS_CELLS;
-  const uint32_t c1 = min(c0 + CS_CELLS, ncell);
-  const uint32_t c = c0 + threadIdx.x;
-  // one pass when the whole range fits (the common case); otherwise runs of
-  // cells found by thread 0
-  const bool whole = start[c1] - start[c0] <= CS_CAP;
-  for (uint32_t ca = c0; ca < c1;) {                 // block-uniform
-    if (whole) {
-      if (threadIdx.x == 0) s_next = c1;
-    } else if (threadIdx.x == 0) {
-      // largest cb in [ca + 1, c1] with start[cb] - start[ca] <= CS_CAP
-      const uint32_t lim = start[ca] + CS_CAP;
-      uint32_t lo = ca + 1, hi = c1;
-      while (lo < hi) {
-        const uint32_t mid = (lo + hi + 1) >> 1;
-        if (start[mid] <= lim) lo = mid;
-        else hi = mid - 1;
-      }
-      s_next = lo;
-    }
-    __syncthreads();
-    const uint32_t cb = s_next;
-    const uint32_t base = start[ca], len = start[cb] - base;
-    if (len <= CS_CAP) {
-      const uint32_t nc = cb - ca;
-      for (uint32_t k = threadIdx.x; k <= nc; k += blockDim.x) cst[k] = start[ca + k] - base;
-      for (uint32_t q = threadIdx.x; q < len; q += blockDim.x) {
-        const uint32_t p = perm[base + q];
-        sv[q] = p;
-        sk[q] = key[p];
-      }
-      __syncthreads();
-      for (uint32_t i = threadIdx.x; i < len; i += blockDim.x) {
-        uint32_t lo = 0, hi = nc;                    // cst[lo] <= i < cst[hi]
-        while (hi - lo > 1) {
-          const uint32_t mid = (lo + hi) >> 1;
-          if (cst[mid] <= i) lo = mid;
-          else hi = mid;
-        }
-        const uint32_t b = cst[lo], e = cst[lo + 1];
-        const uint32_t ki = sk[i];
-        uint32_t rank = 0;
-        for (uint32_t j = b; j < e; ++j) {
-          const uint32_t kj = sk[j];
-          rank += (kj < ki || (kj == ki && j < i)) ? 1u : 0u;
-        }
-        perm[base + b + rank] = sv[i];
-      }
-    } else if (c >= ca && c < cb) {
-      const uint32_t b = start[c], e = start[c + 1];
-      for (uint32_t i = b + 1; i < e; ++i) {
-        const uint32_t p = perm[i];
-        const uint32_t kp = key[p];
-        uint32_t j = i;
-        while (j > b) {
-          const uint32_t q = perm[j - 1];
-          if (key[q] <= kp) break;
-          perm[j] = q;
-          --j;
-        }
-        perm[j] = p;
-      }
-    }
-    __syncthreads();                                 // LDS and s_next are reused
-    ca = cb;
+// The sorted order as arrays: perm, and for the nreal particles pid / bid, and
+// bindex (calcBlockID's outputs, cudaCutoffBlock.cu:233-258).  Bound by its
+// chain of dependent L2 reads (pair, cell start, keys of the cell) and 20 bytes
+// of traffic a particle: 16 us at 796,176 particles in 470,000 cells, where
+// ordering runs of 64 cells in LDS and a pass for the outputs took 19 + 6 us;
+// 4000 particles in 125 cells 11 us (with the rows, in k_reorder) against
+// 29 + 5, since two workgroups had all the cells.
+__global__ void k_cell_order(PbCellOrder O, uint32_t n, uint32_t *perm, uint32_t nreal,
+                             uint32_t ncell, uint32_t *pid, uint32_t *bid, uint32_t *bindex) {
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < ncell) {
+    const uint32_t b = O.start[i];
+    bindex[i] = O.start[i + 1] > b ? b : PB_NONE;
+  }
+  if (i == 0) bindex[ncell] = nreal;
+  if (i >= n) return;
+  uint32_t slot, cell;
+  const uint32_t k = pb_cell_position(O, i, &slot, &cell);
+  perm[k] = slot;
+  if (k < nreal) {
+    pid[k] = O.skey[i];
+    bid[k] = cell;
   }
 }
 
@@ -221,41 +205,45 @@ int pb_ensure_sort_ws(pb_sys *s, uint32_t ncell) {
   int rc;
   if (!s->cellid) {
     if ((rc = pb_alloc(s->ctx, &s->cellid, s->npad)) || (rc = pb_alloc(s->ctx, &s->rank, s->npad)) ||
-        (rc = pb_alloc(s->ctx, &s->perm, s->npad)))
+        (rc = pb_alloc(s->ctx, &s->perm, s->npad)) || (rc = pb_alloc(s->ctx, &s->skey, s->npad)) ||
+        (rc = pb_alloc(s->ctx, &s->sslot, s->npad)) || (rc = pb_alloc(s->ctx, &s->scell, s->npad)))
       return rc;
   }
   if (s->ncell_cap < ncell) {
+    s->ncell_cap = 0;
     if ((rc = pb_alloc(s->ctx, &s->ccount, (size_t)ncell + 1)) ||
         (rc = pb_alloc(s->ctx, &s->cstart, (size_t)ncell + 1)))
       return rc;
+    // the counters are zero between sorts (k_scatter clears them)
+    hipLaunchKernelGGL(k_fill_u32, dim3(pb_blocks((size_t)ncell + 1, 256)), dim3(256), 0,
+                       s->ctx->stream, s->ccount, ncell + 1, 0u);
+    PB_LAUNCH_CHECK(s->ctx, "sort workspace");
     s->ncell_cap = ncell;
   }
   return PB_OK;
 }
 
-int pb_counting_sort(pb_sys *s, uint32_t ncell, const uint32_t *key) {
-  if (int rc = pb_ensure_sort_ws(s, ncell)) return rc;
-  hipStream_t st = s->ctx->stream;
-  const uint32_t n = s->npad;
-  hipLaunchKernelGGL(k_fill_u32, dim3(pb_blocks(ncell + 1, 256)), dim3(256), 0, st, s->ccount,
-                     ncell + 1, 0u);
-  hipLaunchKernelGGL(k_count, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->cellid, n, s->ccount,
-                     s->rank);
-  PB_LAUNCH_CHECK(s->ctx, "k_count");
-  return pb_counting_sort_counted(s, ncell, key);
-}
-
-// the sort after the counting: s->ccount and s->rank filled (by k_count or
-// by a caller's kernel that computes the cell ids and counts in one pass)
-int pb_counting_sort_counted(pb_sys *s, uint32_t ncell, const uint32_t *key) {
+// the sort after the counting (s->ccount and s->rank filled by the caller's
+// cell-id kernel) up to the scattered (key, slot, cell)
+int pb_counting_sort(pb_sys *s, uint32_t ncell, const uint32_t *key, PbCellOrder *O) {
   s->lj_cont = false;             // the fused LJ run's cell order is gone
-  hipStream_t st = s->ctx->stream;
   const uint32_t n = s->npad;
   if (int rc = pb_exclusive_scan(s, s->ccount, s->cstart, ncell)) return rc;
-  hipLaunchKernelGGL(k_scatter, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->cellid, s->rank,
-                     s->cstart, n, s->perm);
-  hipLaunchKernelGGL(k_cell_sort, dim3(pb_blocks(ncell, CS_CELLS)), dim3(CS_THREADS), 0, st,
-                     s->cstart, ncell, key, s->perm);
+  hipLaunchKernelGGL(k_scatter, dim3(pb_blocks(n > ncell ? n : ncell, 256)), dim3(256), 0,
+                     s->ctx->stream, s->cellid, s->rank, s->cstart, key, n, s->skey, s->sslot,
+                     s->scell, s->ccount, ncell);
   PB_LAUNCH_CHECK(s->ctx, "pb_counting_sort");
+  O->start = s->cstart;
+  O->skey = s->skey;
+  O->sslot = s->sslot;
+  O->scell = s->scell;
+  return PB_OK;
+}
+
+int pb_cell_order(pb_sys *s, const PbCellOrder &O, uint32_t ncell) {
+  const uint32_t n = s->npad, m = n > ncell + 1 ? n : ncell + 1;
+  hipLaunchKernelGGL(k_cell_order, dim3(pb_blocks(m, 256)), dim3(256), 0, s->ctx->stream, O, n,
+                     s->perm, s->n, ncell, s->ref_pid, s->ref_bid, s->ref_bindex);
+  PB_LAUNCH_CHECK(s->ctx, "k_cell_order");
   return PB_OK;
 }
