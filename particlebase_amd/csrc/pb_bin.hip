@@ -207,54 +207,6 @@ extern "C" int pb_get_bins(pb_sys *s, uint32_t *pid, uint32_t *bid_sorted, uint3
   return PB_OK;
 }
 
-// ------------------------------------------------------- neighbour counts
-// calcCoordMD_F4 (kernelinline.hh:387-399) over the 27 cells of
-// calcF_IJpairWithBlock_F4 (kerneltemplate.hh:244-293); cells computed on
-// the fly with the wrap of calc_BlockNeighbor (periodic, nb >= 3).
-__global__ void k_coord_counts(const double4 *r, const uint32_t *perm, const uint32_t *cellid,
-                               const uint32_t *start, uint32_t nreal, RefGrid g, float cx,
-                               float cy, float cz, float rmax2t, int periodic, uint32_t *out) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= nreal) return;
-  const uint32_t si = perm[k];
-  const uint32_t c = cellid[si];
-  const uint32_t nyz = g.nb[1] * g.nb[2];
-  const int i0 = (int)(c / nyz), j0 = (int)((c / g.nb[2]) % g.nb[1]), k0 = (int)(c % g.nb[2]);
-  const double4 pi = r[si];
-  const float xi = (float)pi.x, yi = (float)pi.y, zi = (float)pi.z;
-  uint32_t cnt = 0;
-  for (int a = -1; a <= 1; ++a) {
-    int i2 = i0 + a;
-    if (i2 < 0 || i2 >= (int)g.nb[0]) {
-      if (!periodic) continue;
-      i2 = (i2 + (int)g.nb[0]) % (int)g.nb[0];
-    }
-    for (int b = -1; b <= 1; ++b) {
-      int j2 = j0 + b;
-      if (j2 < 0 || j2 >= (int)g.nb[1]) {
-        if (!periodic) continue;
-        j2 = (j2 + (int)g.nb[1]) % (int)g.nb[1];
-      }
-      for (int d = -1; d <= 1; ++d) {
-        int k2 = k0 + d;
-        if (k2 < 0 || k2 >= (int)g.nb[2]) {
-          if (!periodic) continue;
-          k2 = (k2 + (int)g.nb[2]) % (int)g.nb[2];
-        }
-        const uint32_t J = (uint32_t)k2 + (uint32_t)j2 * g.nb[2] + (uint32_t)i2 * nyz;
-        for (uint32_t jj = start[J]; jj < start[J + 1]; ++jj) {
-          const uint32_t sj = perm[jj];
-          if (sj == si) continue;
-          const double4 pj = r[sj];
-          const float R2 = distance2p(xi, yi, zi, (float)pj.x, (float)pj.y, (float)pj.z, cx, cy, cz);
-          if (R2 < rmax2t) ++cnt;
-        }
-      }
-    }
-  }
-  out[si] = cnt;
-}
-
 static void half_cell2(const pb_sys *s, uint32_t q, float c[3]) {
   // cudaFrame::setCell, cudaFrame.cu:85-91, on the FP32 cell values
   for (int a = 0; a < 3; ++a) {
@@ -262,30 +214,6 @@ static void half_cell2(const pb_sys *s, uint32_t q, float c[3]) {
     c[a] = (hi - lo) / 2;
     c[a] *= c[a];
   }
-}
-
-extern "C" int pb_coord_counts(pb_sys *s, float rmax2t, uint32_t *counts) {
-  if (!s || !counts) return PB_ERR_ARG;
-  if (!s->ref_cells || s->ref_single)
-    return pb_fail(s->ctx, PB_ERR_STATE, "pb_coord_counts: needs a 27-neighbour cell grid");
-  float rc = sqrtf(rmax2t);
-  for (int a = 0; a < 3; ++a)
-    if (s->blocklen[a] < rc)
-      return pb_fail(s->ctx, PB_ERR_CELLS, "pb_coord_counts: cell length below the count radius");
-  if (int rc2 = pb_bin(s)) return rc2;
-  float c[3];
-  half_cell2(s, 0, c);
-  uint32_t *dcnt = nullptr;
-  if (int rc2 = pb_alloc(s->ctx, &dcnt, s->npad)) return rc2;
-  hipStream_t st = s->ctx->stream;
-  hipLaunchKernelGGL(k_coord_counts, dim3(pb_blocks(s->n, 256)), dim3(256), 0, st, s->r, s->perm,
-                     s->cellid, s->cstart, s->n, ref_grid(s), c[0], c[1], c[2], rmax2t,
-                     s->ref_periodic, dcnt);
-  int e = PB_OK;
-  if (hipError_t he = hipGetLastError()) e = pb_hip_check(s->ctx, he, "pb_coord_counts");
-  if (e == PB_OK) e = pb_io_gather_u32(s, dcnt, counts);
-  pb_free(dcnt);
-  return e;
 }
 
 // ------------------------------------------------------------------ g(r)
@@ -686,53 +614,135 @@ __device__ __forceinline__ void for_27_cells(const RefGrid &g, uint32_t c, int p
 }
 
 struct NlistArgs {
-  const double4 *r;
-  const uint32_t *perm, *cellid, *start, *orig;
+  const float4 *pos;           // cell order: FP32 position, original index
+  const uint32_t *bid, *start; // cell of a sorted position, first position of a cell
   uint32_t nreal;
   RefGrid g;
+  float L[3];                  // FP32 box edges
   float cx, cy, cz, rmax2t;
   int periodic;
+  uint32_t cap;                // capacity of the column array
 };
 
-__global__ void k_nlist_count(NlistArgs A, uint32_t *rowcnt) {
+__global__ void k_md_gather(const double4 *r, const uint32_t *perm, const uint32_t *pid,
+                            uint32_t n, float4 *pos) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= A.nreal) return;
-  const uint32_t si = A.perm[k];
-  const double4 pi = A.r[si];
-  const float xi = (float)pi.x, yi = (float)pi.y, zi = (float)pi.z;
-  uint32_t cnt = 0;
-  for_27_cells(A.g, A.cellid[si], A.periodic, A.start, A.perm, [&](uint32_t sj) {
-    if (sj == si) return;
-    const double4 pj = A.r[sj];
-    if (distance2p(xi, yi, zi, (float)pj.x, (float)pj.y, (float)pj.z, A.cx, A.cy, A.cz) < A.rmax2t)
-      ++cnt;
-  });
-  rowcnt[A.orig[si]] = cnt;
+  if (k >= n) return;
+  const double4 p = r[perm[k]];
+  pos[k] = make_float4((float)p.x, (float)p.y, (float)p.z, __uint_as_float(pid[k]));
 }
 
-__global__ void k_nlist_fill(NlistArgs A, const uint32_t *rowptr, uint32_t *col) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+// Rows of the list: one wavefront a particle, 64 candidates of the 27 cells
+// at a time (a column of three cells is one contiguous run of the cell order,
+// two where it wraps in z), so a row's candidates are coalesced reads and
+// 32,000 particles are 32,000 wavefronts.  The reference's FP32 distance2p
+// decides; it is evaluated only where the distance from folded axes lies
+// within the rounding bound of rmax2t (the bound of k_gr: 64 u (cx + cy + cz)
+// for |d| <= 1.25 L), a few lanes in a hundred thousand.
+//   FILL = false: the row's length.
+//   FILL = true: the row's original indices, ascending: the hits are compacted
+// into LDS and every hit counts the smaller ones.  Rows longer than the LDS
+// row are written as found and sorted in place by one lane.
+// 32,000 particles of a liquid (about 80 a row): 316 + 1079 us a build with a
+// thread a row and an insertion sort in global memory, 48 + 69 us now.
+#define NL_CAP 512u
+template <bool FILL>
+__global__ void __launch_bounds__(256) k_nlist(NlistArgs A, uint32_t *rowcnt, const uint32_t *rowptr,
+                                               uint32_t *col) {
+  __shared__ __align__(16) uint32_t rows[FILL ? 4 : 1][FILL ? NL_CAP : 1];
+  const uint32_t lane = pb_lane(), wave = threadIdx.x / 64;
+  const uint32_t k = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + wave);
   if (k >= A.nreal) return;
-  const uint32_t si = A.perm[k];
-  const double4 pi = A.r[si];
-  const float xi = (float)pi.x, yi = (float)pi.y, zi = (float)pi.z;
-  const uint32_t b = rowptr[A.orig[si]];
-  uint32_t e = b;
-  for_27_cells(A.g, A.cellid[si], A.periodic, A.start, A.perm, [&](uint32_t sj) {
-    if (sj == si) return;
-    const double4 pj = A.r[sj];
-    if (distance2p(xi, yi, zi, (float)pj.x, (float)pj.y, (float)pj.z, A.cx, A.cy, A.cz) < A.rmax2t)
-      col[e++] = A.orig[sj];
-  });
-  // ascending columns (insertion sort of the row)
-  for (uint32_t i = b + 1; i < e; ++i) {
-    const uint32_t x = col[i];
-    uint32_t j = i;
-    while (j > b && col[j - 1] > x) {
-      col[j] = col[j - 1];
-      --j;
+  const float4 pi = A.pos[k];
+  const uint32_t oi = __float_as_uint(pi.w), c = A.bid[k];
+  uint32_t b = 0, len = 0;
+  if (FILL) {
+    b = rowptr[oi];
+    len = rowptr[oi + 1] - b;
+    if (b + len > A.cap || len == 0) return;          // outgrown: filled again, larger
+  }
+  const float E = 64.0f * 5.9604645e-8f * 1.0001f * (A.cx + A.cy + A.cz);
+  const float lim = A.rmax2t + E, sure = A.rmax2t - E;
+  const float fx = 1.25f * A.L[0], fy = 1.25f * A.L[1], fz = 1.25f * A.L[2];
+  const int nb0 = (int)A.g.nb[0], nb1 = (int)A.g.nb[1], nb2 = (int)A.g.nb[2];
+  const int i0 = (int)(c / (A.g.nb[1] * A.g.nb[2])), j0 = (int)((c / A.g.nb[2]) % A.g.nb[1]),
+            k0 = (int)(c % A.g.nb[2]);
+  uint32_t cnt = 0;
+  auto run = [&](uint32_t q0, uint32_t q1) {          // wave-uniform
+    for (uint32_t q = q0; q < q1; q += 64u) {
+      const uint32_t j = q + lane;
+      bool hit = false;
+      uint32_t oj = 0;
+      if (j < q1 && j != k) {
+        const float4 pj = A.pos[j];
+        oj = __float_as_uint(pj.w);
+        const float dx = fabsf(pi.x - pj.x), dy = fabsf(pi.y - pj.y), dz = fabsf(pi.z - pj.z);
+        const float ax = fminf(dx, fabsf(dx - A.L[0])), ay = fminf(dy, fabsf(dy - A.L[1])),
+                    az = fminf(dz, fabsf(dz - A.L[2]));
+        const float R2 = fmaf(az, az, fmaf(ay, ay, ax * ax));
+        const bool bound = dx <= fx && dy <= fy && dz <= fz;
+        hit = R2 < sure;
+        if (!bound || !(hit || R2 >= lim))
+          hit = distance2p(pi.x, pi.y, pi.z, pj.x, pj.y, pj.z, A.cx, A.cy, A.cz) < A.rmax2t;
+      }
+      const uint64_t m = __ballot(hit);
+      if (FILL && hit) {
+        const uint32_t p = cnt + __builtin_amdgcn_mbcnt_hi(
+                                     (uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (len > NL_CAP) col[b + p] = oj;
+        else rows[wave][p] = oj;
+      }
+      cnt += (uint32_t)__popcll(m);
     }
-    col[j] = x;
+  };
+  for (int a = -1; a <= 1; ++a) {
+    int i2 = i0 + a;
+    if (i2 < 0 || i2 >= nb0) {
+      if (!A.periodic) continue;
+      i2 = i2 < 0 ? nb0 - 1 : 0;
+    }
+    for (int d = -1; d <= 1; ++d) {
+      int j2 = j0 + d;
+      if (j2 < 0 || j2 >= nb1) {
+        if (!A.periodic) continue;
+        j2 = j2 < 0 ? nb1 - 1 : 0;
+      }
+      const uint32_t cb = ((uint32_t)i2 * A.g.nb[1] + (uint32_t)j2) * A.g.nb[2];
+      const int lo = k0 > 0 ? k0 - 1 : 0, hi = k0 + 1 < nb2 ? k0 + 1 : nb2 - 1;
+      run(A.start[cb + (uint32_t)lo], A.start[cb + (uint32_t)hi + 1u]);
+      if (A.periodic && k0 == 0) run(A.start[cb + (uint32_t)nb2 - 1u], A.start[cb + (uint32_t)nb2]);
+      if (A.periodic && k0 == nb2 - 1) run(A.start[cb], A.start[cb + 1u]);
+    }
+  }
+  if (!FILL) {
+    if (lane == 0) rowcnt[oi] = cnt;
+    return;
+  }
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "workgroup");
+  __builtin_amdgcn_wave_barrier();
+  if (len <= NL_CAP) {
+    const uint32_t *row = rows[wave];
+    for (uint32_t base = 0; base < len; base += 64u) {
+      const uint32_t i = base + lane;
+      const uint32_t x = i < len ? row[i] : 0u;
+      uint32_t rank = 0, j = 0;
+      for (; j + 4 <= len; j += 4) {
+        const uint4 y = *reinterpret_cast<const uint4 *>(row + j);
+        rank += (y.x < x ? 1u : 0u) + (y.y < x ? 1u : 0u) + (y.z < x ? 1u : 0u) + (y.w < x ? 1u : 0u);
+      }
+      for (; j < len; ++j) rank += row[j] < x ? 1u : 0u;
+      if (i < len) col[b + rank] = x;
+    }
+  } else if (lane == 0) {
+    for (uint32_t i = b + 1; i < b + len; ++i) {
+      const uint32_t x = col[i];
+      uint32_t j = i;
+      while (j > b && col[j - 1] > x) {
+        col[j] = col[j - 1];
+        --j;
+      }
+      col[j] = x;
+    }
   }
 }
 
@@ -764,16 +774,33 @@ struct PairArgs {
   double *partials;
 };
 
-// LJ forces, PE and virial from the CSR list (pairs with r^2 < rc2)
-__global__ void k_lj_force_nlist(PairArgs A) {
-  const uint32_t si = blockIdx.x * blockDim.x + threadIdx.x;
+// LJ forces, PE and virial from the CSR list (pairs with r^2 < rc2): eight
+// lanes a row, each taking every eighth column, so a row's columns are read
+// together and a lane waits for ten dependent gathers (column, slot, position)
+// instead of eighty.  Bound by that latency: 32,000 rows of about 80 are 4000
+// wavefronts; a thread a row (500 wavefronts) took 79 us, this 20 us.
+// Partials per 64 slots, added in a fixed order.
+#define NF_LANES 8u
+__global__ void __launch_bounds__(64 * NF_LANES) k_lj_force_nlist(PairArgs A) {
+  __shared__ double tab[4][PB_MAXT * PB_MAXT];
+  __shared__ double sums[2][NF_LANES];
+  for (uint32_t t = threadIdx.x; t < PB_MAXT * PB_MAXT; t += blockDim.x) {
+    tab[0][t] = A.lj->s2[t];
+    tab[1][t] = A.lj->e24[t];
+    tab[2][t] = A.lj->e4[t];
+    tab[3][t] = A.lj->shift[t];
+  }
+  __syncthreads();
+  const uint32_t si = blockIdx.x * 64u + threadIdx.x / NF_LANES, sub = threadIdx.x % NF_LANES;
   double pe = 0.0, vir = 0.0;
-  if (si < A.npad && A.orig[si] != PB_NONE) {
-    const uint32_t row = A.orig[si];
+  const uint32_t row = si < A.npad ? A.orig[si] : PB_NONE;
+  if (row != PB_NONE) {
     const double4 pi = A.r[si];
     const uint32_t ti = (uint32_t)pi.w;
     double fx = 0.0, fy = 0.0, fz = 0.0;
-    for (uint32_t k = A.rowptr[row]; k < A.rowptr[row + 1]; ++k) {
+    const uint32_t e = A.rowptr[row + 1];
+#pragma unroll 2
+    for (uint32_t k = A.rowptr[row] + sub; k < e; k += NF_LANES) {
       const double4 pj = A.r[A.inv[A.col[k]]];
       const double dx = min_image(pi.x - pj.x, A.L[0], A.periodic);
       const double dy = min_image(pi.y - pj.y, A.L[1], A.periodic);
@@ -781,22 +808,34 @@ __global__ void k_lj_force_nlist(PairArgs A) {
       const double r2 = dx * dx + dy * dy + dz * dz;
       if (!(r2 < A.rc2)) continue;
       const uint32_t t = ti * PB_MAXT + (uint32_t)pj.w;
-      double s6 = A.lj->s2[t] / r2;
+      double s6 = tab[0][t] / r2;
       s6 = s6 * s6 * s6;
-      const double fr = A.lj->e24[t] * s6 * (2.0 * s6 - 1.0) / r2;
+      const double fr = tab[1][t] * s6 * (2.0 * s6 - 1.0) / r2;
       fx += fr * dx;
       fy += fr * dy;
       fz += fr * dz;
-      pe += 0.5 * (A.lj->e4[t] * s6 * (s6 - 1.0) - A.lj->shift[t]);
+      pe += 0.5 * (tab[2][t] * s6 * (s6 - 1.0) - tab[3][t]);
       vir += 0.5 * fr * r2;
     }
-    A.F[si] = make_double4(fx, fy, fz, 0.0);
+#pragma unroll
+    for (uint32_t o = 1; o < NF_LANES; o <<= 1) {      // a row's lanes take this branch together
+      fx += __shfl_xor(fx, (int)o, 64);
+      fy += __shfl_xor(fy, (int)o, 64);
+      fz += __shfl_xor(fz, (int)o, 64);
+    }
+    if (sub == 0) A.F[si] = make_double4(fx, fy, fz, 0.0);
   }
   pe = pb_wave_sum(pe);
   vir = pb_wave_sum(vir);
-  if (pb_lane() == 0 && si < A.npad) {
-    A.partials[4 * (si / PB_WAVE) + 0] = pe;
-    A.partials[4 * (si / PB_WAVE) + 1] = vir;
+  if (pb_lane() == 0) {
+    sums[0][threadIdx.x / 64] = pe;
+    sums[1][threadIdx.x / 64] = vir;
+  }
+  __syncthreads();
+  if (threadIdx.x < 2) {
+    double t = 0.0;
+    for (uint32_t w = 0; w < NF_LANES; ++w) t += sums[threadIdx.x][w];
+    A.partials[4 * (size_t)blockIdx.x + threadIdx.x] = t;
   }
 }
 
@@ -835,13 +874,19 @@ static int need_binned_grid(pb_sys *s, const char *who) {
   return PB_OK;
 }
 
-static NlistArgs nlist_args(pb_sys *s, float rmax2t) {
-  NlistArgs A;
-  A.r = s->r;
-  A.perm = s->perm;
-  A.cellid = s->cellid;
+// the 27-cell search's arguments, on the positions gathered into cell order
+static int nlist_args(pb_sys *s, float rmax2t, NlistArgs *out) {
+  int rc;
+  if (!s->md_pos &&
+      ((rc = pb_alloc(s->ctx, &s->md_pos, s->npad)) || (rc = pb_alloc(s->ctx, &s->md_cnt, (size_t)s->n + 1))))
+    return rc;
+  hipLaunchKernelGGL(k_md_gather, dim3(pb_blocks(s->n, 256)), dim3(256), 0, s->ctx->stream, s->r,
+                     s->perm, s->ref_pid, s->n, s->md_pos);
+  PB_LAUNCH_CHECK(s->ctx, "k_md_gather");
+  NlistArgs &A = *out;
+  A.pos = s->md_pos;
+  A.bid = s->ref_bid;
   A.start = s->cstart;
-  A.orig = s->orig;
   A.nreal = s->n;
   A.g = ref_grid(s);
   float c[3];
@@ -849,9 +894,30 @@ static NlistArgs nlist_args(pb_sys *s, float rmax2t) {
   A.cx = c[0];
   A.cy = c[1];
   A.cz = c[2];
+  for (int a = 0; a < 3; ++a) A.L[a] = (float)s->cells[2 * a + 1] - (float)s->cells[2 * a];
   A.rmax2t = rmax2t;
   A.periodic = s->ref_periodic;
-  return A;
+  A.cap = 0;
+  return PB_OK;
+}
+
+// calcCoordMD_F4 counts (kernelinline.hh:387-399) over the 27 cells of
+// calcF_IJpairWithBlock_F4 (kerneltemplate.hh:244-293): the rows' lengths
+extern "C" int pb_coord_counts(pb_sys *s, float rmax2t, uint32_t *counts) {
+  if (!s || !counts) return PB_ERR_ARG;
+  if (!s->ref_cells || s->ref_single)
+    return pb_fail(s->ctx, PB_ERR_STATE, "pb_coord_counts: needs a 27-neighbour cell grid");
+  const float rc = sqrtf(rmax2t);
+  for (int a = 0; a < 3; ++a)
+    if (s->blocklen[a] < rc)
+      return pb_fail(s->ctx, PB_ERR_CELLS, "pb_coord_counts: cell length below the count radius");
+  if (int e = pb_bin(s)) return e;
+  NlistArgs A;
+  if (int e = nlist_args(s, rmax2t, &A)) return e;
+  hipLaunchKernelGGL(k_nlist<false>, dim3(pb_blocks(s->n, 4)), dim3(256), 0, s->ctx->stream, A,
+                     s->md_cnt, (const uint32_t *)nullptr, (uint32_t *)nullptr);
+  PB_LAUNCH_CHECK(s->ctx, "k_nlist (counts)");
+  return pb_io_download(s->ctx, counts, s->md_cnt, 4 * (size_t)s->n);
 }
 
 extern "C" int pb_nlist_build(pb_sys *s, float rmax2t, uint32_t *nnz_out) {
@@ -865,27 +931,36 @@ extern "C" int pb_nlist_build(pb_sys *s, float rmax2t, uint32_t *nnz_out) {
   const uint32_t n = s->n;
   int rc2;
   if (!s->md_row && (rc2 = pb_alloc(s->ctx, &s->md_row, (size_t)n + 1))) return rc2;
-  uint32_t *cnt = nullptr;
-  if ((rc2 = pb_alloc(s->ctx, &cnt, (size_t)n + 1))) return rc2;
-  const NlistArgs A = nlist_args(s, rmax2t);
-  hipLaunchKernelGGL(k_nlist_count, dim3(pb_blocks(n, 256)), dim3(256), 0, st, A, cnt);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) {
-    pb_free(cnt);
-    return pb_hip_check(s->ctx, e, "k_nlist_count");
-  }
-  rc2 = pb_exclusive_scan(s, cnt, s->md_row, n);
-  pb_free(cnt);
-  if (rc2) return rc2;
-  uint32_t nnz = 0;
-  PB_HIP(s->ctx, hipMemcpyAsync(&nnz, s->md_row + n, 4, hipMemcpyDeviceToHost, st));
+  if ((rc2 = pb_results(s->ctx))) return rc2;
+  NlistArgs A;
+  if ((rc2 = nlist_args(s, rmax2t, &A))) return rc2;
+  s->md_valid = false;                        // until the rows are whole
+  hipLaunchKernelGGL(k_nlist<false>, dim3(pb_blocks(n, 4)), dim3(256), 0, st, A, s->md_cnt,
+                     (const uint32_t *)nullptr, (uint32_t *)nullptr);
+  PB_LAUNCH_CHECK(s->ctx, "k_nlist (counts)");
+  if ((rc2 = pb_exclusive_scan(s, s->md_cnt, s->md_row, n))) return rc2;
+  // the rows are filled before the host knows their sum, up to the capacity
+  // of the last list; a list that outgrew it is filled again
+  auto fill = [&]() -> int {
+    A.cap = s->md_cap;
+    if (!A.cap) return PB_OK;
+    hipLaunchKernelGGL(k_nlist<true>, dim3(pb_blocks(n, 4)), dim3(256), 0, st, A, s->md_cnt, s->md_row,
+                       s->md_col);
+    PB_LAUNCH_CHECK(s->ctx, "k_nlist (rows)");
+    return PB_OK;
+  };
+  if ((rc2 = fill())) return rc2;
+  PB_HIP(s->ctx, hipMemcpyAsync(s->ctx->res, s->md_row + n, 4, hipMemcpyDeviceToHost, st));
   PB_HIP(s->ctx, hipStreamSynchronize(st));
+  uint32_t nnz;
+  std::memcpy(&nnz, s->ctx->res, 4);
   if (s->md_cap < nnz || !s->md_col) {
-    if ((rc2 = pb_alloc(s->ctx, &s->md_col, (size_t)nnz + 1))) return rc2;
-    s->md_cap = nnz;
+    const uint32_t cap = (uint32_t)std::min<uint64_t>((uint64_t)nnz + nnz / 16 + 64, 0xFFFFFFF0ull);
+    s->md_cap = 0;
+    if ((rc2 = pb_alloc(s->ctx, &s->md_col, cap))) return rc2;
+    s->md_cap = cap;
+    if ((rc2 = fill())) return rc2;
   }
-  hipLaunchKernelGGL(k_nlist_fill, dim3(pb_blocks(n, 256)), dim3(256), 0, st, A, s->md_row, s->md_col);
-  PB_LAUNCH_CHECK(s->ctx, "k_nlist_fill");
   s->md_nnz = nnz;
   s->md_valid = true;
   if (nnz_out) *nnz_out = nnz;
@@ -935,20 +1010,21 @@ extern "C" int pb_lj_force_nlist(pb_sys *s, double *pe, double *virial) {
   hipStream_t st = s->ctx->stream;
   int rc;
   if (!s->md_inv && (rc = pb_alloc(s->ctx, &s->md_inv, (size_t)s->n))) return rc;
-  hipLaunchKernelGGL(k_inverse_perm, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->orig,
-                     s->npad, s->md_inv);
+  if (s->md_inv_order != s->order_gen) {
+    hipLaunchKernelGGL(k_inverse_perm, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->orig,
+                       s->npad, s->md_inv);
+    s->md_inv_order = s->order_gen;
+  }
   PairArgs A = pair_args(s);
   A.inv = s->md_inv;
   A.rowptr = s->md_row;
   A.col = s->md_col;
   A.periodic = 1;       // MD boxes are periodic (MDpairForce folds every pair)
-  hipLaunchKernelGGL(k_lj_force_nlist, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, A);
+  hipLaunchKernelGGL(k_lj_force_nlist, dim3(s->nwave), dim3(64 * NF_LANES), 0, st, A);
   PB_LAUNCH_CHECK(s->ctx, "k_lj_force_nlist");
   if (pe || virial) {
-    if ((rc = pb_reduce_waves(s, 2))) return rc;
-    double h[8];
-    PB_HIP(s->ctx, hipMemcpyAsync(h, s->d_out, sizeof(h), hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
+    const double *h = nullptr;
+    if ((rc = pb_reduce_to_host(s, 2, &h))) return rc;
     if (pe) *pe = h[0];
     if (virial) *virial = h[1];
   }

@@ -43,6 +43,8 @@ struct LJTable {
       shiftf[PB_MAXT * PB_MAXT];
 };
 
+#define PB_RES_DOUBLES 16384u
+
 struct pb_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -51,6 +53,10 @@ struct pb_ctx {
   // per slot
   uint8_t *io_stage = nullptr, *io_dev = nullptr;
   hipEvent_t io_ev[2] = {};
+  // small results that kernels write to the host themselves: PB_RES_DOUBLES
+  // doubles of pinned memory and their device address (pb_results); read
+  // after the stream's synchronisation that every such call ends with
+  double *res = nullptr, *res_dev = nullptr;
   // device address of pb_bin.hip's static g(r) scratch array on this
   // context's device (pb_gr_hist_noalloc); set when the context is created
   void *gr_scratch = nullptr;
@@ -84,11 +90,13 @@ struct pb_sys {
   uint8_t *move = nullptr;
   uint16_t *type = nullptr;
   uint32_t *orig = nullptr;       // storage slot -> original index (PB_NONE: pad)
+  uint32_t order_gen = 1;         // advanced whenever orig is permuted
   uint32_t *waveRep = nullptr;    // wave -> replica
   RepInfo *d_reps = nullptr;
   double *partials = nullptr;     // per-wave partial sums, 4 per wave
   uint32_t *d_counter = nullptr;  // last-block counters / flags (16 words)
   double *d_out = nullptr;        // small reduction outputs (16 per replica)
+  std::vector<double> h_out;      // host copy of them where they exceed the context's results
   uint8_t *io = nullptr;          // a packed field in the caller's order (24 B a particle, lazy)
 
   // reference cell grid (pb_setup_cells), single replica
@@ -163,7 +171,10 @@ struct pb_sys {
 
   // MD neighbour list (cudaParticleMD::makeNList): CSR by original index
   uint32_t *md_row = nullptr, *md_col = nullptr, *md_inv = nullptr;
+  uint32_t *md_cnt = nullptr;      // row lengths
+  float4 *md_pos = nullptr;        // cell order: FP32 position, original index
   uint32_t md_cap = 0, md_nnz = 0;
+  uint32_t md_inv_order = 0;       // order_gen md_inv was made for (0: none)
   bool md_valid = false;
 
   // g(r)
@@ -255,16 +266,20 @@ int pb_counting_sort(pb_sys *sys, uint32_t ncell, const uint32_t *key, PbCellOrd
 // calcBlockID's outputs of the reference cell grid
 int pb_cell_order(pb_sys *sys, const PbCellOrder &O, uint32_t ncell);
 // per-replica reduction of K per-wave partial components into out[rep*8+c]
-int pb_reduce_waves(pb_sys *sys, int K);
+// (device memory, or the context's small results)
+int pb_reduce_waves(pb_sys *sys, int K, double *out);
+// the same, waited for, into host[rep*8+c]
+int pb_reduce_to_host(pb_sys *sys, int K, const double **host);
 // host boundary (pb_io.hip): copies through the context's pinned ring (an
 // upload is stream ordered, a download waits); the packed-field device
 // buffer; a scalar per particle from the caller's order into storage order
-// (squared if asked; padding 0) and a uint32 per slot to the caller's order
+// (squared if asked; padding 0)
 int pb_io_upload(pb_ctx *ctx, void *dev, const void *host, size_t bytes);
 int pb_io_download(pb_ctx *ctx, void *host, const void *dev, size_t bytes);
 int pb_io_buffer(pb_sys *sys);
 int pb_io_scatter(pb_sys *sys, const double *host, double *dst, bool square);
-int pb_io_gather_u32(pb_sys *sys, const uint32_t *src, uint32_t *host);
+// the context's small-result memory, allocated on first use
+int pb_results(pb_ctx *ctx);
 void pb_io_release(pb_ctx *ctx);
 // rotation / radius state, allocated on first use
 int pb_ensure_rotation(pb_sys *sys);

@@ -39,7 +39,19 @@ static int ensure_stage(pb_ctx *ctx) {
   return PB_OK;
 }
 
+int pb_results(pb_ctx *ctx) {
+  if (ctx->res_dev) return PB_OK;
+  if (!ctx->res)
+    PB_HIP(ctx, hipHostMalloc((void **)&ctx->res, sizeof(double) * PB_RES_DOUBLES, hipHostMallocMapped));
+  void *d = nullptr;
+  PB_HIP(ctx, hipHostGetDevicePointer(&d, ctx->res, 0));
+  ctx->res_dev = (double *)d;
+  return PB_OK;
+}
+
 void pb_io_release(pb_ctx *ctx) {
+  if (ctx->res) (void)hipHostFree(ctx->res);
+  ctx->res = ctx->res_dev = nullptr;
   if (ctx->io_stage) (void)hipHostFree(ctx->io_stage);
   ctx->io_stage = ctx->io_dev = nullptr;
   for (hipEvent_t &e : ctx->io_ev) {
@@ -211,12 +223,6 @@ int pb_io_scatter(pb_sys *s, const double *host, double *dst, bool square) {
   else hipLaunchKernelGGL(k_pack1<double>, IO_GRID(s), in, s->orig, s->npad, dst);
   PB_LAUNCH_CHECK(s->ctx, "pb_io_scatter");
   return PB_OK;
-}
-
-int pb_io_gather_u32(pb_sys *s, const uint32_t *src, uint32_t *host) {
-  return download_packed(s, host, 4 * (size_t)s->n, [&](void *d) {
-    hipLaunchKernelGGL(k_unpack1<uint32_t>, IO_GRID(s), src, s->orig, s->npad, (uint32_t *)d);
-  });
 }
 
 extern "C" int pb_sys_import(pb_sys *s, const double *r, const double *v, const double *a,

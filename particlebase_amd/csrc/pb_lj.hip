@@ -1373,6 +1373,7 @@ static int rebuild(pb_sys *s, bool carry_a) {
   std::swap(s->v, s->v2buf);
   if (carry_a) std::swap(s->a, s->a2buf);
   std::swap(s->orig, s->orig2);
+  ++s->order_gen;
   std::swap(s->type, s->type2);
   std::swap(s->move, s->move2);
   hipLaunchKernelGGL(k_build_list, dim3(s->list_nsegs), dim3(TB), 0, st, s->r, s->cstart,
@@ -1977,6 +1978,7 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
         std::swap(s->r, s->r2buf);          // the rebuild's reorder (Fold is not carried)
         std::swap(s->v, s->v2buf);
         std::swap(s->orig, s->orig2);
+        ++s->order_gen;
         std::swap(s->type, s->type2);
         std::swap(s->move, s->move2);
         rebuilds += 1;
@@ -2193,6 +2195,7 @@ out:
     s->tile_w = w0;
     s->tile_fill = f0;
   }
+  ++s->order_gen;                 // orig was restored
   s->lj_cont = false;             // the restored state has no list of its own
   (void)hipStreamSynchronize(st);
   pb_free(sr); pb_free(sv); pb_free(sa); pb_free(sf); pb_free(so); pb_free(sty); pb_free(smv);

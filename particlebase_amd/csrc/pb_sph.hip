@@ -568,11 +568,8 @@ extern "C" int pb_sph_inspect_density(pb_sys *s, double *mean_num) {
   hipLaunchKernelGGL(k_sph_inspect, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, s->ctx->stream,
                      s->sph_num, s->move, s->orig, s->npad, s->partials);
   PB_LAUNCH_CHECK(s->ctx, "k_sph_inspect");
-  if (int rc = pb_reduce_waves(s, 2)) return rc;
-  double h[2];
-  PB_HIP(s->ctx, hipMemcpyAsync(h, s->d_out, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                                s->ctx->stream));
-  PB_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
+  const double *h = nullptr;
+  if (int rc = pb_reduce_to_host(s, 2, &h)) return rc;
   *mean_num = h[0] / h[1];     // 0/0 (no movable particle) is NaN, as the reference divides
   return PB_OK;
 }
