@@ -156,6 +156,7 @@ extern "C" int pb_sys_create(pb_ctx *ctx, uint32_t nrep, const uint32_t *counts,
     pb_sys_destroy(s);
     return rc;
   }
+  s->partials_cap = s->nwave;
   std::vector<uint32_t> wr(s->nwave);
   for (uint32_t q = 0; q < nrep; ++q)
     for (uint32_t k = 0; k < s->reps[q].nwave; ++k) wr[s->reps[q].wave0 + k] = q;
@@ -210,7 +211,7 @@ extern "C" void pb_sys_destroy(pb_sys *s) {
     pb_free(s->cm_row[b]); pb_free(s->cm_col[b]); pb_free(s->cm_val[b]);
   }
   pb_free(s->gr_hist);
-  pb_free(s->list_segs); pb_free(s->list_wtab);
+  pb_free(s->list_segs); pb_free(s->list_wtab); pb_free(s->lj_ebuf);
   if (s->hmon) (void)hipHostFree(s->hmon);
   if (s->ctx) --s->ctx->nsys;
   delete s;
@@ -241,6 +242,7 @@ extern "C" int pb_sys_set_cell(pb_sys *s, const double *cells) {
   std::memcpy(s->cells.data(), cells, sizeof(double) * 6 * s->nrep);
   s->cell_set = true;
   s->lj_cont = false;             // the fused LJ run's list cells follow the box
+  s->plan_lanes = 0;
   return upload_reps(s);
 }
 

@@ -140,6 +140,14 @@ struct pb_sys {
   uint32_t list_nsegs = 0;
   uint4 *list_wtab = nullptr;      // per-segment window tables (cell order of the last sort)
   uint32_t list_wtab_cap = 0;      // segments list_wtab holds
+  uint32_t list_segs_cap = 0;      // segments list_segs holds
+  uint32_t partials_cap = 0;       // records `partials` holds
+  // what the list cells and segments were laid out for (plan_lanes 0: none)
+  uint32_t plan_lanes = 0, plan_tile_w = 0;
+  double plan_rc = 0, plan_fill = 0;
+  std::vector<double> plan_skins;
+  double *lj_ebuf = nullptr;       // energy records
+  size_t lj_ebuf_cap = 0;
   uint32_t tile_w = 2;             // list-cell columns per tile side (1 or 2)
   double tile_fill = 0.72;         // target fill of the LDS window stage
   // Continuation of the fused LJ run: the cell order, Verlet list and list
@@ -315,27 +323,24 @@ __device__ __forceinline__ uint32_t pb_count_rank(uint32_t c, bool valid, uint32
 }
 
 // Sorted position of the pair at i: its cell's start plus the number of
-// smaller keys in the cell (equal keys, which only padding has, by slot).
+// smaller keys in the cell.  Equal keys, which only the padding slots of a
+// replica have, keep the order they stand in: their rows are all alike.
 // Lanes of a wavefront share cells, so the reads are mostly broadcast L1 hits;
 // eight are in flight at a time.
 __device__ __forceinline__ uint32_t pb_cell_position(const PbCellOrder &O, uint32_t i,
                                                      uint32_t *slot, uint32_t *cell) {
-  const uint32_t s = O.sslot[i], k = O.skey[i], c = O.scell[i];
+  const uint32_t k = O.skey[i], c = O.scell[i];
   const uint32_t b = O.start[c], e = O.start[c + 1];
-  uint32_t rank = 0, same = 0;
+  uint32_t rank = 0;
   for (uint32_t j = b; j < e; j += 8) {
     uint32_t q[8];
 #pragma unroll
     for (uint32_t u = 0; u < 8; ++u) q[u] = O.skey[min(j + u, e - 1u)];
 #pragma unroll
-    for (uint32_t u = 0; u < 8; ++u) {
-      rank += (j + u < e && q[u] < k) ? 1u : 0u;
-      same += (j + u < e && q[u] == k) ? 1u : 0u;
-    }
+    for (uint32_t u = 0; u < 8; ++u)
+      rank += (j + u < e && (q[u] < k || (q[u] == k && j + u < i))) ? 1u : 0u;
   }
-  if (same > 1)
-    for (uint32_t j = b; j < e; ++j) rank += (O.skey[j] == k && O.sslot[j] < s) ? 1u : 0u;
-  *slot = s;
+  *slot = O.sslot[i];
   *cell = c;
   return b + rank;
 }

@@ -136,7 +136,8 @@ struct ReorderArgs {
   uint32_t *nn;
   const uint32_t *waveRep;
   const RepInfo *reps;
-  uint32_t *counter;           // displacement / speed maxima, cleared
+  uint32_t *counter;           // words [clear0, clear1) are cleared
+  uint32_t clear0, clear1;
   uint32_t n;
 };
 
@@ -145,7 +146,7 @@ struct ReorderArgs {
 // writes a permutation for this one to read: 1M atoms 34 + 21 us before.
 __global__ void k_reorder(ReorderArgs A) {
   const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i == 0) A.counter[CNT_DISP] = A.counter[CNT_VMAX] = 0;
+  if (i >= A.clear0 && i < A.clear1) A.counter[i] = 0;
   if (i >= A.n) return;
   uint32_t s, cell;
   const uint32_t k = pb_cell_position(A.order, i, &s, &cell);
@@ -233,8 +234,10 @@ static_assert(WCAP < 0xFFF, "12-bit list entries address the staged window and i
 #define NL_ROW (20u * LPA) // list capacity granule: a multiple of both batch sizes
 #define PAD_FAR 1.0e10     // coordinate of that slot
 struct Stage {              // pair kernel: FP64 positions with shifts applied
-  double x[WCAP + 1], y[WCAP + 1], z[WCAP + 1];   // slot WCAP: padding target
-  uint8_t t[WCAP + 1];
+  // slot WCAP: padding target; the last group of a mask (k_lj_direct) reads
+  // up to 31 entries past a range
+  double x[WCAP + 32], y[WCAP + 32], z[WCAP + 32];
+  uint8_t t[WCAP + 32];
   alignas(16) WinTable W;
   unsigned long long hsum[16];  // last step of a run: fingerprint sums (lane mod 16, so
                                 // four lanes of a wavefront share an LDS atomic address)
@@ -832,6 +835,69 @@ __global__ void k_publish_maxima(const uint32_t *counter, uint32_t *mon, uint32_
   if (threadIdx.x == 0) publish_maxima(counter, mon, step);
 }
 
+// Sums over a particle's pairs.  Forces and energies accumulate in FP64 in
+// both modes; MIXED evaluates each pair in FP32 on the FP64 displacement after
+// the FP64 cutoff test.
+template <bool MIXED, bool ENERGY, bool ONE_TYPE>
+struct PairSums {
+  double fx = 0, fy = 0, fz = 0, pe = 0, vir = 0;
+  float pef = 0.f, virf = 0.f;   // MIXED energies: per-lane FP32 sums
+  // displacement r_i - r_j, type pair t; `counts`: not the particle itself and
+  // not a padding entry seen through the minimum image
+  __device__ __forceinline__ void add(const StepArgs &A, double dx, double dy, double dz, uint32_t t,
+                                      bool counts) {
+    const double r2d = dx * dx + dy * dy + dz * dz;
+    const bool in = r2d < A.rc2 && counts;
+    if (MIXED) {
+      // r2 of a padding entry is large but finite; zero r2 (the particle
+      // itself, or an image of a padding entry under the minimum image) gives
+      // inf / NaN that the selects below discard
+      const float r2 = (float)r2d;
+      const float s2 = ONE_TYPE ? A.s2f : A.lj->s2f[t];
+      const float e24 = ONE_TYPE ? A.e24f : A.lj->e24f[t];
+      float ir2 = __builtin_amdgcn_rcpf(r2);
+      ir2 = ir2 * (2.0f - r2 * ir2);               // one Newton step: ~0.5 ulp
+      ir2 = in ? ir2 : 0.0f;                       // outside rc: f/r = 0 (one FP32 select)
+      float s6 = s2 * ir2;
+      s6 = s6 * s6 * s6;
+      // f/r = 24 eps s6 (2 s6 - 1) / r^2 (kernelinline.hh:90-95), written as
+      // ir2 s6 (48 eps s6 - 24 eps): one multiply fewer a pair
+      const float e48 = e24 + e24;                 // exact; hoisted with one type
+      const float fr = ir2 * s6 * fmaf(e48, s6, -e24);
+      const double frd = (double)fr;              // f/r, applied to the FP64 displacement
+      fx = fma(frd, dx, fx);
+      fy = fma(frd, dy, fy);
+      fz = fma(frd, dz, fz);
+      if (ENERGY) {
+        const float e4 = ONE_TYPE ? A.e4f : A.lj->e4f[t];
+        const float sh = ONE_TYPE ? A.shiftf : A.lj->shiftf[t];
+        const float ep = e4 * s6 * (s6 - 1.0f) - sh;
+        pef += in ? ep : 0.0f;
+        virf = fmaf(fr, r2, virf);
+      }
+    } else {
+      const double r2 = r2d;
+      const double s2 = ONE_TYPE ? A.s2 : A.lj->s2[t];
+      const double e24 = ONE_TYPE ? A.e24 : A.lj->e24[t];
+      const double ir2 = rcp64(r2);
+      double s6 = s2 * ir2;
+      s6 = s6 * s6 * s6;
+      double fr = e24 * s6 * (2.0 * s6 - 1.0) * ir2;
+      fr = in ? fr : 0.0;
+      fx += fr * dx;
+      fy += fr * dy;
+      fz += fr * dz;
+      if (ENERGY) {
+        const double e4 = ONE_TYPE ? A.e4 : A.lj->e4[t];
+        const double sh = ONE_TYPE ? A.shift : A.lj->shift[t];
+        const double ep = e4 * s6 * (s6 - 1.0) - sh;
+        pe += in ? ep : 0.0;
+        vir += fr * r2;
+      }
+    }
+  }
+};
+
 // Pairs and integration of one segment's tile particles: one lane a
 // particle (LPA = 1), 64 particles a wavefront.  With FAST (window staged,
 // no minimum image) a lane takes a word pair (ten pairs) a step, the next
@@ -840,7 +906,7 @@ __global__ void k_publish_maxima(const uint32_t *counter, uint32_t *mon, uint32_
 // cutoff is a select.  Other segments take one word (four pairs) a step.
 // (LPA > 1 lanes a particle would sum partial forces over the lanes and
 // let the first lane integrate.)
-template <bool FAST, bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool INTEGRATE>
+template <bool FAST, bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE>
 __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const ListSeg &G,
                                          const RepInfo &R, bool staged, bool mi, double &ke, double &pe_b,
                                          double &vir_b, float &d2m, float &v2m,
@@ -882,7 +948,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
   // requested at the end of the current one (one set of registers live)
   uint32_t norig = 0;
   auto fetch_state = [&](uint32_t ub) {
-    if (INTEGRATE && sl == 0 && ub + grp < ntile) {
+    if (sl == 0 && ub + grp < ntile) {
       np_own = A.rin[ngi];
       nv_own = A.vin[ngi];
       nrb_own = A.rbuild[ngi];
@@ -907,10 +973,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
     if (FAST) pi = make_double4(S.x[li], S.y[li], S.z[li], (double)S.t[li]);
     else pi = act ? window_pos(S, G, R, A.rin, staged, li) : make_double4(0, 0, 0, 0);
     const uint32_t ti = ONE_TYPE ? 0u : (uint32_t)pi.w;
-    // forces and energies accumulate in FP64 in both modes; MIXED evaluates
-    // each pair in FP32 on the FP64 displacement after the FP64 cutoff test
-    double fx = 0, fy = 0, fz = 0, pe = 0, vir = 0;
-    float pef = 0.f, virf = 0.f;   // MIXED energies: per-lane FP32 sums of ~20 pairs
+    PairSums<MIXED, ENERGY, ONE_TYPE> P;
     auto pair = [&](uint32_t q) {
       double4 pj;
       if (FAST) pj = make_double4(S.x[q], S.y[q], S.z[q], ONE_TYPE ? 0.0 : (double)S.t[q]);
@@ -921,57 +984,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
         dy -= L1 * rint(dy * I1);
         dz -= L2 * rint(dz * I2);
       }
-      uint32_t t = 0;
-      if (!ONE_TYPE) t = ti * PB_MAXT + (uint32_t)pj.w;
-      const double r2d = dx * dx + dy * dy + dz * dz;
-      const bool in = r2d < A.rc2 && (FAST || !mi || q != NL_PAD);
-      if (MIXED) {
-        // r2 of a padding entry is large but finite; zero r2 (an image of a
-        // padding entry under the minimum image) gives inf / NaN that the
-        // selects below discard
-        const float r2 = (float)r2d;
-        const float s2 = ONE_TYPE ? A.s2f : A.lj->s2f[t];
-        const float e24 = ONE_TYPE ? A.e24f : A.lj->e24f[t];
-        float ir2 = __builtin_amdgcn_rcpf(r2);
-        ir2 = ir2 * (2.0f - r2 * ir2);               // one Newton step: ~0.5 ulp
-        ir2 = in ? ir2 : 0.0f;                       // outside rc: f/r = 0 (one FP32 select)
-        float s6 = s2 * ir2;
-        s6 = s6 * s6 * s6;
-        // f/r = 24 eps s6 (2 s6 - 1) / r^2 (kernelinline.hh:90-95), written as
-        // ir2 s6 (48 eps s6 - 24 eps): one multiply fewer a pair
-        const float e48 = e24 + e24;                 // exact; hoisted with one type
-        const float fr = ir2 * s6 * fmaf(e48, s6, -e24);
-        const double frd = (double)fr;              // f/r, applied to the FP64 displacement
-        fx = fma(frd, dx, fx);
-        fy = fma(frd, dy, fy);
-        fz = fma(frd, dz, fz);
-        if (ENERGY) {
-          const float e4 = ONE_TYPE ? A.e4f : A.lj->e4f[t];
-          const float sh = ONE_TYPE ? A.shiftf : A.lj->shiftf[t];
-          const float ep = e4 * s6 * (s6 - 1.0f) - sh;
-          pef += in ? ep : 0.0f;
-          virf = fmaf(fr, r2, virf);
-        }
-      } else {
-        const double r2 = r2d;
-        const double s2 = ONE_TYPE ? A.s2 : A.lj->s2[t];
-        const double e24 = ONE_TYPE ? A.e24 : A.lj->e24[t];
-        const double ir2 = rcp64(r2);
-        double s6 = s2 * ir2;
-        s6 = s6 * s6 * s6;
-        double fr = e24 * s6 * (2.0 * s6 - 1.0) * ir2;
-        fr = in ? fr : 0.0;
-        fx += fr * dx;
-        fy += fr * dy;
-        fz += fr * dz;
-        if (ENERGY) {
-          const double e4 = ONE_TYPE ? A.e4 : A.lj->e4[t];
-          const double sh = ONE_TYPE ? A.shift : A.lj->shift[t];
-          const double ep = e4 * s6 * (s6 - 1.0) - sh;
-          pe += in ? ep : 0.0;
-          vir += fr * r2;
-        }
-      }
+      P.add(A, dx, dy, dz, ONE_TYPE ? 0u : ti * PB_MAXT + (uint32_t)pj.w, FAST || !mi || q != NL_PAD);
     };
     // rows are padded with the inert entry to whole word pairs
     constexpr uint32_t EPW = FAST ? 5u : 4u, EB = FAST ? 12u : 16u;
@@ -1025,9 +1038,10 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
         for (uint32_t j = 0; j < EPW; ++j) pair(e[EPW + j]);
       }
     }
+    double fx = P.fx, fy = P.fy, fz = P.fz, pe = P.pe, vir = P.vir;
     if (MIXED && ENERGY) {
-      pe = (double)pef;
-      vir = (double)virf;
+      pe = (double)P.pef;
+      vir = (double)P.virf;
     }
 #pragma unroll
     for (int o = (int)LPA / 2; o > 0; o >>= 1) {
@@ -1042,49 +1056,47 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
     fetch_state(ub + nwv * APW);
     if (!act || sl != 0) continue;
 
-    if (INTEGRATE) {
-      double4 p = p_own;
-      double4 vi = v_own;
-      const float4 rb = rb_own;
-      // the list is valid for this step iff the positions the pair loop used
-      // are within skin/2 of their positions at the last rebuild
-      auto disp2 = [&](const double4 &x) {
-        const float ex = (float)(x.x - (double)rb.x), ey = (float)(x.y - (double)rb.y),
-                    ez = (float)(x.z - (double)rb.z);
-        return ex * ex + ey * ey + ez * ez;
-      };
-      if ((double)disp2(p) > half_skin2) atomicOr(&A.counter[CNT_SKIN], 1u);
-      // kick-drift form of propagateVelocityVerlet_F4 (kernelfuncs.cu:
-      // 347-365): v holds v(t - dt/2) = v_ref(t-dt) + Fold dt/2m
-      const double dtm2 = 0.5 * A.dt * vi.w;
-      const double vx = vi.x + fx * dtm2, vy = vi.y + fy * dtm2, vz = vi.z + fz * dtm2;  // v(t)
-      if (ENERGY) ke += 0.5 * (vx * vx + vy * vy + vz * vz) / vi.w;
-      vi.x = vx + fx * dtm2;
-      vi.y = vy + fy * dtm2;
-      vi.z = vz + fz * dtm2;
-      p.x += vi.x * A.dt;
-      p.y += vi.y * A.dt;
-      p.z += vi.z * A.dt;
-      if (!WRITE_F) {
-        A.rout[gi] = p;
-        A.vout[gi] = vi;
-      }
-      // displacement of the new positions feeds the rebuild schedule
-      // in units of the replica's half skin (replicas may have different skins)
-      d2m = fmaxf(d2m, disp2(p) * inv_hs2);
-      v2m = fmaxf(v2m, (float)(vi.x * vi.x + vi.y * vi.y + vi.z * vi.z) * inv_hs2);
-      if (WRITE_F) {
-        // last step of a run: the reference VV state r(t+dt), v(t), Fold =
-        // F(t), positions wrapped into the box (treatPeriodicCondition), and
-        // the fingerprint of the slot that a next run compares against
-        p.x = wrap1(p.x, R.lo[0], R.hi[0]);
-        p.y = wrap1(p.y, R.lo[1], R.hi[1]);
-        p.z = wrap1(p.z, R.lo[2], R.hi[2]);
-        A.rout[gi] = p;
-        A.vout[gi] = make_double4(vx, vy, vz, vi.w);
-        A.Aout[gi] = make_double4(fx, fy, fz, 0.0);
-        atomicAdd(hsum + (lane & 15u), (unsigned long long)slot_hash(gi, o_own, p));   // LDS
-      }
+    double4 p = p_own;
+    double4 vi = v_own;
+    const float4 rb = rb_own;
+    // the list is valid for this step iff the positions the pair loop used
+    // are within skin/2 of their positions at the last rebuild
+    auto disp2 = [&](const double4 &x) {
+      const float ex = (float)(x.x - (double)rb.x), ey = (float)(x.y - (double)rb.y),
+                  ez = (float)(x.z - (double)rb.z);
+      return ex * ex + ey * ey + ez * ez;
+    };
+    if ((double)disp2(p) > half_skin2) atomicOr(&A.counter[CNT_SKIN], 1u);
+    // kick-drift form of propagateVelocityVerlet_F4 (kernelfuncs.cu:
+    // 347-365): v holds v(t - dt/2) = v_ref(t-dt) + Fold dt/2m
+    const double dtm2 = 0.5 * A.dt * vi.w;
+    const double vx = vi.x + fx * dtm2, vy = vi.y + fy * dtm2, vz = vi.z + fz * dtm2;  // v(t)
+    if (ENERGY) ke += 0.5 * (vx * vx + vy * vy + vz * vz) / vi.w;
+    vi.x = vx + fx * dtm2;
+    vi.y = vy + fy * dtm2;
+    vi.z = vz + fz * dtm2;
+    p.x += vi.x * A.dt;
+    p.y += vi.y * A.dt;
+    p.z += vi.z * A.dt;
+    if (!WRITE_F) {
+      A.rout[gi] = p;
+      A.vout[gi] = vi;
+    }
+    // displacement of the new positions feeds the rebuild schedule
+    // in units of the replica's half skin (replicas may have different skins)
+    d2m = fmaxf(d2m, disp2(p) * inv_hs2);
+    v2m = fmaxf(v2m, (float)(vi.x * vi.x + vi.y * vi.y + vi.z * vi.z) * inv_hs2);
+    if (WRITE_F) {
+      // last step of a run: the reference VV state r(t+dt), v(t), Fold =
+      // F(t), positions wrapped into the box (treatPeriodicCondition), and
+      // the fingerprint of the slot that a next run compares against
+      p.x = wrap1(p.x, R.lo[0], R.hi[0]);
+      p.y = wrap1(p.y, R.lo[1], R.hi[1]);
+      p.z = wrap1(p.z, R.lo[2], R.hi[2]);
+      A.rout[gi] = p;
+      A.vout[gi] = make_double4(vx, vy, vz, vi.w);
+      A.Aout[gi] = make_double4(fx, fy, fz, 0.0);
+      atomicAdd(hsum + (lane & 15u), (unsigned long long)slot_hash(gi, o_own, p));   // LDS
     }
     if (WRITE_F) A.Fout[gi] = make_double4(fx, fy, fz, 0.0);
     if (ENERGY) {
@@ -1096,12 +1108,12 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
 
 // One segment: stage its window, pairs + integration of its tile
 // particles, block maxima and energy partials.
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool INTEGRATE>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE>
 __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   __shared__ Stage S;
   const ListSeg G = A.segs[seg];
   const RepInfo &R = A.reps[G.rep];
-  if (WRITE_F && INTEGRATE && threadIdx.x < 16) S.hsum[threadIdx.x] = 0;   // visible after the staging
+  if (WRITE_F && threadIdx.x < 16) S.hsum[threadIdx.x] = 0;   // visible after the staging
   load_window_table(S.W, A.wtab, seg);
   const bool staged = S.W.total <= WCAP;
   const bool mi = G.whole != 0;
@@ -1109,26 +1121,24 @@ __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   double ke = 0.0, pe_b = 0.0, vir_b = 0.0;
   float d2m = 0.f, v2m = 0.f;
   if (staged && !mi)          // block-uniform: the common case, branch-free pairs
-    lj_tiles<true, MIXED, ENERGY, WRITE_F, ONE_TYPE, INTEGRATE>(A, S, G, R, staged, mi, ke, pe_b, vir_b,
-                                                                d2m, v2m, S.hsum);
+    lj_tiles<true, MIXED, ENERGY, WRITE_F, ONE_TYPE>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
+                                                     v2m, S.hsum);
   else
-    lj_tiles<false, MIXED, ENERGY, WRITE_F, ONE_TYPE, INTEGRATE>(A, S, G, R, staged, mi, ke, pe_b,
-                                                                 vir_b, d2m, v2m, S.hsum);
+    lj_tiles<false, MIXED, ENERGY, WRITE_F, ONE_TYPE>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
+                                                      v2m, S.hsum);
 
   __shared__ float smx[2][TBS / 64];
   __shared__ double sen[3][TBS / 64];
-  if (INTEGRATE) {
-    // block maxima of displacement^2 and speed^2; an atomic only when the
-    // block beats the running maximum (non-negative floats order as uints)
+  // block maxima of displacement^2 and speed^2; an atomic only when the
+  // block beats the running maximum (non-negative floats order as uints)
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-      d2m = fmaxf(d2m, __shfl_xor(d2m, o, 64));
-      v2m = fmaxf(v2m, __shfl_xor(v2m, o, 64));
-    }
-    if (pb_lane() == 0) {
-      smx[0][threadIdx.x / 64] = d2m;
-      smx[1][threadIdx.x / 64] = v2m;
-    }
+  for (int o = 32; o > 0; o >>= 1) {
+    d2m = fmaxf(d2m, __shfl_xor(d2m, o, 64));
+    v2m = fmaxf(v2m, __shfl_xor(v2m, o, 64));
+  }
+  if (pb_lane() == 0) {
+    smx[0][threadIdx.x / 64] = d2m;
+    smx[1][threadIdx.x / 64] = v2m;
   }
   if (ENERGY) {
     const double kw = pb_wave_sum(ke), pw = pb_wave_sum(pe_b), ww = pb_wave_sum(vir_b);
@@ -1141,23 +1151,21 @@ __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   __syncthreads();
   if (threadIdx.x == 0) {
     const uint32_t nw = blockDim.x / 64;
-    if (WRITE_F && INTEGRATE) {
+    if (WRITE_F) {
       unsigned long long t = 0;
       for (int k = 0; k < 16; ++k) t += S.hsum[k];
       if (t) atomicAdd(A.hash + blockIdx.x % HASH_SLOTS, t);
     }
-    if (INTEGRATE) {
-      float bd = 0.f, bv = 0.f;
-      for (uint32_t w = 0; w < nw; ++w) {
-        bd = fmaxf(bd, smx[0][w]);
-        bv = fmaxf(bv, smx[1][w]);
-      }
-      const uint32_t ud = __float_as_uint(bd), uv = __float_as_uint(bv);
-      if (ud > __hip_atomic_load(&A.counter[CNT_DISP], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(&A.counter[CNT_DISP], ud);
-      if (uv > __hip_atomic_load(&A.counter[CNT_VMAX], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
-        atomicMax(&A.counter[CNT_VMAX], uv);
+    float bd = 0.f, bv = 0.f;
+    for (uint32_t w = 0; w < nw; ++w) {
+      bd = fmaxf(bd, smx[0][w]);
+      bv = fmaxf(bv, smx[1][w]);
     }
+    const uint32_t ud = __float_as_uint(bd), uv = __float_as_uint(bv);
+    if (ud > __hip_atomic_load(&A.counter[CNT_DISP], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(&A.counter[CNT_DISP], ud);
+    if (uv > __hip_atomic_load(&A.counter[CNT_VMAX], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicMax(&A.counter[CNT_VMAX], uv);
     if (ENERGY) {
       // per-segment partials (a segment never spans two replicas), summed
       // per replica in a fixed order by k_energy_reduce after this kernel
@@ -1172,7 +1180,7 @@ __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   }
 }
 
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool INTEGRATE, bool PERSIST>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST>
 __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
   publish_prev(A);
   if constexpr (PERSIST) {
@@ -1200,7 +1208,7 @@ __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
         continue;
       }
       const uint32_t seg = __builtin_amdgcn_readfirstlane(q * per + (q < rmd ? q : rmd) + t);
-      lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE, INTEGRATE>(A, seg);
+      lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE>(A, seg);
     }
     if (threadIdx.x == 0) {
       __threadfence();
@@ -1215,20 +1223,155 @@ __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
   // eight consecutive segments per XCD in every 64 (pb_xcd_chunk8): the same
   // as one slab per XCD on a uniform fluid, 3 % faster on the batched
   // replicas, whose segment sizes vary with the replica
-  lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE, INTEGRATE>(A, pb_xcd_chunk8());
+  lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE>(A, pb_xcd_chunk8());
 }
 
 // Two entry points over the same body: the common variants fit 128 VGPRs
 // (4 wavefronts per SIMD, two 512-thread workgroups per CU); the FP64 and
 // multi-type energy variants need more registers and run without the cap
 // (no spills) at lower occupancy.
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool INTEGRATE, bool PERSIST>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST>
 __global__ void __launch_bounds__(TBS) __attribute__((amdgpu_waves_per_eu(4))) k_lj_step(StepArgs A) {
-  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, INTEGRATE, PERSIST>(A);
+  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST>(A);
 }
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool INTEGRATE, bool PERSIST>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST>
 __global__ void __launch_bounds__(TBS) k_lj_step_wide(StepArgs A) {
-  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, INTEGRATE, PERSIST>(A);
+  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST>(A);
+}
+
+// Forces (and energies) of the current positions without a list, for a single
+// evaluation (pb_lj_force): building a list, writing it and reading it back
+// once cost more than testing the candidates where they stand.  The window is
+// staged as in the step kernel; a particle's candidates are the three cells of
+// each of its nine columns.  LN lanes a particle:
+//   1  (large systems): 32 FP64 distance tests a step into a bit mask (the sign
+//      of r2 - rc2, seven instructions each), then the pair body per hit;
+//   more (too few particles to fill the chip): every lane evaluates every LN-th
+//      candidate outright, a short serial chain, and the lanes' sums are added.
+// 1,048,576 atoms: the call, sort included, takes 660 us against 880 with a
+// list (FP64); 864 atoms: this kernel 13 us against 42 (list) + 12.
+template <bool MIXED, bool ENERGY, bool ONE_TYPE, uint32_t LN>
+__global__ void __launch_bounds__(TBS) k_lj_direct(StepArgs A) {
+  __shared__ Stage S;
+  __shared__ double sen[2][TBS / 64];
+  const uint32_t seg = pb_xcd_chunk8();
+  const ListSeg G = A.segs[seg];
+  const RepInfo &R = A.reps[G.rep];
+  WinTable &W = S.W;
+  window_table(W, G, R, A.cstart);
+  const uint32_t ntile = W.rpref[W.nrun];
+  if (W.total >= NL_PAD) {                       // block-uniform; the call is refused
+    if (threadIdx.x == 0) atomicOr(&A.counter[CNT_WIN], 1u);
+    return;
+  }
+  const bool staged = W.total <= WCAP, mi = G.whole != 0;
+  stage_window(S, R, A.rin);
+  constexpr uint32_t APW = 64u / LN;
+  const uint32_t lane = pb_lane(), sl = lane & (LN - 1u), grp = lane / LN;
+  const uint32_t wave = threadIdx.x / 64, nwv = blockDim.x / 64;
+  const double L0 = R.L[0], L1 = R.L[1], L2 = R.L[2];
+  const double I0 = R.Linv[0], I1 = R.Linv[1], I2 = R.Linv[2];
+  // |r|^2 below this passes the mask's test: rc2 and more than its rounding
+  const double rcm = A.rc2 * (1.0 + 1e-12);
+  double pe_b = 0.0, vir_b = 0.0;
+  for (uint32_t ub = wave * APW; ub < ntile; ub += nwv * APW) {   // wave-uniform
+    const uint32_t u = ub + grp;
+    const bool act = u < ntile;
+    uint32_t li = 0, gi = 0, run = 0;
+    if (act) tile_particle(W, u, li, gi, run);
+    PairSums<MIXED, ENERGY, ONE_TYPE> P;
+    if (act) {
+      const double4 pi = staged ? make_double4(S.x[li], S.y[li], S.z[li], (double)S.t[li])
+                                : window_global(W, G, R, A.rin, li);
+      const uint32_t ti = ONE_TYPE ? 0u : (uint32_t)pi.w * PB_MAXT;
+      auto pair = [&](uint32_t q) {             // a staged candidate, images applied
+        P.add(A, pi.x - S.x[q], pi.y - S.y[q], pi.z - S.z[q], ONE_TYPE ? 0u : ti + S.t[q], q != li);
+      };
+      auto scan = [&](uint32_t q0, uint32_t q1) {
+        if (staged && !mi) {
+          if constexpr (LN == 1) {
+            for (uint32_t c0 = q0; c0 < q1; c0 += 32u) {
+              // the last group reads up to 31 entries past q1 (the arrays' slack)
+              uint32_t m = 0;
+#pragma unroll 4
+              for (uint32_t k = 0; k < 32u; ++k) {
+                const double dx = pi.x - S.x[c0 + k], dy = pi.y - S.y[c0 + k], dz = pi.z - S.z[c0 + k];
+                const double t = fma(dz, dz, fma(dy, dy, fma(dx, dx, -rcm)));
+                m = __builtin_amdgcn_alignbit(m, (uint32_t)__double2hiint(t), 31);
+              }
+              if (q1 - c0 < 32u) m &= ~((0x80000000u >> (q1 - c0 - 1u)) - 1u);
+              while (m) {
+                const uint32_t k = (uint32_t)__builtin_clz(m);
+                m &= ~(0x80000000u >> k);
+                pair(c0 + k);
+              }
+            }
+          } else {
+#pragma unroll 4
+            for (uint32_t q = q0 + sl; q < q1; q += LN) pair(q);
+          }
+          return;
+        }
+        for (uint32_t q = q0 + sl; q < q1; q += LN) {
+          const double4 pj = staged ? make_double4(S.x[q], S.y[q], S.z[q], (double)S.t[q])
+                                    : window_global(W, G, R, A.rin, q);
+          double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+          if (mi) {
+            dx -= L0 * rint(dx * I0);
+            dy -= L1 * rint(dy * I1);
+            dz -= L2 * rint(dz * I2);
+          }
+          P.add(A, dx, dy, dz, ONE_TYPE ? 0u : ti + (uint32_t)pj.w, q != li);
+        }
+      };
+      if (mi) {
+        scan(0, W.total);
+      } else {
+        const uint32_t col = W.rcol[run];
+        uint32_t tz = 1;
+        while (tz < G.nz && W.eoff[col * W.zs + tz + 1] <= li) ++tz;
+        const uint32_t wy = G.ty + 2, ca = col / wy, cb = col % wy;
+        for (uint32_t a = ca - 1; a <= ca + 1; ++a)
+          for (uint32_t b = cb - 1; b <= cb + 1; ++b) {
+            const uint32_t e0 = (a * wy + b) * W.zs + tz - 1;
+            scan(W.eoff[e0], W.eoff[e0 + 3]);        // three z slots
+          }
+      }
+    }
+    double fx = P.fx, fy = P.fy, fz = P.fz;
+    double pe = MIXED ? (double)P.pef : P.pe, vir = MIXED ? (double)P.virf : P.vir;
+#pragma unroll
+    for (uint32_t o = 1; o < LN; o <<= 1) {
+      fx += __shfl_xor(fx, (int)o, 64);
+      fy += __shfl_xor(fy, (int)o, 64);
+      fz += __shfl_xor(fz, (int)o, 64);
+    }
+    if (act && sl == 0) A.Fout[gi] = make_double4(fx, fy, fz, 0.0);
+    if (ENERGY) {                                 // every lane's share
+      pe_b += 0.5 * pe;
+      vir_b += 0.5 * vir;
+    }
+  }
+  if (ENERGY) {
+    // per-segment partials, as the step kernel's (no kinetic energy)
+    const double pw = pb_wave_sum(pe_b), ww = pb_wave_sum(vir_b);
+    if (lane == 0) {
+      sen[0][wave] = pw;
+      sen[1][wave] = ww;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      double pe = 0.0, vir = 0.0;
+      for (uint32_t w = 0; w < nwv; ++w) {
+        pe += sen[0][w];
+        vir += sen[1][w];
+      }
+      double *Q = A.partials + 4 * (size_t)seg;
+      Q[0] = 0.0;
+      Q[1] = pe;
+      Q[2] = vir;
+    }
+  }
 }
 
 // ------------------------------------------------------------- host side
@@ -1243,8 +1386,17 @@ static uint32_t expected_maxnb(const pb_sys *s) {
   return (m + NL_ROW - 1u) / NL_ROW * NL_ROW;
 }
 
-// List cells, radii and segments for cutoff rc with skin[q] per replica.
-static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &skin) {
+// Tile particles a segment should hold: a workgroup's lanes take them in one
+// pass, `lanes` to a particle.
+static uint32_t tile_target(uint32_t lanes) { return TBS / lanes; }
+
+// List cells, radii and segments for cutoff rc with skin[q] per replica, kept
+// while nothing they depend on changes (the box clears plan_lanes).
+static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &skin, uint32_t lanes) {
+  if (s->plan_lanes == lanes && s->plan_rc == rc && s->plan_skins == skin &&
+      s->plan_tile_w == s->tile_w && s->plan_fill == s->tile_fill)
+    return PB_OK;
+  s->plan_lanes = 0;
   uint32_t cell0 = 0;
   double rmax_all = 0.0;
   for (uint32_t q = 0; q < s->nrep; ++q) {
@@ -1287,11 +1439,15 @@ static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &ski
                        "a replica thinner than 3 list cells must fit one LDS window");
       segs.push_back(ListSeg{q, 0, 0, 0, 1, 1, 1, 1});
     } else {
-      const uint32_t tw = s->tile_w;
-      const uint32_t tx = R.nb[0] >= tw + 2 ? tw : 1, ty = R.nb[1] >= tw + 2 ? tw : 1;
       const double per_cell = (double)R.natoms / nc;
+      const uint32_t want = tile_target(lanes);
+      // several lanes a particle: no more tile particles than a pass takes
+      const uint32_t tw = lanes == 1 || 4.0 * per_cell <= want ? s->tile_w : 1;
+      const uint32_t tx = R.nb[0] >= tw + 2 ? tw : 1, ty = R.nb[1] >= tw + 2 ? tw : 1;
       int nz = (int)std::floor(s->tile_fill * WCAP /
                                ((tx + 2) * (ty + 2) * std::max(per_cell, 1e-3))) - 2;
+      if (lanes > 1)
+        nz = std::min(nz, (int)std::lround(want / (tx * ty * std::max(per_cell, 1e-3))));
       nz = std::max(1, std::min<int>({nz, MAXZ, (int)R.nb[2] - 2}));
       // the column split into the fewest z runs of at most nz cells, of
       // equal length to within one cell (a short last run would be a
@@ -1310,26 +1466,37 @@ static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &ski
     R.nseg = (uint32_t)segs.size() - R.seg0;
   }
   s->list_nsegs = (uint32_t)segs.size();
-  if (int rc = pb_alloc(s->ctx, &s->list_segs, 8 * segs.size())) return rc;
+  if (segs.size() > s->list_segs_cap) {
+    s->list_segs_cap = 0;
+    if (int rc = pb_alloc(s->ctx, &s->list_segs, 8 * segs.size())) return rc;
+    s->list_segs_cap = (uint32_t)segs.size();
+  }
   // the window tables persist while the segments do (a continued list uses
   // the ones its build stored)
   if (segs.size() > s->list_wtab_cap) {
+    s->list_wtab_cap = 0;
     if (int rc = pb_alloc(s->ctx, &s->list_wtab, (size_t)WTAB_U4 * segs.size())) return rc;
     s->list_wtab_cap = (uint32_t)segs.size();
   }
-  PB_HIP(s->ctx, hipMemcpyAsync(s->list_segs, segs.data(), sizeof(ListSeg) * segs.size(),
-                                hipMemcpyHostToDevice, s->ctx->stream));
   // per-segment energy partials
-  if (s->list_nsegs > s->nwave) {
+  if (s->list_nsegs > s->partials_cap) {
+    s->partials_cap = 0;
     if (int rc = pb_alloc(s->ctx, &s->partials, 4 * (size_t)s->list_nsegs)) return rc;
+    s->partials_cap = s->list_nsegs;
   }
-  PB_HIP(s->ctx, hipMemcpyAsync(s->d_reps, s->reps.data(), sizeof(RepInfo) * s->nrep,
-                                hipMemcpyHostToDevice, s->ctx->stream));
-  PB_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));   // segs is a host temporary
-  return pb_ensure_sort_ws(s, s->list_ncell);
+  if (int rc = pb_io_upload(s->ctx, s->list_segs, segs.data(), sizeof(ListSeg) * segs.size())) return rc;
+  if (int rc = pb_io_upload(s->ctx, s->d_reps, s->reps.data(), sizeof(RepInfo) * s->nrep)) return rc;
+  if (int rc = pb_ensure_sort_ws(s, s->list_ncell)) return rc;
+  s->plan_rc = rc;
+  s->plan_skins = skin;
+  s->plan_tile_w = s->tile_w;
+  s->plan_fill = s->tile_fill;
+  s->plan_lanes = lanes;
+  return PB_OK;
 }
 
-static int ensure_list_buffers(pb_sys *s, uint32_t maxnb) {
+// the other halves of the arrays that a sort permutes
+static int ensure_sort_buffers(pb_sys *s) {
   int rc;
   if (!s->r2buf) {
     if ((rc = pb_alloc(s->ctx, &s->r2buf, s->npad)) || (rc = pb_alloc(s->ctx, &s->v2buf, s->npad)) ||
@@ -1338,6 +1505,12 @@ static int ensure_list_buffers(pb_sys *s, uint32_t maxnb) {
         (rc = pb_alloc(s->ctx, &s->rbuild, s->npad)) || (rc = pb_alloc(s->ctx, &s->nn, s->npad)))
       return rc;
   }
+  return PB_OK;
+}
+
+static int ensure_list_buffers(pb_sys *s, uint32_t maxnb) {
+  int rc;
+  if ((rc = ensure_sort_buffers(s))) return rc;
   if (s->maxnb < maxnb) {
     // + 48 entries per slot: the step kernel prefetches one batch (4 words)
     // past the end
@@ -1347,11 +1520,13 @@ static int ensure_list_buffers(pb_sys *s, uint32_t maxnb) {
   return PB_OK;
 }
 
-// rebuild: cell ids -> counting sort -> reorder into cell order -> list.
-// F is not carried: every caller rewrites it before it is read again.
-// carry_a = false inside a fused run, where Fold (a) is dead between the
-// conversion to the kick-drift state and the final one (which rewrites it).
-static int rebuild(pb_sys *s, bool carry_a) {
+// Sort into the cell order of the list cells: cell ids -> counting sort ->
+// reorder.  F is not carried: every caller rewrites it before it is read
+// again.  carry_a = false inside a fused run, where Fold (a) is dead between
+// the conversion to the kick-drift state and the final one (which rewrites
+// it).  clear_all: every counter of a run, else its displacement and speed
+// maxima.
+static int sort_cells(pb_sys *s, bool carry_a, bool clear_all) {
   hipStream_t st = s->ctx->stream;
   const uint32_t n = s->npad;
   if (int rc = pb_ensure_sort_ws(s, s->list_ncell)) return rc;
@@ -1367,6 +1542,8 @@ static int rebuild(pb_sys *s, bool carry_a) {
   A.rbuild = s->rbuild;
   A.nn = s->nn;
   A.waveRep = s->waveRep; A.reps = s->d_reps; A.counter = s->d_counter; A.n = n;
+  A.clear0 = clear_all ? 0u : (uint32_t)CNT_DISP;
+  A.clear1 = clear_all ? 16u : (uint32_t)CNT_VMAX + 1u;
   hipLaunchKernelGGL(k_reorder, dim3(pb_blocks(n, 256)), dim3(256), 0, st, A);
   PB_LAUNCH_CHECK(s->ctx, "k_reorder");
   std::swap(s->r, s->r2buf);
@@ -1376,11 +1553,17 @@ static int rebuild(pb_sys *s, bool carry_a) {
   ++s->order_gen;
   std::swap(s->type, s->type2);
   std::swap(s->move, s->move2);
-  hipLaunchKernelGGL(k_build_list, dim3(s->list_nsegs), dim3(TB), 0, st, s->r, s->cstart,
-                     (const ListSeg *)s->list_segs, s->d_reps, n, s->maxnb, s->nl, s->nn,
+  s->ref_binned = false;
+  return PB_OK;
+}
+
+// rebuild: sort, then the Verlet list
+static int rebuild(pb_sys *s, bool carry_a, bool clear_all) {
+  if (int rc = sort_cells(s, carry_a, clear_all)) return rc;
+  hipLaunchKernelGGL(k_build_list, dim3(s->list_nsegs), dim3(TB), 0, s->ctx->stream, s->r, s->cstart,
+                     (const ListSeg *)s->list_segs, s->d_reps, s->npad, s->maxnb, s->nl, s->nn,
                      s->d_counter, s->list_wtab);
   PB_LAUNCH_CHECK(s->ctx, "k_build_list");
-  s->ref_binned = false;
   return PB_OK;
 }
 
@@ -1418,52 +1601,49 @@ static StepArgs make_args(pb_sys *s, double dt) {
 // advanced.  A separate launch: stream order makes the partials visible.
 __global__ void __launch_bounds__(256) k_energy_reduce(const double *partials, const RepInfo *reps,
                                                        uint32_t nrep, double *energy,
-                                                       uint32_t *counter) {
+                                                       uint32_t *counter, uint32_t *counts_out) {
   __shared__ double sm[4 * 256];
   const uint32_t rec = counter[CNT_REC];
   pb_block_reduce_reps(partials, 3, reps, nrep, energy + (size_t)rec * 8 * nrep, true, sm);
   __syncthreads();
   if (threadIdx.x == 0) counter[CNT_REC] = rec + 1;
+  if (counts_out && threadIdx.x < 16) counts_out[threadIdx.x] = counter[threadIdx.x];
 }
 
 typedef void (*StepKernel)(StepArgs);
 
-template <bool MIXED, bool ONE, bool E, bool W, bool I, bool P>
+template <bool MIXED, bool ONE, bool E, bool W, bool P>
 static StepKernel pick1() {
   // variants that do not fit 128 VGPRs without spilling
   if constexpr ((E && (!MIXED || !ONE)) || (!MIXED && !ONE))
-    return k_lj_step_wide<MIXED, E, W, ONE, I, P>;
+    return k_lj_step_wide<MIXED, E, W, ONE, P>;
   else
-    return k_lj_step<MIXED, E, W, ONE, I, P>;
+    return k_lj_step<MIXED, E, W, ONE, P>;
 }
 
 template <bool MIXED, bool ONE, bool P>
-static StepKernel pick3(bool energy, bool wf, bool integ) {
-  if (integ) {
-    if (energy) return wf ? pick1<MIXED, ONE, true, true, true, P>() : pick1<MIXED, ONE, true, false, true, P>();
-    return wf ? pick1<MIXED, ONE, false, true, true, P>() : pick1<MIXED, ONE, false, false, true, P>();
-  }
-  return energy ? pick1<MIXED, ONE, true, true, false, false>() : pick1<MIXED, ONE, false, true, false, false>();
+static StepKernel pick3(bool energy, bool wf) {
+  if (energy) return wf ? pick1<MIXED, ONE, true, true, P>() : pick1<MIXED, ONE, true, false, P>();
+  return wf ? pick1<MIXED, ONE, false, true, P>() : pick1<MIXED, ONE, false, false, P>();
 }
 
 template <bool MIXED, bool ONE>
-static StepKernel pick2(bool energy, bool wf, bool integ, bool persist) {
-  return persist ? pick3<MIXED, ONE, true>(energy, wf, integ) : pick3<MIXED, ONE, false>(energy, wf, integ);
+static StepKernel pick2(bool energy, bool wf, bool persist) {
+  return persist ? pick3<MIXED, ONE, true>(energy, wf) : pick3<MIXED, ONE, false>(energy, wf);
 }
 
-// persistent variants exist for the integrating steps of a fused run
-static StepKernel pick_kernel(bool mixed, bool one, bool energy, bool wf, bool integ, bool persist) {
-  if (mixed) return one ? pick2<true, true>(energy, wf, integ, persist) : pick2<true, false>(energy, wf, integ, persist);
-  return one ? pick2<false, true>(energy, wf, integ, persist) : pick2<false, false>(energy, wf, integ, persist);
+static StepKernel pick_kernel(bool mixed, bool one, bool energy, bool wf, bool persist) {
+  if (mixed) return one ? pick2<true, true>(energy, wf, persist) : pick2<true, false>(energy, wf, persist);
+  return one ? pick2<false, true>(energy, wf, persist) : pick2<false, false>(energy, wf, persist);
 }
 
 // With events, their timestamps are the step kernel's own start and end
 // (taken by the dispatch, hipExtLaunchKernelGGL): a marker packet of
 // hipEventRecord between kernels costs about 10 us of idle GPU per step.
 static int launch_step(pb_sys *s, const StepArgs &A, bool mixed, bool energy, bool wf,
-                       bool integ, hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr) {
+                       hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr) {
   const bool one = s->lj.ntypes == 1;
-  StepKernel k = pick_kernel(mixed, one, energy, wf, integ, A.queue != nullptr);
+  StepKernel k = pick_kernel(mixed, one, energy, wf, A.queue != nullptr);
   // persistent form: two 512-thread workgroups per compute unit (the step
   // kernel's LDS and register use), never more than there are segments
   const uint32_t grid = A.queue ? std::min<uint32_t>(s->list_nsegs, 2u * (uint32_t)std::max(s->ctx->cu_count, 1))
@@ -1474,7 +1654,7 @@ static int launch_step(pb_sys *s, const StepArgs &A, bool mixed, bool energy, bo
     hipLaunchKernelGGL(k, dim3(grid), dim3(TBS), 0, s->ctx->stream, A);
   if (energy)
     hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(256), 0, s->ctx->stream, A.partials, A.reps,
-                       A.nrep, A.energy, A.counter);
+                       A.nrep, A.energy, A.counter, (uint32_t *)nullptr);
   PB_LAUNCH_CHECK(s->ctx, "k_lj_step");
   return PB_OK;
 }
@@ -1488,9 +1668,13 @@ static int check_lj_ready(pb_sys *s) {
   return PB_OK;
 }
 
+// the run's counters, waited for (through the context's pinned results)
 static int read_counters(pb_sys *s, uint32_t *c) {
-  PB_HIP(s->ctx, hipMemcpyAsync(c, s->d_counter, 16 * 4, hipMemcpyDeviceToHost, s->ctx->stream));
+  if (int rc = pb_results(s->ctx)) return rc;
+  PB_HIP(s->ctx, hipMemcpyAsync(s->ctx->res, s->d_counter, 16 * 4, hipMemcpyDeviceToHost,
+                                s->ctx->stream));
   PB_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
+  std::memcpy(c, s->ctx->res, 16 * 4);
   return PB_OK;
 }
 
@@ -1505,8 +1689,7 @@ static int build_checked(pb_sys *s, bool carry_a) {
   uint32_t want = std::max(s->maxnb, expected_maxnb(s));
   for (int attempt = 0; attempt < 4; ++attempt) {
     if (int rc = ensure_list_buffers(s, want)) return rc;
-    if (int rc = reset_counters(s)) return rc;
-    if (int rc = rebuild(s, carry_a)) return rc;
+    if (int rc = rebuild(s, carry_a, true)) return rc;
     uint32_t c[16];
     if (int rc = read_counters(s, c)) return rc;
     if (c[CNT_WIN])
@@ -1520,38 +1703,76 @@ static int build_checked(pb_sys *s, bool carry_a) {
   return pb_fail(s->ctx, PB_ERR_NLIST, "neighbour list keeps overflowing");
 }
 
+// Lanes a particle in a single evaluation (us a call with 16, 8 and 1 lanes,
+// FP64, the sort included): 4000 particles 55, 59, 74 (4 lanes); 8000 56, 59,
+// 70 (4); 16,000 69, 62, 74 (4); 32,000 90, 79, 104.  One lane beyond, where
+// the mask form does less work a candidate: 108,000 particles 160 us.
+#define FORCE_L16 12288u
+#define FORCE_L8 65536u
+static uint32_t force_lanes(const pb_sys *s) {
+  return s->npad <= FORCE_L16 ? 16u : s->npad <= FORCE_L8 ? 8u : 1u;
+}
+
+template <bool MIXED, bool ENERGY, bool ONE>
+static StepKernel pick_direct(uint32_t lanes) {
+  return lanes == 16 ? k_lj_direct<MIXED, ENERGY, ONE, 16u>
+                     : lanes == 8 ? k_lj_direct<MIXED, ENERGY, ONE, 8u> : k_lj_direct<MIXED, ENERGY, ONE, 1u>;
+}
+
 extern "C" int pb_lj_force(pb_sys *s, int precision, double *pe, double *virial) {
   if (!s) return PB_ERR_ARG;
   if (int rc = check_lj_ready(s)) return rc;
   PB_HIP(s->ctx, hipSetDevice(s->ctx->device));
   const double rc = std::sqrt(s->rc2);
-  if (int e = setup_list_cells(s, rc, std::vector<double>(s->nrep, rc * 1e-12))) return e;
-  if (int e = build_checked(s, true)) return e;
+  const uint32_t lanes = force_lanes(s);
+  if (int e = setup_list_cells(s, rc, std::vector<double>(s->nrep, rc * 1e-12), lanes)) return e;
+  if (int e = ensure_sort_buffers(s)) return e;
+  if (int e = pb_results(s->ctx)) return e;
+  if (int e = sort_cells(s, true, true)) return e;
   StepArgs A = make_args(s, 0.0);
   A.rin = s->r;
-  A.vin = s->v;
   A.Fout = s->F;
-  const bool energy = (pe || virial);
-  double *ebuf = nullptr;
-  if (energy) {
-    if (int e = pb_alloc(s->ctx, &ebuf, 8 * (size_t)s->nrep)) return e;
-    A.energy = ebuf;
+  const bool energy = (pe || virial), one = s->lj.ntypes == 1;
+  // energies go straight to pinned memory when they fit behind the counters
+  const bool direct = 16 + 8 * (size_t)s->nrep <= PB_RES_DOUBLES;
+  if (energy && !direct) {
+    if (s->lj_ebuf_cap < 8 * (size_t)s->nrep) {
+      if (int e = pb_alloc(s->ctx, &s->lj_ebuf, 8 * (size_t)s->nrep)) return e;
+      s->lj_ebuf_cap = 8 * (size_t)s->nrep;
+    }
   }
-  if (int e = launch_step(s, A, precision == PB_MIXED, energy, true, false)) {
-    pb_free(ebuf);
+  A.energy = direct ? s->ctx->res_dev + 16 : s->lj_ebuf;
+  const StepKernel k =
+      precision == PB_MIXED
+          ? (energy ? (one ? pick_direct<true, true, true>(lanes) : pick_direct<true, true, false>(lanes))
+                    : (one ? pick_direct<true, false, true>(lanes) : pick_direct<true, false, false>(lanes)))
+          : (energy ? (one ? pick_direct<false, true, true>(lanes) : pick_direct<false, true, false>(lanes))
+                    : (one ? pick_direct<false, false, true>(lanes) : pick_direct<false, false, false>(lanes)));
+  hipStream_t st = s->ctx->stream;
+  hipLaunchKernelGGL(k, dim3(s->list_nsegs), dim3(TBS), 0, st, A);
+  if (energy)
+    hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(256), 0, st, A.partials, A.reps, A.nrep, A.energy,
+                       A.counter, (uint32_t *)s->ctx->res_dev);
+  PB_LAUNCH_CHECK(s->ctx, "k_lj_direct");
+  std::vector<double> far;
+  uint32_t c[16];
+  if (energy) {
+    if (direct) {
+      PB_HIP(s->ctx, hipStreamSynchronize(st));
+    } else {
+      far.resize(8 * (size_t)s->nrep);
+      if (int e = pb_io_download(s->ctx, far.data(), s->lj_ebuf, 8 * sizeof(double) * s->nrep)) return e;
+    }
+    std::memcpy(c, s->ctx->res, sizeof(c));
+  } else if (int e = read_counters(s, c)) {
     return e;
   }
-  if (energy) {
-    std::vector<double> h(8 * (size_t)s->nrep);
-    hipError_t e = hipMemcpyAsync(h.data(), ebuf, 8 * sizeof(double) * s->nrep,
-                                  hipMemcpyDeviceToHost, s->ctx->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(s->ctx->stream);
-    pb_free(ebuf);
-    if (e != hipSuccess) return pb_hip_check(s->ctx, e, "pb_lj_force energies");
-    for (uint32_t q = 0; q < s->nrep; ++q) {
-      if (pe) pe[q] = h[8 * q + 1];
-      if (virial) virial[q] = h[8 * q + 2];
-    }
+  if (c[CNT_WIN])
+    return pb_fail(s->ctx, PB_ERR_CELLS, "a list window holds more than 65534 particles");
+  const double *h = direct ? s->ctx->res + 16 : far.data();
+  for (uint32_t q = 0; energy && q < s->nrep; ++q) {
+    if (pe) pe[q] = h[8 * q + 1];
+    if (virial) virial[q] = h[8 * q + 2];
   }
   return PB_OK;
 }
@@ -1670,13 +1891,15 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
       skins[q] = std::max(o->skin, std::min(sk, cap));
     }
   }
-  if (int rc = setup_list_cells(s, std::sqrt(s->rc2), skins)) return rc;
+  if (int rc = setup_list_cells(s, std::sqrt(s->rc2), skins, 1u)) return rc;
   const uint32_t ne = o->energy_every;
   const uint32_t nrec = ne ? (o->nsteps + ne - 1) / ne : 0;
-  double *ebuf = nullptr;
-  if (nrec) {
-    if (int rc = pb_alloc(s->ctx, &ebuf, (size_t)nrec * 8 * s->nrep)) return rc;
+  if (s->lj_ebuf_cap < (size_t)nrec * 8 * s->nrep) {
+    s->lj_ebuf_cap = 0;
+    if (int rc = pb_alloc(s->ctx, &s->lj_ebuf, (size_t)nrec * 8 * s->nrep)) return rc;
+    s->lj_ebuf_cap = (size_t)nrec * 8 * s->nrep;
   }
+  double *ebuf = nrec ? s->lj_ebuf : nullptr;
   int rc = PB_OK;
   uint32_t rebuilds = 0;
   int skin_bad = 0;
@@ -1778,7 +2001,7 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
           if (reb_from) (void)hipEventRecord(reb_from, st);
         }
       }
-      if (int e = rebuild(s, false)) return e;
+      if (int e = rebuild(s, false, false)) return e;
       ++rebuilds;
       last_build = step;
       A.nl = (const uint64_t *)s->nl;
@@ -1881,7 +2104,7 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
         }
         reb_from = nullptr;
       }
-      if (int e = launch_step(s, A, mixed, energy, last, true, e0, e1)) return e;
+      if (int e = launch_step(s, A, mixed, energy, last, e0, e1)) return e;
       prev_stop = e1;
       std::swap(s->r, s->r2buf);
       std::swap(s->v, s->v2buf);
@@ -1923,11 +2146,11 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
           A.vout = s->v2buf;
           A.Fout = s->F;
           A.step = 0;
-          e = launch_step(s, A, mixed, ne && ((step0 + l) % ne == 0), false, true);
+          e = launch_step(s, A, mixed, ne && ((step0 + l) % ne == 0), false);
           std::swap(s->r, s->r2buf);
           std::swap(s->v, s->v2buf);
         }
-        if (e == PB_OK) e = rebuild(s, false);
+        if (e == PB_OK) e = rebuild(s, false, false);
         hipGraph_t g = nullptr;
         hipError_t he = hipStreamEndCapture(st, &g);
         if (e != PB_OK) {
@@ -2068,7 +2291,6 @@ done:
   for (hipEvent_t e : ev_step) (void)hipEventDestroy(e);
   for (hipEvent_t e : ev_mark) (void)hipEventDestroy(e);
   for (hipEvent_t e : ev_graph) (void)hipEventDestroy(e);
-  pb_free(ebuf);
   return rc;
 }
 
