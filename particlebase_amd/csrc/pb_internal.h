@@ -158,7 +158,7 @@ struct pb_sys {
   bool lj_cont = false;
   uint64_t lj_cont_hash = 0;       // fingerprint of r, orig at the end of the run
   double lj_cont_rc2 = 0, lj_cont_fill = 0;
-  uint32_t lj_cont_tile_w = 0;
+  uint32_t lj_cont_tile_w = 0, lj_cont_lanes = 0;
   std::vector<double> lj_cont_skins;
   uint32_t lj_cont_since = 0;      // steps since the list was built
   uint32_t lj_cont_d2 = 0, lj_cont_v2 = 0;   // displacement / speed maxima (float bits)

@@ -185,9 +185,6 @@ struct ListSeg {
 // fluid), one particle a lane here as well: with 384 lanes the build made a
 // second pass for the last few particles of most segments (340 us at 1M
 // atoms; 448 lanes: 326 us; 512: 288 us)
-#ifndef TB
-#define TB 512
-#endif
 #ifndef BUILD_GROUP
 #define BUILD_GROUP 32u   // candidates tested per mask step of the list build (<= 32)
 #endif
@@ -195,6 +192,13 @@ struct ListSeg {
 #define BUILD_UNROLL 4
 #endif
 #define TBS 512           // step workgroup (8 waves; two per CU at <= 128 VGPRs)
+// Workgroup of the list build and the step kernel with LN lanes a particle: two
+// lanes go with 1024 threads, so that a tile keeps the particles (and the window
+// it shares) of the one-lane form while twice the wavefronts stage and evaluate
+// it; four and eight lanes with smaller tiles of 512 threads.
+template <uint32_t LN>
+constexpr uint32_t tile_threads() { return LN == 2u ? 1024u : (uint32_t)TBS; }
+#define MAXWV 16          // wavefronts of the largest workgroup
 #ifndef WCAP
 #define WCAP 2816         // staged window particles per workgroup (LDS)
 #endif
@@ -208,7 +212,7 @@ struct alignas(16) WinTable {
   uint32_t eoff[MAXE + 1], eg0[MAXE], ec[MAXE], esh[MAXE];
   uint32_t nent, total, ncol, zs;
   uint32_t nrun, rloc[4], rpref[5], rg0[4], rcol[4];
-  uint32_t wsum[TBS / 64];
+  uint32_t wsum[MAXWV];
 };
 // Two list formats, chosen per segment by the same test in the build and the
 // step kernel: segments whose window is staged in LDS and that need no
@@ -217,21 +221,16 @@ struct alignas(16) WinTable {
 // 16-bit entries, four to a word.
 // Padding entries: WCAP in 12-bit rows (the inert LDS slot, so the step
 // kernel uses every entry as it stands), all ones in 16-bit rows (tested
-// for).  A batch of the step kernel is one word per lane: 5 * LPA or 4 * LPA
-// entries; rows are padded to whole batches.
+// for).  Rows are padded to whole pairs of words.
+// LN lanes share a particle's row (build and step alike): word pair p of the
+// row belongs to lane p mod LN, each lane fills its own pairs from its own part
+// of the candidates and is padded to the longest of them, so nn holds the
+// padded entries of one lane.
 #define NL_PAD 0xFFFFu     // 16-bit list padding entry
 #define NL_PADW12 ((uint64_t)WCAP * 0x1001001001001ull)   // a 12-bit word of five WCAP entries
 static_assert(WCAP < 0xFFF, "12-bit list entries address the staged window and its inert slot");
-// Step kernel: lanes per particle, each taking every LPA-th list word.  One
-// lane (64 particles a wavefront) measured 125 us a step at 1M atoms
-// against 131 us with two lanes, 151 with four and 178 with eight: rows
-// are padded to 5 * LPA entries, and with fewer lanes to a row less of each
-// wavefront idles on padding, more than making up for the wavefront
-// running its longest row.
-#ifndef LPA
-#define LPA 1u
-#endif
-#define NL_ROW (20u * LPA) // list capacity granule: a multiple of both batch sizes
+#define NL_ROW 20u         // list capacity granule: a multiple of 2 x 5 and 4 entries
+#define NL_SLACK 96u       // entries past a row's capacity that a read one word pair ahead may reach
 #define PAD_FAR 1.0e10     // coordinate of that slot
 struct Stage {              // pair kernel: FP64 positions with shifts applied
   // slot WCAP: padding target; the last group of a mask (k_lj_direct) reads
@@ -243,13 +242,14 @@ struct Stage {              // pair kernel: FP64 positions with shifts applied
                                 // four lanes of a wavefront share an LDS atomic address)
 };
 #define WCAPB WCAP          // build kernel stage (FP32, 12 B a particle): four workgroups per CU
+#define STAGE_SLACK 64u
 struct StageB {             // list build: FP32 window-relative positions, 12 B a
-  float2 xy[WCAPB + 32];     // particle (four workgroups per CU); 32 slack
-  float z[WCAPB + 32];       // entries read by the last group of 32 tests
+  float2 xy[WCAPB + STAGE_SLACK];   // particle (four workgroups per CU); slack
+  float z[WCAPB + STAGE_SLACK];     // entries read by the last group of tests
   alignas(16) WinTable W;
 };
 
-// exclusive block scan (blockDim multiple of 64, <= TBS)
+// exclusive block scan (blockDim multiple of 64, <= 64 MAXWV)
 __device__ __forceinline__ uint32_t tile_scan(uint32_t x, uint32_t *wsum, uint32_t *total) {
   const uint32_t lane = pb_lane(), w = threadIdx.x / 64, nw = blockDim.x / 64;
   uint32_t inc = x;
@@ -535,7 +535,8 @@ __device__ __forceinline__ void tile_particle(const WinTable &W, uint32_t u, uin
 #ifndef BUILD_WPE
 #define BUILD_WPE 8
 #endif
-__global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_WPE))) k_build_list(const double4 *r, const uint32_t *cstart,
+template <uint32_t LN>
+__global__ void __launch_bounds__(tile_threads<LN>()) __attribute__((amdgpu_waves_per_eu(BUILD_WPE))) k_build_list(const double4 *r, const uint32_t *cstart,
                                                    const ListSeg *segs, const RepInfo *reps,
                                                    uint32_t npad, uint32_t maxnb, uint16_t *nl,
                                                    uint32_t *nn, uint32_t *counter, uint4 *wtab) {
@@ -578,18 +579,20 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_W
   auto tile_rows = [&](auto fmt) {
   constexpr uint32_t epw = decltype(fmt)::value, eb = epw == 5u ? 12u : 16u;
   constexpr uint64_t padw = epw == 5u ? NL_PADW12 : ~0ull;   // a word of padding entries
-  for (uint32_t u = threadIdx.x; u < ntile; u += blockDim.x) {
+  const uint32_t sl = threadIdx.x % LN;
+  for (uint32_t u = threadIdx.x / LN; u < ntile; u += blockDim.x / LN) {
     uint32_t li, gi, run;
     tile_particle(W, u, li, gi, run);
     // Kept entries are packed epw to a 64-bit word in registers; word m of
-    // slot gi is written whole at waddr(m), for m < maxnb / epw (the
-    // allocation holds maxnb + 48 entries per slot: slack words for the
-    // step kernel's read one word pair ahead).
-    uint64_t *const wrow = reinterpret_cast<uint64_t *>(nl) + 2u * gi;
+    // slot gi is written whole at waddr(m), for m < wcap (the allocation
+    // holds maxnb + NL_SLACK entries per slot: slack words for the step
+    // kernel's read one word pair ahead).
+    uint64_t *const wrow = reinterpret_cast<uint64_t *>(nl) + 2u * ((size_t)sl * npad + gi);
     auto waddr = [&](uint32_t m) -> uint64_t * {
-      return wrow + (size_t)(m >> 1) * 2u * npad + (m & 1u);
+      return wrow + (size_t)(m >> 1) * (2u * LN) * npad + (m & 1u);
     };
-    const uint32_t wcap = maxnb / epw;
+    const uint32_t wcap = LN == 1u ? maxnb / epw : (maxnb / (epw * LN)) & ~1u;
+    const uint32_t cap = LN == 1u ? maxnb : wcap * epw;      // entries of this lane
     // 12-bit format: an entry enters the word at bit 0 and the word moves up
     // 12 bits per append, behind a marker bit that starts at bit 0; after
     // five appends the marker reaches bit 60, above the five fields (readers
@@ -606,7 +609,7 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_W
     const uint64_t *const wend = waddr(wcap);
     auto store_word = [&]() {
       if (wp < wend) *wp = word;
-      wp += odd ? 2u * npad - 1u : 1u;
+      wp += odd ? 2u * LN * npad - 1u : 1u;
       odd ^= 1u;
     };
     auto append = [&](uint32_t q) {
@@ -624,11 +627,13 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_W
         }
       }
     };
-    // staged candidates [q0, q1) except li: 32 distance tests into a bit
-    // mask, then the hits appended in order (the append runs once per hit,
-    // not once per candidate).  The last group reads up to 31 entries past
-    // q1 (the stage's slack) and li's own test is kept; their bits are
-    // cleared, so every group runs the same unrolled tests.
+    // This lane's staged candidates of [q0, q1), every LN-th from q0 + sl (a
+    // contiguous part would give the lanes in the middle of a range most of
+    // the hits), except li: GRP distance tests into a bit mask, then the hits
+    // appended in order (the append runs once per hit, not once per
+    // candidate).  The last group reads past q1 (the stage's slack) and li's
+    // own test is kept; their bits are cleared, so every group runs the same
+    // unrolled tests.
     auto scan_staged = [&](uint32_t q0, uint32_t q1, bool mi) {
       const float2 pixy = S.xy[li];
       const float piz = S.z[li];
@@ -643,20 +648,25 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_W
         }
         return __float_as_uint(fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, -rb2))));
       };
-      for (uint32_t c0 = q0; c0 < q1; c0 += BUILD_GROUP) {
-        // test k shifts in at bit 0, so candidate c0 + k ends at bit
-        // BUILD_GROUP - 1 - k: alignbit(m, t, 31) = (m << 1) | (t >> 31),
+      // groups end at most STAGE_SLACK entries past q1
+      constexpr uint32_t GRP = LN <= 2u ? BUILD_GROUP : LN == 4u ? 16u : 8u;
+      static_assert(GRP * LN <= STAGE_SLACK, "a group's reads stay in the stage");
+      for (uint32_t c0 = q0 + sl; c0 < q1; c0 += GRP * LN) {
+        // test k shifts in at bit 0, so candidate c0 + LN k ends at bit
+        // GRP - 1 - k: alignbit(m, t, 31) = (m << 1) | (t >> 31),
         // one instruction a candidate for the compare and the mask
         uint32_t m = 0;
 #pragma unroll BUILD_UNROLL
-        for (uint32_t k = 0; k < BUILD_GROUP; ++k) m = __builtin_amdgcn_alignbit(m, near(c0 + k), 31);
-        constexpr uint32_t top = 1u << (BUILD_GROUP - 1u);
-        if (q1 - c0 < BUILD_GROUP) m &= ~((top >> (q1 - c0 - 1u)) - 1u);
-        if (li - c0 < BUILD_GROUP) m &= ~(top >> (li - c0));   // li < c0 wraps past the group
+        for (uint32_t k = 0; k < GRP; ++k) m = __builtin_amdgcn_alignbit(m, near(c0 + LN * k), 31);
+        constexpr uint32_t top = 1u << (GRP - 1u);
+        const uint32_t left = (q1 - c0 + LN - 1u) / LN;            // candidates from c0 on
+        if (left < GRP) m &= ~((top >> (left - 1u)) - 1u);
+        // li < c0 wraps past the group
+        if (li - c0 < GRP * LN && (li - c0) % LN == 0u) m &= ~(top >> ((li - c0) / LN));
         cnt += __popc(m);
         while (m) {
-          const uint32_t k = (uint32_t)__builtin_clz(m) - (32u - BUILD_GROUP);
-          append(c0 + k);
+          const uint32_t k = (uint32_t)__builtin_clz(m) - (32u - GRP);
+          append(c0 + LN * k);
           m &= ~(top >> k);
         }
       }
@@ -664,7 +674,8 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_W
     // window read from global memory (window larger than the stage)
     auto scan_global = [&](uint32_t q0, uint32_t q1, bool mi) {
       const double4 pi = window_global(W, G, R, r, li);
-      for (uint32_t q = q0; q < q1; ++q) {
+      for (uint32_t q = q0 + sl; q < q1; q += LN) {
+        if (q == li) continue;
         const double4 pj = window_global(W, G, R, r, q);
         double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
         if (mi) {
@@ -678,16 +689,9 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_W
         }
       }
     };
-    // candidates [q0, q1) except the particle itself
     auto scan = [&](uint32_t q0, uint32_t q1, bool mi) {
-      if (staged) {
-        scan_staged(q0, q1, mi);
-      } else if (li >= q0 && li < q1) {
-        scan_global(q0, li, mi);
-        scan_global(li + 1, q1, mi);
-      } else {
-        scan_global(q0, q1, mi);
-      }
+      if (staged) scan_staged(q0, q1, mi);
+      else scan_global(q0, q1, mi);
     };
     if (G.whole) {
       scan(0, W.total, true);
@@ -706,10 +710,15 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_W
     }
     // close the partial word and pad to whole batches with the inert entry
     // (nn holds the padded length)
-    const uint32_t used = cnt < maxnb ? cnt : maxnb;
-    const uint32_t batch = 2u * epw * LPA;      // whole word pairs
-    const uint32_t padded = (used + batch - 1u) / batch * batch;
-    if (cnt % epw != 0u && cnt < maxnb) {
+    const uint32_t used = cnt < cap ? cnt : cap;
+    constexpr uint32_t batch = 2u * epw;        // whole word pairs
+    uint32_t padded = (used + batch - 1u) / batch * batch, total = cnt;
+#pragma unroll
+    for (uint32_t o = 1; o < LN; o <<= 1) {     // the longest lane, and the row's length
+      padded = max(padded, (uint32_t)__shfl_xor((int)padded, (int)o, 64));
+      total += (uint32_t)__shfl_xor((int)total, (int)o, 64);
+    }
+    if (cnt % epw != 0u && cnt < cap) {
       // the partial word: its kr entries moved to the word's top fields, the
       // rest filled with the inert entry
       const uint32_t kr = cnt % epw;
@@ -723,9 +732,9 @@ __global__ void __launch_bounds__(TB) __attribute__((amdgpu_waves_per_eu(BUILD_W
       *waddr(cnt / epw) = last;
     }
     for (uint32_t m = (used + epw - 1u) / epw; m < padded / epw; ++m) *waddr(m) = padw;
-    nn[gi] = padded;
-    if (cnt > maxnb) atomicMax(&counter[CNT_OVF], cnt);
-    mymax = max(mymax, cnt);
+    if (sl == 0) nn[gi] = padded;
+    if (cnt > cap) atomicMax(&counter[CNT_OVF], cnt * LN);
+    mymax = max(mymax, total);
   }
   };
   if (fmt12) tile_rows(UConst<5u>{});
@@ -898,15 +907,17 @@ struct PairSums {
   }
 };
 
-// Pairs and integration of one segment's tile particles: one lane a
-// particle (LPA = 1), 64 particles a wavefront.  With FAST (window staged,
-// no minimum image) a lane takes a word pair (ten pairs) a step, the next
-// pair's 16-byte load in flight while they are evaluated; rows are padded
-// with the inert LDS slot, so a pair is a straight-line sequence and the
-// cutoff is a select.  Other segments take one word (four pairs) a step.
-// (LPA > 1 lanes a particle would sum partial forces over the lanes and
-// let the first lane integrate.)
-template <bool FAST, bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE>
+// Pairs and integration of one segment's tile particles, LN lanes a particle
+// (each evaluates its own word pairs of the row; the first integrates).  With
+// FAST (window staged, no minimum image) a lane takes a word pair (ten pairs) a
+// step, the next pair's 16-byte load in flight while they are evaluated; rows
+// are padded with the inert LDS slot, so a pair is a straight-line sequence and
+// the cutoff is a select.  Other segments take one word (four pairs) a step.
+// One lane keeps large systems busy with the least padding (1M atoms: 125 us a
+// step against 131 with two lanes, 151 with four, 178 with eight); with too few
+// particles to fill the chip a row is a serial chain and more lanes shorten it
+// (run_lanes).
+template <bool FAST, bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, uint32_t LN>
 __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const ListSeg &G,
                                          const RepInfo &R, bool staged, bool mi, double &ke, double &pe_b,
                                          double &vir_b, float &d2m, float &v2m,
@@ -914,8 +925,8 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
   const uint32_t ntile = S.W.rpref[S.W.nrun];
   const double L0 = R.L[0], L1 = R.L[1], L2 = R.L[2];
   const double I0 = R.Linv[0], I1 = R.Linv[1], I2 = R.Linv[2];
-  const uint32_t lane = pb_lane(), sl = lane & (LPA - 1u), grp = lane / LPA;
-  constexpr uint32_t APW = 64u / LPA;            // particles per wavefront
+  const uint32_t lane = pb_lane(), sl = lane & (LN - 1u), grp = lane / LN;
+  constexpr uint32_t APW = 64u / LN;             // particles per wavefront
   const uint32_t wave = threadIdx.x / 64, nwv = blockDim.x / 64;
   // replica constants read once, before any store (stores could alias them)
   const double half_skin2 = R.half_skin2;
@@ -941,7 +952,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
     if (u < ntile) {
       tile_particle(S.W, u, nli, ngi, run);
       nnn = A.nn[ngi];
-      nqq = reinterpret_cast<const ulonglong2 *>(A.nl)[ngi];
+      nqq = reinterpret_cast<const ulonglong2 *>(A.nl)[LN == 1u ? ngi : sl * ld + ngi];
     }
   };
   // the next group's integration state, needed at the end of its iteration:
@@ -989,7 +1000,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
     // rows are padded with the inert entry to whole word pairs
     constexpr uint32_t EPW = FAST ? 5u : 4u, EB = FAST ? 12u : 16u;
     constexpr uint32_t EMASK = (1u << EB) - 1u;
-    const uint32_t nbat = act ? nni / (EPW * LPA) : 0u;
+    const uint32_t nbat = act ? nni / EPW : 0u;
     auto batch = [&](uint64_t w64) {
 #pragma unroll
       for (uint32_t j = 0; j < EPW; ++j) {
@@ -997,22 +1008,22 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
         pair(qj);
       }
     };
-    static_assert(LPA == 1u, "word-pair rows assume one lane a particle");
     if (!FAST) {
       // one word a batch (the minimum-image and unstaged paths use more
-      // registers a pair): word m of the row at 2 gi + (m >> 1) 2 npad + (m & 1)
+      // registers a pair): the lane's word m at
+      // 2 (sl npad + gi) + (m >> 1) 2 LN npad + (m & 1)
       uint64_t qw = qq.x;
-      const uint64_t *wp = A.nl + 2u * (size_t)gi + 1u;
+      const uint64_t *wp = A.nl + 2u * (sl * ld + gi) + 1u;
       for (uint32_t b = 0; b < nbat; ++b) {
         const uint64_t w64 = qw;
         qw = *wp;                                 // one word ahead (slack words at the end)
-        wp += (b & 1u) ? 1u : 2u * ld - 1u;
+        wp += (b & 1u) ? 1u : 2u * LN * ld - 1u;
         batch(w64);
       }
     } else {
       // one 16-byte load brings the next two words while ten pairs are
       // evaluated
-      const ulonglong2 *pp = reinterpret_cast<const ulonglong2 *>(A.nl) + ld + gi;
+      const ulonglong2 *pp = reinterpret_cast<const ulonglong2 *>(A.nl) + (sl + LN) * ld + gi;
       const uint32_t npair = act ? nni / (2u * EPW) : 0u;
       for (uint32_t b = 0; b < npair; ++b) {
         // unpack both words first, so the load lands in their registers and
@@ -1030,7 +1041,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
         // the row's next pair; none past the row's end (its cache lines
         // would be fetched for nothing when all their lanes are done)
         if (b + 1u < npair) qq = *pp;
-        pp += ld;
+        pp += LN * ld;
 #pragma unroll
         for (uint32_t j = 0; j < EPW; ++j) pair(e[j]);
         __builtin_amdgcn_sched_barrier(0);
@@ -1044,7 +1055,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
       vir = (double)P.virf;
     }
 #pragma unroll
-    for (int o = (int)LPA / 2; o > 0; o >>= 1) {
+    for (int o = (int)LN / 2; o > 0; o >>= 1) {
       fx += __shfl_xor(fx, o, 64);
       fy += __shfl_xor(fy, o, 64);
       fz += __shfl_xor(fz, o, 64);
@@ -1108,7 +1119,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
 
 // One segment: stage its window, pairs + integration of its tile
 // particles, block maxima and energy partials.
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, uint32_t LN>
 __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   __shared__ Stage S;
   const ListSeg G = A.segs[seg];
@@ -1121,14 +1132,14 @@ __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   double ke = 0.0, pe_b = 0.0, vir_b = 0.0;
   float d2m = 0.f, v2m = 0.f;
   if (staged && !mi)          // block-uniform: the common case, branch-free pairs
-    lj_tiles<true, MIXED, ENERGY, WRITE_F, ONE_TYPE>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
+    lj_tiles<true, MIXED, ENERGY, WRITE_F, ONE_TYPE, LN>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
                                                      v2m, S.hsum);
   else
-    lj_tiles<false, MIXED, ENERGY, WRITE_F, ONE_TYPE>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
+    lj_tiles<false, MIXED, ENERGY, WRITE_F, ONE_TYPE, LN>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
                                                       v2m, S.hsum);
 
-  __shared__ float smx[2][TBS / 64];
-  __shared__ double sen[3][TBS / 64];
+  __shared__ float smx[2][MAXWV];
+  __shared__ double sen[3][MAXWV];
   // block maxima of displacement^2 and speed^2; an atomic only when the
   // block beats the running maximum (non-negative floats order as uints)
 #pragma unroll
@@ -1180,7 +1191,7 @@ __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   }
 }
 
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST, uint32_t LN>
 __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
   publish_prev(A);
   if constexpr (PERSIST) {
@@ -1208,7 +1219,7 @@ __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
         continue;
       }
       const uint32_t seg = __builtin_amdgcn_readfirstlane(q * per + (q < rmd ? q : rmd) + t);
-      lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE>(A, seg);
+      lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE, LN>(A, seg);
     }
     if (threadIdx.x == 0) {
       __threadfence();
@@ -1223,20 +1234,20 @@ __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
   // eight consecutive segments per XCD in every 64 (pb_xcd_chunk8): the same
   // as one slab per XCD on a uniform fluid, 3 % faster on the batched
   // replicas, whose segment sizes vary with the replica
-  lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE>(A, pb_xcd_chunk8());
+  lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE, LN>(A, pb_xcd_chunk8());
 }
 
 // Two entry points over the same body: the common variants fit 128 VGPRs
 // (4 wavefronts per SIMD, two 512-thread workgroups per CU); the FP64 and
 // multi-type energy variants need more registers and run without the cap
 // (no spills) at lower occupancy.
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST>
-__global__ void __launch_bounds__(TBS) __attribute__((amdgpu_waves_per_eu(4))) k_lj_step(StepArgs A) {
-  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST>(A);
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST, uint32_t LN>
+__global__ void __launch_bounds__(tile_threads<LN>()) __attribute__((amdgpu_waves_per_eu(4))) k_lj_step(StepArgs A) {
+  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST, LN>(A);
 }
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST, uint32_t LN>
 __global__ void __launch_bounds__(TBS) k_lj_step_wide(StepArgs A) {
-  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST>(A);
+  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST, LN>(A);
 }
 
 // Forces (and energies) of the current positions without a list, for a single
@@ -1382,13 +1393,15 @@ static uint32_t expected_maxnb(const pb_sys *s) {
     const double rho = (double)R.natoms / (R.L[0] * R.L[1] * R.L[2]);
     mean = std::max(mean, 4.0 / 3.0 * M_PI * R.rlist * R.rlist * R.rlist * rho);
   }
-  uint32_t m = (uint32_t)std::ceil(1.5 * mean + 48.0);
-  return (m + NL_ROW - 1u) / NL_ROW * NL_ROW;
+  // a lane's share varies more than the row: its own margin, in granules
+  const uint32_t lanes = s->plan_lanes;
+  const uint32_t m = (uint32_t)std::ceil(1.5 * mean / lanes + (lanes == 1 ? 48.0 : 16.0));
+  return (m + NL_ROW - 1u) / NL_ROW * NL_ROW * lanes;
 }
 
 // Tile particles a segment should hold: a workgroup's lanes take them in one
 // pass, `lanes` to a particle.
-static uint32_t tile_target(uint32_t lanes) { return TBS / lanes; }
+static uint32_t tile_target(uint32_t lanes) { return lanes <= 2u ? TBS : TBS / lanes; }
 
 // List cells, radii and segments for cutoff rc with skin[q] per replica, kept
 // while nothing they depend on changes (the box clears plan_lanes).
@@ -1442,11 +1455,11 @@ static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &ski
       const double per_cell = (double)R.natoms / nc;
       const uint32_t want = tile_target(lanes);
       // several lanes a particle: no more tile particles than a pass takes
-      const uint32_t tw = lanes == 1 || 4.0 * per_cell <= want ? s->tile_w : 1;
+      const uint32_t tw = lanes <= 2 || 4.0 * per_cell <= want ? s->tile_w : 1;
       const uint32_t tx = R.nb[0] >= tw + 2 ? tw : 1, ty = R.nb[1] >= tw + 2 ? tw : 1;
       int nz = (int)std::floor(s->tile_fill * WCAP /
                                ((tx + 2) * (ty + 2) * std::max(per_cell, 1e-3))) - 2;
-      if (lanes > 1)
+      if (lanes > 2)
         nz = std::min(nz, (int)std::lround(want / (tx * ty * std::max(per_cell, 1e-3))));
       nz = std::max(1, std::min<int>({nz, MAXZ, (int)R.nb[2] - 2}));
       // the column split into the fewest z runs of at most nz cells, of
@@ -1512,9 +1525,8 @@ static int ensure_list_buffers(pb_sys *s, uint32_t maxnb) {
   int rc;
   if ((rc = ensure_sort_buffers(s))) return rc;
   if (s->maxnb < maxnb) {
-    // + 48 entries per slot: the step kernel prefetches one batch (4 words)
-    // past the end
-    if ((rc = pb_alloc(s->ctx, &s->nl, (size_t)(maxnb + 48) * s->npad))) return rc;
+    s->maxnb = 0;
+    if ((rc = pb_alloc(s->ctx, &s->nl, (size_t)(maxnb + NL_SLACK) * s->npad))) return rc;
     s->maxnb = maxnb;
   }
   return PB_OK;
@@ -1560,7 +1572,11 @@ static int sort_cells(pb_sys *s, bool carry_a, bool clear_all) {
 // rebuild: sort, then the Verlet list
 static int rebuild(pb_sys *s, bool carry_a, bool clear_all) {
   if (int rc = sort_cells(s, carry_a, clear_all)) return rc;
-  hipLaunchKernelGGL(k_build_list, dim3(s->list_nsegs), dim3(TB), 0, s->ctx->stream, s->r, s->cstart,
+  auto *build = s->plan_lanes == 8   ? k_build_list<8u>
+                : s->plan_lanes == 4 ? k_build_list<4u>
+                : s->plan_lanes == 2 ? k_build_list<2u>
+                                     : k_build_list<1u>;
+  hipLaunchKernelGGL(build, dim3(s->list_nsegs), dim3(s->plan_lanes == 2 ? 1024 : TBS), 0, s->ctx->stream, s->r, s->cstart,
                      (const ListSeg *)s->list_segs, s->d_reps, s->npad, s->maxnb, s->nl, s->nn,
                      s->d_counter, s->list_wtab);
   PB_LAUNCH_CHECK(s->ctx, "k_build_list");
@@ -1612,29 +1628,51 @@ __global__ void __launch_bounds__(256) k_energy_reduce(const double *partials, c
 
 typedef void (*StepKernel)(StepArgs);
 
-template <bool MIXED, bool ONE, bool E, bool W, bool P>
+template <bool MIXED, bool ONE, bool E, bool W, bool P, uint32_t LN>
 static StepKernel pick1() {
   // variants that do not fit 128 VGPRs without spilling
   if constexpr ((E && (!MIXED || !ONE)) || (!MIXED && !ONE))
-    return k_lj_step_wide<MIXED, E, W, ONE, P>;
+    return k_lj_step_wide<MIXED, E, W, ONE, P, LN>;
   else
-    return k_lj_step<MIXED, E, W, ONE, P>;
+    return k_lj_step<MIXED, E, W, ONE, P, LN>;
 }
 
-template <bool MIXED, bool ONE, bool P>
+template <bool MIXED, bool ONE, bool P, uint32_t LN>
 static StepKernel pick3(bool energy, bool wf) {
-  if (energy) return wf ? pick1<MIXED, ONE, true, true, P>() : pick1<MIXED, ONE, true, false, P>();
-  return wf ? pick1<MIXED, ONE, false, true, P>() : pick1<MIXED, ONE, false, false, P>();
+  if (energy) return wf ? pick1<MIXED, ONE, true, true, P, LN>() : pick1<MIXED, ONE, true, false, P, LN>();
+  return wf ? pick1<MIXED, ONE, false, true, P, LN>() : pick1<MIXED, ONE, false, false, P, LN>();
 }
 
+// the persistent form has one lane a particle
 template <bool MIXED, bool ONE>
-static StepKernel pick2(bool energy, bool wf, bool persist) {
-  return persist ? pick3<MIXED, ONE, true>(energy, wf) : pick3<MIXED, ONE, false>(energy, wf);
+static StepKernel pick2(bool energy, bool wf, bool persist, uint32_t lanes) {
+  if (persist) return pick3<MIXED, ONE, true, 1u>(energy, wf);
+  switch (lanes) {
+    case 8: return pick3<MIXED, ONE, false, 8u>(energy, wf);
+    case 4: return pick3<MIXED, ONE, false, 4u>(energy, wf);
+    case 2: return pick3<MIXED, ONE, false, 2u>(energy, wf);
+    default: return pick3<MIXED, ONE, false, 1u>(energy, wf);
+  }
 }
 
-static StepKernel pick_kernel(bool mixed, bool one, bool energy, bool wf, bool persist) {
-  if (mixed) return one ? pick2<true, true>(energy, wf, persist) : pick2<true, false>(energy, wf, persist);
-  return one ? pick2<false, true>(energy, wf, persist) : pick2<false, false>(energy, wf, persist);
+static StepKernel pick_kernel(bool mixed, bool one, bool energy, bool wf, bool persist, uint32_t lanes) {
+  if (mixed)
+    return one ? pick2<true, true>(energy, wf, persist, lanes) : pick2<true, false>(energy, wf, persist, lanes);
+  return one ? pick2<false, true>(energy, wf, persist, lanes) : pick2<false, false>(energy, wf, persist, lanes);
+}
+
+// Lanes a particle in a run, by the particles of all replicas together (us a
+// step, FP64, rebuilds included, with 8, 4, 2 and 1 lanes): 864 particles 13,
+// 14, -, 21; 4000 17, 19, -, 24; 8000 18, 17.5, 24, 29; 16,000 19, 18.5, 24, 28;
+// 32,000 26, 24, 25, 28; 48,000 -, 32, 26, 30; 80,000 -, 35, 31, 33.5.  Beyond
+// about 100,000 the two-lane form has more workgroups (one a CU at 16
+// wavefronts) than CUs and a second round: 108,000 particles 45 against 37.5.
+#define RUN_L8 6144u
+#define RUN_L4 32768u
+#define RUN_L2 98304u
+static uint32_t run_lanes(const pb_sys *s, bool persistent) {
+  if (persistent) return 1u;
+  return s->npad <= RUN_L8 ? 8u : s->npad <= RUN_L4 ? 4u : s->npad <= RUN_L2 ? 2u : 1u;
 }
 
 // With events, their timestamps are the step kernel's own start and end
@@ -1643,15 +1681,18 @@ static StepKernel pick_kernel(bool mixed, bool one, bool energy, bool wf, bool p
 static int launch_step(pb_sys *s, const StepArgs &A, bool mixed, bool energy, bool wf,
                        hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr) {
   const bool one = s->lj.ntypes == 1;
-  StepKernel k = pick_kernel(mixed, one, energy, wf, A.queue != nullptr);
+  StepKernel k = pick_kernel(mixed, one, energy, wf, A.queue != nullptr, s->plan_lanes);
   // persistent form: two 512-thread workgroups per compute unit (the step
   // kernel's LDS and register use), never more than there are segments
   const uint32_t grid = A.queue ? std::min<uint32_t>(s->list_nsegs, 2u * (uint32_t)std::max(s->ctx->cu_count, 1))
                                 : s->list_nsegs;
+  // the uncapped variants keep the smaller workgroup (their registers)
+  const bool wide = (energy && (!mixed || !one)) || (!mixed && !one);
+  const uint32_t threads = s->plan_lanes == 2 && !wide ? tile_threads<2u>() : (uint32_t)TBS;
   if (ev0 && ev1)
-    hipExtLaunchKernelGGL(k, dim3(grid), dim3(TBS), 0, s->ctx->stream, ev0, ev1, 0u, A);
+    hipExtLaunchKernelGGL(k, dim3(grid), dim3(threads), 0, s->ctx->stream, ev0, ev1, 0u, A);
   else
-    hipLaunchKernelGGL(k, dim3(grid), dim3(TBS), 0, s->ctx->stream, A);
+    hipLaunchKernelGGL(k, dim3(grid), dim3(threads), 0, s->ctx->stream, A);
   if (energy)
     hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(256), 0, s->ctx->stream, A.partials, A.reps,
                        A.nrep, A.energy, A.counter, (uint32_t *)nullptr);
@@ -1698,7 +1739,8 @@ static int build_checked(pb_sys *s, bool carry_a) {
       s->last_maxnn = c[CNT_MAXNN];
       return PB_OK;
     }
-    want = (c[CNT_OVF] * 5 / 4 + 2u * NL_ROW - 1u) / NL_ROW * NL_ROW;
+    const uint32_t granule = NL_ROW * s->plan_lanes;
+    want = (c[CNT_OVF] * 5 / 4 + 2u * granule - 1u) / granule * granule;
   }
   return pb_fail(s->ctx, PB_ERR_NLIST, "neighbour list keeps overflowing");
 }
@@ -1891,7 +1933,7 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
       skins[q] = std::max(o->skin, std::min(sk, cap));
     }
   }
-  if (int rc = setup_list_cells(s, std::sqrt(s->rc2), skins, 1u)) return rc;
+  if (int rc = setup_list_cells(s, std::sqrt(s->rc2), skins, run_lanes(s, o->persistent != 0))) return rc;
   const uint32_t ne = o->energy_every;
   const uint32_t nrec = ne ? (o->nsteps + ne - 1) / ne : 0;
   if (s->lj_ebuf_cap < (size_t)nrec * 8 * s->nrep) {
@@ -1951,7 +1993,8 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
   // period then starts where the eager schedule would rebuild)
   cont = false;
   if (s->lj_cont && s->lj_cont_rc2 == s->rc2 && s->lj_cont_skins == skins &&
-      s->lj_cont_tile_w == s->tile_w && s->lj_cont_fill == s->tile_fill) {
+      s->lj_cont_tile_w == s->tile_w && s->lj_cont_fill == s->tile_fill &&
+      s->lj_cont_lanes == s->plan_lanes) {
     uint64_t h = 0;
     if ((rc = state_hash(s, &h))) goto done;
     cont = h == s->lj_cont_hash;
@@ -2256,6 +2299,7 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
       s->lj_cont_skins = skins;
       s->lj_cont_tile_w = s->tile_w;
       s->lj_cont_fill = s->tile_fill;
+      s->lj_cont_lanes = s->plan_lanes;
       s->lj_cont_since = (uint32_t)std::min<int64_t>(end_since, 0x7FFFFFFF);
       s->lj_cont_d2 = c[CNT_DISP];
       s->lj_cont_v2 = c[CNT_VMAX];
