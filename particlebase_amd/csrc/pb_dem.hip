@@ -9,17 +9,16 @@
 // pointers, a host read of nnz, a column-index pass, a per-row sort, the
 // history carry-over from the previous matrix and the contact-force pass.
 //
-// Here the same stages run as: a gather of (x, y, z, radius) and the
-// original index into cell order -> count (one thread per particle in cell
-// order, 27 or 125 neighbour cells as contiguous ranges of that view) ->
-// LDS-tiled exclusive scan -> fill + in-row insertion sort (rows are short)
-// -> merge carry of the tangential history (both rows sorted) -> contact
-// force and torque.  The column arrays are sized from the previous step's
-// count; the stages after the scan stop at that capacity and the host reads
-// nnz and the time-step check together at the end, repeating the stages
-// after the scan with larger arrays in the rare step where nnz outgrew them
-// (one host synchronisation per call).  Rows are indexed by the original particle index and hold
-// original indices in ascending order.  Contacts use the strict
+// Here the same stages run as: a gather of (x, y, z, radius) into cell order
+// -> count (one thread per particle in cell order, 27 or 125 neighbour cells as
+// contiguous ranges of that view) -> exclusive scan -> one kernel that sorts
+// each row, takes the tangential history over from the previous matrix (both
+// rows sorted) and computes contact force and torque.  The column arrays are
+// sized from the previous step's count; that kernel stops at the capacity and
+// the host reads nnz and the time-step check together at the end, repeating it
+// with larger arrays in the rare step where nnz outgrew them (one host
+// synchronisation per call).  Rows are indexed by the original particle index
+// and hold original indices in ascending order.  Contacts use the strict
 // |r_ij| < r_i + r_j for both the count and the list (the reference lists
 // with <=, which overruns a row on an exact touch, kernelfuncs.cu:1158).
 #include "pb_internal.h"
@@ -30,12 +29,11 @@
 __global__ void k_fill_u32(uint32_t *x, uint32_t n, uint32_t val);
 
 struct DemGrid {
-  const uint32_t *perm, *cellid, *cstart;
+  const uint32_t *perm, *bid, *cstart;
   const double4 *rs;        // cell order: (x, y, z, radius)
   const uint32_t *so;       // cell order: original index
   const uint8_t *move;
   uint32_t nb[3];
-  int w;            // neighbour half-width: 1 (27 cells) or 2 (125, single-particle cells)
   uint32_t n;
   uint32_t cap;     // capacity of the column arrays
   uint32_t *rowbuf; // DEM_ROWBUF contacts per particle, by original index
@@ -45,35 +43,14 @@ struct DemGrid {
 // touching neighbours than any sphere packing gives) are scanned again
 #define DEM_ROWBUF 16u
 
-// positions with the radius in w, and original indices, in cell order
-__global__ void k_dem_gather(const uint32_t *perm, const double4 *r, const double *rad,
-                             const uint32_t *orig, uint32_t n, double4 *rs, uint32_t *so) {
+// positions with the radius in w, in cell order
+__global__ void k_dem_gather(const uint32_t *perm, const double4 *r, const double *rad, uint32_t n,
+                             double4 *rs) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const uint32_t s = perm[k];
   const double4 p = r[s];
   rs[k] = make_double4(p.x, p.y, p.z, rad[s]);
-  so[k] = orig[s];
-}
-
-// visit the sorted slots of the (2w+1)^3 cells around cell c (non-periodic:
-// DEM distances never use an image, kernelinline.hh:248)
-template <typename F>
-__device__ __forceinline__ void dem_cells(const DemGrid &G, uint32_t c, F &&f) {
-  const uint32_t nz = G.nb[2], nyz = G.nb[1] * nz;
-  const int i0 = (int)(c / nyz), j0 = (int)((c / nz) % G.nb[1]), k0 = (int)(c % nz);
-  const int kl = max(k0 - G.w, 0), kh = min(k0 + G.w, (int)nz - 1);
-  for (int a = -G.w; a <= G.w; ++a) {
-    const int i2 = i0 + a;
-    if (i2 < 0 || i2 >= (int)G.nb[0]) continue;
-    for (int b = -G.w; b <= G.w; ++b) {
-      const int j2 = j0 + b;
-      if (j2 < 0 || j2 >= (int)G.nb[1]) continue;
-      const uint32_t cb = (uint32_t)i2 * nyz + (uint32_t)j2 * nz;
-      const uint32_t q0 = G.cstart[cb + (uint32_t)kl], q1 = G.cstart[cb + (uint32_t)kh + 1];
-      for (uint32_t q = q0; q < q1; ++q) f(q);
-    }
-  }
 }
 
 // (x, y, z, radius) of both particles
@@ -84,176 +61,150 @@ __device__ __forceinline__ bool in_contact(const double4 &pi, const double4 &pj)
   return R2 < rc * rc;
 }
 
+// The sorted slots q != k in contact with particle k, over the (2W + 1)^3 cells
+// around its own (non-periodic: DEM distances never use an image,
+// kernelinline.hh:248), in ascending q.  The scan is a chain of dependent reads
+// (cell starts, candidates) at few wavefronts a SIMD, so the starts of a row of
+// columns are read together, and the candidates of a column (one or two on
+// average) four at a time.
+template <int W, typename F>
+__device__ __forceinline__ void dem_contacts(const DemGrid &G, uint32_t k, const double4 &pi, F &&f) {
+  const uint32_t c = G.bid[k], nz = G.nb[2], nyz = G.nb[1] * nz;
+  const int i0 = (int)(c / nyz), j0 = (int)((c / nz) % G.nb[1]), k0 = (int)(c % nz);
+  const uint32_t kl = (uint32_t)max(k0 - W, 0), kh = (uint32_t)min(k0 + W, (int)nz - 1) + 1u;
+  constexpr int NC = W == 1 ? 9 : 5;                  // columns read together
+#pragma unroll 1
+  for (int g = 0; g < (2 * W + 1) * (2 * W + 1); g += NC) {
+    uint32_t q0[NC], q1[NC];
+#pragma unroll
+    for (int t = 0; t < NC; ++t) {
+      const int i2 = i0 + (g + t) / (2 * W + 1) - W, j2 = j0 + (g + t) % (2 * W + 1) - W;
+      const bool ok = i2 >= 0 && i2 < (int)G.nb[0] && j2 >= 0 && j2 < (int)G.nb[1];
+      const uint32_t cb = ok ? (uint32_t)i2 * nyz + (uint32_t)j2 * nz : 0u;
+      q0[t] = G.cstart[cb + kl];
+      q1[t] = ok ? G.cstart[cb + kh] : q0[t];
+    }
+#pragma unroll
+    for (int t = 0; t < NC; ++t)
+      for (uint32_t q = q0[t]; q < q1[t]; q += 4) {
+        double4 pj[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) pj[u] = G.rs[min(q + u, q1[t] - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)
+          if (q + u < q1[t] && q + u != k && in_contact(pi, pj[u])) f(q + u);
+      }
+  }
+}
+
 // calcCoord_F4 (kernelinline.hh:371-382): contacts of movable particles
 // The same scan keeps the first DEM_ROWBUF contacts (original indices, scan
-// order) in the row buffer for the fill.
-__global__ void k_dem_count(DemGrid G, uint32_t *cnt) {
+// order) in the row buffer for the rows.
+template <int W>
+__global__ void k_dem_count(DemGrid G, uint32_t *cnt, uint32_t *bad) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k == 0) *bad = 0;                               // Cundall-Strack violations of this call
   if (k >= G.n) return;
-  const uint32_t s = G.perm[k];
   const uint32_t i = G.so[k];
   uint32_t c = 0;
-  if (G.move[s]) {
-    const double4 pi = G.rs[k];
+  if (G.move[G.perm[k]]) {
     uint32_t *buf = G.rowbuf + (size_t)i * DEM_ROWBUF;
-    dem_cells(G, G.cellid[s], [&](uint32_t q) {
-      if (q != k && in_contact(pi, G.rs[q])) {
-        if (c < DEM_ROWBUF) buf[c] = G.so[q];
-        ++c;
-      }
+    dem_contacts<W>(G, k, G.rs[k], [&](uint32_t q) {
+      if (c < DEM_ROWBUF) buf[c] = G.so[q];
+      ++c;
     });
   }
   cnt[i] = c;
 }
 
-// makeJlist_WithBlock2/4_F4 (kernelfuncs.cu:1120-1216) + sortColIdx
-// (:1262-1290): the thread that owns a row fills it (from the counting
-// scan's row buffer, or by scanning again when the row is longer) and
-// sorts it.
-__global__ void k_dem_fill(DemGrid G, const uint32_t *row, uint32_t *col) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
-  if (k >= G.n) return;
-  const uint32_t s = G.perm[k];
-  if (!G.move[s]) return;
-  const uint32_t i = G.so[k];
-  const uint32_t b = row[i], e = min(row[i + 1], G.cap);   // rows past the capacity: redone
-  if (b >= e) return;
-  uint32_t p = b;
-  if (row[i + 1] - b <= DEM_ROWBUF) {     // the counting scan kept the whole row
-    const uint32_t *buf = G.rowbuf + (size_t)i * DEM_ROWBUF;
-    for (; p < e; ++p) col[p] = buf[p - b];
-  } else {
-    const double4 pi = G.rs[k];
-    dem_cells(G, G.cellid[s], [&](uint32_t q) {
-      if (q != k && in_contact(pi, G.rs[q]) && p < e) col[p++] = G.so[q];
-    });
-  }
-  for (uint32_t x = b + 1; x < e; ++x) {
-    const uint32_t v = col[x];
-    uint32_t y = x;
-    while (y > b && col[y - 1] > v) {
-      col[y] = col[y - 1];
-      --y;
-    }
-    col[y] = v;
-  }
-}
-
-// succeedPrevState (kernelfuncs.cu:1292-1309): both rows are sorted, so a
-// merge finds the contacts present in both matrices; new contacts start at 0.
-// hw history doubles per contact (1: Hertz slip length, 3: tangential spring).
-__global__ void k_dem_carry(const uint32_t *prow, const uint32_t *pcol, const double *pval,
-                            const uint32_t *crow, const uint32_t *ccol, double *cval,
-                            uint32_t n, uint32_t cap, uint32_t hw) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  uint32_t p = prow ? prow[i] : 0u;
-  const uint32_t pe = prow ? prow[i + 1] : 0u;
-  const uint32_t qe = min(crow[i + 1], cap);
-  for (uint32_t q = crow[i]; q < qe; ++q) {
-    const uint32_t j = ccol[q];
-    while (p < pe && pcol[p] < j) ++p;
-    const bool hit = p < pe && pcol[p] == j;
-    for (uint32_t k = 0; k < hw; ++k)
-      cval[(size_t)q * hw + k] = hit ? pval[(size_t)p * hw + k] : 0.0;
-  }
-}
-
 struct DemForceArgs {
-  const uint32_t *orig, *inv;          // storage -> original, original -> storage
-  const uint32_t *row, *col;
+  const uint32_t *inv;                 // original -> storage
+  const uint32_t *prow, *pcol;         // previous matrix (null: none)
+  const double *pval;
+  const uint32_t *row;
+  uint32_t *col;
   double *val;
   const double4 *r, *v, *w;
   const double *rad;
   const uint8_t *move;
   double4 *F, *T;
   uint32_t *bad;                         // Cundall-Strack violations
-  uint32_t n, npad;
-  uint32_t cap;                          // capacity of col / val
   double E, mu, s2, gamma2, mu_r, dt;
   double kn, zeta, kt;                   // linear law
 };
 
-// DEMContact_F4 (kernelinline.hh:235-363) over the CSR rows
-// (calcF_IJpairWithList_F4, kerneltemplate.hh:135-168), FP64.  F and T are
-// overwritten (the reference clears both first, cudaParticleDEM.cu:168-169).
-// One thread per storage slot, so the particle's own state and its F and T
-// are coalesced; padding slots are skipped (they stay zero).
-__global__ void __launch_bounds__(256) k_dem_force(DemForceArgs A) {
-  const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= A.npad) return;
-  const uint32_t i = A.orig[s];
-  if (i == PB_NONE) return;
-  const double4 pi = A.r[s], vi = A.v[s], wi = A.w[s];
-  const double ri = A.rad[s];
+// a particle's state and sums
+struct DemBody {
+  double4 p, v, w;
+  double rad;
   double f[3] = {0, 0, 0}, t[3] = {0, 0, 0};
   uint32_t bad = 0;
+};
+
+// DEMContact_F4 (kernelinline.hh:235-363), FP64.  h: the contact's history (1
+// double: the slip length), updated in place.
+__device__ __forceinline__ void contact_hertz(const DemForceArgs &A, DemBody &B, uint32_t sj, double *h) {
+  const double4 &pi = B.p, &vi = B.v, &wi = B.w;
+  const double ri = B.rad;
   const bool wnz = wi.x != 0 && wi.y != 0 && wi.z != 0;
-  const uint32_t qe = min(A.row[i + 1], A.cap);
-  for (uint32_t q = A.row[i]; q < qe; ++q) {
-    const uint32_t sj = A.inv[A.col[q]];
-    const double4 pj = A.r[sj], vj = A.v[sj], wj = A.w[sj];
-    const double rj = A.rad[sj];
-    const double d[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
-    const double R2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-    const double rs = ri + rj;
-    if (!(R2 < rs * rs)) continue;
-    const double R = sqrt(R2);
-    const double nv[3] = {d[0] / R, d[1] / R, d[2] / R};
-    const double c = -ri / rs;
-    const double Rij[3] = {c * d[0], c * d[1], c * d[2]};
-    const double vij[3] = {vi.x - vj.x, vi.y - vj.y, vi.z - vj.z};
-    const double xi = rs - R;
-    const double C3 = vij[0] * nv[0] + vij[1] * nv[1] + vij[2] * nv[2];
-    const double Rbar = ri * rj / rs;
-    const double mbar = 1.0 / (vi.w + vj.w);
-    const double Kn = 2.0 / 3.0 * A.E * sqrt(Rbar * xi);
-    const double C4 = Kn * xi - A.gamma2 * sqrt(mbar * Kn) * C3;
-    const double Fn[3] = {nv[0] * C4, nv[1] * C4, nv[2] * C4};
-    if (!(A.dt < 2.0 * sqrt(mbar / Kn))) ++bad;    // Cundall-Strack, kernelinline.hh:285-286
-    const double F0 = sqrt(Fn[0] * Fn[0] + Fn[1] * Fn[1] + Fn[2] * Fn[2]);
-    const double ws[3] = {wi.x + wj.x, wi.y + wj.y, wi.z + wj.z};
-    double vt[3] = {vij[0] - C3 * nv[0], vij[1] - C3 * nv[1], vij[2] - C3 * nv[2]};
-    vt[0] += ws[1] * Rij[2] - ws[2] * Rij[1];
-    vt[1] += ws[2] * Rij[0] - ws[0] * Rij[2];
-    vt[2] += ws[0] * Rij[1] - ws[1] * Rij[0];
-    double Fs[3] = {0, 0, 0};
-    if (vt[0] != 0 && vt[1] != 0 && vt[2] != 0) {   // as the reference, kernelinline.hh:296
-      const double xsm = A.mu * A.s2 * xi;
-      const double vn = sqrt(vt[0] * vt[0] + vt[1] * vt[1] + vt[2] * vt[2]);
-      const double xs = A.val[q];
-      const double v1 = -A.mu * F0 * ((xs < xsm) ? (xs / xsm) : 1.0) / vn;
-      Fs[0] = v1 * vt[0];
-      Fs[1] = v1 * vt[1];
-      Fs[2] = v1 * vt[2];
-      A.val[q] = xs + vn * A.dt;                    // history, owned by this row
-    }
-    const double Ts[3] = {Rij[1] * Fs[2] - Rij[2] * Fs[1], Rij[2] * Fs[0] - Rij[0] * Fs[2],
-                          Rij[0] * Fs[1] - Rij[1] * Fs[0]};
-    double Tr[3] = {0, 0, 0};
-    if (wnz) {
-      const double wn = sqrt(wi.x * wi.x + wi.y * wi.y + wi.z * wi.z);
-      const double cr = -A.mu_r * ri * F0 / wn;
-      Tr[0] = cr * wi.x;
-      Tr[1] = cr * wi.y;
-      Tr[2] = cr * wi.z;
-    }
-    const double Q = 2.0 - (double)A.move[sj];
-#pragma unroll
-    for (int x = 0; x < 3; ++x) {
-      f[x] += (Fn[x] + Fs[x]) * Q;
-      t[x] += (Ts[x] + Tr[x]) * Q;
-    }
+  const double4 pj = A.r[sj], vj = A.v[sj], wj = A.w[sj];
+  const double rj = A.rad[sj];
+  const double d[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+  const double R2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+  const double rs = ri + rj;
+  if (!(R2 < rs * rs)) return;
+  const double R = sqrt(R2);
+  const double nv[3] = {d[0] / R, d[1] / R, d[2] / R};
+  const double c = -ri / rs;
+  const double Rij[3] = {c * d[0], c * d[1], c * d[2]};
+  const double vij[3] = {vi.x - vj.x, vi.y - vj.y, vi.z - vj.z};
+  const double xi = rs - R;
+  const double C3 = vij[0] * nv[0] + vij[1] * nv[1] + vij[2] * nv[2];
+  const double Rbar = ri * rj / rs;
+  const double mbar = 1.0 / (vi.w + vj.w);
+  const double Kn = 2.0 / 3.0 * A.E * sqrt(Rbar * xi);
+  const double C4 = Kn * xi - A.gamma2 * sqrt(mbar * Kn) * C3;
+  const double Fn[3] = {nv[0] * C4, nv[1] * C4, nv[2] * C4};
+  if (!(A.dt < 2.0 * sqrt(mbar / Kn))) ++B.bad;    // Cundall-Strack, kernelinline.hh:285-286
+  const double F0 = sqrt(Fn[0] * Fn[0] + Fn[1] * Fn[1] + Fn[2] * Fn[2]);
+  const double ws[3] = {wi.x + wj.x, wi.y + wj.y, wi.z + wj.z};
+  double vt[3] = {vij[0] - C3 * nv[0], vij[1] - C3 * nv[1], vij[2] - C3 * nv[2]};
+  vt[0] += ws[1] * Rij[2] - ws[2] * Rij[1];
+  vt[1] += ws[2] * Rij[0] - ws[0] * Rij[2];
+  vt[2] += ws[0] * Rij[1] - ws[1] * Rij[0];
+  double Fs[3] = {0, 0, 0};
+  if (vt[0] != 0 && vt[1] != 0 && vt[2] != 0) {   // as the reference, kernelinline.hh:296
+    const double xsm = A.mu * A.s2 * xi;
+    const double vn = sqrt(vt[0] * vt[0] + vt[1] * vt[1] + vt[2] * vt[2]);
+    const double xs = h[0];
+    const double v1 = -A.mu * F0 * ((xs < xsm) ? (xs / xsm) : 1.0) / vn;
+    Fs[0] = v1 * vt[0];
+    Fs[1] = v1 * vt[1];
+    Fs[2] = v1 * vt[2];
+    h[0] = xs + vn * A.dt;                        // history, owned by this row
   }
-  A.F[s] = make_double4(f[0], f[1], f[2], 0.0);
-  A.T[s] = make_double4(t[0], t[1], t[2], 0.0);
-  if (bad) atomicAdd(A.bad, bad);
+  const double Ts[3] = {Rij[1] * Fs[2] - Rij[2] * Fs[1], Rij[2] * Fs[0] - Rij[0] * Fs[2],
+                        Rij[0] * Fs[1] - Rij[1] * Fs[0]};
+  double Tr[3] = {0, 0, 0};
+  if (wnz) {
+    const double wn = sqrt(wi.x * wi.x + wi.y * wi.y + wi.z * wi.z);
+    const double cr = -A.mu_r * ri * F0 / wn;
+    Tr[0] = cr * wi.x;
+    Tr[1] = cr * wi.y;
+    Tr[2] = cr * wi.z;
+  }
+  const double Q = 2.0 - (double)A.move[sj];
+#pragma unroll
+  for (int x = 0; x < 3; ++x) {
+    B.f[x] += (Fn[x] + Fs[x]) * Q;
+    B.t[x] += (Ts[x] + Tr[x]) * Q;
+  }
 }
 
 // Linear spring-dashpot normal force with a tangential spring and a Coulomb
 // cap (Cundall & Strack, Geotechnique 29 (1979) 47-65; no reference
 // counterpart: the granular settle workload's law, behind the same calls as
-// the Hertz kernel above).  Per contact, n = (r_i - r_j)/|r_ij|,
+// the Hertz law above).  Per contact, n = (r_i - r_j)/|r_ij|,
 // delta = rad_i + rad_j - |r_ij|, 1/meff = minv_i + minv_j (0 for a fixed j):
 //   Fn = (kn delta - 2 zeta sqrt(meff kn) v_ij.n) n
 //   vt = tangential part of v_ij - (rad_i w_i + rad_j w_j) x n
@@ -261,70 +212,189 @@ __global__ void __launch_bounds__(256) k_dem_force(DemForceArgs A) {
 //        capped at mu |Fn| (the spring then follows the cap, s = -Ft/kt)
 //   F_i += Fn + Ft, T_i += (-rad_i n) x Ft
 // The history (3 doubles per contact) belongs to row i and is updated in
-// place.  FP64, one thread per storage slot as k_dem_force.
-__global__ void __launch_bounds__(256) k_dem_force_lsd(DemForceArgs A) {
-  const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= A.npad) return;
-  const uint32_t i = A.orig[s];
-  if (i == PB_NONE) return;
-  const double4 pi = A.r[s], vi = A.v[s], wi = A.w[s];
-  const double ri = A.rad[s];
-  double f[3] = {0, 0, 0}, t[3] = {0, 0, 0};
-  uint32_t bad = 0;
-  const uint32_t qe = min(A.row[i + 1], A.cap);
-  for (uint32_t q = A.row[i]; q < qe; ++q) {
-    const uint32_t sj = A.inv[A.col[q]];
-    const double4 pj = A.r[sj], vj = A.v[sj], wj = A.w[sj];
-    const double rj = A.rad[sj];
-    const double d[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
-    const double R2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
-    const double rs = ri + rj;
-    if (!(R2 < rs * rs)) continue;
-    const double R = sqrt(R2);
-    const double nv[3] = {d[0] / R, d[1] / R, d[2] / R};
-    const double delta = rs - R;
-    const double meff = 1.0 / (vi.w + (A.move[sj] ? vj.w : 0.0));
-    const double gn = 2.0 * A.zeta * sqrt(meff * A.kn);
-    if (!(A.dt < 2.0 * sqrt(meff / A.kn))) ++bad;
-    const double vij[3] = {vi.x - vj.x, vi.y - vj.y, vi.z - vj.z};
-    const double vn = vij[0] * nv[0] + vij[1] * nv[1] + vij[2] * nv[2];
-    const double fn = A.kn * delta - gn * vn;
-    const double W[3] = {ri * wi.x + rj * wj.x, ri * wi.y + rj * wj.y, ri * wi.z + rj * wj.z};
-    const double Wxn[3] = {W[1] * nv[2] - W[2] * nv[1], W[2] * nv[0] - W[0] * nv[2],
-                           W[0] * nv[1] - W[1] * nv[0]};
-    double *h = A.val + (size_t)q * 3;
-    const double h0 = h[0], h1 = h[1], h2 = h[2];
-    const double hn = h0 * nv[0] + h1 * nv[1] + h2 * nv[2];
-    double sp[3], ft[3];
-    sp[0] = h0 - hn * nv[0] + (vij[0] - Wxn[0] - vn * nv[0]) * A.dt;
-    sp[1] = h1 - hn * nv[1] + (vij[1] - Wxn[1] - vn * nv[1]) * A.dt;
-    sp[2] = h2 - hn * nv[2] + (vij[2] - Wxn[2] - vn * nv[2]) * A.dt;
+// place.
+__device__ __forceinline__ void contact_linear(const DemForceArgs &A, DemBody &B, uint32_t sj, double *h) {
+  const double4 &pi = B.p, &vi = B.v, &wi = B.w;
+  const double ri = B.rad;
+  const double4 pj = A.r[sj], vj = A.v[sj], wj = A.w[sj];
+  const double rj = A.rad[sj];
+  const double d[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
+  const double R2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
+  const double rs = ri + rj;
+  if (!(R2 < rs * rs)) return;
+  const double R = sqrt(R2);
+  const double nv[3] = {d[0] / R, d[1] / R, d[2] / R};
+  const double delta = rs - R;
+  const double meff = 1.0 / (vi.w + (A.move[sj] ? vj.w : 0.0));
+  const double gn = 2.0 * A.zeta * sqrt(meff * A.kn);
+  if (!(A.dt < 2.0 * sqrt(meff / A.kn))) ++B.bad;
+  const double vij[3] = {vi.x - vj.x, vi.y - vj.y, vi.z - vj.z};
+  const double vn = vij[0] * nv[0] + vij[1] * nv[1] + vij[2] * nv[2];
+  const double fn = A.kn * delta - gn * vn;
+  const double W[3] = {ri * wi.x + rj * wj.x, ri * wi.y + rj * wj.y, ri * wi.z + rj * wj.z};
+  const double Wxn[3] = {W[1] * nv[2] - W[2] * nv[1], W[2] * nv[0] - W[0] * nv[2],
+                         W[0] * nv[1] - W[1] * nv[0]};
+  const double h0 = h[0], h1 = h[1], h2 = h[2];
+  const double hn = h0 * nv[0] + h1 * nv[1] + h2 * nv[2];
+  double sp[3], ft[3];
+  sp[0] = h0 - hn * nv[0] + (vij[0] - Wxn[0] - vn * nv[0]) * A.dt;
+  sp[1] = h1 - hn * nv[1] + (vij[1] - Wxn[1] - vn * nv[1]) * A.dt;
+  sp[2] = h2 - hn * nv[2] + (vij[2] - Wxn[2] - vn * nv[2]) * A.dt;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) ft[k] = -A.kt * sp[k];
-    const double ftm = sqrt(ft[0] * ft[0] + ft[1] * ft[1] + ft[2] * ft[2]);
-    const double cap = A.mu * fabs(fn);
-    if (ftm > cap) {
-      const double c = cap / ftm;
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        ft[k] *= c;
-        sp[k] = -ft[k] / A.kt;
-      }
-    }
-    h[0] = sp[0];
-    h[1] = sp[1];
-    h[2] = sp[2];
-    const double nxf[3] = {nv[1] * ft[2] - nv[2] * ft[1], nv[2] * ft[0] - nv[0] * ft[2],
-                           nv[0] * ft[1] - nv[1] * ft[0]};
+  for (int k = 0; k < 3; ++k) ft[k] = -A.kt * sp[k];
+  const double ftm = sqrt(ft[0] * ft[0] + ft[1] * ft[1] + ft[2] * ft[2]);
+  const double cap = A.mu * fabs(fn);
+  if (ftm > cap) {
+    const double c = cap / ftm;
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      f[k] += fn * nv[k] + ft[k];
-      t[k] += -ri * nxf[k];
+      ft[k] *= c;
+      sp[k] = -ft[k] / A.kt;
     }
   }
-  A.F[s] = make_double4(f[0], f[1], f[2], 0.0);
-  A.T[s] = make_double4(t[0], t[1], t[2], 0.0);
-  if (bad) atomicAdd(A.bad, bad);
+  h[0] = sp[0];
+  h[1] = sp[1];
+  h[2] = sp[2];
+  const double nxf[3] = {nv[1] * ft[2] - nv[2] * ft[1], nv[2] * ft[0] - nv[0] * ft[2],
+                         nv[0] * ft[1] - nv[1] * ft[0]};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    B.f[k] += fn * nv[k] + ft[k];
+    B.t[k] += -ri * nxf[k];
+  }
+}
+
+// ascending order of N registers (Batcher's odd-even merge sort)
+template <int N>
+__device__ __forceinline__ void sort_registers(uint32_t (&a)[DEM_ROWBUF]) {
+#pragma unroll
+  for (int p = 1; p < N; p *= 2)
+#pragma unroll
+    for (int k = p; k >= 1; k /= 2)
+#pragma unroll
+      for (int j = k % p; j <= N - 1 - k; j += 2 * k)
+#pragma unroll
+        for (int i = 0; i < k; ++i)
+          if (i + j + k < N && (i + j) / (2 * p) == (i + j + k) / (2 * p)) {
+            const uint32_t x = min(a[i + j], a[i + j + k]), y = max(a[i + j], a[i + j + k]);
+            a[i + j] = x;
+            a[i + j + k] = y;
+          }
+}
+
+// The rows of the contact matrix, their history and the forces, one thread per
+// particle in cell order: makeJlist_WithBlock2/4_F4 (kernelfuncs.cu:1120-1216),
+// sortColIdx (:1262-1290), succeedPrevState (:1292-1309) and
+// calcF_IJpairWithList_F4 (kerneltemplate.hh:135-168) in one pass.  F and T are
+// overwritten (the reference clears both first, cudaParticleDEM.cu:168-169);
+// padding slots are not visited (they stay zero).
+// Bound by latency (a particle has none to a dozen contacts and every stage is
+// a dependent read), so a row that the counting scan kept whole is sorted in
+// registers, and its columns' slots and the previous row are read together
+// before the first contact; longer rows (more touching neighbours than any
+// sphere packing gives) are scanned again and merged in memory.  A contact
+// present in both matrices keeps its history (both rows are sorted); new ones
+// start at 0.  60,000 spheres of 6 contacts: 24 us, 200,000 with almost none:
+// 8 us; fill, carry and force as kernels of their own took 31 and 16 us.
+#define DEM_ROWS_BS 128
+template <int LAW, int W>
+__global__ void __launch_bounds__(DEM_ROWS_BS) k_dem_rows(DemGrid G, DemForceArgs A) {
+  __shared__ uint32_t sslot[DEM_ROWBUF][DEM_ROWS_BS];   // storage slot of a contact
+  __shared__ uint32_t sprev[DEM_ROWBUF][DEM_ROWS_BS];   // its place in the previous matrix
+  constexpr uint32_t HW = LAW == 1 ? 3u : 1u;
+  const uint32_t k = blockIdx.x * DEM_ROWS_BS + threadIdx.x, tid = threadIdx.x;
+  if (k >= G.n) return;
+  const uint32_t s = G.perm[k], i = G.so[k];
+  const uint32_t b = A.row[i], full = A.row[i + 1] - b;
+  // rows past the capacity: redone
+  const uint32_t e = min(b + full, G.cap), len = e > b ? e - b : 0u;
+  DemBody B;
+  if (len) {
+    B.p = A.r[s];
+    B.v = A.v[s];
+    B.w = A.w[s];
+    B.rad = A.rad[s];
+    uint32_t p = 0, pe = 0;
+    if (A.prow) {
+      p = A.prow[i];
+      pe = A.prow[i + 1];
+    }
+    auto contact = [&](uint32_t q, uint32_t sj, uint32_t from) {
+      double h[HW];
+#pragma unroll
+      for (uint32_t x = 0; x < HW; ++x) h[x] = from != PB_NONE ? A.pval[(size_t)from * HW + x] : 0.0;
+      if (LAW == 1) contact_linear(A, B, sj, h);
+      else contact_hertz(A, B, sj, h);
+#pragma unroll
+      for (uint32_t x = 0; x < HW; ++x) A.val[(size_t)q * HW + x] = h[x];
+    };
+    if (full <= DEM_ROWBUF) {               // the counting scan kept the whole row
+      uint32_t a[DEM_ROWBUF];
+      const uint4 *buf = reinterpret_cast<const uint4 *>(G.rowbuf + (size_t)i * DEM_ROWBUF);
+#pragma unroll
+      for (uint32_t x = 0; x < DEM_ROWBUF; x += 4) {
+        uint4 y = make_uint4(PB_NONE, PB_NONE, PB_NONE, PB_NONE);
+        if (x < full) y = buf[x / 4];
+        a[x] = x < full ? y.x : PB_NONE;
+        a[x + 1] = x + 1 < full ? y.y : PB_NONE;
+        a[x + 2] = x + 2 < full ? y.z : PB_NONE;
+        a[x + 3] = x + 3 < full ? y.w : PB_NONE;
+      }
+      if (__ballot(full > 8) == 0ull) sort_registers<8>(a);
+      else sort_registers<(int)DEM_ROWBUF>(a);
+#pragma unroll
+      for (uint32_t x = 0; x < DEM_ROWBUF; ++x)
+        if (x < len) {
+          A.col[b + x] = a[x];
+          sslot[x][tid] = A.inv[a[x]];
+          sprev[x][tid] = PB_NONE;
+        }
+      // the previous row, four columns at a time, against the sorted row
+      for (uint32_t q = p; q < pe; q += 4) {
+        uint32_t y[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) y[u] = A.pcol[min(q + u, pe - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+          if (q + u >= pe) continue;
+#pragma unroll
+          for (uint32_t x = 0; x < DEM_ROWBUF; ++x)
+            if (x < len && a[x] == y[u]) sprev[x][tid] = q + u;
+        }
+      }
+      for (uint32_t x = 0; x < len; ++x) contact(b + x, sslot[x][tid], sprev[x][tid]);
+    } else {
+      uint32_t m = b;
+      dem_contacts<W>(G, k, G.rs[k], [&](uint32_t q) {
+        if (m < e) A.col[m++] = G.so[q];
+      });
+      for (uint32_t x = b + 1; x < e; ++x) {
+        const uint32_t v = A.col[x];
+        uint32_t y = x;
+        while (y > b && A.col[y - 1] > v) {
+          A.col[y] = A.col[y - 1];
+          --y;
+        }
+        A.col[y] = v;
+      }
+      for (uint32_t q = b; q < e; ++q) {
+        const uint32_t j = A.col[q];
+        while (p < pe && A.pcol[p] < j) ++p;
+        contact(q, A.inv[j], p < pe && A.pcol[p] == j ? p : PB_NONE);
+      }
+    }
+  }
+  A.F[s] = make_double4(B.f[0], B.f[1], B.f[2], 0.0);
+  A.T[s] = make_double4(B.t[0], B.t[1], B.t[2], 0.0);
+  if (B.bad) atomicAdd(A.bad, B.bad);
+}
+
+// nnz and the time-step check to pinned memory
+__global__ void k_dem_result(const uint32_t *nnz, const uint32_t *bad, uint32_t *out) {
+  if (threadIdx.x == 0) {
+    out[0] = *nnz;
+    out[1] = *bad;
+  }
 }
 
 __global__ void k_dem_inv(const uint32_t *orig, uint32_t n, uint32_t *inv) {
@@ -494,45 +564,48 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
   hipStream_t st = s->ctx->stream;
   const uint32_t n = s->n;
   int rc;
-  if (!s->dem_inv) {
-    if ((rc = pb_alloc(s->ctx, &s->dem_inv, (size_t)n + 1))) return rc;
-  }
-  hipLaunchKernelGGL(k_dem_inv, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->orig, s->npad,
-                     s->dem_inv);
+  if ((rc = pb_results(s->ctx))) return rc;
   if (!s->dem_rs) {
-    if ((rc = pb_alloc(s->ctx, &s->dem_rs, s->npad)) || (rc = pb_alloc(s->ctx, &s->dem_so, s->npad)) ||
-        (rc = pb_alloc(s->ctx, &s->dem_rowbuf, (size_t)s->npad * DEM_ROWBUF)))
+    if ((rc = pb_alloc(s->ctx, &s->dem_inv, (size_t)n + 1)) ||
+        (rc = pb_alloc(s->ctx, &s->dem_rowbuf, (size_t)s->npad * DEM_ROWBUF)) ||
+        (rc = pb_alloc(s->ctx, &s->dem_rs, s->npad)))
       return rc;
   }
-  if (n)
-    hipLaunchKernelGGL(k_dem_gather, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->perm, s->r,
-                       s->radius, s->orig, n, s->dem_rs, s->dem_so);
+  if (s->dem_inv_order != s->order_gen) {
+    hipLaunchKernelGGL(k_dem_inv, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->orig, s->npad,
+                       s->dem_inv);
+    s->dem_inv_order = s->order_gen;
+  }
+  hipLaunchKernelGGL(k_dem_gather, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->perm, s->r,
+                     s->radius, n, s->dem_rs);
   DemGrid G;
   G.perm = s->perm;
-  G.cellid = s->cellid;
+  G.bid = s->ref_bid;
   G.cstart = s->cstart;
   G.rs = s->dem_rs;
-  G.so = s->dem_so;
+  G.so = s->ref_pid;
   G.rowbuf = s->dem_rowbuf;
   G.move = s->move;
   for (int a = 0; a < 3; ++a) G.nb[a] = s->blocknum[a];
-  G.w = s->ref_single ? 2 : 1;
   G.n = n;
   const int b = (s->cm_cur + 1) & 1;         // the other buffer keeps the previous matrix
   // capacity from the previous matrix (ensure_csr adds a quarter)
   if ((rc = ensure_csr(s, b, s->cm_cur >= 0 ? s->cm_nnz[s->cm_cur] : 0))) return rc;
+  G.cap = s->cm_cap[b];
   // per-row counts go to the sort workspace's rank array (free once pb_bin
   // has produced perm / cstart), their exclusive scan to the new row array
-  uint32_t *cnt = s->rank;
-  const uint32_t grid = pb_blocks(n ? n : 1, 256);
-  if (n) {
-    hipLaunchKernelGGL(k_dem_count, dim3(grid), dim3(256), 0, st, G, cnt);
-    PB_LAUNCH_CHECK(s->ctx, "k_dem_count");
-  }
+  uint32_t *cnt = s->rank, *bad = s->d_counter + 8;
+  const bool single = s->ref_single != 0;    // 125 cells of one particle, else 27
+  hipLaunchKernelGGL(single ? k_dem_count<2> : k_dem_count<1>, dim3(pb_blocks(n, 256)), dim3(256), 0,
+                     st, G, cnt, bad);
+  PB_LAUNCH_CHECK(s->ctx, "k_dem_count");
   if ((rc = pb_exclusive_scan(s, cnt, s->cm_row[b], n))) return rc;
+  const int p = s->cm_cur;
   DemForceArgs A;
-  A.orig = s->orig;
   A.inv = s->dem_inv;
+  A.prow = p >= 0 ? s->cm_row[p] : nullptr;
+  A.pcol = p >= 0 ? s->cm_col[p] : nullptr;
+  A.pval = p >= 0 ? s->cm_val[p] : nullptr;
   A.r = s->r;
   A.v = s->v;
   A.w = s->w;
@@ -540,9 +613,7 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
   A.move = s->move;
   A.F = s->F;
   A.T = s->T;
-  A.bad = s->d_counter + 8;
-  A.n = n;
-  A.npad = s->npad;
+  A.bad = bad;
   A.E = s->dem_E;
   A.mu = s->dem_mu;
   A.s2 = s->dem_s2;
@@ -552,52 +623,37 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
   A.kn = s->dem_kn;
   A.zeta = s->dem_zeta;
   A.kt = s->dem_kt;
-  const int p = s->cm_cur;
-  // fill + sort, history carry, contact forces and torques up to the
-  // capacity; then nnz and the time-step check in one read
+  auto rows = s->dem_law == 1 ? (single ? k_dem_rows<1, 2> : k_dem_rows<1, 1>)
+                              : (single ? k_dem_rows<0, 2> : k_dem_rows<0, 1>);
+  // rows, history and forces up to the capacity; then nnz and the time-step
+  // check in one wait
+  uint32_t nnz = 0, nbad = 0;
   auto contacts_and_force = [&]() -> int {
-    G.cap = A.cap = s->cm_cap[b];
+    G.cap = s->cm_cap[b];
     A.row = s->cm_row[b];
     A.col = s->cm_col[b];
     A.val = s->cm_val[b];
-    if (n) {
-      hipLaunchKernelGGL(k_dem_fill, dim3(grid), dim3(256), 0, st, G, s->cm_row[b], s->cm_col[b]);
-      hipLaunchKernelGGL(k_dem_carry, dim3(grid), dim3(256), 0, st,
-                         p >= 0 ? s->cm_row[p] : (const uint32_t *)nullptr,
-                         p >= 0 ? s->cm_col[p] : (const uint32_t *)nullptr,
-                         p >= 0 ? s->cm_val[p] : (const double *)nullptr, s->cm_row[b],
-                         s->cm_col[b], s->cm_val[b], n, s->cm_cap[b], s->dem_hw);
-      PB_LAUNCH_CHECK(s->ctx, "k_dem_fill/carry");
-    }
-    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, s->d_counter + 8, 1u, 0u);
-    // every real particle's F and T is written (empty rows give zero);
-    // padding slots are never written and stay zero
-    if (n) {
-      if (s->dem_law == 1)
-        hipLaunchKernelGGL(k_dem_force_lsd, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, A);
-      else
-        hipLaunchKernelGGL(k_dem_force, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, A);
-    }
-    PB_LAUNCH_CHECK(s->ctx, "k_dem_force");
+    hipLaunchKernelGGL(rows, dim3(pb_blocks(n, DEM_ROWS_BS)), dim3(DEM_ROWS_BS), 0, st, G, A);
+    hipLaunchKernelGGL(k_dem_result, dim3(1), dim3(64), 0, st, s->cm_row[b] + n, bad,
+                       (uint32_t *)s->ctx->res_dev);
+    PB_LAUNCH_CHECK(s->ctx, "k_dem_rows");
+    PB_HIP(s->ctx, hipStreamSynchronize(st));
+    nnz = ((const uint32_t *)s->ctx->res)[0];
+    nbad = ((const uint32_t *)s->ctx->res)[1];
     return PB_OK;
   };
   if ((rc = contacts_and_force())) return rc;
-  uint32_t nnz = 0, bad = 0;
-  PB_HIP(s->ctx, hipMemcpyAsync(&nnz, s->cm_row[b] + n, 4, hipMemcpyDeviceToHost, st));
-  PB_HIP(s->ctx, hipMemcpyAsync(&bad, s->d_counter + 8, 4, hipMemcpyDeviceToHost, st));
-  PB_HIP(s->ctx, hipStreamSynchronize(st));
   if (nnz > s->cm_cap[b]) {                  // the matrix outgrew the arrays: again, larger
+    hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(64), 0, st, bad, 1u, 0u);
     if ((rc = ensure_csr(s, b, nnz)) || (rc = contacts_and_force())) return rc;
-    PB_HIP(s->ctx, hipMemcpyAsync(&bad, s->d_counter + 8, 4, hipMemcpyDeviceToHost, st));
-    PB_HIP(s->ctx, hipStreamSynchronize(st));
   }
   s->cm_nnz[b] = nnz;
   s->cm_prev = p >= 0;
   s->cm_rewound = false;
   s->cm_cur = b;
-  s->dem_bad = bad;
+  s->dem_bad = nbad;
   if (nnz_out) *nnz_out = nnz;
-  if (bad && !autotune)
+  if (nbad && !autotune)
     return pb_fail(s->ctx, PB_ERR_DT, "DEM: time step above the Cundall-Strack bound 2 sqrt(m/Kn)");
   return PB_OK;
 }

@@ -217,8 +217,8 @@ struct pb_sys {
   bool cm_prev = false;                        // the other buffer holds the matrix before it
   bool cm_rewound = false;                     // the last matrix operation was pb_dem_rewind
   uint32_t *dem_inv = nullptr;                 // original index -> storage slot
+  uint32_t dem_inv_order = 0;                  // order_gen dem_inv was made for (0: none)
   double4 *dem_rs = nullptr;                   // cell order: (x, y, z, radius)
-  uint32_t *dem_so = nullptr;                  // cell order: original index
   uint32_t *dem_rowbuf = nullptr;              // contacts kept by the counting scan
   uint32_t dem_bad = 0;                        // Cundall-Strack violations of the last call
 };

@@ -57,13 +57,31 @@ __device__ __forceinline__ uint32_t block_excl_scan(uint32_t x, uint32_t *total)
   return off + inc - x;
 }
 
+// a thread's SCAN_PER consecutive elements (0 past the end), 16 bytes a load
+__device__ __forceinline__ void scan_load(const uint32_t *in, uint32_t n, uint32_t base,
+                                          uint32_t (&v)[SCAN_PER]) {
+  if (base + SCAN_PER <= n) {
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; k += 4) {
+      const uint4 y = *reinterpret_cast<const uint4 *>(in + base + k);
+      v[k] = y.x;
+      v[k + 1] = y.y;
+      v[k + 2] = y.z;
+      v[k + 3] = y.w;
+    }
+  } else {
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; ++k) v[k] = base + k < n ? in[base + k] : 0u;
+  }
+}
+
 __global__ void __launch_bounds__(SCAN_BS) k_scan_reduce(const uint32_t *in, uint32_t n,
                                                          uint32_t *bsum) {
   const uint32_t base = blockIdx.x * SCAN_CH + threadIdx.x * SCAN_PER;
-  uint32_t x = 0;
+  uint32_t v[SCAN_PER], x = 0;
+  scan_load(in, n, base, v);
 #pragma unroll
-  for (int k = 0; k < SCAN_PER; ++k)
-    if (base + k < n) x += in[base + k];
+  for (int k = 0; k < SCAN_PER; ++k) x += v[k];
   uint32_t tot;
   (void)block_excl_scan(x, &tot);
   if (threadIdx.x == 0) bsum[blockIdx.x] = tot;
@@ -79,21 +97,27 @@ __global__ void __launch_bounds__(SCAN_BS) k_scan_final(const uint32_t *in, uint
   uint32_t before;
   (void)block_excl_scan(pre, &before);
   const uint32_t base = blockIdx.x * SCAN_CH + threadIdx.x * SCAN_PER;
-  uint32_t v[SCAN_PER];
-  uint32_t x = 0;
+  uint32_t v[SCAN_PER], x = 0;
+  scan_load(in, n, base, v);
 #pragma unroll
-  for (int k = 0; k < SCAN_PER; ++k) {
-    v[k] = (base + k < n) ? in[base + k] : 0u;
-    x += v[k];
-  }
+  for (int k = 0; k < SCAN_PER; ++k) x += v[k];
   uint32_t tot;
   uint32_t run = block_excl_scan(x, &tot) + before;
 #pragma unroll
-  for (int k = 0; k < SCAN_PER; ++k)
-    if (base + k < n) {
-      out[base + k] = run;
-      run += v[k];
-    }
+  for (int k = 0; k < SCAN_PER; ++k) {
+    const uint32_t y = v[k];
+    v[k] = run;
+    run += y;
+  }
+  if (base + SCAN_PER <= n) {
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; k += 4)
+      *reinterpret_cast<uint4 *>(out + base + k) = make_uint4(v[k], v[k + 1], v[k + 2], v[k + 3]);
+  } else {
+#pragma unroll
+    for (int k = 0; k < SCAN_PER; ++k)
+      if (base + k < n) out[base + k] = v[k];
+  }
   if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) out[n] = before + tot;
 }
 
