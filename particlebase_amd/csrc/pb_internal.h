@@ -192,7 +192,10 @@ struct pb_sys {
   // SPH (cudaParticleSPH_NS), storage order unless noted
   double *sph_mu0 = nullptr, *sph_c2 = nullptr, *sph_rhoinv = nullptr;
   double4 *sph_num = nullptr;                  // (number density, rho, mu or p, 0)
-  double4 *sph_rs = nullptr, *sph_vs = nullptr, *sph_ds = nullptr;   // cell-sorted views
+  double4 *sph_rs = nullptr, *sph_vs = nullptr;   // cell-sorted views
+  double2 *sph_ds = nullptr;
+  double *sph_mus = nullptr;
+  float4 *sph_fq = nullptr;
   double sph_h = 0.0, sph_rho0 = 1.0;
   bool sph_set = false, sph_dens = false;
   // 0: reference physics (Lucy, linear EOS, mu); 1: weakly compressible
@@ -355,6 +358,12 @@ __device__ __forceinline__ uint32_t pb_wave_sum_u32(uint32_t x) {
   for (int o = 32; o > 0; o >>= 1) x += (uint32_t)__shfl_xor((int)x, o, 64);
   return x;
 }
+// LDS written by some lanes of a wavefront and read by others of it: LDS
+// operations of one wavefront complete in order, so only the compiler is held
+__device__ __forceinline__ void pb_wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
 __device__ __forceinline__ double pb_wave_max(double x) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
@@ -369,6 +378,13 @@ __device__ __forceinline__ double pb_wave_max(double x) {
 __device__ __forceinline__ uint32_t pb_xcd_chunk8() {
   const uint32_t b = blockIdx.x, full = gridDim.x & ~63u;
   return b < full ? (b & ~63u) + (b & 7u) * 8u + ((b >> 3) & 7u) : b;
+}
+
+// the same with C consecutive logical blocks a XCD within every 8 C
+template <uint32_t C>
+__device__ __forceinline__ uint32_t pb_xcd_chunk() {
+  const uint32_t b = blockIdx.x, full = gridDim.x / (8u * C) * (8u * C);
+  return b < full ? b / (8u * C) * (8u * C) + (b & 7u) * C + (b >> 3) % C : b;
 }
 
 __device__ __forceinline__ double pb_load_relaxed(const double *p) {

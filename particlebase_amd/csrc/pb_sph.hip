@@ -27,16 +27,18 @@
 
 struct SphGrid {
   uint32_t nb[3];
+  float len[3], lo[3];
 };
 
 struct SphArgs {
   const uint32_t *perm;      // sorted slot -> storage slot
-  const uint32_t *cellid;    // storage slot -> cell
+  const uint32_t *bid;       // sorted slot -> cell
   const uint32_t *cstart;    // cell -> first sorted slot (cstart[c+1] ends it)
+  const float4 *fq;          // sorted filter view (sph_view)
   const double4 *rs;         // sorted (x, y, z, m)
-  const double4 *vs;         // sorted (vx, vy, vz, mu0 or mu)
-  double4 *ds;               // sorted (1/rho, P, mu, 0) from the density pass;
-                             // (rho, p/rho^2, 0, 0) under the config physics
+  const double4 *vs;         // acceleration: sorted (vx, vy, vz, 1/rho; rho under the config physics)
+  const double2 *ds;         // acceleration: sorted (P, mu); (p/rho^2, 0) under the config physics
+  const double *mus;         // density: sorted mu0
   SphGrid g;
   uint32_t n;
   double h, w0, w1, rho0;
@@ -45,73 +47,96 @@ struct SphArgs {
   double sup2, hinv, ws, wf, B, rho0inv, gamma, pmin, avh, eh2;
 };
 
-// positions (mass in w), velocities, mu0 in cell order (density call)
-__global__ void k_sph_gather(const uint32_t *perm, const double4 *r, const double4 *v,
-                             const double *mu0, uint32_t n, double4 *rs, double4 *vs) {
+// FP32 filter: the bound on |r_ij|^2 with the rounding margin, and the ranges of
+// the coordinates that the margin covers
+struct SphFilter {
+  float r2, l2, zmax;
+};
+
+// Filter view of a particle of cell c: x and y from the middle of its cell
+// column, z from the grid's edge, and x^2 + y^2; a particle beyond the margin's
+// ranges (outside the grid, binned into its edge cells; NaN) passes every test.
+__device__ __forceinline__ float4 sph_view(const SphGrid &g, const SphFilter &FB, uint32_t c,
+                                           const double4 &p) {
+  const uint32_t col = c / g.nb[2], i = col / g.nb[1], j = col % g.nb[1];
+  const float x = (float)(p.x - ((double)g.lo[0] + ((double)i + 0.5) * (double)g.len[0]));
+  const float y = (float)(p.y - ((double)g.lo[1] + ((double)j + 0.5) * (double)g.len[1]));
+  const float z = (float)(p.z - (double)g.lo[2]);
+  const float w = x * x + y * y;
+  return w <= FB.l2 && fabsf(z) <= FB.zmax ? make_float4(x, y, z, w)
+                                           : make_float4(0.f, 0.f, 0.f, -INFINITY);
+}
+
+// positions (mass in w), the filter view and mu0 in cell order (density call)
+__global__ void k_sph_gather(const uint32_t *perm, const uint32_t *bid, const double4 *r,
+                             const double4 *v, const double *mu0, SphGrid g, SphFilter FB,
+                             uint32_t n, double4 *rs, float4 *fq, double *mus) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const uint32_t s = perm[k];
-  const double4 p = r[s], u = v[s];
-  rs[k] = make_double4(p.x, p.y, p.z, 1.0 / u.w);
-  vs[k] = make_double4(u.x, u.y, u.z, mu0 ? mu0[s] : 0.0);
+  const double4 p = r[s];
+  rs[k] = make_double4(p.x, p.y, p.z, 1.0 / v[s].w);
+  fq[k] = sph_view(g, FB, bid[k], p);
+  if (mu0) mus[k] = mu0[s];
 }
 
 // Acceleration call: positions, velocities and the per-particle terms of the
 // last density call, read from the storage-order outputs, so a pb_bin
-// between the two calls is harmless.  Reference physics: ds = (1/rho,
-// c2/rho (1 - rho0/rho), mu); config physics: ds = (rho, p/rho^2).
-__global__ void k_sph_gather_acc(const uint32_t *perm, const double4 *r, const double4 *v,
-                                 const double4 *num, const double *rhoinv, const double *c2,
-                                 double rho0, int wc, uint32_t n, double4 *rs, double4 *vs,
-                                 double4 *ds) {
+// between the two calls is harmless.  Reference physics: 1/rho, and ds =
+// (c2/rho (1 - rho0/rho), mu); config physics: rho, and ds = (p/rho^2, -).
+__global__ void k_sph_gather_acc(const uint32_t *perm, const uint32_t *bid, const double4 *r,
+                                 const double4 *v, const double4 *num, const double *rhoinv,
+                                 const double *c2, double rho0, int wc, SphGrid g, SphFilter FB,
+                                 uint32_t n, double4 *rs, float4 *fq, double4 *vs, double2 *ds) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const uint32_t s = perm[k];
   const double4 p = r[s], u = v[s], d = num[s];
   const double ri = rhoinv[s];
   rs[k] = make_double4(p.x, p.y, p.z, 1.0 / u.w);
-  vs[k] = make_double4(u.x, u.y, u.z, 0.0);
-  ds[k] = wc ? make_double4(d.y, d.z * ri * ri, 0.0, 0.0)
-             : make_double4(ri, c2[s] * ri * (1.0 - rho0 * ri), d.z, 0.0);
+  fq[k] = sph_view(g, FB, bid[k], p);
+  vs[k] = make_double4(u.x, u.y, u.z, wc ? d.y : ri);
+  ds[k] = wc ? make_double2(d.z * ri * ri, 0.0)
+             : make_double2(c2[s] * ri * (1.0 - rho0 * ri), d.z);
 }
 
 // ---------------------------------------------------------------------------
-// Pair kernels.  One workgroup per segment of zseg cells of a cell column
-// (i, j): the segment's sorted slots are taken 256 at a time, one thread
-// each.  For each of the 9 neighbour columns the candidates of cells
-// z-1 .. z+1 of every thread in the chunk form one contiguous sorted range;
-// it is staged into LDS (coalesced loads, sph_cap<M>() at a time) and each
-// thread scans its own 3-cell window of it:
-//   * a conservative FP32 filter, 32 candidates per step into a bit mask:
-//     |ri - rj|^2 = |ri|^2 + |rj|^2 - 2 ri.rj in coordinates relative to
-//     the segment's first particle, against r2max plus a margin that covers
-//     the FP32 rounding of that form;
-//   * the FP64 pair body per set bit, from the staged FP64 fields, which
-//     applies the exact support test itself (so the margin changes nothing).
-// Pairs are visited in the order of a per-particle 27-cell loop (neighbour
-// columns in (a, b) order, slots ascending).
-constexpr uint32_t SC_T = 256;     // threads per workgroup, one sorted slot each
-
-// FP32 pre-filter bound r2 (r2max plus the rounding margin) and the squared
-// coordinate range l2 that the margin covers
-struct SphFilter {
-  float r2, l2;
-};
+// Pair kernels.  LN lanes per sorted slot, 64 / LN consecutive slots a wavefront.
+// In each of the 9 neighbour columns the cells z-1 .. z+1 of a slot are one
+// contiguous sorted range (its window), and the windows of a wavefront's slots
+// overlap: their union is staged into LDS, SC_CAP filter views at a time (loaded
+// while the column before is tested), and each lane scans its share of its own
+// window, every LN-th candidate:
+//   * a conservative FP32 filter, up to 32 candidates into a bit mask:
+//     |ri - rj|^2 < r2max plus a margin that covers the FP32 rounding, from
+//     coordinates relative to the candidates' column (6 instructions a test);
+//   * the hits are appended to the lane's list in LDS, and the lists are worked
+//     off together when one of them is full and at the end, so that lanes wait
+//     for the largest number of hits of all columns instead of the largest of
+//     each (Lucy, h = 1.7 dx: 21 in place of 36 a wavefront for 20 a particle);
+//   * the FP64 pair body on the cell-order views, which applies the exact
+//     support test itself (so the margin changes nothing).
+// A wavefront whose slots lie thinly (a floor, a splash) can span many dense
+// neighbour columns of which it needs little: past SC_DIRECT candidates the lanes
+// read their windows from memory.  Such wavefronts, one in a hundred, took up
+// to eight times the others' time and were the kernel's end (796,176 particles:
+// 97 us with this, 114 without).
+// Bound by vector instructions (about 60 % of the time) and by the latency of
+// the loads between them.  Density and acceleration of 796,176 particles, Lucy,
+// 20 pairs each: 202 and 270 us with a workgroup a column segment (wavefronts
+// two thirds full, two barriers a column), now 95 and 134 us; 133,904 of the
+// config physics, 66 pairs: 99 and 174, now 56 and 78 us.
+// A slot's pairs are visited in the order of a 27-cell loop (neighbour columns in
+// (a, b) order, slots ascending), each lane its share of them; the lanes' sums
+// are added in a fixed order.
+constexpr uint32_t SC_T = 64;       // a wavefront is a workgroup: none waits for another's end
+constexpr uint32_t SC_CAP = 128;    // candidates staged at a time
+constexpr uint32_t SC_DIRECT = 256; // longer unions are read directly
+constexpr uint32_t SC_HITS = 20;    // hits a lane keeps
+constexpr uint32_t SC_W = 2;        // hits worked off at a time
+constexpr uint32_t SC_G = 8;        // tests at a time
 
 enum { SPH_LUCY_DENS = 0, SPH_LUCY_ACC = 1, SPH_WC_DENS = 2, SPH_WC_ACC = 3 };
-
-// staged FP64 fields per candidate: x, y, z, m, then
-//   Lucy density: mu0 | Lucy accel: vx, vy, vz, 1/rho, P, mu |
-//   config density: - | config accel: vx, vy, vz, rho, P
-template <int M>
-constexpr int sph_nf() {
-  return M == SPH_LUCY_DENS ? 5 : M == SPH_LUCY_ACC ? 10 : M == SPH_WC_DENS ? 4 : 9;
-}
-// candidates per batch: LDS of a workgroup stays below 40 KB (4 per CU)
-template <int M>
-constexpr uint32_t sph_cap() {
-  return (M == SPH_LUCY_ACC || M == SPH_WC_ACC) ? 384u : 512u;
-}
 
 // 1/sqrt(x), x > 0: the hardware estimate and two Newton steps (about one
 // ulp); and 1/x the same way
@@ -142,225 +167,266 @@ __device__ __forceinline__ double sph_norm(double r2, double *rinv) {
   return r2 * y;
 }
 
+// the fields of a particle that pass M reads
+struct SphBody {
+  double4 p, v;
+  double2 d;
+  double mu;
+};
 template <int M>
-__device__ __forceinline__ void sph_pairs(const SphArgs &A, uint32_t zseg, SphFilter FB,
-                                          double4 *out4, double *out1) {
-  constexpr int NF = sph_nf<M>();
-  constexpr uint32_t CAP = sph_cap<M>();
-  __shared__ double L[NF][CAP];
-  __shared__ float4 Fq[CAP + 64];             // filter view; 64 spare for the last step
-  const uint32_t nz = A.g.nb[2], ny = A.g.nb[1];
-  const uint32_t ncol = A.g.nb[0] * ny;
-  // 1-D grid of (z segment, column), columns fastest.  Workgroups go to the
-  // XCDs round-robin; within every 64 workgroups XCD x takes 8 consecutive
-  // columns, which share neighbour columns in its L2, while the fine
-  // interleave keeps dense and empty regions spread over all XCDs.
-  const uint32_t lb = pb_xcd_chunk8();
-  const uint32_t col = lb % ncol;
-  const int ci = (int)(col / ny), cj = (int)(col % ny);
-  // this workgroup's cells: z in [zs, ze) of column col
-  const uint32_t zs = (lb / ncol) * zseg, ze = zs + zseg < nz ? zs + zseg : nz;
-  const uint32_t s0 = A.cstart[col * nz + zs], s1 = A.cstart[col * nz + ze];
-  if (s0 >= s1) return;
-  const double4 O = A.rs[s0];                 // origin of the filter coordinates
-  for (uint32_t c0 = s0; c0 < s1; c0 += SC_T) {
-    const uint32_t c1 = c0 + SC_T < s1 ? c0 + SC_T : s1;
-    const uint32_t k = c0 + threadIdx.x;
-    const bool act = k < c1;
-    uint32_t s = 0, kz = 0;
-    double4 pi = O, vi = make_double4(0.0, 0.0, 0.0, 0.0), di = vi;
-    if (act) {
-      s = A.perm[k];
-      kz = A.cellid[s] % nz;
-      pi = A.rs[k];
-      if constexpr (M == SPH_LUCY_ACC || M == SPH_WC_ACC) {
-        vi = A.vs[k];
-        di = A.ds[k];
-      }
+__device__ __forceinline__ SphBody sph_load(const SphArgs &A, uint32_t q) {
+  SphBody B;
+  B.p = A.rs[q];
+  if constexpr (M == SPH_LUCY_DENS) B.mu = A.mus[q];
+  if constexpr (M == SPH_LUCY_ACC || M == SPH_WC_ACC) {
+    B.v = A.vs[q];
+    B.d = A.ds[q];
+  }
+  return B;
+}
+
+// one pair; self: the particle with itself
+template <int M>
+__device__ __forceinline__ void sph_pair(const SphArgs &A, const SphBody &I, const SphBody &J,
+                                         bool self, double &acc0, double &acc1, double &acc2) {
+  const double4 &pi = I.p, &vi = I.v, &pj = J.p, &vj = J.v;
+  if constexpr (M == SPH_LUCY_DENS) {
+    // SPHcalcDensity<SPHKernelLucy> (kerneltemplate.hh:636-656):
+    // W = w0 (h + 3R)(h - R)^3, 0 beyond h (kernelinline.hh:182-188)
+    const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+    double ri;
+    const double R = sph_norm(dx * dx + dy * dy + dz * dz, &ri);
+    const double tt = fmax(A.h - R, 0.0);
+    const double W = A.w0 * (A.h + 3.0 * R) * (tt * tt * tt);
+    const double mW = pj.w * W;
+    acc0 += W;
+    acc1 += mW;
+    acc2 = fma(J.mu, mW, acc2);
+  } else if constexpr (M == SPH_LUCY_ACC) {
+    // SPHNavierStokes<SPHKernelLucyDW> (kerneltemplate.hh:666-709)
+    const double dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+    double ri;
+    const double R = sph_norm(dx * dx + dy * dy + dz * dz, &ri);
+    const double tt = A.h - R;
+    if (tt > 0.0 && !self) {                    // no self term, 0 beyond h
+      const double mw = pj.w * (A.w1 * tt * tt);  // m_j (dW/dr)/r, kernelinline.hh:209-214
+      const double p1 = I.d.x + J.d.x;
+      const double v1 = (I.d.y + J.d.y) * vi.w * vj.w;
+      acc0 += mw * (dx * p1 - (vj.x - vi.x) * v1);
+      acc1 += mw * (dy * p1 - (vj.y - vi.y) * v1);
+      acc2 += mw * (dz * p1 - (vj.z - vi.z) * v1);
     }
-    // filter constants: -2 ri and r2 margin - |ri|^2, FP32, relative to O;
-    // a particle farther from O than the margin covers (outside the cell
-    // grid) passes every candidate to the exact test
-    const float xf = (float)(pi.x - O.x), yf = (float)(pi.y - O.y), zf = (float)(pi.z - O.z);
-    const float fx = -2.0f * xf, fy = -2.0f * yf, fz = -2.0f * zf;
-    const float bi = xf * xf + yf * yf + zf * zf;
-    const float lim = bi <= FB.l2 ? FB.r2 - bi : INFINITY;
-    // z range of the chunk (slots are sorted by cell, so by z in a column)
-    const uint32_t za = A.cellid[A.perm[c0]] % nz, zb = A.cellid[A.perm[c1 - 1]] % nz;
-    const uint32_t zlo = za > 0 ? za - 1 : 0, zhi = zb + 1 < nz ? zb + 1 : zb;
-    const uint32_t klo = kz > 0 ? kz - 1 : 0, khi = kz + 1 < nz ? kz + 1 : kz;
-    double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
-    for (int a = -1; a <= 1; ++a) {
-      const int i2 = ci + a;
-      if (i2 < 0 || i2 >= (int)A.g.nb[0]) continue;
-      for (int b = -1; b <= 1; ++b) {
-        const int j2 = cj + b;
-        if (j2 < 0 || j2 >= (int)ny) continue;
-        const uint32_t cb = ((uint32_t)i2 * ny + (uint32_t)j2) * nz;
-        const uint32_t r0 = A.cstart[cb + zlo], r1 = A.cstart[cb + zhi + 1];
-        uint32_t w0 = 0, w1 = 0;          // this thread's window (empty if inactive)
-        if (act) {
-          w0 = A.cstart[cb + klo];
-          w1 = A.cstart[cb + khi + 1];
-        }
-        for (uint32_t b0 = r0; b0 < r1; b0 += CAP) {
-          const uint32_t b1 = b0 + CAP < r1 ? b0 + CAP : r1;
-          __syncthreads();                // the previous batch is consumed
-          for (uint32_t t = threadIdx.x; t < b1 - b0; t += SC_T) {
-            const double4 pj = A.rs[b0 + t];
-            L[0][t] = pj.x;
-            L[1][t] = pj.y;
-            L[2][t] = pj.z;
-            L[3][t] = pj.w;
-            const float xr = (float)(pj.x - O.x), yr = (float)(pj.y - O.y),
-                        zr = (float)(pj.z - O.z);
-            const float bj = xr * xr + yr * yr + zr * zr;
-            // beyond the margin's range: a filter entry every thread passes
-            Fq[t] = bj <= FB.l2 ? make_float4(xr, yr, zr, bj) : make_float4(0.f, 0.f, 0.f, -INFINITY);
-            if constexpr (M == SPH_LUCY_DENS) {
-              L[4][t] = A.vs[b0 + t].w;
-            } else if constexpr (M == SPH_LUCY_ACC || M == SPH_WC_ACC) {
-              const double4 vj = A.vs[b0 + t], dj = A.ds[b0 + t];
-              L[4][t] = vj.x;
-              L[5][t] = vj.y;
-              L[6][t] = vj.z;
-              L[7][t] = dj.x;
-              L[8][t] = dj.y;
-              if constexpr (M == SPH_LUCY_ACC) L[9][t] = dj.z;
-            }
-          }
-          __syncthreads();
-          const uint32_t q0 = w0 > b0 ? w0 : b0, q1 = w1 < b1 ? w1 : b1;
-          for (uint32_t base = q0; base < q1; base += 64) {
-            const uint32_t t0 = base - b0;
-            // 64 tests, two 32-bit halves (entries past the window are
-            // masked off below; Fq has 64 spare entries so the reads stay
-            // inside the array).  A window of three cells usually fits in
-            // one step, so the pair loop below runs the largest per-lane hit
-            // count of the window once.
-            uint32_t lo = 0, hi = 0;
-#pragma unroll 1
-            for (uint32_t g = 0; g < 32; g += 8) {
-#pragma unroll
-              for (uint32_t u = 0; u < 8; ++u) {
-                const float4 f = Fq[t0 + g + u];
-                if (fmaf(fx, f.x, fmaf(fy, f.y, fmaf(fz, f.z, f.w))) < lim) lo |= 1u << (g + u);
-              }
-            }
-            if (q1 - base > 32u) {
-#pragma unroll 1
-              for (uint32_t g = 0; g < 32; g += 8) {
-#pragma unroll
-                for (uint32_t u = 0; u < 8; ++u) {
-                  const float4 f = Fq[t0 + 32 + g + u];
-                  if (fmaf(fx, f.x, fmaf(fy, f.y, fmaf(fz, f.z, f.w))) < lim) hi |= 1u << (g + u);
-                }
-              }
-            }
-            uint64_t mask = ((uint64_t)hi << 32) | lo;
-            if (q1 - base < 64u) mask &= (1ull << (q1 - base)) - 1ull;
-            while (mask) {
-              const uint32_t u = (uint32_t)__builtin_ctzll(mask);
-              mask &= mask - 1;
-              const uint32_t j = t0 + u, q = base + u;
-              const double xj = L[0][j], yj = L[1][j], zj = L[2][j], mj = L[3][j];
-              if constexpr (M == SPH_LUCY_DENS) {
-                // SPHcalcDensity<SPHKernelLucy> (kerneltemplate.hh:636-656):
-                // W = w0 (h + 3R)(h - R)^3, 0 beyond h (kernelinline.hh:182-188)
-                const double dx = pi.x - xj, dy = pi.y - yj, dz = pi.z - zj;
-                double ri;
-                const double R = sph_norm(dx * dx + dy * dy + dz * dz, &ri);
-                const double tt = fmax(A.h - R, 0.0);
-                const double W = A.w0 * (A.h + 3.0 * R) * (tt * tt * tt);
-                const double mW = mj * W;
-                acc0 += W;
-                acc1 += mW;
-                acc2 = fma(L[4][j], mW, acc2);
-              } else if constexpr (M == SPH_LUCY_ACC) {
-                // SPHNavierStokes<SPHKernelLucyDW> (kerneltemplate.hh:666-709)
-                const double dx = xj - pi.x, dy = yj - pi.y, dz = zj - pi.z;
-                double ri;
-                const double R = sph_norm(dx * dx + dy * dy + dz * dz, &ri);
-                const double tt = A.h - R;
-                if (tt > 0.0 && q != k) {                 // no self term, 0 beyond h
-                  const double mw = mj * (A.w1 * tt * tt);  // m_j (dW/dr)/r, kernelinline.hh:209-214
-                  const double p1 = di.y + L[8][j];
-                  const double v1 = (di.z + L[9][j]) * di.x * L[7][j];
-                  acc0 += mw * (dx * p1 - (L[4][j] - vi.x) * v1);
-                  acc1 += mw * (dy * p1 - (L[5][j] - vi.y) * v1);
-                  acc2 += mw * (dz * p1 - (L[6][j] - vi.z) * v1);
-                }
-              } else if constexpr (M == SPH_WC_DENS) {
-                // M4 spline inside the support: W = ws (t2^3/4 - t1^3),
-                // t1 = max(1 - q, 0), t2 = 2 - q, q = r/h
-                const double dx = pi.x - xj, dy = pi.y - yj, dz = pi.z - zj;
-                const double R2 = dx * dx + dy * dy + dz * dz;
-                if (R2 < A.sup2) {
-                  double ri;
-                  const double qq = sph_norm(R2, &ri) * A.hinv;
-                  const double t1 = fmax(1.0 - qq, 0.0), t2 = 2.0 - qq;
-                  const double W = 0.25 * (t2 * t2 * t2) - t1 * t1 * t1;
-                  acc0 += W;
-                  acc1 = fma(mj, W, acc1);
-                }
-              } else {
-                // a_i = -sum m_j (P_i + P_j + Pi_ij) F(r) r_ij, F = (dW/dr)/r
-                // = wf (-3 + 9/4 q) for q < 1, wf (-3/4 (2 - q)^2 / q) below 2;
-                // Pi_ij = -alpha c0 h (v_ij . r_ij) / ((r^2 + 0.01 h^2) rho_bar)
-                // for approaching pairs
-                const double dx = pi.x - xj, dy = pi.y - yj, dz = pi.z - zj;
-                const double R2 = dx * dx + dy * dy + dz * dz;
-                if (R2 < A.sup2 && q != k) {
-                  double ri;
-                  const double qq = sph_norm(R2, &ri) * A.hinv, t2 = 2.0 - qq;
-                  const double g = qq < 1.0 ? fma(2.25, qq, -3.0) : -0.75 * t2 * t2 * (A.h * ri);
-                  const double vr =
-                      (vi.x - L[4][j]) * dx + (vi.y - L[5][j]) * dy + (vi.z - L[6][j]) * dz;
-                  const double visc =
-                      vr < 0.0 ? -A.avh * vr * sph_rcp((R2 + A.eh2) * (0.5 * (di.x + L[7][j])))
-                               : 0.0;
-                  const double f = -mj * (di.y + L[8][j] + visc) * g;
-                  acc0 = fma(f, dx, acc0);
-                  acc1 = fma(f, dy, acc1);
-                  acc2 = fma(f, dz, acc2);
-                }
-              }
-            }
-          }
-        }
-      }
+  } else if constexpr (M == SPH_WC_DENS) {
+    // M4 spline inside the support: W = ws (t2^3/4 - t1^3),
+    // t1 = max(1 - q, 0), t2 = 2 - q, q = r/h
+    const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+    const double R2 = dx * dx + dy * dy + dz * dz;
+    if (R2 < A.sup2) {
+      double ri;
+      const double qq = sph_norm(R2, &ri) * A.hinv;
+      const double t1 = fmax(1.0 - qq, 0.0), t2 = 2.0 - qq;
+      const double W = 0.25 * (t2 * t2 * t2) - t1 * t1 * t1;
+      acc0 += W;
+      acc1 = fma(pj.w, W, acc1);
     }
-    if (act) {
-      if constexpr (M == SPH_LUCY_DENS) {
-        // calcDensityPost (cudaParticleSPH_NS.cu:184-207)
-        const double ri = 1.0 / acc1;
-        out4[s] = make_double4(acc0, acc1, acc2 * ri, 0.0);
-        out1[s] = ri;
-      } else if constexpr (M == SPH_WC_DENS) {
-        // Tait: p = max(B ((rho/rho0)^gamma - 1), pmin)
-        const double n0 = acc0 * A.ws, rho = acc1 * A.ws;
-        const double p = sph_tait(rho, A.rho0inv, A.gamma, A.B, A.pmin);
-        out4[s] = make_double4(n0, rho, p, 0.0);
-        out1[s] = 1.0 / rho;
-      } else if constexpr (M == SPH_LUCY_ACC) {
-        out4[s] = make_double4(acc0, acc1, acc2, 0.0);
-      } else {
-        out4[s] = make_double4(acc0 * A.wf, acc1 * A.wf, acc2 * A.wf, 0.0);
-      }
+  } else {
+    // a_i = -sum m_j (P_i + P_j + Pi_ij) F(r) r_ij, F = (dW/dr)/r
+    // = wf (-3 + 9/4 q) for q < 1, wf (-3/4 (2 - q)^2 / q) below 2;
+    // Pi_ij = -alpha c0 h (v_ij . r_ij) / ((r^2 + 0.01 h^2) rho_bar)
+    // for approaching pairs
+    const double dx = pi.x - pj.x, dy = pi.y - pj.y, dz = pi.z - pj.z;
+    const double R2 = dx * dx + dy * dy + dz * dz;
+    if (R2 < A.sup2 && !self) {
+      double ri;
+      const double qq = sph_norm(R2, &ri) * A.hinv, t2 = 2.0 - qq;
+      const double g = qq < 1.0 ? fma(2.25, qq, -3.0) : -0.75 * t2 * t2 * (A.h * ri);
+      const double vr = (vi.x - vj.x) * dx + (vi.y - vj.y) * dy + (vi.z - vj.z) * dz;
+      const double visc =
+          vr < 0.0 ? -A.avh * vr * sph_rcp((R2 + A.eh2) * (0.5 * (vi.w + vj.w))) : 0.0;
+      const double f = -pj.w * (I.d.x + J.d.x + visc) * g;
+      acc0 = fma(f, dx, acc0);
+      acc1 = fma(f, dy, acc1);
+      acc2 = fma(f, dz, acc2);
     }
   }
 }
 
-// The config density fits six wavefronts per SIMD (80 VGPRs, 25 KB of
-// LDS); the other passes need more registers and run at four or five.
-template <int M>
-__global__ void __launch_bounds__(SC_T) k_sph_pairs(SphArgs A, uint32_t zseg, SphFilter FB,
-                                                    double4 *out4, double *out1) {
-  sph_pairs<M>(A, zseg, FB, out4, out1);
+template <int M, uint32_t LN>
+__device__ __forceinline__ void sph_pairs(const SphArgs &A, SphFilter FB, double4 *out4,
+                                          double *out1) {
+  static_assert(SC_T == PB_WAVE, "the lists and the stage are a wavefront's own");
+  __shared__ float4 F[SC_CAP + SC_G * LN];       // spare for a window's last tests
+  __shared__ uint32_t Hs[SC_HITS][SC_T];
+  const uint32_t lane = threadIdx.x;
+  // consecutive workgroups share neighbour columns in an XCD's L2
+  const uint32_t blk = pb_xcd_chunk<64>();
+  const uint32_t k = blk * (SC_T / LN) + lane / LN, sl = lane % LN;
+  const bool act = k < A.n;
+  const uint32_t kk = act ? k : A.n - 1u;
+  const uint32_t nz = A.g.nb[2], ny = A.g.nb[1], nx = A.g.nb[0];
+  const uint32_t c = A.bid[kk], col = c / nz, z = c % nz, ci = col / ny, cj = col % ny;
+  const uint32_t klo = z > 0 ? z - 1 : 0, khi = z + 1 < nz ? z + 1 : z;
+  const SphBody I = sph_load<M>(A, kk);
+  const float4 fi = A.fq[kk];
+  double acc0 = 0.0, acc1 = 0.0, acc2 = 0.0;
+  uint32_t cnt = 0;
+  auto work_off = [&]() {
+    for (uint32_t e = 0; e < cnt; e += SC_W) {
+      SphBody J[SC_W];
+      uint32_t q[SC_W];
+#pragma unroll
+      for (uint32_t u = 0; u < SC_W; ++u) q[u] = Hs[e + u < cnt ? e + u : e][lane];
+#pragma unroll
+      for (uint32_t u = 0; u < SC_W; ++u) J[u] = sph_load<M>(A, q[u]);
+#pragma unroll
+      for (uint32_t u = 0; u < SC_W; ++u)
+        if (e + u < cnt) sph_pair<M>(A, I, J[u], q[u] == k, acc0, acc1, acc2);
+    }
+    cnt = 0;
+    // no load of a skipped pair stays open: its registers would hold up every
+    // later use of them behind the prefetches (vmcnt(0))
+    __builtin_amdgcn_s_waitcnt(0x0f70);
+  };
+  // the lane's window in column t (false: none)
+  auto window = [&](int t, uint32_t &w0, uint32_t &w1) {
+    const int a = t / 3 - 1, b = t % 3 - 1;
+    const bool in = act && t < 9 && (a >= 0 || ci > 0) && (a <= 0 || ci + 1 < nx) &&
+                    (b >= 0 || cj > 0) && (b <= 0 || cj + 1 < ny);
+    w0 = w1 = 0;
+    if (in) {
+      const uint32_t cb = (col + (uint32_t)(a * (int)ny + b)) * nz;
+      w0 = A.cstart[cb + klo];
+      w1 = A.cstart[cb + khi + 1];
+    }
+    return in;
+  };
+  // the union of the windows, which ascend with the slots
+  auto span = [&](bool in, uint32_t w0, uint32_t w1, uint32_t &r0, uint32_t &r1) {
+    const uint64_t any = __ballot(in);
+    r0 = r1 = 0;
+    if (any) {
+      r0 = (uint32_t)__builtin_amdgcn_readlane((int)w0, __builtin_ctzll(any));
+      r1 = (uint32_t)__builtin_amdgcn_readlane((int)w1, 63 - __builtin_clzll(any));
+    }
+  };
+  static_assert(SC_CAP == 2 * PB_WAVE, "a batch is two views a lane");
+  float4 stage0, stage1;                         // a batch on its way to LDS
+  auto fetch = [&](uint32_t b0) {
+    stage0 = A.fq[min(b0 + lane, A.n - 1u)];
+    stage1 = A.fq[min(b0 + PB_WAVE + lane, A.n - 1u)];
+  };
+  uint32_t w0, w1, r0, r1, nw0, nw1;
+  span(window(0, w0, w1), w0, w1, r0, r1);
+  fetch(r0);
+  bool nin = window(1, nw0, nw1);
+#pragma unroll 1
+  for (int t = 0; t < 9; ++t) {
+    // the lane against this column: -2 ri and the bound less |ri|^2
+    const int a = t / 3 - 1, b = t % 3 - 1;
+    const float x = fi.x - (float)a * A.g.len[0], y = fi.y - (float)b * A.g.len[1];
+    const bool far = fi.w < 0.f;
+    const float fx = far ? 0.f : -2.0f * x, fy = far ? 0.f : -2.0f * y, fz = fi.z;
+    const float lim = far ? INFINITY : FB.r2 - (x * x + y * y);
+    uint32_t nr0 = 0, nr1 = 0;
+    const bool direct = r1 - r0 > SC_DIRECT;
+#pragma unroll 1
+    for (uint32_t b0 = r0;;) {
+      const uint32_t b1 = b0 + SC_CAP < r1 && !direct ? b0 + SC_CAP : r1;
+      pb_wave_lds_sync();                        // the previous batch is consumed
+      F[lane] = stage0;
+      F[PB_WAVE + lane] = stage1;
+      pb_wave_lds_sync();
+      const bool last = b1 >= r1;
+      if (last) span(nin, nw0, nw1, nr0, nr1);
+      fetch(last ? nr0 : b1);
+      // the lane's candidates: every LN-th of the window
+      uint32_t q0 = w0 + sl;
+      if (q0 < b0) q0 += (b0 - q0 + LN - 1u) / LN * LN;
+      const uint32_t q1 = w1 < b1 ? w1 : b1;
+#pragma unroll 1
+      while (__any(q0 < q1)) {
+        const uint32_t len = q0 < q1 ? min((q1 - q0 + LN - 1u) / LN, 32u) : 0u;
+        // first test in the highest bit; tests past the window are cut off
+        uint32_t mask = 0, done = 0;
+        auto tests = [&](const float4 (&f)[SC_G]) {
+#pragma unroll
+          for (uint32_t u = 0; u < SC_G; ++u) {
+            const float dz = f[u].z - fz;
+            const float d = fmaf(dz, dz, fmaf(fx, f[u].x, fmaf(fy, f[u].y, f[u].w - lim)));
+            mask = __builtin_amdgcn_alignbit(mask, __float_as_uint(d), 31);
+          }
+        };
+        if (!direct) {
+          const float4 *f0 = F + (q0 < q1 ? q0 - b0 : 0u);
+#pragma unroll 1
+          for (; done < len; done += SC_G) {
+            float4 f[SC_G];
+#pragma unroll
+            for (uint32_t u = 0; u < SC_G; ++u) f[u] = f0[(done + u) * LN];
+            tests(f);
+          }
+        } else {
+#pragma unroll 1
+          for (; done < len; done += SC_G) {
+            float4 f[SC_G];
+#pragma unroll
+            for (uint32_t u = 0; u < SC_G; ++u) f[u] = A.fq[min(q0 + (done + u) * LN, A.n - 1u)];
+            tests(f);
+          }
+        }
+        mask = len ? (mask << (32u - done)) & (~0u << (32u - len)) : 0u;
+        for (;;) {
+          while (mask && cnt < SC_HITS) {
+            const uint32_t u = (uint32_t)__builtin_clz(mask);
+            mask &= ~(0x80000000u >> u);
+            Hs[cnt++][lane] = q0 + u * LN;
+          }
+          if (!__any(mask)) break;
+          work_off();
+        }
+        q0 += 32u * LN;
+      }
+      if (last) break;
+      b0 = b1;
+    }
+    w0 = nw0;
+    w1 = nw1;
+    r0 = nr0;
+    r1 = nr1;
+    nin = window(t + 2, nw0, nw1);
+  }
+  work_off();
+#pragma unroll
+  for (uint32_t o = 1; o < LN; o <<= 1) {
+    acc0 += __shfl_xor(acc0, (int)o, 64);
+    acc1 += __shfl_xor(acc1, (int)o, 64);
+    acc2 += __shfl_xor(acc2, (int)o, 64);
+  }
+  if (act && sl == 0) {
+    const uint32_t s = A.perm[k];
+    if constexpr (M == SPH_LUCY_DENS) {
+      // calcDensityPost (cudaParticleSPH_NS.cu:184-207)
+      const double ri = 1.0 / acc1;
+      out4[s] = make_double4(acc0, acc1, acc2 * ri, 0.0);
+      out1[s] = ri;
+    } else if constexpr (M == SPH_WC_DENS) {
+      // Tait: p = max(B ((rho/rho0)^gamma - 1), pmin)
+      const double n0 = acc0 * A.ws, rho = acc1 * A.ws;
+      const double p = sph_tait(rho, A.rho0inv, A.gamma, A.B, A.pmin);
+      out4[s] = make_double4(n0, rho, p, 0.0);
+      out1[s] = 1.0 / rho;
+    } else if constexpr (M == SPH_LUCY_ACC) {
+      out4[s] = make_double4(acc0, acc1, acc2, 0.0);
+    } else {
+      out4[s] = make_double4(acc0 * A.wf, acc1 * A.wf, acc2 * A.wf, 0.0);
+    }
+  }
 }
-__global__ void __launch_bounds__(SC_T) __attribute__((amdgpu_waves_per_eu(6)))
-k_sph_pairs_wc_density(SphArgs A, uint32_t zseg, SphFilter FB, double4 *out4, double *out1) {
-  sph_pairs<SPH_WC_DENS>(A, zseg, FB, out4, out1);
+
+template <int M, uint32_t LN>
+__global__ void __launch_bounds__(SC_T) k_sph_pairs(SphArgs A, SphFilter FB, double4 *out4,
+                                                    double *out1) {
+  sph_pairs<M, LN>(A, FB, out4, out1);
 }
 
 // inspectDense_x (kernelfuncs.cu:772-801): per-wave partial sums of the
@@ -395,12 +461,18 @@ static int sph_ready(pb_sys *s) {
 static SphArgs sph_args(pb_sys *s) {
   SphArgs A;
   A.perm = s->perm;
-  A.cellid = s->cellid;
+  A.bid = s->ref_bid;
   A.cstart = s->cstart;
+  A.fq = s->sph_fq;
   A.rs = s->sph_rs;
   A.vs = s->sph_vs;
   A.ds = s->sph_ds;
-  for (int a = 0; a < 3; ++a) A.g.nb[a] = s->blocknum[a];
+  A.mus = s->sph_mus;
+  for (int a = 0; a < 3; ++a) {
+    A.g.nb[a] = s->blocknum[a];
+    A.g.len[a] = s->blocklen[a];
+    A.g.lo[a] = s->blocklen[a + 3];
+  }
   A.n = s->n;
   A.h = s->sph_h;
   A.w0 = 105.0 / (16.0 * M_PI * std::pow(s->sph_h, 7));   // cudaParticleSPHBase.cu:121
@@ -420,33 +492,48 @@ static SphArgs sph_args(pb_sys *s) {
   return A;
 }
 
-// Pair-kernel grid: (columns, z segments).  A segment of zseg cells holds
-// 64 particles at the mean cell occupancy, and two to three times that in
-// the filled part of a partly filled box, so dense columns are spread over
-// several workgroups of one or two 256-slot chunks each.
-static dim3 sph_pair_grid(pb_sys *s, uint32_t *zseg) {
-  const uint32_t nz = s->blocknum[2];
-  const double ncell = (double)s->blocknum[0] * s->blocknum[1] * nz;
-  const double occ = s->n / (ncell > 0 ? ncell : 1.0);
-  uint32_t z = (uint32_t)std::lround(64.0 / (occ > 1e-9 ? occ : 1e-9));
-  z = z < 1 ? 1 : (z > nz ? nz : z);
-  *zseg = z;
-  return dim3(s->blocknum[0] * s->blocknum[1] * ((nz + z - 1) / z));
+// FP32 filter bound: r2max and what rounding can add.  With (cx, cy) the cell
+// lengths, x^2 + y^2 of a candidate from its column's middle is at most cx^2 +
+// cy^2 = L2/4 (l2) and that of a lane, up to a column away, at most L2; the
+// expanded form then errs by at most ten units of 2^-24 L2 and its inputs'
+// rounding by as much again.  z within [-cz, zmax] is rounded twice and
+// subtracted: e = 3 units of 2^-24 zmax on |dz| <= sqrt(r2max).  Where the squares
+// leave the FP32 range every pair is left to the exact test.
+static SphFilter sph_filter(pb_sys *s, double r2max) {
+  const double cx = s->blocklen[0], cy = s->blocklen[1], cz = s->blocklen[2];
+  const double L2 = 4.0 * (cx * cx + cy * cy), zmax = (s->blocknum[2] + 1.0) * cz;
+  const double e = 3.0 * 6e-8 * zmax;
+  SphFilter F;
+  F.r2 = (float)(r2max * (1.0 + 1e-6) + 4e-6 * L2 + 2.0 * std::sqrt(r2max) * e + e * e);
+  F.l2 = L2 + zmax * zmax < 1e30 && r2max > 1e-30 ? (float)(0.25 * L2) : -1.f;
+  F.zmax = (float)zmax;
+  return F;
 }
 
-// FP32 filter bound: r2max plus 1e-6 Lmax^2, where Lmax bounds the filter
-// coordinates' magnitude for particles inside the cell grid (two cells
-// across x and y, the segment and one cell along z); the rounding of the
-// expanded |ri - rj|^2 in FP32 stays below ten units of 2^-24 Lmax^2, so no
-// pair within r2max is filtered out.  Coordinates beyond Lmax (particles
-// outside the grid, binned into its edge cells) bypass the filter.
-static SphFilter sph_filter(pb_sys *s, uint32_t zseg, double r2max) {
-  const double cx = s->blocklen[0], cy = s->blocklen[1], cz = s->blocklen[2];
-  const double l2 = 4.0 * cx * cx + 4.0 * cy * cy + (zseg + 1.0) * (zseg + 1.0) * cz * cz;
-  SphFilter F;
-  F.r2 = (float)(r2max * (1.0 + 1e-6) + 1e-6 * l2);
-  F.l2 = (float)l2;
-  return F;
+// Lanes a slot: as many as fill the chip's 1024 SIMDs several times over; more only
+// repeat the staging.  Density + acceleration, gathers included, us with 1, 2, 4
+// and 8 lanes:
+//   Lucy (14 candidates a window):  15,876: 55, 41, 33, 33;  48,148: 61, 47, 46, 65;
+//     133,904: 82, 83, 95, 135;  796,176: 279, 301, 402, 664
+//   config (34 a window, support 2h):  7,036: 162, 79, 50, 38;  48,148: 184, 97, 70, 84;
+//     133,904: 214, 147, 153, 183;  796,176: 700, 630, 705, 920
+static uint32_t sph_lanes(const pb_sys *s) {
+  const bool wc = s->sph_kind == 1;
+  if (s->n <= 24576u) return 8u;
+  if (s->n <= (wc ? 98304u : 49152u)) return 4u;
+  return wc || s->n <= 131072u ? 2u : 1u;
+}
+
+template <int M>
+static void sph_launch_pairs(pb_sys *s, const SphArgs &A, const SphFilter &FB, double4 *out4,
+                             double *out1) {
+  const uint32_t ln = sph_lanes(s);
+  auto kernel = ln == 8   ? k_sph_pairs<M, 8>
+                : ln == 4 ? k_sph_pairs<M, 4>
+                : ln == 2 ? k_sph_pairs<M, 2>
+                          : k_sph_pairs<M, 1>;
+  hipLaunchKernelGGL(kernel, dim3(pb_blocks(A.n, SC_T / ln)), dim3(SC_T), 0, s->ctx->stream, A, FB,
+                     out4, out1);
 }
 
 // density, 1/rho and the cell-order views, shared by both physics
@@ -456,7 +543,8 @@ static int sph_alloc_views(pb_sys *s) {
   if (!s->sph_rs) {
     if ((rc = pb_alloc(s->ctx, &s->sph_rhoinv, np)) || (rc = pb_alloc(s->ctx, &s->sph_num, np)) ||
         (rc = pb_alloc(s->ctx, &s->sph_rs, np)) || (rc = pb_alloc(s->ctx, &s->sph_vs, np)) ||
-        (rc = pb_alloc(s->ctx, &s->sph_ds, np)))
+        (rc = pb_alloc(s->ctx, &s->sph_ds, np)) || (rc = pb_alloc(s->ctx, &s->sph_mus, np)) ||
+        (rc = pb_alloc(s->ctx, &s->sph_fq, np)))
       return rc;
   }
   hipStream_t st = s->ctx->stream;
@@ -518,16 +606,12 @@ extern "C" int pb_sph_density(pb_sys *s) {
   if (n == 0) return PB_OK;
   SphArgs A = sph_args(s);
   const bool wc = s->sph_kind == 1;
-  uint32_t zseg = 0;
-  const dim3 grid = sph_pair_grid(s, &zseg);
-  hipLaunchKernelGGL(k_sph_gather, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->perm, s->r, s->v,
-                     wc ? (const double *)nullptr : s->sph_mu0, n, s->sph_rs, s->sph_vs);
-  if (wc)
-    hipLaunchKernelGGL(k_sph_pairs_wc_density, grid, dim3(SC_T), 0, st, A, zseg,
-                       sph_filter(s, zseg, A.sup2), s->sph_num, s->sph_rhoinv);
-  else
-    hipLaunchKernelGGL(k_sph_pairs<SPH_LUCY_DENS>, grid, dim3(SC_T), 0, st, A, zseg,
-                       sph_filter(s, zseg, A.h * A.h), s->sph_num, s->sph_rhoinv);
+  const SphFilter FB = sph_filter(s, wc ? A.sup2 : A.h * A.h);
+  hipLaunchKernelGGL(k_sph_gather, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->perm, s->ref_bid,
+                     s->r, s->v, wc ? (const double *)nullptr : s->sph_mu0, A.g, FB, n, s->sph_rs,
+                     s->sph_fq, s->sph_mus);
+  if (wc) sph_launch_pairs<SPH_WC_DENS>(s, A, FB, s->sph_num, s->sph_rhoinv);
+  else sph_launch_pairs<SPH_LUCY_DENS>(s, A, FB, s->sph_num, s->sph_rhoinv);
   PB_LAUNCH_CHECK(s->ctx, "k_sph_pairs (density)");
   s->sph_dens = true;
   return PB_OK;
@@ -543,21 +627,16 @@ extern "C" int pb_sph_acceleration(pb_sys *s) {
   if (n == 0) return PB_OK;
   SphArgs A = sph_args(s);
   const bool wc = s->sph_kind == 1;
-  uint32_t zseg = 0;
-  const dim3 grid = sph_pair_grid(s, &zseg);
+  const SphFilter FB = sph_filter(s, wc ? A.sup2 : A.h * A.h);
   // current positions and velocities, and the density call's rho, 1/rho,
   // mu or p, in the current cell order
-  hipLaunchKernelGGL(k_sph_gather_acc, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->perm, s->r,
-                     s->v, s->sph_num, s->sph_rhoinv,
+  hipLaunchKernelGGL(k_sph_gather_acc, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->perm,
+                     s->ref_bid, s->r, s->v, s->sph_num, s->sph_rhoinv,
                      s->sph_c2 ? s->sph_c2 : s->sph_rhoinv,   // not read under the config physics
-                     s->sph_rho0, wc ? 1 : 0, n,
-                     s->sph_rs, s->sph_vs, s->sph_ds);
-  if (wc)
-    hipLaunchKernelGGL(k_sph_pairs<SPH_WC_ACC>, grid, dim3(SC_T), 0, st, A, zseg,
-                       sph_filter(s, zseg, A.sup2), s->a, (double *)nullptr);
-  else
-    hipLaunchKernelGGL(k_sph_pairs<SPH_LUCY_ACC>, grid, dim3(SC_T), 0, st, A, zseg,
-                       sph_filter(s, zseg, A.h * A.h), s->a, (double *)nullptr);
+                     s->sph_rho0, wc ? 1 : 0, A.g, FB, n, s->sph_rs, s->sph_fq, s->sph_vs,
+                     s->sph_ds);
+  if (wc) sph_launch_pairs<SPH_WC_ACC>(s, A, FB, s->a, nullptr);
+  else sph_launch_pairs<SPH_LUCY_ACC>(s, A, FB, s->a, nullptr);
   PB_LAUNCH_CHECK(s->ctx, "k_sph_pairs (acceleration)");
   return PB_OK;
 }
