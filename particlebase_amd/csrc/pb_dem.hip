@@ -10,8 +10,8 @@
 // history carry-over from the previous matrix and the contact-force pass.
 //
 // Here the same stages run as: a gather of (x, y, z, radius) into cell order
-// -> count (one thread per particle in cell order, 27 or 125 neighbour cells as
-// contiguous ranges of that view) -> exclusive scan -> one kernel that sorts
+// and an FP32 view of it -> count (one thread per particle in cell order, 27 or
+// 125 neighbour cells as contiguous ranges) -> exclusive scan -> one kernel that sorts
 // each row, takes the tangential history over from the previous matrix (both
 // rows sorted) and computes contact force and torque.  The column arrays are
 // sized from the previous step's count; that kernel stops at the capacity and
@@ -31,6 +31,7 @@ __global__ void k_fill_u32(uint32_t *x, uint32_t n, uint32_t val);
 struct DemGrid {
   const uint32_t *perm, *bid, *cstart;
   const double4 *rs;        // cell order: (x, y, z, radius)
+  const float4 *fq;         // cell order: the same for the FP32 filter (dem_view)
   const uint32_t *so;       // cell order: original index
   const uint8_t *move;
   uint32_t nb[3];
@@ -43,14 +44,34 @@ struct DemGrid {
 // touching neighbours than any sphere packing gives) are scanned again
 #define DEM_ROWBUF 16u
 
-// positions with the radius in w, in cell order
+// FP32 view for a first test that passes every pair in contact: positions from
+// the grid's corner, up to `span` from it, and the radius with half the margin
+// that covers their rounding: 2^-24 span a coordinate and particle, so less than
+// 4e-7 span a distance, and a few units of relative rounding.  A particle beyond
+// the span (outside the grid, binned into its edge cells; NaN) gets an infinite
+// radius.
+struct DemView {
+  double lo[3];
+  float span;
+};
+__device__ __forceinline__ float4 dem_view(const DemView &V, const double4 &p) {
+  const float x = (float)(p.x - V.lo[0]), y = (float)(p.y - V.lo[1]), z = (float)(p.z - V.lo[2]);
+  if (!(fabsf(x) <= V.span && fabsf(y) <= V.span && fabsf(z) <= V.span))
+    return make_float4(0.f, 0.f, 0.f, INFINITY);
+  // at least 1e-18, so that the squares stay normal
+  return make_float4(x, y, z, fmaxf(fabsf((float)p.w) * 1.000001f + 2e-7f * V.span, 1e-18f));
+}
+
+// positions with the radius in w and their view, in cell order
 __global__ void k_dem_gather(const uint32_t *perm, const double4 *r, const double *rad, uint32_t n,
-                             double4 *rs) {
+                             DemView V, double4 *rs, float4 *fq) {
   const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k >= n) return;
   const uint32_t s = perm[k];
   const double4 p = r[s];
-  rs[k] = make_double4(p.x, p.y, p.z, rad[s]);
+  const double4 o = make_double4(p.x, p.y, p.z, rad[s]);
+  rs[k] = o;
+  fq[k] = dem_view(V, o);
 }
 
 // (x, y, z, radius) of both particles
@@ -61,56 +82,114 @@ __device__ __forceinline__ bool in_contact(const double4 &pi, const double4 &pj)
   return R2 < rc * rc;
 }
 
-// The sorted slots q != k in contact with particle k, over the (2W + 1)^3 cells
-// around its own (non-periodic: DEM distances never use an image,
-// kernelinline.hh:248), in ascending q.  The scan is a chain of dependent reads
-// (cell starts, candidates) at few wavefronts a SIMD, so the starts of a row of
-// columns are read together, and the candidates of a column (one or two on
-// average) four at a time.
-template <int W, typename F>
-__device__ __forceinline__ void dem_contacts(const DemGrid &G, uint32_t k, const double4 &pi, F &&f) {
+// f(original index) for every particle in contact with particle k, over the
+// (2W + 1)^3 cells around its own (non-periodic: DEM distances never use an image,
+// kernelinline.hh:248), in no particular order.  The scan is a chain of dependent
+// reads (cell starts, candidates) at few wavefronts a SIMD, so the starts of a
+// row of columns are read together, and the first candidates of several columns
+// (a column holds one to three) in one go, as FP32 views; what passes is listed
+// in the thread's LDS and tested exactly four at a time.
+template <int W, typename F, size_t T>
+__device__ __forceinline__ void dem_contacts(const DemGrid &G, uint32_t k,
+                                             uint32_t (&list)[DEM_ROWBUF][T], F &&f) {
+  const uint32_t tid = threadIdx.x;
   const uint32_t c = G.bid[k], nz = G.nb[2], nyz = G.nb[1] * nz;
   const int i0 = (int)(c / nyz), j0 = (int)((c / nz) % G.nb[1]), k0 = (int)(c % nz);
   const uint32_t kl = (uint32_t)max(k0 - W, 0), kh = (uint32_t)min(k0 + W, (int)nz - 1) + 1u;
-  constexpr int NC = W == 1 ? 9 : 5;                  // columns read together
-#pragma unroll 1
-  for (int g = 0; g < (2 * W + 1) * (2 * W + 1); g += NC) {
-    uint32_t q0[NC], q1[NC];
+  const double4 pi = G.rs[k];
+  const float4 fi = G.fq[k];
+  uint32_t cnt = 0;
+  auto work_off = [&]() {
+    for (uint32_t e = 0; e < cnt; e += 4) {
+      uint32_t q[4], o[4];
+      double4 pj[4];
 #pragma unroll
-    for (int t = 0; t < NC; ++t) {
-      const int i2 = i0 + (g + t) / (2 * W + 1) - W, j2 = j0 + (g + t) % (2 * W + 1) - W;
-      const bool ok = i2 >= 0 && i2 < (int)G.nb[0] && j2 >= 0 && j2 < (int)G.nb[1];
+      for (uint32_t u = 0; u < 4; ++u) q[u] = list[min(e + u, cnt - 1u)][tid];
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u) {
+        pj[u] = G.rs[q[u]];
+        o[u] = G.so[q[u]];
+      }
+#pragma unroll
+      for (uint32_t u = 0; u < 4; ++u)
+        if (e + u < cnt && in_contact(pi, pj[u])) f(o[u]);
+    }
+    cnt = 0;
+  };
+  constexpr int NG = 2 * W + 1;                       // columns of a row, tested together,
+  constexpr uint32_t U = W == 1 ? 4u : 2u;            // that many candidates each
+  static_assert(NG * U <= DEM_ROWBUF, "a round's candidates fit the list");
+  auto starts = [&](int a, uint32_t (&q0)[NG], uint32_t (&q1)[NG]) {
+    const int i2 = i0 + a;
+#pragma unroll
+    for (int t = 0; t < NG; ++t) {
+      const int j2 = j0 + t - W;
+      const bool ok = a <= W && i2 >= 0 && i2 < (int)G.nb[0] && j2 >= 0 && j2 < (int)G.nb[1];
       const uint32_t cb = ok ? (uint32_t)i2 * nyz + (uint32_t)j2 * nz : 0u;
       q0[t] = G.cstart[cb + kl];
       q1[t] = ok ? G.cstart[cb + kh] : q0[t];
     }
+  };
+  uint32_t q0[NG], q1[NG], n0[NG], n1[NG];
+  starts(-W, q0, q1);
+#pragma unroll 1
+  for (int a = -W; a <= W; ++a) {
+    starts(a + 1, n0, n1);                            // the next row on its way
+    bool more;
+    uint32_t o = 0;
+#pragma unroll 1
+    do {
+      float4 fj[NG][U];
 #pragma unroll
-    for (int t = 0; t < NC; ++t)
-      for (uint32_t q = q0[t]; q < q1[t]; q += 4) {
-        double4 pj[4];
+      for (int t = 0; t < NG; ++t)
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) pj[u] = G.rs[min(q + u, q1[t] - 1u)];
+        for (uint32_t u = 0; u < U; ++u) {
+          const uint32_t q = q0[t] + o + u;
+          fj[t][u] = G.fq[q < q1[t] ? q : k];         // past the end: the particle itself
+        }
+      more = false;
 #pragma unroll
-        for (uint32_t u = 0; u < 4; ++u)
-          if (q + u < q1[t] && q + u != k && in_contact(pi, pj[u])) f(q + u);
+      for (int t = 0; t < NG; ++t) {
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+          const uint32_t q = q0[t] + o + u;
+          const float dx = fi.x - fj[t][u].x, dy = fi.y - fj[t][u].y, dz = fi.z - fj[t][u].z;
+          const float rr = fi.w + fj[t][u].w;
+          if (q < q1[t] && q != k && dx * dx + dy * dy + dz * dz < rr * rr) list[cnt++][tid] = q;
+        }
+        more |= q0[t] + o + U < q1[t];
       }
+      o += U;
+      // room for the next round; the last row's rounds end here too
+      if (cnt > DEM_ROWBUF - NG * U || (a == W && !more)) work_off();
+    } while (more);
+#pragma unroll
+    for (int t = 0; t < NG; ++t) {
+      q0[t] = n0[t];
+      q1[t] = n1[t];
+    }
   }
 }
 
 // calcCoord_F4 (kernelinline.hh:371-382): contacts of movable particles
-// The same scan keeps the first DEM_ROWBUF contacts (original indices, scan
-// order) in the row buffer for the rows.
+// The same scan keeps the first DEM_ROWBUF contacts (original indices, in no
+// particular order) in the row buffer for the rows.
+// 200,000 dispersed spheres 15 us, a bed of 60,000 15 us (18 and 15 with FP64
+// candidates column by column); at most 128 registers, so that four wavefronts
+// fit a SIMD.
 template <int W>
-__global__ void k_dem_count(DemGrid G, uint32_t *cnt, uint32_t *bad) {
-  const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
+k_dem_count(DemGrid G, uint32_t *cnt, uint32_t *bad) {
+  __shared__ uint32_t list[DEM_ROWBUF][256];
+  const uint32_t k = pb_xcd_chunk8() * 256u + threadIdx.x;
   if (k == 0) *bad = 0;                               // Cundall-Strack violations of this call
   if (k >= G.n) return;
   const uint32_t i = G.so[k];
   uint32_t c = 0;
   if (G.move[G.perm[k]]) {
     uint32_t *buf = G.rowbuf + (size_t)i * DEM_ROWBUF;
-    dem_contacts<W>(G, k, G.rs[k], [&](uint32_t q) {
-      if (c < DEM_ROWBUF) buf[c] = G.so[q];
+    dem_contacts<W>(G, k, list, [&](uint32_t o) {
+      if (c < DEM_ROWBUF) buf[c] = o;
       ++c;
     });
   }
@@ -129,6 +208,7 @@ struct DemForceArgs {
   const uint8_t *move;
   double4 *F, *T;
   uint32_t *bad;                         // Cundall-Strack violations
+  uint32_t *res;                         // pinned: nnz, and 1 if there are any violations
   double E, mu, s2, gamma2, mu_r, dt;
   double kn, zeta, kt;                   // linear law
 };
@@ -141,14 +221,24 @@ struct DemBody {
   uint32_t bad = 0;
 };
 
+// the other particle of a contact
+struct DemOther {
+  double4 p, v, w;
+  double rad;
+  uint32_t move;
+};
+__device__ __forceinline__ DemOther dem_other(const DemForceArgs &A, uint32_t sj) {
+  return DemOther{A.r[sj], A.v[sj], A.w[sj], A.rad[sj], A.move[sj]};
+}
+
 // DEMContact_F4 (kernelinline.hh:235-363), FP64.  h: the contact's history (1
 // double: the slip length), updated in place.
-__device__ __forceinline__ void contact_hertz(const DemForceArgs &A, DemBody &B, uint32_t sj, double *h) {
+__device__ __forceinline__ void contact_hertz(const DemForceArgs &A, DemBody &B, const DemOther &J, double *h) {
   const double4 &pi = B.p, &vi = B.v, &wi = B.w;
   const double ri = B.rad;
   const bool wnz = wi.x != 0 && wi.y != 0 && wi.z != 0;
-  const double4 pj = A.r[sj], vj = A.v[sj], wj = A.w[sj];
-  const double rj = A.rad[sj];
+  const double4 &pj = J.p, &vj = J.v, &wj = J.w;
+  const double rj = J.rad;
   const double d[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
   const double R2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
   const double rs = ri + rj;
@@ -193,7 +283,7 @@ __device__ __forceinline__ void contact_hertz(const DemForceArgs &A, DemBody &B,
     Tr[1] = cr * wi.y;
     Tr[2] = cr * wi.z;
   }
-  const double Q = 2.0 - (double)A.move[sj];
+  const double Q = 2.0 - (double)J.move;
 #pragma unroll
   for (int x = 0; x < 3; ++x) {
     B.f[x] += (Fn[x] + Fs[x]) * Q;
@@ -213,11 +303,11 @@ __device__ __forceinline__ void contact_hertz(const DemForceArgs &A, DemBody &B,
 //   F_i += Fn + Ft, T_i += (-rad_i n) x Ft
 // The history (3 doubles per contact) belongs to row i and is updated in
 // place.
-__device__ __forceinline__ void contact_linear(const DemForceArgs &A, DemBody &B, uint32_t sj, double *h) {
+__device__ __forceinline__ void contact_linear(const DemForceArgs &A, DemBody &B, const DemOther &J, double *h) {
   const double4 &pi = B.p, &vi = B.v, &wi = B.w;
   const double ri = B.rad;
-  const double4 pj = A.r[sj], vj = A.v[sj], wj = A.w[sj];
-  const double rj = A.rad[sj];
+  const double4 &pj = J.p, &vj = J.v, &wj = J.w;
+  const double rj = J.rad;
   const double d[3] = {pi.x - pj.x, pi.y - pj.y, pi.z - pj.z};
   const double R2 = d[0] * d[0] + d[1] * d[1] + d[2] * d[2];
   const double rs = ri + rj;
@@ -225,7 +315,7 @@ __device__ __forceinline__ void contact_linear(const DemForceArgs &A, DemBody &B
   const double R = sqrt(R2);
   const double nv[3] = {d[0] / R, d[1] / R, d[2] / R};
   const double delta = rs - R;
-  const double meff = 1.0 / (vi.w + (A.move[sj] ? vj.w : 0.0));
+  const double meff = 1.0 / (vi.w + (J.move ? vj.w : 0.0));
   const double gn = 2.0 * A.zeta * sqrt(meff * A.kn);
   if (!(A.dt < 2.0 * sqrt(meff / A.kn))) ++B.bad;
   const double vij[3] = {vi.x - vj.x, vi.y - vj.y, vi.z - vj.z};
@@ -288,22 +378,25 @@ __device__ __forceinline__ void sort_registers(uint32_t (&a)[DEM_ROWBUF]) {
 // calcF_IJpairWithList_F4 (kerneltemplate.hh:135-168) in one pass.  F and T are
 // overwritten (the reference clears both first, cudaParticleDEM.cu:168-169);
 // padding slots are not visited (they stay zero).
-// Bound by latency (a particle has none to a dozen contacts and every stage is
-// a dependent read), so a row that the counting scan kept whole is sorted in
-// registers, and its columns' slots and the previous row are read together
-// before the first contact; longer rows (more touching neighbours than any
-// sphere packing gives) are scanned again and merged in memory.  A contact
-// present in both matrices keeps its history (both rows are sorted); new ones
-// start at 0.  60,000 spheres of 6 contacts: 24 us, 200,000 with almost none:
-// 8 us; fill, carry and force as kernels of their own took 31 and 16 us.
+// Bound by latency and uncoalesced reads (a particle has none to a dozen
+// contacts).  A row that the counting scan kept whole is sorted in registers;
+// longer rows (more touching neighbours than any sphere packing gives) are
+// scanned again and sorted in memory.  A contact present in both matrices keeps
+// its history (both rows are sorted); new ones start at 0.  LN lanes take every
+// LN-th contact of a row (each walks the previous row by itself), and the sums
+// are added in a fixed order.  Code is kept short (rolled loops): a wavefront
+// passes most of it once, so its fetch counts.  Neighbouring workgroups share an
+// XCD's L2.  A bed of 60,000 spheres of 6 contacts: 19 us with two lanes, 21 with
+// one, 27 with four; 200,000 dispersed ones with almost none: 8.0 and 7.6;
+// fill, carry and force as kernels of their own took 31 and 16 us.
 #define DEM_ROWS_BS 128
-template <int LAW, int W>
+template <int LAW, int W, uint32_t LN>
 __global__ void __launch_bounds__(DEM_ROWS_BS) k_dem_rows(DemGrid G, DemForceArgs A) {
-  __shared__ uint32_t sslot[DEM_ROWBUF][DEM_ROWS_BS];   // storage slot of a contact
-  __shared__ uint32_t sprev[DEM_ROWBUF][DEM_ROWS_BS];   // its place in the previous matrix
+  __shared__ uint32_t scol[DEM_ROWBUF][DEM_ROWS_BS];    // a row
   constexpr uint32_t HW = LAW == 1 ? 3u : 1u;
-  const uint32_t k = blockIdx.x * DEM_ROWS_BS + threadIdx.x, tid = threadIdx.x;
-  if (k >= G.n) return;
+  const uint32_t tid = threadIdx.x, k = (pb_xcd_chunk<16>() * DEM_ROWS_BS + tid) / LN, sl = tid % LN;
+  if (k >= G.n) return;                               // a particle's lanes leave together
+  if (k == 0 && sl == 0) A.res[0] = A.row[G.n];
   const uint32_t s = G.perm[k], i = G.so[k];
   const uint32_t b = A.row[i], full = A.row[i + 1] - b;
   // rows past the capacity: redone
@@ -319,22 +412,13 @@ __global__ void __launch_bounds__(DEM_ROWS_BS) k_dem_rows(DemGrid G, DemForceArg
       p = A.prow[i];
       pe = A.prow[i + 1];
     }
-    auto contact = [&](uint32_t q, uint32_t sj, uint32_t from) {
-      double h[HW];
-#pragma unroll
-      for (uint32_t x = 0; x < HW; ++x) h[x] = from != PB_NONE ? A.pval[(size_t)from * HW + x] : 0.0;
-      if (LAW == 1) contact_linear(A, B, sj, h);
-      else contact_hertz(A, B, sj, h);
-#pragma unroll
-      for (uint32_t x = 0; x < HW; ++x) A.val[(size_t)q * HW + x] = h[x];
-    };
-    if (full <= DEM_ROWBUF) {               // the counting scan kept the whole row
+    const bool kept = full <= DEM_ROWBUF;   // the counting scan kept the whole row
+    if (kept) {
       uint32_t a[DEM_ROWBUF];
       const uint4 *buf = reinterpret_cast<const uint4 *>(G.rowbuf + (size_t)i * DEM_ROWBUF);
 #pragma unroll
       for (uint32_t x = 0; x < DEM_ROWBUF; x += 4) {
-        uint4 y = make_uint4(PB_NONE, PB_NONE, PB_NONE, PB_NONE);
-        if (x < full) y = buf[x / 4];
+        const uint4 y = buf[x / 4];
         a[x] = x < full ? y.x : PB_NONE;
         a[x + 1] = x + 1 < full ? y.y : PB_NONE;
         a[x + 2] = x + 2 < full ? y.z : PB_NONE;
@@ -343,30 +427,11 @@ __global__ void __launch_bounds__(DEM_ROWS_BS) k_dem_rows(DemGrid G, DemForceArg
       if (__ballot(full > 8) == 0ull) sort_registers<8>(a);
       else sort_registers<(int)DEM_ROWBUF>(a);
 #pragma unroll
-      for (uint32_t x = 0; x < DEM_ROWBUF; ++x)
-        if (x < len) {
-          A.col[b + x] = a[x];
-          sslot[x][tid] = A.inv[a[x]];
-          sprev[x][tid] = PB_NONE;
-        }
-      // the previous row, four columns at a time, against the sorted row
-      for (uint32_t q = p; q < pe; q += 4) {
-        uint32_t y[4];
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) y[u] = A.pcol[min(q + u, pe - 1u)];
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-          if (q + u >= pe) continue;
-#pragma unroll
-          for (uint32_t x = 0; x < DEM_ROWBUF; ++x)
-            if (x < len && a[x] == y[u]) sprev[x][tid] = q + u;
-        }
-      }
-      for (uint32_t x = 0; x < len; ++x) contact(b + x, sslot[x][tid], sprev[x][tid]);
-    } else {
+      for (uint32_t x = 0; x < DEM_ROWBUF; ++x) scol[x][tid] = a[x];
+    } else if (sl == 0) {
       uint32_t m = b;
-      dem_contacts<W>(G, k, G.rs[k], [&](uint32_t q) {
-        if (m < e) A.col[m++] = G.so[q];
+      dem_contacts<W>(G, k, scol, [&](uint32_t o) {
+        if (m < e) A.col[m++] = o;
       });
       for (uint32_t x = b + 1; x < e; ++x) {
         const uint32_t v = A.col[x];
@@ -377,23 +442,42 @@ __global__ void __launch_bounds__(DEM_ROWS_BS) k_dem_rows(DemGrid G, DemForceArg
         }
         A.col[y] = v;
       }
-      for (uint32_t q = b; q < e; ++q) {
-        const uint32_t j = A.col[q];
-        while (p < pe && A.pcol[p] < j) ++p;
-        contact(q, A.inv[j], p < pe && A.pcol[p] == j ? p : PB_NONE);
+    }
+    uint32_t pj = p < pe ? A.pcol[p] : PB_NONE;       // both rows ascend
+    const uint32_t step = kept ? LN : 1u, first = kept || sl == 0 ? sl : len;
+#pragma unroll 1
+    for (uint32_t x = first; x < len; x += step) {
+      const uint32_t j = kept ? scol[x][tid] : A.col[b + x];
+      if (kept) A.col[b + x] = j;
+      const DemOther J = dem_other(A, A.inv[j]);
+      while (pj < j) {
+        ++p;
+        pj = p < pe ? A.pcol[p] : PB_NONE;
       }
+      double h[HW];
+#pragma unroll
+      for (uint32_t y = 0; y < HW; ++y) h[y] = pj == j ? A.pval[(size_t)p * HW + y] : 0.0;
+      if (LAW == 1) contact_linear(A, B, J, h);
+      else contact_hertz(A, B, J, h);
+#pragma unroll
+      for (uint32_t y = 0; y < HW; ++y) A.val[(size_t)(b + x) * HW + y] = h[y];
     }
   }
-  A.F[s] = make_double4(B.f[0], B.f[1], B.f[2], 0.0);
-  A.T[s] = make_double4(B.t[0], B.t[1], B.t[2], 0.0);
-  if (B.bad) atomicAdd(A.bad, B.bad);
-}
-
-// nnz and the time-step check to pinned memory
-__global__ void k_dem_result(const uint32_t *nnz, const uint32_t *bad, uint32_t *out) {
-  if (threadIdx.x == 0) {
-    out[0] = *nnz;
-    out[1] = *bad;
+#pragma unroll
+  for (uint32_t o = 1; o < LN; o <<= 1) {
+#pragma unroll
+    for (int x = 0; x < 3; ++x) {
+      B.f[x] += __shfl_xor(B.f[x], (int)o, PB_WAVE);
+      B.t[x] += __shfl_xor(B.t[x], (int)o, PB_WAVE);
+    }
+  }
+  if (sl == 0) {
+    A.F[s] = make_double4(B.f[0], B.f[1], B.f[2], 0.0);
+    A.T[s] = make_double4(B.t[0], B.t[1], B.t[2], 0.0);
+  }
+  if (B.bad) {
+    atomicAdd(A.bad, B.bad);
+    A.res[1] = 1u;
   }
 }
 
@@ -556,6 +640,17 @@ static int ensure_csr(pb_sys *s, int b, uint32_t nnz) {
   return PB_OK;
 }
 
+// lanes a particle in k_dem_rows: two while one leaves SIMDs without a wavefront
+static uint32_t dem_lanes(uint32_t n) {
+  return n <= 98304u ? 2u : 1u;
+}
+
+template <int LAW>
+static void (*dem_rows_kernel(bool single, uint32_t ln))(DemGrid, DemForceArgs) {
+  if (ln == 2) return single ? k_dem_rows<LAW, 2, 2> : k_dem_rows<LAW, 1, 2>;
+  return single ? k_dem_rows<LAW, 2, 1> : k_dem_rows<LAW, 1, 1>;
+}
+
 extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *nnz_out) {
   if (!s) return PB_ERR_ARG;
   if (!s->dem_set) return pb_fail(s->ctx, PB_ERR_STATE, "DEM properties not set");
@@ -568,7 +663,7 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
   if (!s->dem_rs) {
     if ((rc = pb_alloc(s->ctx, &s->dem_inv, (size_t)n + 1)) ||
         (rc = pb_alloc(s->ctx, &s->dem_rowbuf, (size_t)s->npad * DEM_ROWBUF)) ||
-        (rc = pb_alloc(s->ctx, &s->dem_rs, s->npad)))
+        (rc = pb_alloc(s->ctx, &s->dem_fq, s->npad)) || (rc = pb_alloc(s->ctx, &s->dem_rs, s->npad)))
       return rc;
   }
   if (s->dem_inv_order != s->order_gen) {
@@ -576,13 +671,21 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
                        s->dem_inv);
     s->dem_inv_order = s->order_gen;
   }
+  DemView V;
+  double span = 0.0;
+  for (int a = 0; a < 3; ++a) {
+    V.lo[a] = s->blocklen[3 + a];
+    span = std::max(span, (s->blocknum[a] + 1.0) * s->blocklen[a]);
+  }
+  V.span = span < 1e18 ? (float)span : -1.f;  // squares outside FP32: every pair exactly
   hipLaunchKernelGGL(k_dem_gather, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->perm, s->r,
-                     s->radius, n, s->dem_rs);
+                     s->radius, n, V, s->dem_rs, s->dem_fq);
   DemGrid G;
   G.perm = s->perm;
   G.bid = s->ref_bid;
   G.cstart = s->cstart;
   G.rs = s->dem_rs;
+  G.fq = s->dem_fq;
   G.so = s->ref_pid;
   G.rowbuf = s->dem_rowbuf;
   G.move = s->move;
@@ -623,24 +726,25 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
   A.kn = s->dem_kn;
   A.zeta = s->dem_zeta;
   A.kt = s->dem_kt;
-  auto rows = s->dem_law == 1 ? (single ? k_dem_rows<1, 2> : k_dem_rows<1, 1>)
-                              : (single ? k_dem_rows<0, 2> : k_dem_rows<0, 1>);
-  // rows, history and forces up to the capacity; then nnz and the time-step
-  // check in one wait
+  A.res = (uint32_t *)s->ctx->res_dev;
+  const uint32_t ln = dem_lanes(n);
+  auto rows = s->dem_law == 1 ? dem_rows_kernel<1>(single, ln) : dem_rows_kernel<0>(single, ln);
+  // rows, history and forces up to the capacity; that kernel reports nnz and
+  // whether the time-step check failed (its count is fetched only then)
   uint32_t nnz = 0, nbad = 0;
   auto contacts_and_force = [&]() -> int {
     G.cap = s->cm_cap[b];
     A.row = s->cm_row[b];
     A.col = s->cm_col[b];
     A.val = s->cm_val[b];
-    hipLaunchKernelGGL(rows, dim3(pb_blocks(n, DEM_ROWS_BS)), dim3(DEM_ROWS_BS), 0, st, G, A);
-    hipLaunchKernelGGL(k_dem_result, dim3(1), dim3(64), 0, st, s->cm_row[b] + n, bad,
-                       (uint32_t *)s->ctx->res_dev);
+    volatile uint32_t *res = (volatile uint32_t *)s->ctx->res;
+    res[1] = 0;
+    hipLaunchKernelGGL(rows, dim3(pb_blocks(n, DEM_ROWS_BS / ln)), dim3(DEM_ROWS_BS), 0, st, G, A);
     PB_LAUNCH_CHECK(s->ctx, "k_dem_rows");
     PB_HIP(s->ctx, hipStreamSynchronize(st));
-    nnz = ((const uint32_t *)s->ctx->res)[0];
-    nbad = ((const uint32_t *)s->ctx->res)[1];
-    return PB_OK;
+    nnz = res[0];
+    nbad = 0;
+    return res[1] ? pb_io_download(s->ctx, &nbad, bad, sizeof(nbad)) : PB_OK;
   };
   if ((rc = contacts_and_force())) return rc;
   if (nnz > s->cm_cap[b]) {                  // the matrix outgrew the arrays: again, larger

@@ -222,6 +222,7 @@ struct pb_sys {
   uint32_t *dem_inv = nullptr;                 // original index -> storage slot
   uint32_t dem_inv_order = 0;                  // order_gen dem_inv was made for (0: none)
   double4 *dem_rs = nullptr;                   // cell order: (x, y, z, radius)
+  float4 *dem_fq = nullptr;                    // the same in FP32
   uint32_t *dem_rowbuf = nullptr;              // contacts kept by the counting scan
   uint32_t dem_bad = 0;                        // Cundall-Strack violations of the last call
 };

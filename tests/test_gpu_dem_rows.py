@@ -80,3 +80,37 @@ def test_row_lengths(ctx, orc, law):
             if want.size:
                 assert np.abs(got - want).max() <= 1e-11 * np.abs(want).max(), call
         prow, pcol, pval = orow, ocol, h
+
+
+@pytest.mark.parametrize("scale", [1e-20, 1.0, 1e19])
+@pytest.mark.parametrize("single", [False, True])
+def test_contacts_beyond_fp32(ctx, orc, scale, single):
+    """Contacts of particles outside the grid (binned into its edge cells), and at
+    scales whose squares leave FP32: the CSR bit for bit."""
+    print(f"\n[case] contacts outside the grid, scale {scale}, 125 cells {single}", flush=True)
+    rng = np.random.default_rng(6)
+    if single:                                # at most one particle a cell of the grid
+        g = (np.arange(8) + 0.5) * 0.98
+        x = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+        x += rng.uniform(-5e-3, 5e-3, x.shape)
+        rad, box = np.full(len(x), 0.5), 8 * 0.98
+    else:
+        x, box = rng.uniform(0.0, 8.0, (800, 3)), 8.0
+        rad = rng.uniform(0.4, 0.6, len(x))
+    far = [(1e3, 4.0, 4.0), (1e3, 4.3, 4.0), (-40.0, -40.0, -40.0), (4.0, 4.0, 1e9), (4.0, 4.4, 1e9)]
+    x = np.concatenate([x, far]) * scale
+    rad = np.concatenate([rad, np.full(len(far), 0.5)]) * scale
+    n = len(x)
+    s = pb.System(ctx, [n])
+    s.set_cell(np.array([0.0, box, 0.0, box, 0.0, box]) * scale)
+    s.import_particles(x, np.ones(n))
+    s.dem_set_properties(E, MU, SIG, G2, MU_R, rad)
+    s.rot_set_inertia(rad)
+    s.setup_cells(scale * (2 * 0.5 / np.sqrt(3.0) if single else 1.2), periodic=False,
+                  single_particle=single)
+    s.bin()
+    nnz = s.dem_calc_force(1e-9, autotune=True)
+    row, col, _ = s.dem_contacts()
+    orow, ocol = orc.dem_contacts(x, rad, np.ones(n, np.uint8))
+    assert nnz == len(ocol) and np.array_equal(row, orow) and np.array_equal(col, ocol)
+    assert np.diff(orow)[-2:].tolist() == [1, 1]        # a pair outside touches
