@@ -137,6 +137,7 @@ struct pb_sys {
   uint32_t list_ncell = 0;
   double list_rlist = 0.0;         // largest list radius over the replicas
   uint32_t *list_segs = nullptr;   // list-build work units (8 words each)
+  bool list_thin = false;         // some replica is one whole segment
   uint32_t list_nsegs = 0;
   uint4 *list_wtab = nullptr;      // per-segment window tables (cell order of the last sort)
   uint32_t list_wtab_cap = 0;      // segments list_wtab holds

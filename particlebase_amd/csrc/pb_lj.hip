@@ -907,6 +907,10 @@ struct PairSums {
   }
 };
 
+// variants whose pair bodies are long: FP64 energies, table look-ups with either
+template <bool MIXED, bool ENERGY, bool ONE_TYPE>
+constexpr bool lj_heavy() { return (ENERGY && (!MIXED || !ONE_TYPE)) || (!MIXED && !ONE_TYPE); }
+
 // Pairs and integration of one segment's tile particles, LN lanes a particle
 // (each evaluates its own word pairs of the row; the first integrates).  With
 // FAST (window staged, no minimum image) a lane takes a word pair (ten pairs) a
@@ -917,7 +921,7 @@ struct PairSums {
 // step against 131 with two lanes, 151 with four, 178 with eight); with too few
 // particles to fill the chip a row is a serial chain and more lanes shorten it
 // (run_lanes).
-template <bool FAST, bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, uint32_t LN>
+template <bool FAST, bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, uint32_t LN, bool WIDE>
 __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const ListSeg &G,
                                          const RepInfo &R, bool staged, bool mi, double &ke, double &pe_b,
                                          double &vir_b, float &d2m, float &v2m,
@@ -997,6 +1001,10 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
       }
       P.add(A, dx, dy, dz, ONE_TYPE ? 0u : ti * PB_MAXT + (uint32_t)pj.w, FAST || !mi || q != NL_PAD);
     };
+    // pairs whose instructions may interleave: five, or two of the variants with
+    // long pair bodies (400,000 atoms, two types: 122 us an energy step against
+    // 134 with five, FP64; 85 against 96 without energies)
+    constexpr bool HEAVY = lj_heavy<MIXED, ENERGY, ONE_TYPE>();
     // rows are padded with the inert entry to whole word pairs
     constexpr uint32_t EPW = FAST ? 5u : 4u, EB = FAST ? 12u : 16u;
     constexpr uint32_t EMASK = (1u << EB) - 1u;
@@ -1018,7 +1026,12 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
         const uint64_t w64 = qw;
         qw = *wp;                                 // one word ahead (slack words at the end)
         wp += (b & 1u) ? 1u : 2u * LN * ld - 1u;
-        batch(w64);
+        if constexpr (HEAVY && !WIDE) {           // fewer registers: one pair at a time
+#pragma unroll 1
+          for (uint32_t j = 0; j < EPW; ++j) pair((uint32_t)(w64 >> (EB * j)) & EMASK);
+        } else {
+          batch(w64);
+        }
       }
     } else {
       // one 16-byte load brings the next two words while ten pairs are
@@ -1042,11 +1055,19 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
         // would be fetched for nothing when all their lanes are done)
         if (b + 1u < npair) qq = *pp;
         pp += LN * ld;
+        if constexpr (HEAVY) {
 #pragma unroll
-        for (uint32_t j = 0; j < EPW; ++j) pair(e[j]);
-        __builtin_amdgcn_sched_barrier(0);
+          for (uint32_t j = 0; j < 2 * EPW; ++j) {
+            pair(e[j]);
+            if (j % 2u) __builtin_amdgcn_sched_barrier(0);
+          }
+        } else {
 #pragma unroll
-        for (uint32_t j = 0; j < EPW; ++j) pair(e[EPW + j]);
+          for (uint32_t j = 0; j < EPW; ++j) pair(e[j]);
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (uint32_t j = 0; j < EPW; ++j) pair(e[EPW + j]);
+        }
       }
     }
     double fx = P.fx, fy = P.fy, fz = P.fz, pe = P.pe, vir = P.vir;
@@ -1119,7 +1140,7 @@ __device__ __forceinline__ void lj_tiles(const StepArgs &A, Stage &S, const List
 
 // One segment: stage its window, pairs + integration of its tile
 // particles, block maxima and energy partials.
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, uint32_t LN>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, uint32_t LN, bool WIDE>
 __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   __shared__ Stage S;
   const ListSeg G = A.segs[seg];
@@ -1132,10 +1153,10 @@ __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   double ke = 0.0, pe_b = 0.0, vir_b = 0.0;
   float d2m = 0.f, v2m = 0.f;
   if (staged && !mi)          // block-uniform: the common case, branch-free pairs
-    lj_tiles<true, MIXED, ENERGY, WRITE_F, ONE_TYPE, LN>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
+    lj_tiles<true, MIXED, ENERGY, WRITE_F, ONE_TYPE, LN, WIDE>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
                                                      v2m, S.hsum);
   else
-    lj_tiles<false, MIXED, ENERGY, WRITE_F, ONE_TYPE, LN>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
+    lj_tiles<false, MIXED, ENERGY, WRITE_F, ONE_TYPE, LN, WIDE>(A, S, G, R, staged, mi, ke, pe_b, vir_b, d2m,
                                                       v2m, S.hsum);
 
   __shared__ float smx[2][MAXWV];
@@ -1191,7 +1212,7 @@ __device__ __forceinline__ void lj_segment(const StepArgs &A, uint32_t seg) {
   }
 }
 
-template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST, uint32_t LN>
+template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST, uint32_t LN, bool WIDE>
 __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
   publish_prev(A);
   if constexpr (PERSIST) {
@@ -1219,7 +1240,7 @@ __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
         continue;
       }
       const uint32_t seg = __builtin_amdgcn_readfirstlane(q * per + (q < rmd ? q : rmd) + t);
-      lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE, LN>(A, seg);
+      lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE, LN, WIDE>(A, seg);
     }
     if (threadIdx.x == 0) {
       __threadfence();
@@ -1234,20 +1255,22 @@ __device__ __forceinline__ void lj_step_impl(const StepArgs &A) {
   // eight consecutive segments per XCD in every 64 (pb_xcd_chunk8): the same
   // as one slab per XCD on a uniform fluid, 3 % faster on the batched
   // replicas, whose segment sizes vary with the replica
-  lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE, LN>(A, pb_xcd_chunk8());
+  lj_segment<MIXED, ENERGY, WRITE_F, ONE_TYPE, LN, WIDE>(A, pb_xcd_chunk8());
 }
 
-// Two entry points over the same body: the common variants fit 128 VGPRs
-// (4 wavefronts per SIMD, two 512-thread workgroups per CU); the FP64 and
-// multi-type energy variants need more registers and run without the cap
-// (no spills) at lower occupancy.
+// Two entry points over the same body, the first within 128 VGPRs (4 wavefronts
+// per SIMD, two 512-thread workgroups per CU).  The heavy variants fit them with
+// the pairs of unstaged windows one at a time; replicas thinner than three cells,
+// whose pairs all take that path, run those variants without the cap instead
+// (400 particles, FP64 energies: 42 us a step against 44, two types 49 against 52;
+// 400,000 particles the other way: 122 against 88 and 170 against 122).
 template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST, uint32_t LN>
 __global__ void __launch_bounds__(tile_threads<LN>()) __attribute__((amdgpu_waves_per_eu(4))) k_lj_step(StepArgs A) {
-  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST, LN>(A);
+  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST, LN, false>(A);
 }
 template <bool MIXED, bool ENERGY, bool WRITE_F, bool ONE_TYPE, bool PERSIST, uint32_t LN>
 __global__ void __launch_bounds__(TBS) k_lj_step_wide(StepArgs A) {
-  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST, LN>(A);
+  lj_step_impl<MIXED, ENERGY, WRITE_F, ONE_TYPE, PERSIST, LN, true>(A);
 }
 
 // Forces (and energies) of the current positions without a list, for a single
@@ -1442,6 +1465,7 @@ static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &ski
   // nz <= nb2 - 2 so a window never holds one cell twice.  A replica with
   // fewer than 3 list cells along an axis is one whole segment.
   std::vector<ListSeg> segs;
+  s->list_thin = false;
   for (uint32_t q = 0; q < s->nrep; ++q) {
     RepInfo &R = s->reps[q];
     R.seg0 = (uint32_t)segs.size();
@@ -1451,6 +1475,7 @@ static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &ski
         return pb_fail(s->ctx, PB_ERR_CELLS,
                        "a replica thinner than 3 list cells must fit one LDS window");
       segs.push_back(ListSeg{q, 0, 0, 0, 1, 1, 1, 1});
+      s->list_thin = true;
     } else {
       const double per_cell = (double)R.natoms / nc;
       const uint32_t want = tile_target(lanes);
@@ -1629,36 +1654,39 @@ __global__ void __launch_bounds__(256) k_energy_reduce(const double *partials, c
 typedef void (*StepKernel)(StepArgs);
 
 template <bool MIXED, bool ONE, bool E, bool W, bool P, uint32_t LN>
-static StepKernel pick1() {
-  // variants that do not fit 128 VGPRs without spilling
-  if constexpr ((E && (!MIXED || !ONE)) || (!MIXED && !ONE))
-    return k_lj_step_wide<MIXED, E, W, ONE, P, LN>;
-  else
-    return k_lj_step<MIXED, E, W, ONE, P, LN>;
+static StepKernel pick1(bool thin) {
+  if constexpr (lj_heavy<MIXED, E, ONE>())
+    if (thin) return k_lj_step_wide<MIXED, E, W, ONE, P, LN>;
+  return k_lj_step<MIXED, E, W, ONE, P, LN>;
 }
 
 template <bool MIXED, bool ONE, bool P, uint32_t LN>
-static StepKernel pick3(bool energy, bool wf) {
-  if (energy) return wf ? pick1<MIXED, ONE, true, true, P, LN>() : pick1<MIXED, ONE, true, false, P, LN>();
-  return wf ? pick1<MIXED, ONE, false, true, P, LN>() : pick1<MIXED, ONE, false, false, P, LN>();
+static StepKernel pick3(bool energy, bool wf, bool thin) {
+  if (energy)
+    return wf ? pick1<MIXED, ONE, true, true, P, LN>(thin) : pick1<MIXED, ONE, true, false, P, LN>(thin);
+  return wf ? pick1<MIXED, ONE, false, true, P, LN>(thin) : pick1<MIXED, ONE, false, false, P, LN>(thin);
 }
 
 // the persistent form has one lane a particle
 template <bool MIXED, bool ONE>
-static StepKernel pick2(bool energy, bool wf, bool persist, uint32_t lanes) {
-  if (persist) return pick3<MIXED, ONE, true, 1u>(energy, wf);
+static StepKernel pick2(bool energy, bool wf, bool persist, uint32_t lanes, bool thin) {
+  if (persist) return pick3<MIXED, ONE, true, 1u>(energy, wf, thin);
   switch (lanes) {
-    case 8: return pick3<MIXED, ONE, false, 8u>(energy, wf);
-    case 4: return pick3<MIXED, ONE, false, 4u>(energy, wf);
-    case 2: return pick3<MIXED, ONE, false, 2u>(energy, wf);
-    default: return pick3<MIXED, ONE, false, 1u>(energy, wf);
+    case 8: return pick3<MIXED, ONE, false, 8u>(energy, wf, thin);
+    case 4: return pick3<MIXED, ONE, false, 4u>(energy, wf, thin);
+    case 2: return pick3<MIXED, ONE, false, 2u>(energy, wf, thin);
+    default: return pick3<MIXED, ONE, false, 1u>(energy, wf, thin);
   }
 }
 
-static StepKernel pick_kernel(bool mixed, bool one, bool energy, bool wf, bool persist, uint32_t lanes) {
+// thin: some replica is one whole segment
+static StepKernel pick_kernel(bool mixed, bool one, bool energy, bool wf, bool persist, uint32_t lanes,
+                              bool thin) {
   if (mixed)
-    return one ? pick2<true, true>(energy, wf, persist, lanes) : pick2<true, false>(energy, wf, persist, lanes);
-  return one ? pick2<false, true>(energy, wf, persist, lanes) : pick2<false, false>(energy, wf, persist, lanes);
+    return one ? pick2<true, true>(energy, wf, persist, lanes, thin)
+               : pick2<true, false>(energy, wf, persist, lanes, thin);
+  return one ? pick2<false, true>(energy, wf, persist, lanes, thin)
+             : pick2<false, false>(energy, wf, persist, lanes, thin);
 }
 
 // Lanes a particle in a run, by the particles of all replicas together (us a
@@ -1681,13 +1709,13 @@ static uint32_t run_lanes(const pb_sys *s, bool persistent) {
 static int launch_step(pb_sys *s, const StepArgs &A, bool mixed, bool energy, bool wf,
                        hipEvent_t ev0 = nullptr, hipEvent_t ev1 = nullptr) {
   const bool one = s->lj.ntypes == 1;
-  StepKernel k = pick_kernel(mixed, one, energy, wf, A.queue != nullptr, s->plan_lanes);
+  StepKernel k = pick_kernel(mixed, one, energy, wf, A.queue != nullptr, s->plan_lanes, s->list_thin);
   // persistent form: two 512-thread workgroups per compute unit (the step
   // kernel's LDS and register use), never more than there are segments
   const uint32_t grid = A.queue ? std::min<uint32_t>(s->list_nsegs, 2u * (uint32_t)std::max(s->ctx->cu_count, 1))
                                 : s->list_nsegs;
   // the uncapped variants keep the smaller workgroup (their registers)
-  const bool wide = (energy && (!mixed || !one)) || (!mixed && !one);
+  const bool wide = s->list_thin && ((energy && (!mixed || !one)) || (!mixed && !one));
   const uint32_t threads = s->plan_lanes == 2 && !wide ? tile_threads<2u>() : (uint32_t)TBS;
   if (ev0 && ev1)
     hipExtLaunchKernelGGL(k, dim3(grid), dim3(threads), 0, s->ctx->stream, ev0, ev1, 0u, A);
