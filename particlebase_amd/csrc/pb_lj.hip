@@ -1282,6 +1282,10 @@ __global__ void __launch_bounds__(TBS) k_lj_step_wide(StepArgs A) {
 //      of r2 - rc2, seven instructions each), then the pair body per hit;
 //   more (too few particles to fill the chip): every lane evaluates every LN-th
 //      candidate outright, a short serial chain, and the lanes' sums are added.
+//      Its loops stay rolled: a wavefront passes the code once, and fetching the
+//      unrolled form (28 KB) took longer than what it hid (4924 atoms, the call:
+//      52.5 against 49.5 us, two types 61 against 53; 64,000, two types 137
+//      against 125).
 // 1,048,576 atoms: the call, sort included, takes 660 us against 880 with a
 // list (FP64); 864 atoms: this kernel 13 us against 42 (list) + 12.
 template <bool MIXED, bool ENERGY, bool ONE_TYPE, uint32_t LN>
@@ -1341,7 +1345,7 @@ __global__ void __launch_bounds__(TBS) k_lj_direct(StepArgs A) {
               }
             }
           } else {
-#pragma unroll 4
+#pragma unroll 1
             for (uint32_t q = q0 + sl; q < q1; q += LN) pair(q);
           }
           return;
@@ -1365,7 +1369,9 @@ __global__ void __launch_bounds__(TBS) k_lj_direct(StepArgs A) {
         uint32_t tz = 1;
         while (tz < G.nz && W.eoff[col * W.zs + tz + 1] <= li) ++tz;
         const uint32_t wy = G.ty + 2, ca = col / wy, cb = col % wy;
+#pragma unroll 1
         for (uint32_t a = ca - 1; a <= ca + 1; ++a)
+#pragma unroll 1
           for (uint32_t b = cb - 1; b <= cb + 1; ++b) {
             const uint32_t e0 = (a * wy + b) * W.zs + tz - 1;
             scan(W.eoff[e0], W.eoff[e0 + 3]);        // three z slots
