@@ -393,6 +393,9 @@ __device__ __forceinline__ double pb_load_relaxed(const double *p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// replicas from which a reduction takes a wavefront for each (and callers a
+// workgroup of 1024)
+constexpr uint32_t PB_REDUCE_WAVES = 4;
 // sum of K per-wave partial components for every replica, executed by one
 // block (used by the last-block reductions and by k_reduce_waves).
 __device__ __forceinline__ void pb_block_reduce_reps(const double *partials, int K, const RepInfo *reps,
@@ -406,15 +409,40 @@ __device__ __forceinline__ void pb_block_reduce_reps(const double *partials, int
   // scratch: 4 x 256 doubles of the caller's LDS
   double (*sm)[256] = reinterpret_cast<double (*)[256]>(scratch);
   const uint32_t t = threadIdx.x, bs = blockDim.x;
-  if (nrep >= 16) {
-    for (uint32_t q = t; q < nrep; q += bs) {
-      const RepInfo R = reps[q];
-      const uint32_t w0 = by_segment ? R.seg0 : R.wave0, nw = by_segment ? R.nseg : R.nwave;
-      double acc[4] = {0, 0, 0, 0};
-      for (uint32_t w = w0; w < w0 + nw; ++w)
-        for (int c = 0; c < K; ++c)
-          acc[c] += partials[4 * w + c];
-      for (int c = 0; c < K; ++c) out[8 * q + c] = acc[c];
+  const RepInfo &last = reps[nrep - 1u];
+  const uint32_t parts = by_segment ? last.seg0 + last.nseg : last.wave0 + last.nwave;
+  if (nrep >= PB_REDUCE_WAVES && parts <= 2048u * nrep) {
+    // a wavefront a replica, four of them in flight (a thread a replica was a
+    // chain of its partials: 256 replicas of 8000 particles 104 us, with 16
+    // wavefronts 22; one replica after the other by the whole workgroup, 15 of
+    // 500 to 4000 particles: mv2 37.5 us a call, now 19.4).  Few replicas of very
+    // many partials keep the whole workgroup on each (4 of 400,000 particles:
+    // 61 us a call against 62.5).
+    constexpr uint32_t Q = 4;
+    const uint32_t lane = pb_lane(), nwv = bs / PB_WAVE;
+    for (uint32_t q0 = t / PB_WAVE; q0 < nrep; q0 += nwv * Q) {
+      uint32_t w0[Q], nw[Q], most = 0;
+      double acc[Q][4] = {};
+#pragma unroll
+      for (uint32_t k = 0; k < Q; ++k) {
+        const RepInfo &R = reps[min(q0 + k * nwv, nrep - 1u)];
+        w0[k] = by_segment ? R.seg0 : R.wave0;
+        nw[k] = q0 + k * nwv < nrep ? (by_segment ? R.nseg : R.nwave) : 0u;
+        most = max(most, nw[k]);
+      }
+      for (uint32_t w = lane; w < most; w += PB_WAVE)
+#pragma unroll
+        for (uint32_t k = 0; k < Q; ++k)
+          if (w < nw[k])
+            for (int c = 0; c < K; ++c) acc[k][c] += partials[4 * (size_t)(w0[k] + w) + c];
+#pragma unroll
+      for (uint32_t k = 0; k < Q; ++k)
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+          if (c < K) {
+            const double x = pb_wave_sum(acc[k][c]);
+            if (lane == 0 && q0 + k * nwv < nrep) out[8 * (q0 + k * nwv) + c] = x;
+          }
     }
     return;
   }
@@ -427,16 +455,14 @@ __device__ __forceinline__ void pb_block_reduce_reps(const double *partials, int
     if (t < T)
       for (uint32_t w = t; w < nw; w += T)
         for (int c = 0; c < K; ++c) acc[c] += partials[4 * (w0 + w) + c];
-    if (t < T)
-      for (int c = 0; c < K; ++c) sm[c][t] = acc[c];
+#pragma unroll
+    for (int c = 0; c < 4; ++c)
+      if (t < T && c < K) {
+        const double x = pb_wave_sum(acc[c]);
+        if (t % PB_WAVE == 0) sm[c][t / PB_WAVE] = x;
+      }
     __syncthreads();
-    for (uint32_t o = T / 2; o > 0; o >>= 1) {
-      if (t < o)
-        for (int c = 0; c < K; ++c) sm[c][t] += sm[c][t + o];
-      __syncthreads();
-    }
-    if (t == 0)
-      for (int c = 0; c < K; ++c) out[8 * q + c] = sm[c][0];
+    if (t < (uint32_t)K) out[8 * q + t] = (sm[t][0] + sm[t][1]) + (sm[t][2] + sm[t][3]);
     __syncthreads();
   }
 }

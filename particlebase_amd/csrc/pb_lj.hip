@@ -1646,7 +1646,7 @@ static StepArgs make_args(pb_sys *s, double dt) {
 // Energy record of a step: per-replica sums of the per-segment partials in a
 // fixed order (deterministic), into record counter[CNT_REC], which is then
 // advanced.  A separate launch: stream order makes the partials visible.
-__global__ void __launch_bounds__(256) k_energy_reduce(const double *partials, const RepInfo *reps,
+__global__ void __launch_bounds__(1024) k_energy_reduce(const double *partials, const RepInfo *reps,
                                                        uint32_t nrep, double *energy,
                                                        uint32_t *counter, uint32_t *counts_out) {
   __shared__ double sm[4 * 256];
@@ -1656,6 +1656,9 @@ __global__ void __launch_bounds__(256) k_energy_reduce(const double *partials, c
   if (threadIdx.x == 0) counter[CNT_REC] = rec + 1;
   if (counts_out && threadIdx.x < 16) counts_out[threadIdx.x] = counter[threadIdx.x];
 }
+
+// workgroup of a reduction over all replicas
+static uint32_t reduce_threads(const pb_sys *s) { return s->nrep >= PB_REDUCE_WAVES ? 1024u : 256u; }
 
 typedef void (*StepKernel)(StepArgs);
 
@@ -1728,7 +1731,7 @@ static int launch_step(pb_sys *s, const StepArgs &A, bool mixed, bool energy, bo
   else
     hipLaunchKernelGGL(k, dim3(grid), dim3(threads), 0, s->ctx->stream, A);
   if (energy)
-    hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(256), 0, s->ctx->stream, A.partials, A.reps,
+    hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(reduce_threads(s)), 0, s->ctx->stream, A.partials, A.reps,
                        A.nrep, A.energy, A.counter, (uint32_t *)nullptr);
   PB_LAUNCH_CHECK(s->ctx, "k_lj_step");
   return PB_OK;
@@ -1827,7 +1830,7 @@ extern "C" int pb_lj_force(pb_sys *s, int precision, double *pe, double *virial)
   hipStream_t st = s->ctx->stream;
   hipLaunchKernelGGL(k, dim3(s->list_nsegs), dim3(TBS), 0, st, A);
   if (energy)
-    hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(256), 0, st, A.partials, A.reps, A.nrep, A.energy,
+    hipLaunchKernelGGL(k_energy_reduce, dim3(1), dim3(reduce_threads(s)), 0, st, A.partials, A.reps, A.nrep, A.energy,
                        A.counter, (uint32_t *)s->ctx->res_dev);
   PB_LAUNCH_CHECK(s->ctx, "k_lj_direct");
   std::vector<double> far;
