@@ -253,7 +253,7 @@ static void half_cell2(const pb_sys *s, uint32_t q, float c[3]) {
 // A tile pair adds at most GR_T * GR_T = 2^16 pairs to one bin of the
 // workgroup's uint32 LDS histogram; flushing at least every 2^14 work items
 // keeps every bin and the pair count below 2^31, whatever the replica's size.
-#define GR_FLUSH_ITEMS 16384u
+#define GR_FLUSH_TILES 16384u
 struct GrRep {
   uint32_t atom0, natoms, ntile;
   uint64_t pair0;      // first tile-pair index of this replica
@@ -401,8 +401,8 @@ __global__ void __launch_bounds__(GR_T) k_gr(const double4 *r, const GrRep *reps
       if (qn) work_off(qn);                // fewer than 64
     }
     // flush when the replica changes, at the end (histograms are per
-    // replica) and every GR_FLUSH_ITEMS items (no uint32 count can wrap)
-    const bool flush = w + 1 >= w1 || ++since >= GR_FLUSH_ITEMS ||
+    // replica) and every GR_FLUSH_TILES work items (no uint32 count can wrap)
+    const bool flush = w + 1 >= w1 || ++since >= GR_FLUSH_TILES ||
                        (rep + 1 < nrep && (w + 1) / slices >= reps[rep + 1].pair0);
     if (flush) {
       __syncthreads();
