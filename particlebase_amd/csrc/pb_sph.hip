@@ -9,12 +9,11 @@
 // particles are gathered into cell order once per call (positions with the
 // mass in w, velocities, per-particle material terms); one kernel computes
 // the number density, rho, 1/rho and the field mu in a single pass over
-// the 27 cells, and one kernel computes the acceleration.  Both stage the
-// cell-sorted views through LDS column by column (neighbour cells of a
-// column are one contiguous range) and write straight to the particle's
-// storage slot: no partial buffers, no reductions.  Distances are
-// non-periodic (distance2,
-// kernelinline.hh:19-29); the density sum includes the particle itself, the
+// the 27 cells, and one kernel computes the acceleration.  Both test FP32
+// views of the candidates, staged in LDS column by column (neighbour cells of a
+// column are one contiguous range), evaluate what passes in FP64 and write
+// straight to the particle's storage slot: no partial buffers, no reductions.
+// Distances are non-periodic (distance2, kernelinline.hh:19-29); the density sum includes the particle itself, the
 // acceleration sum excludes it; rho0 = 1 (cudaParticleSPH_NS.cu:91).
 //
 // The same calls also run the dam-break workload's config physics, which the
@@ -541,10 +540,11 @@ static int sph_alloc_views(pb_sys *s) {
   const size_t np = s->npad;
   int rc = PB_OK;
   if (!s->sph_rs) {
+    // sph_rs last: the others exist where it does
     if ((rc = pb_alloc(s->ctx, &s->sph_rhoinv, np)) || (rc = pb_alloc(s->ctx, &s->sph_num, np)) ||
-        (rc = pb_alloc(s->ctx, &s->sph_rs, np)) || (rc = pb_alloc(s->ctx, &s->sph_vs, np)) ||
-        (rc = pb_alloc(s->ctx, &s->sph_ds, np)) || (rc = pb_alloc(s->ctx, &s->sph_mus, np)) ||
-        (rc = pb_alloc(s->ctx, &s->sph_fq, np)))
+        (rc = pb_alloc(s->ctx, &s->sph_vs, np)) || (rc = pb_alloc(s->ctx, &s->sph_ds, np)) ||
+        (rc = pb_alloc(s->ctx, &s->sph_mus, np)) || (rc = pb_alloc(s->ctx, &s->sph_fq, np)) ||
+        (rc = pb_alloc(s->ctx, &s->sph_rs, np)))
       return rc;
   }
   hipStream_t st = s->ctx->stream;
