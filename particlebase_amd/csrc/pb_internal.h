@@ -176,6 +176,7 @@ struct pb_sys {
   // Gaussian thermostat: per replica {xi, 1/c} of the last step, and the
   // count of steps whose implicit velocity equation had no solution
   double *gt = nullptr;
+  double *gt_part = nullptr;       // partials of its second pass, one set a wavefront
   uint32_t *gt_bad = nullptr;
 
   // MD neighbour list (cudaParticleMD::makeNList): CSR by original index

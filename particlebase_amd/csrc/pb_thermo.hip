@@ -17,8 +17,9 @@
 // xi; when that pass already moves v by no more than tol (always so when
 // xi(t-dt) = 0, as on the first step) the reference stops there with the
 // one-pass velocity and xi of it, so that pass is evaluated too and decides
-// the branch exactly as the loop's test does.  Five launches, no host
-// synchronisation:
+// the branch exactly as the loop's test does.  Three to five launches, no host
+// synchronisation (the solves are part of the kernels after them for small
+// replicas):
 //   k_gt_a       A into v, v' = v + dt/2m (F + Fold) into a; partials
 //                F.A, m A.A, m v'.v'
 //   k_gt_solve1  per replica (fixed order): 1/c, xi of the fixed point,
@@ -30,8 +31,10 @@
 //                Fold = F
 // Per-replica xi persists on the device between steps (GaussianThermo::xi).
 #include "pb_internal.h"
+#include <algorithm>
 
 #define GT_BLOCK 256
+#define GT_SOLVE_WAVES 512u   // largest replica solved without launches of its own
 
 namespace {
 
@@ -74,8 +77,57 @@ __global__ void __launch_bounds__(GT_BLOCK)
   }
 }
 
-// One workgroup.  A replica whose A vanishes (all particles at rest, no
-// force) has no defined xi: g = 0.
+// Sums of a replica's partials in every lane of a wavefront (fixed order)
+struct GtSums {
+  double x[3];
+  __device__ __forceinline__ GtSums(const double *partials, const RepInfo &R) {
+    double a[3] = {0.0, 0.0, 0.0};
+    for (uint32_t w = pb_lane(); w < R.nwave; w += PB_WAVE)
+#pragma unroll
+      for (int c = 0; c < 3; ++c) a[c] += partials[4 * (size_t)(R.wave0 + w) + c];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) x[c] = pb_wave_sum(a[c]);
+  }
+};
+
+// 1/c, xi of the fixed point and 1 / sum m v'^2 from the sums of k_gt_a.  A
+// replica whose A vanishes (all particles at rest, no force) has no defined
+// xi: g = 0.
+struct GtSolve1 {
+  double cinv, mv2inv, xi;
+  __device__ __forceinline__ GtSolve1(double fa, double ma2, double mv2, double dt) {
+    const double g = ma2 > 0.0 ? fa / ma2 : 0.0;
+    cinv = 1.0 - 0.5 * dt * g;
+    mv2inv = mv2 > 0.0 ? 1.0 / mv2 : 0.0;
+    xi = g / cinv;
+  }
+};
+
+// The loop's test after its first pass, v0 = sqrt(sum q^2 / 3N) <= tol, picks
+// the one-pass result (1/c = -1); otherwise the fixed point, which has no
+// solution when 1/c <= 0 (dt too large for the forces; the reference's loop does
+// not converge there): bad, and taken as xi = 0, v = A.
+struct GtSolve2 {
+  double xi, cinv;
+  bool bad;
+  __device__ __forceinline__ GtSolve2(const double (&x)[3], double natoms, double tol, double cinv1,
+                                      double xi1) {
+    const double v0 = sqrt(x[0] / (3.0 * natoms));
+    bad = false;
+    xi = xi1;
+    cinv = cinv1;
+    if (!(v0 > tol)) {
+      xi = x[2] > 0.0 ? x[1] / x[2] : 0.0;
+      cinv = -1.0;
+    } else if (!(cinv1 > 0.0 && isfinite(xi1))) {
+      bad = true;
+      xi = 0.0;
+      cinv = 1.0;
+    }
+  }
+};
+
+// One workgroup.
 __global__ void __launch_bounds__(256)
     k_gt_solve1(const double *partials, const RepInfo *reps, uint32_t nrep, double dt,
                 double *out, double *gt) {
@@ -83,26 +135,42 @@ __global__ void __launch_bounds__(256)
   pb_block_reduce_reps(partials, 3, reps, nrep, out, false, sm);
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < nrep; q += blockDim.x) {
-    const double fa = out[8 * q], ma2 = out[8 * q + 1], mv2 = out[8 * q + 2];
-    const double g = ma2 > 0.0 ? fa / ma2 : 0.0;
-    const double cinv = 1.0 - 0.5 * dt * g;
-    gt[4 * q + 1] = cinv;
-    gt[4 * q + 2] = mv2 > 0.0 ? 1.0 / mv2 : 0.0;
-    gt[4 * q + 3] = g / cinv;
+    const GtSolve1 S(out[8 * q], out[8 * q + 1], out[8 * q + 2], dt);
+    gt[4 * q + 1] = S.cinv;
+    gt[4 * q + 2] = S.mv2inv;
+    gt[4 * q + 3] = S.xi;
   }
 }
 
 // The first pass of calcGaussianThermoFoverF_F4 (kernelfuncs.cu:407-454):
 // f = A - (dt/2 xi + 1) v', f' = -dt/2 (xi + (F - 2 xi m v') v' / sum m v'^2) - 1.
+// SOLVE: every wavefront sums its replica's partials `in` and solves for itself,
+// the first one stores the result (k_gt_solve1's).
+template <bool SOLVE>
 __global__ void __launch_bounds__(GT_BLOCK)
     k_gt_pass1(const double4 *v, const double4 *F, double4 *Fold, const uint32_t *orig,
-               const uint32_t *waveRep, const double *gt, uint32_t n, double dt,
-               double *partials) {
+               const uint32_t *waveRep, const RepInfo *reps, const double *in, double *gt,
+               uint32_t n, double dt, double *partials) {
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s >= n) return;                            // whole wavefronts
   double qq = 0.0, fv = 0.0, mv2 = 0.0;
-  if (s < n && orig[s] != PB_NONE) {
-    const double *G = gt + 4 * waveRep[s / PB_WAVE];
-    const double xi = G[0], mv2inv = G[2], dt2 = 0.5 * dt;
+  double *G = gt + 4 * waveRep[s / PB_WAVE];
+  double mv2inv;
+  if constexpr (SOLVE) {
+    const RepInfo &R = reps[waveRep[s / PB_WAVE]];
+    const GtSums T(in, R);
+    const GtSolve1 S(T.x[0], T.x[1], T.x[2], dt);
+    mv2inv = S.mv2inv;
+    if (pb_lane() == 0 && s / PB_WAVE == R.wave0) {
+      G[1] = S.cinv;
+      G[2] = S.mv2inv;
+      G[3] = S.xi;
+    }
+  } else {
+    mv2inv = G[2];
+  }
+  if (orig[s] != PB_NONE) {
+    const double xi = G[0], dt2 = 0.5 * dt;
     const double4 A = v[s], f = F[s], p = Fold[s];
     const double m = 1.0 / A.w, k1 = dt2 * xi + 1.0, k2 = 2.0 * xi * m;
     const double qx = (A.x - k1 * p.x) / (-dt2 * (xi + (f.x - k2 * p.x) * p.x * mv2inv) - 1.0);
@@ -117,7 +185,7 @@ __global__ void __launch_bounds__(GT_BLOCK)
   qq = pb_wave_sum(qq);
   fv = pb_wave_sum(fv);
   mv2 = pb_wave_sum(mv2);
-  if (pb_lane() == 0 && s < n) {
+  if (pb_lane() == 0) {
     double *P = partials + 4 * (s / PB_WAVE);
     P[0] = qq;
     P[1] = fv;
@@ -125,11 +193,7 @@ __global__ void __launch_bounds__(GT_BLOCK)
   }
 }
 
-// One workgroup: the loop's test after its first pass, v0 = sqrt(sum q^2 /
-// 3N) <= tol, picks the one-pass result; otherwise the fixed point, which
-// has no solution when 1/c <= 0 (dt too large for the forces; the
-// reference's loop does not converge there): counted in bad[0] and taken
-// as xi = 0, v = A.
+// One workgroup; steps without a solution are counted in bad[0].
 __global__ void __launch_bounds__(256)
     k_gt_solve2(const double *partials, const RepInfo *reps, uint32_t nrep, double tol,
                 double *out, double *gt, uint32_t *bad) {
@@ -138,28 +202,40 @@ __global__ void __launch_bounds__(256)
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < nrep; q += blockDim.x) {
     double *G = gt + 4 * q;
-    const double v0 = sqrt(out[8 * q] / (3.0 * reps[q].natoms));
-    if (!(v0 > tol)) {
-      const double mv2 = out[8 * q + 2];
-      G[0] = mv2 > 0.0 ? out[8 * q + 1] / mv2 : 0.0;
-      G[1] = -1.0;
-    } else if (G[1] > 0.0 && isfinite(G[3])) {
-      G[0] = G[3];
-    } else {
-      atomicAdd(bad, 1u);
-      G[0] = 0.0;
-      G[1] = 1.0;
-    }
+    const double x[3] = {out[8 * q], out[8 * q + 1], out[8 * q + 2]};
+    const GtSolve2 S(x, reps[q].natoms, tol, G[1], G[3]);
+    G[0] = S.xi;
+    G[1] = S.cinv;
+    if (S.bad) atomicAdd(bad, 1u);
   }
 }
 
+// SOLVE: as in k_gt_pass1, for k_gt_solve2; the first wavefront stores xi (the
+// others may still read the fixed point's terms, which stay).
+template <bool SOLVE>
 __global__ void __launch_bounds__(GT_BLOCK)
     k_gt_drift(double4 *r, double4 *v, const double4 *F, double4 *Fold, const uint32_t *orig,
-               const uint32_t *waveRep, const double *gt, uint32_t n, double dt) {
+               const uint32_t *waveRep, const RepInfo *reps, const double *in, double *gt,
+               uint32_t n, double dt, double tol, uint32_t *bad) {
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-  if (s >= n || orig[s] == PB_NONE) return;
-  const double *G = gt + 4 * waveRep[s / PB_WAVE];
-  const double xi = G[0], cinv = G[1];
+  if (s >= n) return;
+  double *G = gt + 4 * waveRep[s / PB_WAVE];
+  double xi, cinv;
+  if constexpr (SOLVE) {
+    const RepInfo &R = reps[waveRep[s / PB_WAVE]];
+    const GtSums T(in, R);
+    const GtSolve2 S(T.x, R.natoms, tol, G[1], G[3]);
+    xi = S.xi;
+    cinv = S.cinv;
+    if (pb_lane() == 0 && s / PB_WAVE == R.wave0) {
+      G[0] = xi;
+      if (S.bad) atomicAdd(bad, 1u);
+    }
+  } else {
+    xi = G[0];
+    cinv = G[1];
+  }
+  if (orig[s] == PB_NONE) return;
   double4 V = v[s];
   const double4 f = F[s];
   if (cinv < 0.0) {
@@ -311,6 +387,7 @@ __global__ void __launch_bounds__(GT_BLOCK)
 int ensure_gt(pb_sys *s) {
   if (s->gt) return PB_OK;
   if (int rc = pb_alloc(s->ctx, &s->gt_bad, 1)) return rc;
+  if (int rc = pb_alloc(s->ctx, &s->gt_part, 4 * (size_t)s->nwave)) return rc;
   if (int rc = pb_alloc(s->ctx, &s->gt, 4 * (size_t)s->nrep)) return rc;
   const uint32_t zero = 0;
   PB_HIP(s->ctx, hipMemcpyAsync(s->gt_bad, &zero, sizeof(uint32_t), hipMemcpyHostToDevice,
@@ -334,14 +411,28 @@ extern "C" int pb_gt_step(pb_sys *s, double dt, double tol) {
   hipStream_t st = s->ctx->stream;
   hipLaunchKernelGGL(k_gt_a, GT_GRID(s->npad), s->v, s->F, s->a, s->orig, s->waveRep, s->gt,
                      s->npad, dt, s->partials);
-  hipLaunchKernelGGL(k_gt_solve1, dim3(1), dim3(256), 0, st, s->partials, s->d_reps, s->nrep, dt,
-                     s->d_out, s->gt);
-  hipLaunchKernelGGL(k_gt_pass1, GT_GRID(s->npad), s->v, s->F, s->a, s->orig, s->waveRep, s->gt,
-                     s->npad, dt, s->partials);
-  hipLaunchKernelGGL(k_gt_solve2, dim3(1), dim3(256), 0, st, s->partials, s->d_reps, s->nrep, tol,
-                     s->d_out, s->gt, s->gt_bad);
-  hipLaunchKernelGGL(k_gt_drift, GT_GRID(s->npad), s->r, s->v, s->F, s->a, s->orig, s->waveRep,
-                     s->gt, s->npad, dt);
+  // Replicas of few wavefronts are solved by every wavefront of the kernels that
+  // need the result, two launches of one workgroup fewer; each reads all of its
+  // replica's partials, so larger ones keep the launches (us a step with 3 and
+  // with 5 launches: 500 particles 12.5, 20; 4924 11.4, 15.1; 16,000 12.8, 16.3;
+  // 32,000 15.4, 16.5; 64,000 20.9, 18.9).
+  uint32_t most = 0;
+  for (const RepInfo &R : s->reps) most = std::max(most, R.nwave);
+  if (most <= GT_SOLVE_WAVES) {
+    hipLaunchKernelGGL(k_gt_pass1<true>, GT_GRID(s->npad), s->v, s->F, s->a, s->orig, s->waveRep,
+                       s->d_reps, s->partials, s->gt, s->npad, dt, s->gt_part);
+    hipLaunchKernelGGL(k_gt_drift<true>, GT_GRID(s->npad), s->r, s->v, s->F, s->a, s->orig, s->waveRep,
+                       s->d_reps, s->gt_part, s->gt, s->npad, dt, tol, s->gt_bad);
+  } else {
+    hipLaunchKernelGGL(k_gt_solve1, dim3(1), dim3(256), 0, st, s->partials, s->d_reps, s->nrep, dt,
+                       s->d_out, s->gt);
+    hipLaunchKernelGGL(k_gt_pass1<false>, GT_GRID(s->npad), s->v, s->F, s->a, s->orig, s->waveRep,
+                       s->d_reps, (const double *)nullptr, s->gt, s->npad, dt, s->partials);
+    hipLaunchKernelGGL(k_gt_solve2, dim3(1), dim3(256), 0, st, s->partials, s->d_reps, s->nrep, tol,
+                       s->d_out, s->gt, s->gt_bad);
+    hipLaunchKernelGGL(k_gt_drift<false>, GT_GRID(s->npad), s->r, s->v, s->F, s->a, s->orig, s->waveRep,
+                       s->d_reps, (const double *)nullptr, s->gt, s->npad, dt, tol, s->gt_bad);
+  }
   PB_LAUNCH_CHECK(s->ctx, "pb_gt_step");
   return PB_OK;
 }
