@@ -183,6 +183,7 @@ extern "C" int pb_bin(pb_sys *s) {
   if (!s->ref_cells) return pb_fail(s->ctx, PB_ERR_STATE, "pb_bin: pb_setup_cells first");
   hipStream_t st = s->ctx->stream;
   const uint32_t nc = s->ref_ncell;
+  if (int rc = pb_counts_begin(s)) return rc;
   hipLaunchKernelGGL(k_ref_bid, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->r, s->orig,
                      s->npad, ref_grid(s), nc, s->cellid, s->ccount, s->rank);
   PB_LAUNCH_CHECK(s->ctx, "k_ref_bid");

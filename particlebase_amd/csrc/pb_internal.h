@@ -114,6 +114,7 @@ struct pb_sys {
   uint32_t *skey = nullptr, *sslot = nullptr, *scell = nullptr;   // grouped by cell
   uint32_t *ccount = nullptr, *cstart = nullptr;  // ncell_cap + 1
   uint32_t ncell_cap = 0;
+  bool counts_used = false;       // a sort began and its scatter, which clears ccount, was not launched
   uint32_t *scan_tmp = nullptr;
   size_t scan_tmp_n = 0;
 
@@ -273,6 +274,9 @@ struct PbCellOrder {
   const uint32_t *start;       // cell -> first position (start[c + 1] ends it)
   const uint32_t *skey, *sslot, *scell;
 };
+// before a counting kernel: ccount is zero (a sort given up in between leaves
+// counts, and ranks on top of them lie past the arrays)
+int pb_counts_begin(pb_sys *sys);
 // cellid[s] (PB_NONE never), the counts of every cell and the rank of s among
 // them given; cells start in sys->cstart
 int pb_counting_sort(pb_sys *sys, uint32_t ncell, const uint32_t *key, PbCellOrder *O);

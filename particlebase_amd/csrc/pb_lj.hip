@@ -97,7 +97,7 @@ __global__ void k_list_cellid(const double4 *r, const uint32_t *orig, const uint
                               const RepInfo *reps, uint32_t n, uint32_t *cellid,
                               uint32_t *counts, uint32_t *rank) {
   // the list cell of slot s (padding: the replica's pad cell), counted in
-  // the same pass (the counting sort's k_count)
+  // the same pass
   const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
   const bool valid = s < n;
   uint32_t c = PB_NONE;
@@ -1573,6 +1573,7 @@ static int sort_cells(pb_sys *s, bool carry_a, bool clear_all) {
   hipStream_t st = s->ctx->stream;
   const uint32_t n = s->npad;
   if (int rc = pb_ensure_sort_ws(s, s->list_ncell)) return rc;
+  if (int rc = pb_counts_begin(s)) return rc;
   hipLaunchKernelGGL(k_list_cellid, dim3(pb_blocks(n, 256)), dim3(256), 0, st, s->r, s->orig,
                      s->waveRep, s->d_reps, n, s->cellid, s->ccount, s->rank);
   PB_LAUNCH_CHECK(s->ctx, "k_list_cellid");

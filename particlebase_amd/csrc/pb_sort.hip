@@ -178,6 +178,7 @@ int pb_exclusive_scan(pb_sys *s, const uint32_t *in, uint32_t *out, uint32_t n) 
   const uint32_t nb = (n + SCAN_CH - 1) / SCAN_CH;
   const size_t need = (size_t)nb + 1;
   if (s->scan_tmp_n < need) {
+    s->scan_tmp_n = 0;
     if (int rc = pb_alloc(s->ctx, &s->scan_tmp, need)) return rc;
     s->scan_tmp_n = need;
   }
@@ -243,7 +244,18 @@ int pb_ensure_sort_ws(pb_sys *s, uint32_t ncell) {
                        s->ctx->stream, s->ccount, ncell + 1, 0u);
     PB_LAUNCH_CHECK(s->ctx, "sort workspace");
     s->ncell_cap = ncell;
+    s->counts_used = false;
   }
+  return PB_OK;
+}
+
+int pb_counts_begin(pb_sys *s) {
+  if (s->counts_used) {
+    hipLaunchKernelGGL(k_fill_u32, dim3(pb_blocks((size_t)s->ncell_cap + 1, 256)), dim3(256), 0,
+                       s->ctx->stream, s->ccount, s->ncell_cap + 1, 0u);
+    PB_LAUNCH_CHECK(s->ctx, "pb_counts_begin");
+  }
+  s->counts_used = true;
   return PB_OK;
 }
 
@@ -257,6 +269,7 @@ int pb_counting_sort(pb_sys *s, uint32_t ncell, const uint32_t *key, PbCellOrder
                      s->ctx->stream, s->cellid, s->rank, s->cstart, key, n, s->skey, s->sslot,
                      s->scell, s->ccount, ncell);
   PB_LAUNCH_CHECK(s->ctx, "pb_counting_sort");
+  s->counts_used = false;
   O->start = s->cstart;
   O->skey = s->skey;
   O->sslot = s->sslot;

@@ -1,0 +1,73 @@
+"""Calls that fail on the host part of the way (an allocation, a launch, an error
+left by other code) leave a system that the next call can use.  The library's
+host code runs against a stand-in for the HIP runtime (cpp/hip_host_stub.cpp)
+that fails a chosen call; kernels are recorded, not run.  No GPU."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+PRE = """
+import ctypes as C, sys
+stub = C.CDLL(sys.argv[1], mode=C.RTLD_GLOBAL)
+stub.stub_live_bytes.restype = stub.stub_most_items.restype = C.c_uint64
+for f in ("calls", "live", "dirty_counts", "launches"):
+    getattr(stub, "stub_" + f).restype = C.c_long
+fail = lambda name, k=1: stub.stub_fail(name.encode(), C.c_long(k))
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+import particlebase_amd as pb
+
+def raises(f, *a, **k):
+    try:
+        f(*a, **k)
+    except pb.PBError:
+        return True
+    return False
+
+def system(n=500, L=10.0, cells=None):
+    s = pb.System(pb.Context(0), [n])
+    s.set_cell([0, L] * 3)
+    s.import_particles(np.zeros((n, 3)), np.ones(n))
+    s.lj_set_params([1.0, 1.0], 1)
+    s.lj_set_cutoff(6.25, shifted=True)
+    if cells:
+        s.setup_cells(cells)
+    return s
+"""
+
+
+@pytest.fixture(scope="module")
+def stub(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("stub") / "libhipstub.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-std=c++17", "-I/opt/rocm/include", "-o", out,
+                    os.path.join(HERE, "cpp", "hip_host_stub.cpp")], check=True)
+
+    def run(code):
+        p = subprocess.run([sys.executable, "-c", PRE + textwrap.dedent(code), out, os.path.dirname(HERE)],
+                           capture_output=True, text=True, timeout=300)
+        assert p.returncode == 0, p.stdout + p.stderr
+    return run
+
+
+@pytest.mark.parametrize("call", ["s.bin()", "s.lj_force()", "s.lj_run(0.001, 1)"])
+@pytest.mark.parametrize("failure", ["stub.stub_pending_error()", "fail('k_scan')", "fail('k_scatter')",
+                                     "fail('hipMalloc')"])
+def test_sort_given_up_between_count_and_scatter(stub, call, failure):
+    """The cells' counters are zero when the next sort counts (29791 cells: the
+    scan allocates its block sums)."""
+    stub(f"""
+        s = system(500, 31.0, 1.0)
+        s.lj_set_cutoff(1.0, shifted=True)
+        {failure}
+        raises(lambda: {call})
+        stub.stub_fail(b"", C.c_long(0))
+        for _ in range(2):
+            s.bin()
+            s.lj_force()
+        assert stub.stub_launches(b"k_scatter") >= 4
+        assert stub.stub_dirty_counts() == 0, stub.stub_dirty_counts()
+    """)
