@@ -878,7 +878,7 @@ static int need_binned_grid(pb_sys *s, const char *who) {
 // the 27-cell search's arguments, on the positions gathered into cell order
 static int nlist_args(pb_sys *s, float rmax2t, NlistArgs *out) {
   int rc;
-  if (!s->md_pos &&
+  if (!s->md_cnt &&                          // the last of them
       ((rc = pb_alloc(s->ctx, &s->md_pos, s->npad)) || (rc = pb_alloc(s->ctx, &s->md_cnt, (size_t)s->n + 1))))
     return rc;
   hipLaunchKernelGGL(k_md_gather, dim3(pb_blocks(s->n, 256)), dim3(256), 0, s->ctx->stream, s->r,

@@ -248,9 +248,9 @@ extern "C" int pb_sys_set_cell(pb_sys *s, const double *cells) {
 
 int pb_ensure_rotation(pb_sys *s) {
   if (s->w) return PB_OK;
-  int rc;
-  if ((rc = pb_alloc(s->ctx, &s->w, s->npad)) || (rc = pb_alloc(s->ctx, &s->Lm, s->npad)) ||
-      (rc = pb_alloc(s->ctx, &s->T, s->npad)))
+  int rc;                                  // w last: the others exist where it does
+  if ((rc = pb_alloc(s->ctx, &s->Lm, s->npad)) || (rc = pb_alloc(s->ctx, &s->T, s->npad)) ||
+      (rc = pb_alloc(s->ctx, &s->w, s->npad)))
     return rc;
   hipStream_t st = s->ctx->stream;
   PB_HIP(s->ctx, hipMemsetAsync(s->w, 0, sizeof(double4) * s->npad, st));

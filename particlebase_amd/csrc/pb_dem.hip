@@ -630,8 +630,12 @@ extern "C" int pb_rot_step(pb_sys *s, double dt) {
 static int ensure_csr(pb_sys *s, int b, uint32_t nnz) {
   int rc;
   if (!s->cm_row[b] && (rc = pb_alloc(s->ctx, &s->cm_row[b], (size_t)s->n + 1))) return rc;
-  if (s->cm_cap[b] < nnz || !s->cm_col[b]) {
+  if (s->cm_cap[b] < nnz || !s->cm_cap[b]) {
     const uint32_t cap = (uint32_t)std::min<uint64_t>(((uint64_t)nnz * 5 / 4 + 512), 0xFFFFFFFFull);
+    // the matrix that the arrays held is gone, also if the new ones can't be had
+    s->cm_cap[b] = 0;
+    if (s->cm_cur == b) s->cm_cur = -1;
+    s->cm_prev = false;
     if ((rc = pb_alloc(s->ctx, &s->cm_col[b], cap)) ||
         (rc = pb_alloc(s->ctx, &s->cm_val[b], (size_t)cap * s->dem_hw)))
       return rc;

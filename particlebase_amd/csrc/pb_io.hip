@@ -272,8 +272,8 @@ static double4 *vec_field(pb_sys *s, int field) {
     case PB_FIELD_A: return s->a;
     case PB_FIELD_F: return s->F;
     case PB_FIELD_W: return s->w;
-    case PB_FIELD_L: return s->Lm;
-    case PB_FIELD_T: return s->T;
+    case PB_FIELD_L: return s->w ? s->Lm : nullptr;
+    case PB_FIELD_T: return s->w ? s->T : nullptr;
     case PB_FIELD_SPH_NUM: return s->sph_num;
     default: return nullptr;
   }

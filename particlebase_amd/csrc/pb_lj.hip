@@ -1519,6 +1519,7 @@ static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &ski
   // the ones its build stored)
   if (segs.size() > s->list_wtab_cap) {
     s->list_wtab_cap = 0;
+    s->lj_cont = false;
     if (int rc = pb_alloc(s->ctx, &s->list_wtab, (size_t)WTAB_U4 * segs.size())) return rc;
     s->list_wtab_cap = (uint32_t)segs.size();
   }
@@ -1542,13 +1543,22 @@ static int setup_list_cells(pb_sys *s, double rc, const std::vector<double> &ski
 // the other halves of the arrays that a sort permutes
 static int ensure_sort_buffers(pb_sys *s) {
   int rc;
-  if (!s->r2buf) {
-    if ((rc = pb_alloc(s->ctx, &s->r2buf, s->npad)) || (rc = pb_alloc(s->ctx, &s->v2buf, s->npad)) ||
-        (rc = pb_alloc(s->ctx, &s->a2buf, s->npad)) || (rc = pb_alloc(s->ctx, &s->orig2, s->npad)) ||
-        (rc = pb_alloc(s->ctx, &s->type2, s->npad)) || (rc = pb_alloc(s->ctx, &s->move2, s->npad)) ||
-        (rc = pb_alloc(s->ctx, &s->rbuild, s->npad)) || (rc = pb_alloc(s->ctx, &s->nn, s->npad)))
+  if (!s->r2buf) {                         // the last of them
+    if ((rc = pb_alloc(s->ctx, &s->v2buf, s->npad)) || (rc = pb_alloc(s->ctx, &s->a2buf, s->npad)) ||
+        (rc = pb_alloc(s->ctx, &s->orig2, s->npad)) || (rc = pb_alloc(s->ctx, &s->type2, s->npad)) ||
+        (rc = pb_alloc(s->ctx, &s->move2, s->npad)) || (rc = pb_alloc(s->ctx, &s->rbuild, s->npad)) ||
+        (rc = pb_alloc(s->ctx, &s->nn, s->npad)) || (rc = pb_alloc(s->ctx, &s->r2buf, s->npad)))
       return rc;
   }
+  return PB_OK;
+}
+
+// room for `words` doubles of energy records
+static int ensure_energy_records(pb_sys *s, size_t words) {
+  if (s->lj_ebuf_cap >= words) return PB_OK;
+  s->lj_ebuf_cap = 0;
+  if (int rc = pb_alloc(s->ctx, &s->lj_ebuf, words)) return rc;
+  s->lj_ebuf_cap = words;
   return PB_OK;
 }
 
@@ -1815,12 +1825,8 @@ extern "C" int pb_lj_force(pb_sys *s, int precision, double *pe, double *virial)
   const bool energy = (pe || virial), one = s->lj.ntypes == 1;
   // energies go straight to pinned memory when they fit behind the counters
   const bool direct = 16 + 8 * (size_t)s->nrep <= PB_RES_DOUBLES;
-  if (energy && !direct) {
-    if (s->lj_ebuf_cap < 8 * (size_t)s->nrep) {
-      if (int e = pb_alloc(s->ctx, &s->lj_ebuf, 8 * (size_t)s->nrep)) return e;
-      s->lj_ebuf_cap = 8 * (size_t)s->nrep;
-    }
-  }
+  if (energy && !direct)
+    if (int e = ensure_energy_records(s, 8 * (size_t)s->nrep)) return e;
   A.energy = direct ? s->ctx->res_dev + 16 : s->lj_ebuf;
   const StepKernel k =
       precision == PB_MIXED
@@ -1974,11 +1980,7 @@ extern "C" int pb_lj_run(pb_sys *s, const pb_run_opts *o, double *energies) {
   if (int rc = setup_list_cells(s, std::sqrt(s->rc2), skins, run_lanes(s, o->persistent != 0))) return rc;
   const uint32_t ne = o->energy_every;
   const uint32_t nrec = ne ? (o->nsteps + ne - 1) / ne : 0;
-  if (s->lj_ebuf_cap < (size_t)nrec * 8 * s->nrep) {
-    s->lj_ebuf_cap = 0;
-    if (int rc = pb_alloc(s->ctx, &s->lj_ebuf, (size_t)nrec * 8 * s->nrep)) return rc;
-    s->lj_ebuf_cap = (size_t)nrec * 8 * s->nrep;
-  }
+  if (int rc = ensure_energy_records(s, (size_t)nrec * 8 * s->nrep)) return rc;
   double *ebuf = nrec ? s->lj_ebuf : nullptr;
   int rc = PB_OK;
   uint32_t rebuilds = 0;

@@ -228,10 +228,10 @@ __global__ void k_cell_order(PbCellOrder O, uint32_t n, uint32_t *perm, uint32_t
 
 int pb_ensure_sort_ws(pb_sys *s, uint32_t ncell) {
   int rc;
-  if (!s->cellid) {
-    if ((rc = pb_alloc(s->ctx, &s->cellid, s->npad)) || (rc = pb_alloc(s->ctx, &s->rank, s->npad)) ||
-        (rc = pb_alloc(s->ctx, &s->perm, s->npad)) || (rc = pb_alloc(s->ctx, &s->skey, s->npad)) ||
-        (rc = pb_alloc(s->ctx, &s->sslot, s->npad)) || (rc = pb_alloc(s->ctx, &s->scell, s->npad)))
+  if (!s->cellid) {                        // the last of them
+    if ((rc = pb_alloc(s->ctx, &s->rank, s->npad)) || (rc = pb_alloc(s->ctx, &s->perm, s->npad)) ||
+        (rc = pb_alloc(s->ctx, &s->skey, s->npad)) || (rc = pb_alloc(s->ctx, &s->sslot, s->npad)) ||
+        (rc = pb_alloc(s->ctx, &s->scell, s->npad)) || (rc = pb_alloc(s->ctx, &s->cellid, s->npad)))
       return rc;
   }
   if (s->ncell_cap < ncell) {

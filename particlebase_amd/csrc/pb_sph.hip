@@ -559,8 +559,8 @@ extern "C" int pb_sph_set_properties(pb_sys *s, const double *mu0, const double 
   PB_HIP(s->ctx, hipSetDevice(s->ctx->device));
   int rc = PB_OK;
   const size_t np = s->npad;
-  if (!s->sph_mu0) {
-    if ((rc = pb_alloc(s->ctx, &s->sph_mu0, np)) || (rc = pb_alloc(s->ctx, &s->sph_c2, np)))
+  if (!s->sph_mu0) {                       // the last of them
+    if ((rc = pb_alloc(s->ctx, &s->sph_c2, np)) || (rc = pb_alloc(s->ctx, &s->sph_mu0, np)))
       return rc;
   }
   if ((rc = sph_alloc_views(s))) return rc;

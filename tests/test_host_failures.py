@@ -71,3 +71,72 @@ def test_sort_given_up_between_count_and_scatter(stub, call, failure):
         assert stub.stub_launches(b"k_scatter") >= 4
         assert stub.stub_dirty_counts() == 0, stub.stub_dirty_counts()
     """)
+
+
+ALLOCATING = {
+    "cells": "s.setup_cells(1.0); s.bin()",
+    "nlist": "s.setup_cells(2.5); s.coord_counts(6.25); s.nlist_build(6.25); s.lj_force_nlist()",
+    "force": "s.lj_force()",
+    "run": "s.lj_run(0.001, 1, energy_every=1); s.lj_run(0.001, 1, persistent=True)",
+    "g(r)": "s.gr_hist(np.full(1, 0.1, np.float32), 50)",
+    "sph": "s.setup_cells(1.0, periodic=False); s.sph_set_properties(one, one, 1.0); s.bin();"
+           "s.sph_density(); s.sph_acceleration(); s.sph_inspect_density()",
+    "wcsph": "s.setup_cells(1.0, periodic=False); s.sph_set_wcsph(0.5, 1.0, 10.0); s.bin();"
+             "s.sph_density(); s.sph_acceleration()",
+    "dem": "s.setup_cells(1.0, periodic=False); s.dem_set_properties(1e3, 0.5, 0.3, 0.1, 0.01, 0.4 * one);"
+           "s.rot_set_inertia(0.4 * one); s.bin(); s.dem_calc_force(1e-4); s.dem_calc_force(1e-4);"
+           "s.rot_step(1e-4)",
+    "thermostat": "s.gt_step(0.001); s.mv2()",
+}
+
+
+@pytest.mark.parametrize("calls", list(ALLOCATING))
+def test_failed_allocation(stub, calls):
+    """Whichever allocation fails, the same calls made again end with all the
+    device arrays of calls that never failed."""
+    stub(f"""
+        one = np.ones(500)
+        def calls(s):
+            {ALLOCATING[calls]}
+        def mine(f):
+            before = stub.stub_live(), stub.stub_live_bytes()
+            f()
+            return stub.stub_live() - before[0], stub.stub_live_bytes() - before[1]
+        s = system()
+        stub.stub_reset()
+        want = mine(lambda: calls(s))
+        n = stub.stub_calls(b"hipMalloc")
+        assert n > 0
+        for k in range(1, n + 1):
+            s = system()
+            def both():
+                fail("hipMalloc", k)
+                assert raises(calls, s), k
+                calls(s)
+            assert mine(both) == want, (k, n)
+    """)
+
+
+DEM = """
+        one = np.ones(500)
+        s = system(500, 10.0)
+        s.setup_cells(1.0, periodic=False)
+        s.dem_set_properties(1e3, 0.5, 0.3, 0.1, 0.01, 0.4 * one)
+        s.rot_set_inertia(0.4 * one)
+        s.bin()
+        for _ in range(2):
+            s.dem_calc_force(1e-4)
+        s.dem_contacts()
+"""
+
+
+def test_contacts_whose_arrays_could_not_be_had(stub):
+    """A restored matrix too large for its arrays (512) and for the memory: neither it
+    nor the one before is there afterwards."""
+    stub(DEM + """
+        row = np.minimum(2 * np.arange(501), 998).astype(np.uint32)
+        fail("hipMalloc")
+        assert raises(s.dem_set_contacts, row, np.tile(np.arange(2, dtype=np.uint32), 499), np.zeros(998))
+        assert raises(s.dem_contacts)
+        s.dem_calc_force(1e-4)
+    """)
