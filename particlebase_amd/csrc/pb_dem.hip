@@ -699,6 +699,7 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
   // capacity from the previous matrix (ensure_csr adds a quarter)
   if ((rc = ensure_csr(s, b, s->cm_cur >= 0 ? s->cm_nnz[s->cm_cur] : 0))) return rc;
   G.cap = s->cm_cap[b];
+  s->cm_prev = false;                        // the other buffer is overwritten from here on
   // per-row counts go to the sort workspace's rank array (free once pb_bin
   // has produced perm / cstart), their exclusive scan to the new row array
   uint32_t *cnt = s->rank, *bad = s->d_counter + 8;

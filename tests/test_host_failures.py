@@ -130,6 +130,19 @@ DEM = """
 """
 
 
+@pytest.mark.parametrize("kernel", ["k_dem_count", "k_scan", "k_dem_rows"])
+def test_rewind_after_a_failed_contact_search(stub, kernel):
+    """A search that fails has overwritten the rows of the matrix before the last:
+    there is none to go back to."""
+    stub(DEM + f"""
+        fail("{kernel}")
+        assert raises(s.dem_calc_force, 1e-4)
+        s.dem_rewind()
+        assert raises(s.dem_contacts)
+        s.dem_calc_force(1e-4)
+    """)
+
+
 def test_contacts_whose_arrays_could_not_be_had(stub):
     """A restored matrix too large for its arrays (512) and for the memory: neither it
     nor the one before is there afterwards."""
