@@ -1014,6 +1014,7 @@ extern "C" int pb_lj_force_nlist(pb_sys *s, double *pe, double *virial) {
   if (s->md_inv_order != s->order_gen) {
     hipLaunchKernelGGL(k_inverse_perm, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->orig,
                        s->npad, s->md_inv);
+    PB_LAUNCH_CHECK(s->ctx, "k_inverse_perm");
     s->md_inv_order = s->order_gen;
   }
   PairArgs A = pair_args(s);

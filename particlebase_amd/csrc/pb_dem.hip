@@ -673,6 +673,7 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
   if (s->dem_inv_order != s->order_gen) {
     hipLaunchKernelGGL(k_dem_inv, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->orig, s->npad,
                        s->dem_inv);
+    PB_LAUNCH_CHECK(s->ctx, "k_dem_inv");
     s->dem_inv_order = s->order_gen;
   }
   DemView V;

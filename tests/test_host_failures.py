@@ -153,3 +153,23 @@ def test_contacts_whose_arrays_could_not_be_had(stub):
         assert raises(s.dem_contacts)
         s.dem_calc_force(1e-4)
     """)
+
+
+@pytest.mark.parametrize("kernel,call", [("k_inverse_perm", "s.lj_force_nlist()"),
+                                         ("k_dem_inv", "s.dem_calc_force(1e-4)")])
+def test_inverse_order_that_was_not_made(stub, kernel, call):
+    stub(f"""
+        one = np.ones(500)
+        s = system(500, 10.0, 2.5)
+        if "{kernel}" == "k_dem_inv":
+            s.dem_set_properties(1e3, 0.5, 0.3, 0.1, 0.01, 0.4 * one)
+            s.rot_set_inertia(0.4 * one)
+        s.bin()
+        if "{kernel}" == "k_inverse_perm":
+            s.nlist_build(6.25)
+        stub.stub_reset()
+        fail("{kernel}")
+        assert raises(lambda: {call})
+        {call}
+        assert stub.stub_launches(b"{kernel}") == 1
+    """)
