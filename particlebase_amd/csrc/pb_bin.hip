@@ -932,7 +932,6 @@ extern "C" int pb_nlist_build(pb_sys *s, float rmax2t, uint32_t *nnz_out) {
   const uint32_t n = s->n;
   int rc2;
   if (!s->md_row && (rc2 = pb_alloc(s->ctx, &s->md_row, (size_t)n + 1))) return rc2;
-  if ((rc2 = pb_results(s->ctx))) return rc2;
   NlistArgs A;
   if ((rc2 = nlist_args(s, rmax2t, &A))) return rc2;
   s->md_valid = false;                        // until the rows are whole

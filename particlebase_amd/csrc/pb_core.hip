@@ -45,7 +45,8 @@ extern "C" int pb_ctx_create(int device, pb_ctx **out) {
     delete c;
     return PB_ERR_HIP;
   }
-  if (pb_gr_scratch_init(c) != PB_OK) {
+  if (pb_gr_scratch_init(c) != PB_OK || pb_io_create(c) != PB_OK) {
+    pb_io_release(c);
     (void)hipStreamDestroy(c->stream);
     delete c;
     return PB_ERR_HIP;
@@ -559,7 +560,6 @@ int pb_reduce_waves(pb_sys *s, int K, double *out) {
 // 10 us of host time and a 3 us kernel).
 int pb_reduce_to_host(pb_sys *s, int K, const double **host) {
   if (8 * (size_t)s->nrep <= PB_RES_DOUBLES) {
-    if (int rc = pb_results(s->ctx)) return rc;
     if (int rc = pb_reduce_waves(s, K, s->ctx->res_dev)) return rc;
     PB_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
     *host = s->ctx->res;
@@ -693,7 +693,6 @@ extern "C" int pb_inspect_velocity(pb_sys *s, double vlim, double lim_u, double 
   // truncated before the division.
   const double vl = (double)(uint32_t)(vlim > 0 ? vlim : 0);
   if (vl <= 0) return pb_fail(s->ctx, PB_ERR_ARG, "pb_inspect_velocity: vlim truncates to 0");
-  if (int rc = pb_results(s->ctx)) return rc;
   const uint32_t blocks = std::min(pb_blocks(s->npad, 256), INSPECT_BLOCKS);
   hipLaunchKernelGGL(k_inspect, dim3(blocks), dim3(256), 0, s->ctx->stream, s->v, s->orig, s->npad, vl,
                      s->partials);

@@ -663,7 +663,6 @@ extern "C" int pb_dem_calc_force(pb_sys *s, double dt, int autotune, uint32_t *n
   hipStream_t st = s->ctx->stream;
   const uint32_t n = s->n;
   int rc;
-  if ((rc = pb_results(s->ctx))) return rc;
   if (!s->dem_rs) {
     if ((rc = pb_alloc(s->ctx, &s->dem_inv, (size_t)n + 1)) ||
         (rc = pb_alloc(s->ctx, &s->dem_rowbuf, (size_t)s->npad * DEM_ROWBUF)) ||

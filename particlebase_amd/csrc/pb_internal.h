@@ -48,13 +48,13 @@ struct LJTable {
 struct pb_ctx {
   int device = 0;
   hipStream_t stream = nullptr;
-  // pinned staging ring of the host boundary (pb_io.hip; 2 MiB, allocated on
-  // first use, released with the context), its device address and an event
-  // per slot
+  // pinned staging ring of the host boundary (pb_io.hip; 2 MiB, made and
+  // released with the context, so that no later call allocates it), its device
+  // address and an event per slot
   uint8_t *io_stage = nullptr, *io_dev = nullptr;
   hipEvent_t io_ev[2] = {};
   // small results that kernels write to the host themselves: PB_RES_DOUBLES
-  // doubles of pinned memory and their device address (pb_results); read
+  // doubles of pinned memory and their device address; read
   // after the stream's synchronisation that every such call ends with
   double *res = nullptr, *res_dev = nullptr;
   // device address of pb_bin.hip's static g(r) scratch array on this
@@ -296,8 +296,8 @@ int pb_io_upload(pb_ctx *ctx, void *dev, const void *host, size_t bytes);
 int pb_io_download(pb_ctx *ctx, void *host, const void *dev, size_t bytes);
 int pb_io_buffer(pb_sys *sys);
 int pb_io_scatter(pb_sys *sys, const double *host, double *dst, bool square);
-// the context's small-result memory, allocated on first use
-int pb_results(pb_ctx *ctx);
+// the context's ring, its events and the small-result memory
+int pb_io_create(pb_ctx *ctx);
 void pb_io_release(pb_ctx *ctx);
 // rotation / radius state, allocated on first use
 int pb_ensure_rotation(pb_sys *sys);

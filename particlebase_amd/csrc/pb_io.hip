@@ -27,25 +27,17 @@
 #define IO_DIRECT ((size_t)256 << 10)
 
 // ------------------------------------------------------------ staging ring
-static int ensure_stage(pb_ctx *ctx) {
-  if (ctx->io_dev) return PB_OK;
-  if (!ctx->io_stage)
-    PB_HIP(ctx, hipHostMalloc((void **)&ctx->io_stage, 2 * IO_CHUNK, hipHostMallocMapped));
-  for (hipEvent_t &e : ctx->io_ev)
-    if (!e) PB_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
-  void *d = nullptr;
-  PB_HIP(ctx, hipHostGetDevicePointer(&d, ctx->io_stage, 0));
-  ctx->io_dev = (uint8_t *)d;
-  return PB_OK;
-}
-
-int pb_results(pb_ctx *ctx) {
-  if (ctx->res_dev) return PB_OK;
-  if (!ctx->res)
-    PB_HIP(ctx, hipHostMalloc((void **)&ctx->res, sizeof(double) * PB_RES_DOUBLES, hipHostMallocMapped));
-  void *d = nullptr;
-  PB_HIP(ctx, hipHostGetDevicePointer(&d, ctx->res, 0));
-  ctx->res_dev = (double *)d;
+int pb_io_create(pb_ctx *ctx) {
+  auto pinned = [&](void **host, void **dev, size_t bytes) -> int {
+    PB_HIP(ctx, hipHostMalloc(host, bytes, hipHostMallocMapped));
+    PB_HIP(ctx, hipHostGetDevicePointer(dev, *host, 0));
+    return PB_OK;
+  };
+  int rc;
+  if ((rc = pinned((void **)&ctx->io_stage, (void **)&ctx->io_dev, 2 * IO_CHUNK)) ||
+      (rc = pinned((void **)&ctx->res, (void **)&ctx->res_dev, sizeof(double) * PB_RES_DOUBLES)))
+    return rc;
+  for (hipEvent_t &e : ctx->io_ev) PB_HIP(ctx, hipEventCreateWithFlags(&e, hipEventDisableTiming));
   return PB_OK;
 }
 
@@ -62,7 +54,6 @@ void pb_io_release(pb_ctx *ctx) {
 
 // Device to host.  Every DMA that wrote the ring has completed on return.
 int pb_io_download(pb_ctx *ctx, void *host, const void *dev, size_t bytes) {
-  if (int rc = ensure_stage(ctx)) return rc;
   hipStream_t st = ctx->stream;
   const size_t nchunk = (bytes + IO_CHUNK - 1) / IO_CHUNK;
   for (size_t c = 0; c <= nchunk; ++c) {
@@ -85,7 +76,6 @@ int pb_io_download(pb_ctx *ctx, void *host, const void *dev, size_t bytes) {
 // slot's last event tells when the host may write it again (an event that was
 // never recorded, or one of a finished download, does not wait).
 int pb_io_upload(pb_ctx *ctx, void *dev, const void *host, size_t bytes) {
-  if (int rc = ensure_stage(ctx)) return rc;
   hipStream_t st = ctx->stream;
   const size_t nchunk = (bytes + IO_CHUNK - 1) / IO_CHUNK;
   for (size_t c = 0; c < nchunk; ++c) {
@@ -202,7 +192,6 @@ template <typename F>
 static int download_packed(pb_sys *s, void *host, size_t bytes, F &&pack) {
   pb_ctx *ctx = s->ctx;
   if (bytes <= IO_DIRECT) {
-    if (int rc = ensure_stage(ctx)) return rc;
     pack((void *)ctx->io_dev);
     PB_LAUNCH_CHECK(ctx, "pb_sys_get");
     PB_HIP(ctx, hipStreamSynchronize(ctx->stream));

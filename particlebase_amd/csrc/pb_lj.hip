@@ -1759,7 +1759,6 @@ static int check_lj_ready(pb_sys *s) {
 
 // the run's counters, waited for (through the context's pinned results)
 static int read_counters(pb_sys *s, uint32_t *c) {
-  if (int rc = pb_results(s->ctx)) return rc;
   PB_HIP(s->ctx, hipMemcpyAsync(s->ctx->res, s->d_counter, 16 * 4, hipMemcpyDeviceToHost,
                                 s->ctx->stream));
   PB_HIP(s->ctx, hipStreamSynchronize(s->ctx->stream));
@@ -1817,7 +1816,6 @@ extern "C" int pb_lj_force(pb_sys *s, int precision, double *pe, double *virial)
   const uint32_t lanes = force_lanes(s);
   if (int e = setup_list_cells(s, rc, std::vector<double>(s->nrep, rc * 1e-12), lanes)) return e;
   if (int e = ensure_sort_buffers(s)) return e;
-  if (int e = pb_results(s->ctx)) return e;
   if (int e = sort_cells(s, true, true)) return e;
   StepArgs A = make_args(s, 0.0);
   A.rin = s->r;

@@ -173,3 +173,28 @@ def test_inverse_order_that_was_not_made(stub, kernel, call):
         {call}
         assert stub.stub_launches(b"{kernel}") == 1
     """)
+
+
+def test_gr_noalloc_takes_nothing(stub):
+    """pb_gr_hist_noalloc as the first call that moves data on its context: no device
+    or pinned memory and no events are taken."""
+    stub("""
+        s = pb.System(pb.Context(0), [300])
+        s.set_cell([0, 10.0] * 3)
+        stub.stub_reset()
+        step, hist = np.full(1, 0.1, np.float32), np.zeros(50, np.uint64)
+        rc = s.lib.pb_gr_hist_noalloc(s.h, step.ctypes.data_as(C.POINTER(C.c_float)), 50,
+                                      hist.ctypes.data_as(C.POINTER(C.c_uint64)))
+        assert rc == pb.PB_OK
+        assert [stub.stub_calls(x) for x in (b"hipMalloc", b"hipHostMalloc", b"hipEventCreate")] == [0, 0, 0]
+    """)
+
+
+@pytest.mark.parametrize("call", ["hipHostMalloc", "hipEventCreate"])
+def test_context_that_could_not_be_made(stub, call):
+    stub(f"""
+        for k in (1, 2):
+            fail("{call}", k)
+            assert raises(pb.Context, 0), k
+        system().get("r")
+    """)
