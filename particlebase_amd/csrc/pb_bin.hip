@@ -623,6 +623,7 @@ struct NlistArgs {
   float cx, cy, cz, rmax2t;
   int periodic;
   uint32_t cap;                // capacity of the column array
+  uint32_t k0;                 // first sorted position of the launch
 };
 
 __global__ void k_md_gather(const double4 *r, const uint32_t *perm, const uint32_t *pid,
@@ -646,13 +647,16 @@ __global__ void k_md_gather(const double4 *r, const uint32_t *perm, const uint32
 // row are written as found and sorted in place by one lane.
 // 32,000 particles of a liquid (about 80 a row): 316 + 1079 us a build with a
 // thread a row and an insertion sort in global memory, 48 + 69 us now.
+// A launch takes NL_LAUNCH rows: its work items must fit in 32 bits, and a million
+// wavefronts leave no tail worth a longer launch.
 #define NL_CAP 512u
+#define NL_LAUNCH (1u << 20)
 template <bool FILL>
 __global__ void __launch_bounds__(256) k_nlist(NlistArgs A, uint32_t *rowcnt, const uint32_t *rowptr,
                                                uint32_t *col) {
   __shared__ __align__(16) uint32_t rows[FILL ? 4 : 1][FILL ? NL_CAP : 1];
   const uint32_t lane = pb_lane(), wave = threadIdx.x / 64;
-  const uint32_t k = __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + wave);
+  const uint32_t k = A.k0 + __builtin_amdgcn_readfirstlane(blockIdx.x * 4u + wave);
   if (k >= A.nreal) return;
   const float4 pi = A.pos[k];
   const uint32_t oi = __float_as_uint(pi.w), c = A.bid[k];
@@ -765,6 +769,7 @@ struct PairArgs {
   const uint32_t *rowptr, *col;     // list path
   const uint32_t *perm, *cellid, *start;   // cell path
   uint32_t npad;
+  uint32_t block0;                  // list path: first 64 slots of the launch
   RefGrid g;
   double L[3];
   int periodic;
@@ -792,7 +797,8 @@ __global__ void __launch_bounds__(64 * NF_LANES) k_lj_force_nlist(PairArgs A) {
     tab[3][t] = A.lj->shift[t];
   }
   __syncthreads();
-  const uint32_t si = blockIdx.x * 64u + threadIdx.x / NF_LANES, sub = threadIdx.x % NF_LANES;
+  const uint32_t block = A.block0 + blockIdx.x;
+  const uint32_t si = block * 64u + threadIdx.x / NF_LANES, sub = threadIdx.x % NF_LANES;
   double pe = 0.0, vir = 0.0;
   const uint32_t row = si < A.npad ? A.orig[si] : PB_NONE;
   if (row != PB_NONE) {
@@ -836,7 +842,7 @@ __global__ void __launch_bounds__(64 * NF_LANES) k_lj_force_nlist(PairArgs A) {
   if (threadIdx.x < 2) {
     double t = 0.0;
     for (uint32_t w = 0; w < NF_LANES; ++w) t += sums[threadIdx.x][w];
-    A.partials[4 * (size_t)blockIdx.x + threadIdx.x] = t;
+    A.partials[4 * (size_t)block + threadIdx.x] = t;
   }
 }
 
@@ -902,6 +908,16 @@ static int nlist_args(pb_sys *s, float rmax2t, NlistArgs *out) {
   return PB_OK;
 }
 
+// all rows: their lengths to md_cnt (FILL = false), or their columns to md_col
+template <bool FILL>
+static int nlist_rows(pb_sys *s, NlistArgs A) {
+  for (A.k0 = 0; A.k0 < A.nreal; A.k0 += NL_LAUNCH)
+    hipLaunchKernelGGL(k_nlist<FILL>, dim3(pb_blocks(std::min(A.nreal - A.k0, NL_LAUNCH), 4)), dim3(256),
+                       0, s->ctx->stream, A, s->md_cnt, s->md_row, s->md_col);
+  PB_LAUNCH_CHECK(s->ctx, FILL ? "k_nlist (rows)" : "k_nlist (counts)");
+  return PB_OK;
+}
+
 // calcCoordMD_F4 counts (kernelinline.hh:387-399) over the 27 cells of
 // calcF_IJpairWithBlock_F4 (kerneltemplate.hh:244-293): the rows' lengths
 extern "C" int pb_coord_counts(pb_sys *s, float rmax2t, uint32_t *counts) {
@@ -915,9 +931,7 @@ extern "C" int pb_coord_counts(pb_sys *s, float rmax2t, uint32_t *counts) {
   if (int e = pb_bin(s)) return e;
   NlistArgs A;
   if (int e = nlist_args(s, rmax2t, &A)) return e;
-  hipLaunchKernelGGL(k_nlist<false>, dim3(pb_blocks(s->n, 4)), dim3(256), 0, s->ctx->stream, A,
-                     s->md_cnt, (const uint32_t *)nullptr, (uint32_t *)nullptr);
-  PB_LAUNCH_CHECK(s->ctx, "k_nlist (counts)");
+  if (int e = nlist_rows<false>(s, A)) return e;
   return pb_io_download(s->ctx, counts, s->md_cnt, 4 * (size_t)s->n);
 }
 
@@ -935,19 +949,13 @@ extern "C" int pb_nlist_build(pb_sys *s, float rmax2t, uint32_t *nnz_out) {
   NlistArgs A;
   if ((rc2 = nlist_args(s, rmax2t, &A))) return rc2;
   s->md_valid = false;                        // until the rows are whole
-  hipLaunchKernelGGL(k_nlist<false>, dim3(pb_blocks(n, 4)), dim3(256), 0, st, A, s->md_cnt,
-                     (const uint32_t *)nullptr, (uint32_t *)nullptr);
-  PB_LAUNCH_CHECK(s->ctx, "k_nlist (counts)");
+  if ((rc2 = nlist_rows<false>(s, A))) return rc2;
   if ((rc2 = pb_exclusive_scan(s, s->md_cnt, s->md_row, n))) return rc2;
   // the rows are filled before the host knows their sum, up to the capacity
   // of the last list; a list that outgrew it is filled again
   auto fill = [&]() -> int {
     A.cap = s->md_cap;
-    if (!A.cap) return PB_OK;
-    hipLaunchKernelGGL(k_nlist<true>, dim3(pb_blocks(n, 4)), dim3(256), 0, st, A, s->md_cnt, s->md_row,
-                       s->md_col);
-    PB_LAUNCH_CHECK(s->ctx, "k_nlist (rows)");
-    return PB_OK;
+    return A.cap ? nlist_rows<true>(s, A) : PB_OK;
   };
   if ((rc2 = fill())) return rc2;
   PB_HIP(s->ctx, hipMemcpyAsync(s->ctx->res, s->md_row + n, 4, hipMemcpyDeviceToHost, st));
@@ -1021,7 +1029,9 @@ extern "C" int pb_lj_force_nlist(pb_sys *s, double *pe, double *virial) {
   A.rowptr = s->md_row;
   A.col = s->md_col;
   A.periodic = 1;       // MD boxes are periodic (MDpairForce folds every pair)
-  hipLaunchKernelGGL(k_lj_force_nlist, dim3(s->nwave), dim3(64 * NF_LANES), 0, st, A);
+  for (A.block0 = 0; A.block0 < s->nwave; A.block0 += NL_LAUNCH / 64u)
+    hipLaunchKernelGGL(k_lj_force_nlist, dim3(std::min(s->nwave - A.block0, NL_LAUNCH / 64u)),
+                       dim3(64 * NF_LANES), 0, st, A);
   PB_LAUNCH_CHECK(s->ctx, "k_lj_force_nlist");
   if (pe || virial) {
     const double *h = nullptr;

@@ -198,3 +198,21 @@ def test_context_that_could_not_be_made(stub, call):
             assert raises(pb.Context, 0), k
         system().get("r")
     """)
+
+
+def test_list_of_the_largest_systems(stub):
+    """Rows take a wavefront each: at 2^26 particles and more the work items of one
+    launch would no longer fit in 32 bits."""
+    stub("""
+        n = (1 << 26) + 1
+        s = pb.System(pb.Context(0), [n])
+        s.set_cell([0, 10.0] * 3)
+        s.lj_set_params([1.0, 1.0], 1)
+        s.lj_set_cutoff(6.25)
+        s.setup_cells(2.5)
+        s.bin()
+        s.coord_counts(6.25)
+        s.nlist_build(6.25)
+        s.lj_force_nlist()
+        assert stub.stub_most_items() < 2 * n      # of all launches, whatever the lanes a row
+    """)
