@@ -541,15 +541,16 @@ __global__ void __launch_bounds__(256) k_inspect_final(const double *partials, u
 }
 
 // ============================================================ reductions
-__global__ void __launch_bounds__(1024) k_reduce_waves(const double *partials, int K,
-                                                      const RepInfo *reps, uint32_t nrep,
-                                                      double *out) {
+template <int K>
+__global__ void __launch_bounds__(1024) k_reduce_waves(const double *partials, const RepInfo *reps,
+                                                      uint32_t nrep, double *out) {
   __shared__ double sm[4 * 256];
-  pb_block_reduce_reps(partials, K, reps, nrep, out, false, sm);
+  pb_block_reduce_reps<K>(partials, reps, nrep, out, false, sm);
 }
 
 int pb_reduce_waves(pb_sys *s, int K, double *out) {
-  hipLaunchKernelGGL(k_reduce_waves, dim3(1), dim3(s->nrep >= PB_REDUCE_WAVES ? 1024 : 256), 0, s->ctx->stream, s->partials, K,
+  hipLaunchKernelGGL(K == 1 ? k_reduce_waves<1> : k_reduce_waves<2>, dim3(1),
+                     dim3(s->nrep >= PB_REDUCE_WAVES ? 1024 : 256), 0, s->ctx->stream, s->partials,
                      s->d_reps, s->nrep, out);
   PB_LAUNCH_CHECK(s->ctx, "k_reduce_waves");
   return PB_OK;

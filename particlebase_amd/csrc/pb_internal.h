@@ -283,7 +283,7 @@ int pb_counting_sort(pb_sys *sys, uint32_t ncell, const uint32_t *key, PbCellOrd
 // sys->perm (sorted position -> storage slot, by cell and key) and
 // calcBlockID's outputs of the reference cell grid
 int pb_cell_order(pb_sys *sys, const PbCellOrder &O, uint32_t ncell);
-// per-replica reduction of K per-wave partial components into out[rep*8+c]
+// per-replica reduction of K = 1 or 2 per-wave partial components into out[rep*8+c]
 // (device memory, or the context's small results)
 int pb_reduce_waves(pb_sys *sys, int K, double *out);
 // the same, waited for, into host[rep*8+c]
@@ -401,73 +401,99 @@ __device__ __forceinline__ double pb_load_relaxed(const double *p) {
 // replicas from which a reduction takes a wavefront for each (and callers a
 // workgroup of 1024)
 constexpr uint32_t PB_REDUCE_WAVES = 4;
+// The order of a replica's sum is the same in every form that takes it, so its
+// bits don't depend on the other replicas: partial w goes to running sum w mod
+// 256, sums l, l + 64, l + 128 and l + 192 are added in pairs to lane l's, and the
+// lanes' by pb_wave_sum.
+constexpr uint32_t PB_REDUCE_SUMS = 256;
+
+// a wavefront's part of it: Q replicas (first partial w0, number nw) at once, the
+// sums of their K components in every lane
+template <int K, uint32_t Q>
+__device__ __forceinline__ void pb_wave_reduce(const double *partials, const uint32_t (&w0)[Q],
+                                               const uint32_t (&nw)[Q], double (&out)[Q][K]) {
+  constexpr uint32_t J = PB_REDUCE_SUMS / PB_WAVE;
+  uint32_t most = 0;
+#pragma unroll
+  for (uint32_t k = 0; k < Q; ++k) most = max(most, nw[k]);
+  double acc[J][Q][K] = {};
+  for (uint32_t w = pb_lane(); w < most; w += PB_REDUCE_SUMS)
+#pragma unroll
+    for (uint32_t j = 0; j < J; ++j)
+#pragma unroll
+      for (uint32_t k = 0; k < Q; ++k)
+        if (w + j * PB_WAVE < nw[k])
+#pragma unroll
+          for (int c = 0; c < K; ++c)
+            acc[j][k][c] += partials[4 * (size_t)(w0[k] + w + j * PB_WAVE) + c];
+#pragma unroll
+  for (uint32_t k = 0; k < Q; ++k)
+#pragma unroll
+    for (int c = 0; c < K; ++c)
+      out[k][c] = pb_wave_sum((acc[0][k][c] + acc[1][k][c]) + (acc[2][k][c] + acc[3][k][c]));
+}
+
 // sum of K per-wave partial components for every replica, executed by one
 // block (used by the last-block reductions and by k_reduce_waves).
-__device__ __forceinline__ void pb_block_reduce_reps(const double *partials, int K, const RepInfo *reps,
+template <int K>
+__device__ __forceinline__ void pb_block_reduce_reps(const double *partials, const RepInfo *reps,
                                      uint32_t nrep, double *out, bool by_segment,
                                      double *scratch) {
-  // Deterministic: every replica's partials (one per wave, or one per
-  // pair-kernel segment when by_segment) are summed in a fixed order that
-  // depends only on the launch shape of this block.  Callers that read
-  // partials written by other workgroups issue a device-scope fence first
-  // (it invalidates this CU's vector L1), so plain loads are coherent.
-  // scratch: 4 x 256 doubles of the caller's LDS
+  // Every replica's partials: one per wave, or one per pair-kernel segment when
+  // by_segment.  Callers that read partials written by other workgroups issue a
+  // device-scope fence first (it invalidates this CU's vector L1), so plain loads
+  // are coherent.  scratch: 4 x 256 doubles of the caller's LDS
   double (*sm)[256] = reinterpret_cast<double (*)[256]>(scratch);
-  const uint32_t t = threadIdx.x, bs = blockDim.x;
+  const uint32_t t = threadIdx.x, bs = blockDim.x, lane = pb_lane();
   const RepInfo &last = reps[nrep - 1u];
   const uint32_t parts = by_segment ? last.seg0 + last.nseg : last.wave0 + last.nwave;
   if (nrep >= PB_REDUCE_WAVES && parts <= 2048u * nrep) {
-    // a wavefront a replica, four of them in flight (a thread a replica was a
-    // chain of its partials: 256 replicas of 8000 particles 104 us, with 16
-    // wavefronts 22; one replica after the other by the whole workgroup, 15 of
-    // 500 to 4000 particles: mv2 37.5 us a call, now 19.4).  Few replicas of very
-    // many partials keep the whole workgroup on each (4 of 400,000 particles:
-    // 61 us a call against 62.5).
-    constexpr uint32_t Q = 4;
-    const uint32_t lane = pb_lane(), nwv = bs / PB_WAVE;
+    // a wavefront a replica, two of them and eight partials a lane in flight (mv2
+    // of 256 replicas of 8000 particles: a thread a replica, a chain of its
+    // partials, 125 us a call, this 45; 15 of 500 to 4000: one after the other by
+    // the whole workgroup 37.5, this 18.4).  Few replicas of very many partials
+    // keep the whole workgroup on each (4 of 400,000 particles: 55 us a call
+    // against 56).
+    constexpr uint32_t Q = 2;
+    const uint32_t nwv = bs / PB_WAVE;
     for (uint32_t q0 = t / PB_WAVE; q0 < nrep; q0 += nwv * Q) {
-      uint32_t w0[Q], nw[Q], most = 0;
-      double acc[Q][4] = {};
+      uint32_t w0[Q], nw[Q];
 #pragma unroll
       for (uint32_t k = 0; k < Q; ++k) {
         const RepInfo &R = reps[min(q0 + k * nwv, nrep - 1u)];
         w0[k] = by_segment ? R.seg0 : R.wave0;
         nw[k] = q0 + k * nwv < nrep ? (by_segment ? R.nseg : R.nwave) : 0u;
-        most = max(most, nw[k]);
       }
-      for (uint32_t w = lane; w < most; w += PB_WAVE)
-#pragma unroll
-        for (uint32_t k = 0; k < Q; ++k)
-          if (w < nw[k])
-            for (int c = 0; c < K; ++c) acc[k][c] += partials[4 * (size_t)(w0[k] + w) + c];
+      double x[Q][K];
+      pb_wave_reduce<K>(partials, w0, nw, x);
 #pragma unroll
       for (uint32_t k = 0; k < Q; ++k)
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          if (c < K) {
-            const double x = pb_wave_sum(acc[k][c]);
-            if (lane == 0 && q0 + k * nwv < nrep) out[8 * (q0 + k * nwv) + c] = x;
-          }
+        for (int c = 0; c < K; ++c)
+          if (lane == 0 && q0 + k * nwv < nrep) out[8 * (q0 + k * nwv) + c] = x[k][c];
     }
     return;
   }
-  // the first 256 threads reduce (any block size >= 256 may call this)
-  const uint32_t T = 256;
+  // the first 256 threads hold the running sums (any block size >= 256 may call
+  // this), a wavefront a component adds them
+  const uint32_t T = PB_REDUCE_SUMS;
   for (uint32_t q = 0; q < nrep; ++q) {
     const uint32_t w0 = by_segment ? reps[q].seg0 : reps[q].wave0;
     const uint32_t nw = by_segment ? reps[q].nseg : reps[q].nwave;
-    double acc[4] = {0, 0, 0, 0};
-    if (t < T)
+    double acc[K] = {};
+    if (t < T) {
       for (uint32_t w = t; w < nw; w += T)
-        for (int c = 0; c < K; ++c) acc[c] += partials[4 * (w0 + w) + c];
 #pragma unroll
-    for (int c = 0; c < 4; ++c)
-      if (t < T && c < K) {
-        const double x = pb_wave_sum(acc[c]);
-        if (t % PB_WAVE == 0) sm[c][t / PB_WAVE] = x;
-      }
+        for (int c = 0; c < K; ++c) acc[c] += partials[4 * (size_t)(w0 + w) + c];
+#pragma unroll
+      for (int c = 0; c < K; ++c) sm[c][t] = acc[c];
+    }
     __syncthreads();
-    if (t < (uint32_t)K) out[8 * q + t] = (sm[t][0] + sm[t][1]) + (sm[t][2] + sm[t][3]);
+    const uint32_t c = t / PB_WAVE;
+    if (c < (uint32_t)K) {
+      const double x = pb_wave_sum((sm[c][lane] + sm[c][lane + 64]) + (sm[c][lane + 128] + sm[c][lane + 192]));
+      if (lane == 0) out[8 * q + c] = x;
+    }
     __syncthreads();
   }
 }

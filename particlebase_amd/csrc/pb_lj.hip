@@ -1662,7 +1662,7 @@ __global__ void __launch_bounds__(1024) k_energy_reduce(const double *partials, 
                                                        uint32_t *counter, uint32_t *counts_out) {
   __shared__ double sm[4 * 256];
   const uint32_t rec = counter[CNT_REC];
-  pb_block_reduce_reps(partials, 3, reps, nrep, energy + (size_t)rec * 8 * nrep, true, sm);
+  pb_block_reduce_reps<3>(partials, reps, nrep, energy + (size_t)rec * 8 * nrep, true, sm);
   __syncthreads();
   if (threadIdx.x == 0) counter[CNT_REC] = rec + 1;
   if (counts_out && threadIdx.x < 16) counts_out[threadIdx.x] = counter[threadIdx.x];

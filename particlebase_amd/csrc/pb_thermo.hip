@@ -77,16 +77,15 @@ __global__ void __launch_bounds__(GT_BLOCK)
   }
 }
 
-// Sums of a replica's partials in every lane of a wavefront (fixed order)
+// Sums of a replica's partials in every lane of a wavefront
 struct GtSums {
   double x[3];
   __device__ __forceinline__ GtSums(const double *partials, const RepInfo &R) {
-    double a[3] = {0.0, 0.0, 0.0};
-    for (uint32_t w = pb_lane(); w < R.nwave; w += PB_WAVE)
+    const uint32_t w0[1] = {R.wave0}, nw[1] = {R.nwave};
+    double y[1][3];
+    pb_wave_reduce<3>(partials, w0, nw, y);
 #pragma unroll
-      for (int c = 0; c < 3; ++c) a[c] += partials[4 * (size_t)(R.wave0 + w) + c];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) x[c] = pb_wave_sum(a[c]);
+    for (int c = 0; c < 3; ++c) x[c] = y[0][c];
   }
 };
 
@@ -132,7 +131,7 @@ __global__ void __launch_bounds__(256)
     k_gt_solve1(const double *partials, const RepInfo *reps, uint32_t nrep, double dt,
                 double *out, double *gt) {
   __shared__ double sm[4 * 256];
-  pb_block_reduce_reps(partials, 3, reps, nrep, out, false, sm);
+  pb_block_reduce_reps<3>(partials, reps, nrep, out, false, sm);
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < nrep; q += blockDim.x) {
     const GtSolve1 S(out[8 * q], out[8 * q + 1], out[8 * q + 2], dt);
@@ -198,7 +197,7 @@ __global__ void __launch_bounds__(256)
     k_gt_solve2(const double *partials, const RepInfo *reps, uint32_t nrep, double tol,
                 double *out, double *gt, uint32_t *bad) {
   __shared__ double sm[4 * 256];
-  pb_block_reduce_reps(partials, 3, reps, nrep, out, false, sm);
+  pb_block_reduce_reps<3>(partials, reps, nrep, out, false, sm);
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < nrep; q += blockDim.x) {
     double *G = gt + 4 * q;
@@ -328,7 +327,7 @@ __global__ void __launch_bounds__(256)
     k_vstats(const double *partials, const RepInfo *reps, uint32_t nrep, double *out,
              double *stats, int pass) {
   __shared__ double sm[4 * 256];
-  pb_block_reduce_reps(partials, 3, reps, nrep, out, false, sm);
+  pb_block_reduce_reps<3>(partials, reps, nrep, out, false, sm);
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < nrep; q += blockDim.x) {
     const double inv = 1.0 / (double)reps[q].natoms;
@@ -359,7 +358,7 @@ __global__ void __launch_bounds__(GT_BLOCK)
 __global__ void __launch_bounds__(256)
     k_ct_solve(const double *partials, const RepInfo *reps, uint32_t nrep, double *out) {
   __shared__ double sm[4 * 256];
-  pb_block_reduce_reps(partials, 2, reps, nrep, out, false, sm);
+  pb_block_reduce_reps<2>(partials, reps, nrep, out, false, sm);
   __syncthreads();
   for (uint32_t q = threadIdx.x; q < nrep; q += blockDim.x) {
     const double fv = out[8 * q], mv2 = out[8 * q + 1];
