@@ -106,41 +106,45 @@ extern "C" int pb_setup_cells(pb_sys *s, float rmax, int periodic, int single_pa
   float cell[6];
   for (int i = 0; i < 6; ++i) cell[i] = (float)s->cells[i];
   float c[3];
+  uint32_t num[3];               // the system's grid only when all is known to be good
+  float len[6];
   for (int i = 0; i < 3; ++i) {
     c[i] = cell[i * 2 + 1] - cell[i * 2];
     if (periodic) {
-      s->blocknum[i] = f2u_sat(c[i] / rmax);
-      if (s->blocknum[i] == 0) return pb_fail(s->ctx, PB_ERR_CELLS, "pb_setup_cells: box smaller than rmax");
-      s->blocklen[i] = c[i] / (float)s->blocknum[i];
+      num[i] = f2u_sat(c[i] / rmax);
+      if (num[i] == 0) return pb_fail(s->ctx, PB_ERR_CELLS, "pb_setup_cells: box smaller than rmax");
+      len[i] = c[i] / (float)num[i];
     } else {
-      s->blocklen[i] = rmax;
-      s->blocknum[i] = f2u_sat(c[i] / rmax) + 1u;
+      len[i] = rmax;
+      num[i] = f2u_sat(c[i] / rmax) + 1u;
     }
-    if (s->blocknum[i] <= 2)
+    if (num[i] <= 2)
       return pb_fail(s->ctx, PB_ERR_CELLS, "pb_setup_cells: fewer than 3 cells along an axis");
-    s->blocklen[i + 3] = cell[i * 2];
+    len[i + 3] = cell[i * 2];
   }
   if (single_particle) {
     // cudaCutoffBlock.cu:115-138: shrink cells until the cell diagonal is
     // below the particle diameter (r0 = rmax*sqrt(3)/2)
     const double r0 = rmax * sqrt(3.0) / 2.0;
     const double R02 = (r0 * 2.0) * (r0 * 2.0);
-    while ((double)(s->blocklen[0] * s->blocklen[0] + s->blocklen[1] * s->blocklen[1] +
-                    s->blocklen[2] * s->blocklen[2]) > R02) {
-      if ((s->blocklen[0] > s->blocklen[1]) && (s->blocklen[0] > s->blocklen[2])) {
-        ++s->blocknum[0];
-        s->blocklen[0] = c[0] / s->blocknum[0];
-      } else if (s->blocklen[1] > s->blocklen[2]) {
-        ++s->blocknum[1];
-        s->blocklen[1] = c[1] / s->blocknum[1];
+    while ((double)(len[0] * len[0] + len[1] * len[1] + len[2] * len[2]) > R02) {
+      if ((len[0] > len[1]) && (len[0] > len[2])) {
+        ++num[0];
+        len[0] = c[0] / num[0];
+      } else if (len[1] > len[2]) {
+        ++num[1];
+        len[1] = c[1] / num[1];
       } else {
-        ++s->blocknum[2];
-        s->blocklen[2] = c[2] / s->blocknum[2];
+        ++num[2];
+        len[2] = c[2] / num[2];
       }
     }
   }
-  const uint64_t nc = (uint64_t)s->blocknum[0] * s->blocknum[1] * s->blocknum[2];
+  const uint64_t nc = (uint64_t)num[0] * num[1] * num[2];
   if (nc >= 0x7FFFFFFFull) return pb_fail(s->ctx, PB_ERR_CELLS, "pb_setup_cells: too many cells");
+  s->ref_cells = s->ref_binned = false;
+  std::memcpy(s->blocknum, num, sizeof(num));
+  std::memcpy(s->blocklen, len, sizeof(len));
   s->ref_ncell = (uint32_t)nc;
   s->ref_periodic = periodic ? 1 : 0;
   s->ref_single = single_particle ? 1 : 0;
@@ -150,7 +154,6 @@ extern "C" int pb_setup_cells(pb_sys *s, float rmax, int periodic, int single_pa
     return rc;
   if ((rc = pb_ensure_sort_ws(s, s->ref_ncell + 1))) return rc;
   s->ref_cells = true;
-  s->ref_binned = false;
   return PB_OK;
 }
 
@@ -183,6 +186,7 @@ extern "C" int pb_bin(pb_sys *s) {
   if (!s->ref_cells) return pb_fail(s->ctx, PB_ERR_STATE, "pb_bin: pb_setup_cells first");
   hipStream_t st = s->ctx->stream;
   const uint32_t nc = s->ref_ncell;
+  s->ref_binned = false;         // until the new order is whole
   if (int rc = pb_counts_begin(s)) return rc;
   hipLaunchKernelGGL(k_ref_bid, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->r, s->orig,
                      s->npad, ref_grid(s), nc, s->cellid, s->ccount, s->rank);

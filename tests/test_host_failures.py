@@ -216,3 +216,34 @@ def test_list_of_the_largest_systems(stub):
         s.lj_force_nlist()
         assert stub.stub_most_items() < 2 * n      # of all launches, whatever the lanes a row
     """)
+
+
+@pytest.mark.parametrize("rmax", [4.0, 1e-7])        # two cells along an axis; too many cells
+def test_refused_cells_leave_the_grid(stub, rmax):
+    stub(f"""
+        s = pb.System(pb.Context(0), [500])
+        s.set_cell([0, 30.0, 0, 10.0, 0, 10.0])
+        s.setup_cells(1.0)
+        s.bin()
+        before = s.cell_info()
+        assert raises(s.setup_cells, {rmax})
+        after = s.cell_info()
+        assert all(np.array_equal(a, b) for a, b in zip(before, after)), after
+        s.get_bins()
+    """)
+
+
+def test_cells_whose_arrays_could_not_be_had(stub):
+    stub("""
+        for k in range(1, 6):
+            s = system(500, 10.0, 2.0)
+            s.bin()
+            fail("hipMalloc", k)
+            assert raises(s.setup_cells, 1.0), k
+            stub.stub_fail(b"", C.c_long(0))
+            assert raises(s.bin) and raises(s.get_bins), k
+            s.setup_cells(1.0)
+            s.bin()
+            fail("k_scatter")
+            assert raises(s.bin) and raises(s.get_bins), k
+    """)
