@@ -229,11 +229,13 @@ static int upload_reps(pb_sys *s) {
 
 extern "C" int pb_sys_set_cell(pb_sys *s, const double *cells) {
   if (!s || !cells) return PB_ERR_ARG;
+  // nothing is written before all boxes are known to be good
+  for (size_t k = 0; k < 3 * (size_t)s->nrep; ++k)
+    if (!(cells[2 * k + 1] > cells[2 * k])) return pb_fail(s->ctx, PB_ERR_ARG, "pb_sys_set_cell: empty box");
   for (uint32_t q = 0; q < s->nrep; ++q) {
     RepInfo &R = s->reps[q];
     for (int a = 0; a < 3; ++a) {
       const double lo = cells[6 * q + 2 * a], hi = cells[6 * q + 2 * a + 1];
-      if (!(hi > lo)) return pb_fail(s->ctx, PB_ERR_ARG, "pb_sys_set_cell: empty box");
       R.lo[a] = lo;
       R.hi[a] = hi;
       R.L[a] = hi - lo;
