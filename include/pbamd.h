@@ -169,7 +169,11 @@ int pb_lj_set_params(pb_sys *sys, const double *sigma_eps, int ntypes);
 int pb_lj_set_cutoff(pb_sys *sys, double rc2, int shifted);
 /* cudaParticleMD::calcForce + a correct calcPotentialE
  * (cudaParticleMD.cu:24-122): F from the current positions; pe, virial
- * (FP64 per replica, may be NULL) = 1/2 sum phi, 1/2 sum f.r. */
+ * (FP64 per replica, may be NULL) = 1/2 sum phi, 1/2 sum f.r.
+ * The same system gives the same bits on every call.  The order in which a
+ * particle's pairs are added, and with it the last bits of its force, follows
+ * the number of lanes that share its pairs, which goes by the particles of all
+ * replicas together: a replica alone and in a batch agree to rounding. */
 int pb_lj_force(pb_sys *sys, int precision, double *pe, double *virial);
 /* calcCoordMD_F4 counts via makeNList step 1 (cudaParticleMD.cu:343-366,
  * kernelinline.hh:387-399): FP32-exact number of j != i with distance2p <
@@ -195,8 +199,10 @@ typedef struct {
                               step costs about 9 us of idle GPU before it */
   int      persistent;     /* 1: the step kernel runs as a persistent grid (two
                               workgroups per compute unit) draining the
-                              (replica x tile) segments from per-XCD work queues;
-                              0: one workgroup per segment */
+                              (replica x tile) segments from per-XCD work queues,
+                              one lane a particle; 0: one workgroup per segment,
+                              1 to 8 lanes a particle by the system's size.  The
+                              two agree to rounding */
 } pb_run_opts;
 
 /* Fused cudaParticleMD loop (the testMD1.cu:135-169 step: calcBlockID,

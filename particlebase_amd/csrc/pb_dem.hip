@@ -174,9 +174,9 @@ __device__ __forceinline__ void dem_contacts(const DemGrid &G, uint32_t k,
 // calcCoord_F4 (kernelinline.hh:371-382): contacts of movable particles
 // The same scan keeps the first DEM_ROWBUF contacts (original indices, in no
 // particular order) in the row buffer for the rows.
-// 200,000 dispersed spheres 15 us, a bed of 60,000 15 us (18 and 15 with FP64
-// candidates column by column); at most 128 registers, so that four wavefronts
-// fit a SIMD.
+// 200,000 dispersed spheres 14 us stored in lattice order and 16 in random order, a
+// bed of 60,000 14 us (FP64 candidates column by column: 18 for the first, 15 for
+// the bed); at most 128 registers, so that four wavefronts fit a SIMD.
 template <int W>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4)))
 k_dem_count(DemGrid G, uint32_t *cnt, uint32_t *bad) {
@@ -387,8 +387,9 @@ __device__ __forceinline__ void sort_registers(uint32_t (&a)[DEM_ROWBUF]) {
 // are added in a fixed order.  Code is kept short (rolled loops): a wavefront
 // passes most of it once, so its fetch counts.  Neighbouring workgroups share an
 // XCD's L2.  A bed of 60,000 spheres of 6 contacts: 19 us with two lanes, 21 with
-// one, 27 with four; 200,000 dispersed ones with almost none: 8.0 and 7.6;
-// fill, carry and force as kernels of their own took 31 and 16 us.
+// one, 27 with four; 200,000 dispersed ones with almost none: 8.0 with two, 7.5 with
+// one (9.3 stored in random order); fill, carry and force as kernels of their own
+// took 31 and 16 us.
 #define DEM_ROWS_BS 128
 template <int LAW, int W, uint32_t LN>
 __global__ void __launch_bounds__(DEM_ROWS_BS) k_dem_rows(DemGrid G, DemForceArgs A) {

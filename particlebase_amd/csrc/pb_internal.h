@@ -371,11 +371,6 @@ __device__ __forceinline__ void pb_wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
   __builtin_amdgcn_wave_barrier();
 }
-__device__ __forceinline__ double pb_wave_max(double x) {
-#pragma unroll
-  for (int o = 32; o > 0; o >>= 1) x = fmax(x, __shfl_xor(x, o, 64));
-  return x;
-}
 
 // XCD-aware logical block of a 1-D grid (MI355X dispatches workgroups
 // round-robin over its 8 XCDs, each with its own L2): within every 64
