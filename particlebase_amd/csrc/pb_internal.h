@@ -442,7 +442,7 @@ __device__ __forceinline__ void pb_block_reduce_reps(const double *partials, con
   const uint32_t t = threadIdx.x, bs = blockDim.x, lane = pb_lane();
   const RepInfo &last = reps[nrep - 1u];
   const uint32_t parts = by_segment ? last.seg0 + last.nseg : last.wave0 + last.nwave;
-  if (nrep >= PB_REDUCE_WAVES && parts <= 2048u * nrep) {
+  if (nrep >= PB_REDUCE_WAVES && parts / 2048u < nrep) {   // a product would wrap from 2^21 replicas
     // a wavefront a replica, two of them and eight partials a lane in flight (mv2
     // of 256 replicas of 8000 particles: a thread a replica, a chain of its
     // partials, 125 us a call, this 45; 15 of 500 to 4000: one after the other by
