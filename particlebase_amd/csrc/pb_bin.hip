@@ -186,14 +186,13 @@ extern "C" int pb_bin(pb_sys *s) {
   if (!s->ref_cells) return pb_fail(s->ctx, PB_ERR_STATE, "pb_bin: pb_setup_cells first");
   hipStream_t st = s->ctx->stream;
   const uint32_t nc = s->ref_ncell;
-  s->ref_binned = false;         // until the new order is whole
-  if (int rc = pb_counts_begin(s)) return rc;
+  int rc;
+  if ((rc = pb_ensure_sort_ws(s, nc + 1)) || (rc = pb_counts_begin(s))) return rc;
   hipLaunchKernelGGL(k_ref_bid, dim3(pb_blocks(s->npad, 256)), dim3(256), 0, st, s->r, s->orig,
                      s->npad, ref_grid(s), nc, s->cellid, s->ccount, s->rank);
   PB_LAUNCH_CHECK(s->ctx, "k_ref_bid");
   PbCellOrder O;
-  if (int rc = pb_counting_sort(s, nc + 1, s->orig, &O)) return rc;
-  if (int rc = pb_cell_order(s, O, nc)) return rc;
+  if ((rc = pb_counting_sort(s, nc + 1, s->orig, &O)) || (rc = pb_cell_order(s, O, nc))) return rc;
   s->ref_binned = true;
   return PB_OK;
 }

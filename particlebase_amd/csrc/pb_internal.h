@@ -275,7 +275,8 @@ struct PbCellOrder {
   const uint32_t *skey, *sslot, *scell;
 };
 // before a counting kernel: ccount is zero (a sort given up in between leaves
-// counts, and ranks on top of them lie past the arrays)
+// counts, and ranks on top of them lie past the arrays), and the order of the
+// reference cell grid no longer holds
 int pb_counts_begin(pb_sys *sys);
 // cellid[s] (PB_NONE never), the counts of every cell and the rank of s among
 // them given; cells start in sys->cstart

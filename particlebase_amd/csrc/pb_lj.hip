@@ -1607,7 +1607,6 @@ static int sort_cells(pb_sys *s, bool carry_a, bool clear_all) {
   ++s->order_gen;
   std::swap(s->type, s->type2);
   std::swap(s->move, s->move2);
-  s->ref_binned = false;
   return PB_OK;
 }
 

@@ -236,6 +236,7 @@ int pb_ensure_sort_ws(pb_sys *s, uint32_t ncell) {
   }
   if (s->ncell_cap < ncell) {
     s->ncell_cap = 0;
+    s->ref_binned = false;                   // the order's cell starts go
     if ((rc = pb_alloc(s->ctx, &s->ccount, (size_t)ncell + 1)) ||
         (rc = pb_alloc(s->ctx, &s->cstart, (size_t)ncell + 1)))
       return rc;
@@ -250,6 +251,7 @@ int pb_ensure_sort_ws(pb_sys *s, uint32_t ncell) {
 }
 
 int pb_counts_begin(pb_sys *s) {
+  s->ref_binned = false;                     // the arrays of the order before are written from here on
   if (s->counts_used) {
     hipLaunchKernelGGL(k_fill_u32, dim3(pb_blocks((size_t)s->ncell_cap + 1, 256)), dim3(256), 0,
                        s->ctx->stream, s->ccount, s->ncell_cap + 1, 0u);

@@ -247,3 +247,36 @@ def test_cells_whose_arrays_could_not_be_had(stub):
             fail("k_scatter")
             assert raises(s.bin) and raises(s.get_bins), k
     """)
+
+
+def test_cell_order_after_a_failed_force(stub):
+    """An LJ force that fails inside its own cell sort (here with more cells than the
+    grid's) has given up the order that pb_bin made: calls that need it are errors
+    until pb_bin ran again."""
+    stub("""
+        def fresh():
+            s = system(500, 31.0, 5.0)
+            s.lj_set_cutoff(1.0, shifted=True)
+            s.bin()
+            s.nlist_build(6.25)
+            return s
+        s = fresh()
+        stub.stub_reset()
+        s.lj_force()
+        n = stub.stub_calls(b"hipMalloc")
+        sort = [("hipMalloc", k) for k in range(1, n + 1)]
+        sort += [(k, 1) for k in ("k_list_cellid", "k_scan", "k_scatter", "k_reorder")]
+        lost = 0
+        for what, k in sort:
+            s = fresh()
+            fail(what, k)
+            assert raises(s.lj_force), (what, k)
+            stub.stub_fail(b"", C.c_long(0))
+            gone = raises(s.nlist_build, 6.25)
+            assert gone == raises(s.get_bins), (what, k)
+            lost += gone
+            assert gone or what == "hipMalloc"
+            s.bin()
+            s.nlist_build(6.25)
+        assert lost >= 6                          # two arrays of the cells, four kernels
+    """)
